@@ -140,6 +140,33 @@ hipError_t launch_read_rows(const void *layer_base, int elem_f16, const PoolGeom
                             uint32_t first_row, uint32_t rows, uint32_t ring, void *keys_out,
                             void *values_out, hipStream_t stream);
 
+// The same for a stretch of a snapshot's payload: runs of elements of one layer's and side's rows
+// ([row][kv_head][d], row 0 at position first_row) to out + out0, as f32 or (out_f16) as they are.
+constexpr int kMaxReadRuns = 64;
+struct ReadRun {
+    uint32_t layer;      // index within its group of planes
+    uint32_t side;
+    uint32_t first_row;
+    uint32_t ring;       // windowed layers: storage rows of the ring; 0 = a global layer
+    uint64_t elem0;
+    uint64_t count;
+    uint64_t out0;
+};
+struct ReadRuns {
+    uint32_t n;
+    uint32_t slot;
+    ReadRun run[kMaxReadRuns];
+};
+hipError_t launch_read_runs(const void *base, const void *base_w, int elem_f16, int out_f16, const PoolGeom &g,
+                            const PoolGeom &gw, const ReadRuns &b, void *out, hipStream_t stream);
+
+// ---- FNV-1a 64 on the device (fnv_kernels.hip) ------------------------------------------
+// *state (device memory) = the hash after `bytes` bytes at `data` (device memory, 16-byte aligned)
+// from *state. `bytes` is a multiple of kFnvRun; scratch holds fnv_scratch_bytes(bytes).
+constexpr uint32_t kFnvRun = 64;
+uint64_t fnv_scratch_bytes(uint64_t bytes);
+hipError_t launch_fnv(const void *data, uint64_t bytes, void *scratch, unsigned long long *state, hipStream_t stream);
+
 // ---- ring rows aside and back (checkpoints deeper than a ring's headroom) -----------------
 // Copies rows of windowed layers between their rings and a side buffer that holds, per entry,
 // [side][saved_rows][kv_head][d] elements at saved_off: row saved_row0 + r of the buffer is
@@ -165,8 +192,6 @@ hipError_t launch_ring_rows(void *pool_base_w, int elem_f16, const PoolGeom &gw,
                             const RingRowsBatch &b, void *saved, bool to_ring, hipStream_t stream);
 
 hipError_t launch_convert_f16(const float *src, uint16_t *dst, uint64_t count, hipStream_t stream);
-// f16 bits -> f32, exact (the widening a snapshot capture of an f16 pool needs).
-hipError_t launch_widen_f16(const uint16_t *src, float *dst, uint64_t count, hipStream_t stream);
 // Host-pointer calls: `bytes` (rounded up to 16) from pinned host memory into device memory by
 // a kernel, and a word in pinned host memory set to `value` once everything before it on the
 // stream has finished.

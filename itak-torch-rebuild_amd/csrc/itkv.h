@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <functional>
 #include <string>
 #include <thread>
 #include <vector>
@@ -116,8 +117,11 @@ bool itkv_validate(const ItkvHeader &h, const ItkvLayer *layers, uint64_t blocks
 // KvSnapshot::from_bytes (snapshot.rs:405-509): strict; fills offsets instead of copying rows.
 // `known_sum`, when given, is the checksum of bytes[0, len-8) the caller already computed (while
 // the bytes were still arriving, say); the decoder then compares instead of walking them again.
+// `sum_of`, when given, computes it when the decoder gets there: from the decoded header, the
+// layers with their offsets and the payload's own offset (the rows run from there to the trailer).
+using ItkvSum = std::function<uint64_t(const ItkvHeader &, uint64_t payload)>;
 bool itkv_decode(const uint8_t *bytes, uint64_t len, ItkvHeader &h, std::vector<ItkvLayer> &layers,
-                 ItkvError &err, const uint64_t *known_sum = nullptr);
+                 ItkvError &err, const uint64_t *known_sum = nullptr, const ItkvSum &sum_of = nullptr);
 
 // Bytes of everything before the row payload, and of the whole encoding (payload and the
 // trailing checksum included), for a header whose layers carry `rows` rows each.
@@ -131,9 +135,12 @@ void itkv_write_header(uint8_t *out, const ItkvHeader &h, const char *fingerprin
 // `layers` are the decoder's outputs for `bytes`. The geometry and fingerprint checks of
 // restore_checked (snapshot.rs:351-371) run; the bytes are not walked a second time. For the
 // prefix store, which verifies an entry in its own private buffer and installs from there.
+// `rows`, when given, is device memory that holds the payload (what lies in `bytes` from the first
+// layer's keys on); the rows are then gathered from there.
 int32_t restore_decoded_itkv(itak_pool *pool, uint32_t slot, const uint8_t *bytes,
                              const ItkvHeader &h, const std::vector<ItkvLayer> &layers,
-                             const char *expected_fingerprint, uint64_t expected_fingerprint_len);
+                             const char *expected_fingerprint, uint64_t expected_fingerprint_len,
+                             const uint8_t *rows = nullptr);
 
 // itak_kv_capture_itkv / itak_kv_capture_itkv_f16 with the 8 trailer bytes left zero: for a
 // caller that runs the byte-serial checksum itself while it does something else with the bytes

@@ -245,7 +245,7 @@ bool itkv_validate(const ItkvHeader &h, const ItkvLayer *layers, uint64_t blocks
 }
 
 bool itkv_decode(const uint8_t *bytes, uint64_t len, ItkvHeader &h, std::vector<ItkvLayer> &layers,
-                 ItkvError &err, const uint64_t *known_sum) {
+                 ItkvError &err, const uint64_t *known_sum, const ItkvSum &sum_of) {
     Reader r{bytes, len, 0, err};
     const uint8_t *magic = r.take(4);
     if (!magic) return false;
@@ -307,6 +307,7 @@ bool itkv_decode(const uint8_t *bytes, uint64_t len, ItkvHeader &h, std::vector<
         return inconsistent(err, "KV row width overflows: %llu heads of dim %llu have no usize product",
                             ULL(h.num_kv_heads), ULL(h.head_dim));
     std::vector<uint64_t> floats(layer_count);
+    const uint64_t payload = r.at;
     for (uint32_t i = 0; i < layer_count; ++i) {
         uint64_t bytes_per_side = 0;
         if (!checked_mul(layers[i].rows, row, &floats[i]))
@@ -322,7 +323,9 @@ bool itkv_decode(const uint8_t *bytes, uint64_t len, ItkvHeader &h, std::vector<
     if (!r.u64(&stored)) return false;
     if (r.remaining() != 0)
         return inconsistent(err, "%llu trailing bytes after the checksum", ULL(r.remaining()));
-    const uint64_t computed = known_sum ? *known_sum : itkv_trailer(h.version, bytes, len - 8);
+    const uint64_t computed = known_sum ? *known_sum
+                              : sum_of  ? sum_of(h, payload)
+                                        : itkv_trailer(h.version, bytes, len - 8);
     if (stored != computed)
         return refuse(err, ITAK_KV_CHECKSUM_MISMATCH, stored, computed,
                       "snapshot checksum mismatch: stored 0x%016llx, computed 0x%016llx",

@@ -5,6 +5,8 @@
 // and value planes of f16 pools in 32-row transposed blocks (see PoolGeom).
 #include "internal.h"
 
+#include <algorithm>
+
 namespace itak {
 
 __device__ __forceinline__ void store4(float *dst, const float4 &v) {
@@ -350,6 +352,76 @@ __global__ __launch_bounds__(256) void kv_read_rows(const T *__restrict__ layer_
     }
 }
 
+// Runs of a snapshot's payload: elements [elem0, elem0 + count) of one layer's and side's rows in
+// [row][kv_head][d] order, widened where the payload is f32 and the pool f16 (exact for every half,
+// crates/gguf/src/dequant.rs:12-34 is the host rule). VEC consecutive channels a thread: a key's
+// eight are one 16-byte piece of its plane, a value's eight come from lines that the threads of the
+// neighbouring rows use too. One launch takes the runs of a 32 MiB stretch of the payload, where a
+// launch per layer, two widening launches and a copy per side took 25 us for 8 MB.
+template <typename T, typename OUT, int VEC>
+__global__ __launch_bounds__(256) void kv_read_runs(const T *__restrict__ base, const T *__restrict__ base_w,
+                                                    PoolGeom g, PoolGeom gw, ReadRuns b, OUT *__restrict__ out) {
+    const ReadRun R = b.run[blockIdx.y];
+    const PoolGeom &G = R.ring ? gw : g;
+    const T *src = (R.ring ? base_w : base) + R.layer * G.layer_stride + b.slot * G.slot_stride + R.side * G.side_stride;
+    const uint32_t width = G.kv_heads * G.head_dim;
+    OUT *to = out + R.out0;
+    for (uint64_t i = (blockIdx.x * 256ull + threadIdx.x) * VEC; i < R.count; i += gridDim.x * 256ull * VEC) {
+        const uint64_t e = R.elem0 + i;
+        const uint32_t row = uint32_t(e / width), rem = uint32_t(e % width);
+        const uint32_t head = rem / G.head_dim, d = rem % G.head_dim;
+        const uint32_t srow = R.ring ? (R.first_row + row) % R.ring : R.first_row + row;
+        const T *plane = src + head * G.head_stride;
+        T v[VEC];
+        if (VEC > 1 && (R.side == 0 || G.v_block == 0)) {
+            const T *at = plane + kv_offset(G, R.side, srow, d);
+            __builtin_memcpy(v, __builtin_assume_aligned(at, VEC * sizeof(T) > 16 ? 16 : VEC * sizeof(T)), sizeof(v));
+        } else {
+#pragma unroll
+            for (int k = 0; k < VEC; ++k) v[k] = plane[kv_offset(G, R.side, srow, d + k)];
+        }
+        OUT w[VEC];
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+            if constexpr (sizeof(OUT) == sizeof(T))
+                w[k] = v[k];
+            else
+                w[k] = static_cast<float>(__builtin_bit_cast(_Float16, v[k]));
+        }
+        __builtin_memcpy(__builtin_assume_aligned(to + i, VEC * sizeof(OUT) > 16 ? 16 : VEC * sizeof(OUT)), w, sizeof(w));
+    }
+}
+
+hipError_t launch_read_runs(const void *base, const void *base_w, int elem_f16, int out_f16, const PoolGeom &g,
+                            const PoolGeom &gw, const ReadRuns &b, void *out, hipStream_t stream) {
+    if (b.n == 0) return hipSuccess;
+    uint64_t most = 0;
+    bool by_eight = g.head_dim % 8 == 0;
+    for (uint32_t i = 0; i < b.n; ++i) {
+        most = std::max(most, b.run[i].count);
+        by_eight = by_eight && b.run[i].elem0 % 8 == 0 && b.run[i].count % 8 == 0 && b.run[i].out0 % 8 == 0;
+    }
+    const uint64_t per_group = 256ull * (by_eight ? 8 : 1);
+    const dim3 grid(uint32_t(std::min<uint64_t>((most + per_group - 1) / per_group, 4096)), b.n, 1);
+#define ITAK_RUNS(T, OUT)                                                                                  \
+    do {                                                                                                   \
+        if (by_eight)                                                                                      \
+            kv_read_runs<T, OUT, 8><<<grid, 256, 0, stream>>>(static_cast<const T *>(base),                \
+                static_cast<const T *>(base_w), g, gw, b, static_cast<OUT *>(out));                        \
+        else                                                                                               \
+            kv_read_runs<T, OUT, 1><<<grid, 256, 0, stream>>>(static_cast<const T *>(base),                \
+                static_cast<const T *>(base_w), g, gw, b, static_cast<OUT *>(out));                        \
+    } while (0)
+    if (!elem_f16)
+        ITAK_RUNS(float, float);
+    else if (out_f16)
+        ITAK_RUNS(uint16_t, uint16_t);
+    else
+        ITAK_RUNS(uint16_t, float);
+#undef ITAK_RUNS
+    return hipGetLastError();
+}
+
 // ------------------------------------------------------- ring rows aside and back
 // One element per thread and step: a checkpoint deeper than the headroom is taken once per
 // speculative round at most and moves a few MB.
@@ -427,21 +499,6 @@ hipError_t launch_convert_f16(const float *src, uint16_t *dst, uint64_t count, h
     uint64_t blocks = (count + 255) / 256;
     if (blocks > 65536) blocks = 65536;
     convert_f32_to_f16<<<uint32_t(blocks), 256, 0, stream>>>(src, dst, count);
-    return hipGetLastError();
-}
-
-// f16 -> f32 is exact for every half (crates/gguf/src/dequant.rs:12-34 is the host rule).
-__global__ __launch_bounds__(256) void widen_f16_to_f32(const uint16_t *__restrict__ src,
-                                                        float *__restrict__ dst, uint64_t count) {
-    for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < count; i += gridDim.x * 256ull)
-        dst[i] = static_cast<float>(__builtin_bit_cast(_Float16, src[i]));
-}
-
-hipError_t launch_widen_f16(const uint16_t *src, float *dst, uint64_t count, hipStream_t stream) {
-    if (count == 0) return hipSuccess;
-    uint64_t blocks = (count + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    widen_f16_to_f32<<<uint32_t(blocks), 256, 0, stream>>>(src, dst, count);
     return hipGetLastError();
 }
 

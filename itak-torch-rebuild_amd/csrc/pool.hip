@@ -4,7 +4,10 @@
 // All validation happens here, in the reference's order, before anything is enqueued.
 #include "../../include/itak_hip_kv.h"
 #include "internal.h"
+#include "host_ring.h"
 #include "itkv.h"
+
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <atomic>
@@ -168,6 +171,8 @@ struct itak_pool {
     // and go up in one copy; its kernels write the output here directly.
     unsigned char *hstage = nullptr;
     uint64_t hstage_bytes = 0;
+    // Pinned slots through which snapshot rows move between ordinary host memory and the device.
+    HostRing ring;
     uint32_t call_number = 0;  // what the last host-pointer call asked to be told when done
     mutable ErrorState err;
 };
@@ -991,7 +996,7 @@ namespace itak {
 
 int32_t restore_decoded_itkv(itak_pool *pool, uint32_t slot, const uint8_t *b8, const ItkvHeader &h,
                              const std::vector<ItkvLayer> &ls, const char *expected_fingerprint,
-                             uint64_t expected_fingerprint_len) {
+                             uint64_t expected_fingerprint_len, const uint8_t *rows) {
     if (!pool) return ITAK_INVALID_ARGUMENT;
     if (!find_slot(pool, slot)) return invalid_argument(pool->err, "slot is not in use");
     // restore_checked (snapshot.rs:351-371): geometry first, then the fingerprint.
@@ -1017,9 +1022,10 @@ int32_t restore_decoded_itkv(itak_pool *pool, uint32_t slot, const uint8_t *b8, 
                          int(std::min<uint64_t>(h.fingerprint_len, 400)),
                          reinterpret_cast<const char *>(b8 + h.fingerprint_offset));
     std::vector<itak_snapshot_layer> layers(ls.size());
+    const uint8_t *at = rows ? rows - ls[0].keys_offset : b8;
     for (size_t i = 0; i < ls.size(); ++i)
-        layers[i] = itak_snapshot_layer{ls[i].first_position, ls[i].rows, b8 + ls[i].keys_offset,
-                                        b8 + ls[i].values_offset};
+        layers[i] = itak_snapshot_layer{ls[i].first_position, ls[i].rows, at + ls[i].keys_offset,
+                                        at + ls[i].values_offset};
     return itak_kv_restore_snapshot(pool, slot, h.token_count, layers.data(), layers.size(),
                                     h.elem ? ITAK_ELEM_F16 : ITAK_ELEM_F32);
 }
@@ -1251,6 +1257,7 @@ void itak_pool_destroy(itak_pool *pool) {
     for (void *buf : pool->ring_saved)
         if (buf) (void)hipFree(buf);
     if (pool->hstage) (void)hipHostFree(pool->hstage);
+    pool->ring.close();
     delete pool;
 }
 
@@ -1505,6 +1512,23 @@ static itak_status restore_layers(itak_pool *pool, uint32_t slot, Slot &s,
     if (stage_need) HIP_TRY(pool, hipMalloc(reinterpret_cast<void **>(&temp), stage_need), "allocate restore staging");
     uint64_t temp_off = 0;
     itak_status st = ITAK_OK;
+    std::vector<RingSpan> staged;
+    std::vector<const void *> staged_at(2 * count, nullptr);
+    for (uint64_t i = 0; i < count && stage_need; ++i) {
+        const uint64_t bytes = layers[i].rows * pool->row * src_bytes_per_elem;
+        const void *src[2] = {layers[i].keys, layers[i].values};
+        for (int side = 0; side < 2 && bytes; ++side)
+            if (must_stage(kind_of, src[side], src_bytes_per_elem)) {
+                staged.push_back(RingSpan{src[side], temp + temp_off, bytes});
+                staged_at[2 * i + side] = temp + temp_off;
+                temp_off += align_up(bytes, 256);
+            }
+    }
+    if (hipError_t he = ring_upload(pool->ring, staged, pool->stream); he != hipSuccess) {
+        (void)hipStreamSynchronize(pool->stream);
+        if (temp) (void)hipFree(temp);
+        return hip_error(pool->err, he, "stage snapshot rows");
+    }
     // One gather batch per group of planes (global, windowed), launched when it fills up. A
     // windowed layer's rows go to storage rows position % ring: one run, or two when the
     // positions wrap past the end of the ring (session.rs:320-346 states the same split).
@@ -1541,25 +1565,16 @@ static itak_status restore_layers(itak_pool *pool, uint32_t slot, Slot &s,
         if (L.rows == 0) continue;
         const uint64_t layer = layer_ids ? layer_ids[i] : i;
         const LayerInfo &info = pool->layers[layer];
-        const uint64_t bytes = L.rows * pool->row * src_bytes_per_elem;
         const void *src[2] = {L.keys, L.values};
         for (int side = 0; side < 2; ++side) {
             const void *usable;
-            if (!must_stage(kind_of, src[side], src_bytes_per_elem)) {
+            if (staged_at[2 * i + side]) {
+                src[side] = staged_at[2 * i + side];
+            } else {
                 kind_of(src[side], &usable);
                 src[side] = usable;
-                continue;
             }
-            hipError_t he = hipMemcpyAsync(temp + temp_off, src[side], bytes, hipMemcpyHostToDevice,
-                                           pool->stream);
-            if (he != hipSuccess) {
-                st = hip_error(pool->err, he, "stage snapshot rows");
-                break;
-            }
-            src[side] = temp + temp_off;
-            temp_off += align_up(bytes, 256);
         }
-        if (st != ITAK_OK) break;
         const int w = info.windowed ? 1 : 0;
         uint64_t done = 0;
         while (done < L.rows && st == ITAK_OK) {
@@ -1781,6 +1796,29 @@ itak_status itak_kv_capture_itkv_f16(itak_pool *pool, uint32_t slot, const char 
     return capture_itkv(pool, slot, fingerprint, fingerprint_len, true, out, capacity, written);
 }
 
+// A snapshot's payload passes through device memory this many bytes at a time (a multiple of the
+// ring's chunk and of the hash's runs). From kDeviceSumBytes on version 1's checksum is the
+// device's: the ten launches take 40 us there, what a host core needs for 48 KiB, and the rule
+// leaves a margin for their coming one behind the other on a busy stream.
+constexpr uint64_t kPayloadPiece = 32ull << 20;
+constexpr uint64_t kDeviceSumBytes = 128ull << 10;
+static_assert(kPayloadPiece % kRingChunk == 0 && kRingChunk % kFnvRun == 0, "pieces are whole chunks and runs");
+
+// A large output buffer is often fresh from the allocator: its pages are touched here for the
+// first time, and 4 KiB at a time that costs more than the copy. Only a hint; a refusal is no loss.
+static void advise_huge_pages(void *p, uint64_t bytes) {
+    const uint64_t huge = 2ull << 20;
+    const uint64_t from = align_up(reinterpret_cast<uint64_t>(p), huge), to = (reinterpret_cast<uint64_t>(p) + bytes) / huge * huge;
+    if (to > from && to - from >= 4 * huge) (void)madvise(reinterpret_cast<void *>(from), to - from, MADV_HUGEPAGE);
+}
+
+static itak_status finish_capture(uint8_t *bytes, uint64_t total, uint32_t version, bool with_checksum,
+                                  const uint64_t *known) {
+    const uint64_t sum = known ? *known : with_checksum ? itkv_trailer(version, bytes, total - 8) : 0;
+    for (int b = 0; b < 8; ++b) bytes[total - 8 + b] = uint8_t(sum >> (8 * b));
+    return ITAK_OK;
+}
+
 static itak_status capture_itkv(itak_pool *pool, uint32_t slot, const char *fingerprint,
                                 uint64_t fingerprint_len, bool f16_rows, void *out,
                                 uint64_t capacity, uint64_t *written, bool with_checksum) {
@@ -1828,53 +1866,80 @@ static itak_status capture_itkv(itak_pool *pool, uint32_t slot, const char *fing
         return invalid_argument(pool->err, "output buffer is smaller than the encoding");
     uint8_t *bytes = static_cast<uint8_t *>(out);
     itkv_write_header(bytes, h, fingerprint, ls.data());
-    // Rows come back through the readback kernel in chunks that bound the staging buffer:
-    // planes -> [row][kv_head][d] in the pool's element type, widened to f32 for an f16 pool.
-    const uint64_t chunk_rows = std::max<uint64_t>(1, (uint64_t(16) << 20) / (pool->row * 4));
-    const uint64_t raw = align_up(chunk_rows * pool->row * pool->elem_bytes, 256);
-    const uint64_t wide = align_up(chunk_rows * pool->row * 4, 256);
-    itak_status st = ensure_stage(pool, 2 * raw + (pool->elem_f16 ? 2 * wide : 0));
+    if (token_count == 0) return finish_capture(bytes, total, h.version, with_checksum, nullptr);
+    // The payload (every layer's keys, then its values) is made in device memory 32 MiB at a time,
+    // summed there when the trailer is version 1's, and goes out through the pinned ring.
+    const uint64_t payload = ls[0].keys_offset, payload_bytes = total - 8 - payload;
+    const uint64_t piece = std::min(align_up(payload_bytes, 256), kPayloadPiece);
+    const bool device_sum = with_checksum && h.version == kItkvVersion && payload_bytes >= kDeviceSumBytes;
+    itak_status st = ensure_stage(pool, piece + 256 + (device_sum ? fnv_scratch_bytes(piece) : 0));
     if (st != ITAK_OK) return st;
-    for (uint64_t layer = 0; layer < h.layer_count; ++layer) {
-        for (uint64_t first = 0; first < ls[layer].rows; first += chunk_rows) {
-            const uint64_t rows = std::min(chunk_rows, ls[layer].rows - first);
-            const uint64_t elems = rows * pool->row;
-            unsigned char *kd = pool->stage, *vd = pool->stage + raw;
-            HIP_TRY(pool,
-                    launch_read_rows(layer_base(pool, layer), pool->elem_f16, geom_of(pool, layer),
-                                     slot, uint32_t(ls[layer].first_position + first),
-                                     uint32_t(rows), pool->layers[layer].ring, kd, vd,
-                                     pool->stream),
-                    "launch row readback");
-            const void *ksrc = kd, *vsrc = vd;
-            if (pool->elem_f16 && !f16_rows) {
-                float *kw = reinterpret_cast<float *>(pool->stage + 2 * raw);
-                float *vw = reinterpret_cast<float *>(pool->stage + 2 * raw + wide);
-                HIP_TRY(pool,
-                        launch_widen_f16(reinterpret_cast<const uint16_t *>(kd), kw, elems, pool->stream),
-                        "launch widening");
-                HIP_TRY(pool,
-                        launch_widen_f16(reinterpret_cast<const uint16_t *>(vd), vw, elems, pool->stream),
-                        "launch widening");
-                ksrc = kw;
-                vsrc = vw;
+    unsigned long long *state = reinterpret_cast<unsigned long long *>(pool->stage);
+    unsigned char *rows_dev = pool->stage + 256, *scratch = rows_dev + piece;
+    advise_huge_pages(bytes, total);
+    if (device_sum)
+        HIP_TRY(pool, launch_fill_words(state, 1, fnv1a64(bytes, payload, kFnvOffset), pool->stream), "start checksum");
+    uint64_t run = 0, run_at = 0;  // the (layer, side) the next byte belongs to, and the first byte of it
+    auto make_piece = [&](uint64_t at, uint64_t bytes_here) -> hipError_t {
+        ReadRuns b{};
+        b.slot = slot;
+        const uint64_t end = at + bytes_here;
+        for (uint64_t to = at; to < end;) {
+            const ItkvLayer &L = ls[run / 2];
+            const LayerInfo &info = pool->layers[run / 2];
+            const uint64_t run_bytes = L.rows * pool->row * out_elem;
+            const uint64_t n = std::min(end, run_at + run_bytes) - to;
+            if (n) {
+                b.run[b.n++] = ReadRun{info.index, uint32_t(run & 1), uint32_t(L.first_position),
+                                       info.windowed ? uint32_t(info.ring) : 0, (to - run_at) / out_elem, n / out_elem,
+                                       (to - at) / out_elem};
+                to += n;
             }
-            HIP_TRY(pool,
-                    hipMemcpyAsync(bytes + ls[layer].keys_offset + first * pool->row * out_elem,
-                                   ksrc, elems * out_elem, hipMemcpyDeviceToHost, pool->stream),
-                    "download keys");
-            HIP_TRY(pool,
-                    hipMemcpyAsync(bytes + ls[layer].values_offset + first * pool->row * out_elem,
-                                   vsrc, elems * out_elem, hipMemcpyDeviceToHost, pool->stream),
-                    "download values");
-            // The staging buffer is reused by the next chunk.
-            HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after readback");
+            if (to == run_at + run_bytes) {
+                run_at += run_bytes;
+                ++run;
+            }
+            if (b.n == kMaxReadRuns || to == end) {
+                hipError_t e = launch_read_runs(pool->base, pool->base_w, pool->elem_f16, f16_rows, pool->g, pool->gw, b,
+                                                rows_dev, pool->stream);
+                if (e != hipSuccess) return e;
+                b.n = 0;
+            }
         }
-    }
-    const uint64_t sum = with_checksum ? itkv_trailer(h.version, bytes, total - 8) : 0;
-    for (int b = 0; b < 8; ++b) bytes[total - 8 + b] = uint8_t(sum >> (8 * b));
-    return ITAK_OK;
+        return device_sum ? launch_fnv(rows_dev, bytes_here / kFnvRun * kFnvRun, scratch, state, pool->stream) : hipSuccess;
+    };
+    HIP_TRY(pool,
+            ring_download(pool->ring, bytes + payload, payload_bytes, pool->stream,
+                          [&](uint64_t at, uint64_t, const void **src) -> hipError_t {
+                              *src = rows_dev + at % kPayloadPiece;
+                              if (at % kPayloadPiece) return hipSuccess;
+                              return make_piece(at, std::min(kPayloadPiece, payload_bytes - at));
+                          }),
+            "download snapshot rows");
+    if (!device_sum) return finish_capture(bytes, total, h.version, with_checksum, nullptr);
+    uint64_t sum = 0;
+    HIP_TRY(pool, hipMemcpyAsync(&sum, state, 8, hipMemcpyDeviceToHost, pool->stream), "download checksum");
+    HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after readback");
+    const uint64_t tail = payload_bytes % kFnvRun;  // only the last piece can have one
+    sum = fnv1a64(bytes + total - 8 - tail, tail, sum);
+    return finish_capture(bytes, total, h.version, true, &sum);
 }
+
+// Device memory for the length of a call; freeing it waits for what the call enqueued.
+struct DeviceBuffer {
+    unsigned char *p = nullptr;
+    hipError_t make(uint64_t bytes) {
+        const hipError_t e = hipMalloc(reinterpret_cast<void **>(&p), bytes);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            p = nullptr;
+        }
+        return e;
+    }
+    ~DeviceBuffer() {
+        if (p) (void)hipFree(p);
+    }
+};
 
 itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *bytes, uint64_t len,
                                  const char *expected_fingerprint,
@@ -1892,8 +1957,50 @@ itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *byt
     std::vector<ItkvLayer> ls;
     ItkvError err;
     const uint8_t *b8 = static_cast<const uint8_t *>(bytes);
-    if (!itkv_decode(b8, len, h, ls, err)) return set_itkv_error(pool->err, err);
-    return restore_decoded_itkv(pool, slot, b8, h, ls, expected_fingerprint, expected_fingerprint_len);
+    // From kDeviceSumBytes on the payload goes to the device first, is summed there (version 1) or
+    // by host threads meanwhile (version 2), and is gathered from there once the sum is known good.
+    DeviceBuffer rows;
+    hipError_t moved = hipSuccess;
+    const ItkvSum sum_of = [&](const ItkvHeader &header, uint64_t payload) -> uint64_t {
+        const uint64_t n = len - 8 - payload, piece = std::min(align_up(n, 256), kPayloadPiece);
+        const bool device_sum = header.version == kItkvVersion;
+        const uint64_t scratch_at = align_up(n, 256) + 256;
+        if (n < kDeviceSumBytes ||
+            rows.make(scratch_at + (device_sum ? fnv_scratch_bytes(piece) : 0)) != hipSuccess)
+            return itkv_trailer(header.version, b8, len - 8);
+        unsigned long long *state = reinterpret_cast<unsigned long long *>(rows.p + align_up(n, 256));
+        if (device_sum)
+            moved = launch_fill_words(state, 1, fnv1a64(b8, payload, kFnvOffset), pool->stream);
+        uint64_t summed = 0;
+        const auto sum_up_to = [&](uint64_t sent) -> hipError_t {
+            if (!device_sum || (sent < n && sent - summed < kPayloadPiece)) return hipSuccess;
+            hipError_t e = launch_fnv(rows.p + summed, (sent - summed) / kFnvRun * kFnvRun, rows.p + scratch_at, state, pool->stream);
+            summed = sent;
+            return e;
+        };
+        const void *usable;
+        if (moved == hipSuccess && classify(b8, &usable) == PtrKind::PinnedHost) {
+            for (uint64_t at = 0; at < n && moved == hipSuccess; at += kPayloadPiece) {
+                const uint64_t here = std::min(kPayloadPiece, n - at);
+                moved = hipMemcpyAsync(rows.p + at, b8 + payload + at, here, hipMemcpyHostToDevice, pool->stream);
+                if (moved == hipSuccess) moved = sum_up_to(at + here);
+            }
+        } else if (moved == hipSuccess) {
+            moved = ring_upload(pool->ring, {RingSpan{b8 + payload, rows.p, n}}, pool->stream, sum_up_to);
+        }
+        uint64_t sum = 0;
+        if (!device_sum) sum = itkv_trailer(header.version, b8, len - 8);
+        if (moved == hipSuccess && device_sum)
+            moved = hipMemcpyAsync(&sum, state, 8, hipMemcpyDeviceToHost, pool->stream);
+        const hipError_t done = hipStreamSynchronize(pool->stream);
+        if (moved == hipSuccess) moved = done;
+        if (device_sum) sum = fnv1a64(b8 + len - 8 - n % kFnvRun, n % kFnvRun, sum);
+        return sum;
+    };
+    const bool decoded = itkv_decode(b8, len, h, ls, err, nullptr, sum_of);
+    if (moved != hipSuccess) return hip_error(pool->err, moved, "move snapshot rows to the device");
+    if (!decoded) return set_itkv_error(pool->err, err);
+    return restore_decoded_itkv(pool, slot, b8, h, ls, expected_fingerprint, expected_fingerprint_len, rows.p);
 }
 
 itak_status itak_kv_stats(itak_pool *pool, uint32_t slot, itak_layer_stats *out) {

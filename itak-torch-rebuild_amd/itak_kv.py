@@ -231,9 +231,13 @@ def capture_bytes(cache: KvCache, model_fingerprint: str, elem: str = "f32") -> 
     written = C.c_uint64()
     h = cache.pool._h
     _check_kv(h, fn(h, cache.slot, fp, len(fp), None, 0, C.byref(written)))
-    out = np.empty(written.value, dtype=np.uint8)
-    _check_kv(h, fn(h, cache.slot, fp, len(fp), out.ctypes.data, out.size, C.byref(written)))
-    return out.tobytes()
+    # The bytes object is filled before anyone else sees it, instead of an array copied into one.
+    make, at = C.pythonapi.PyBytes_FromStringAndSize, C.pythonapi.PyBytes_AsString
+    make.restype, make.argtypes = C.py_object, (C.c_void_p, C.c_ssize_t)
+    at.restype, at.argtypes = C.c_void_p, (C.py_object,)
+    out = make(None, written.value)
+    _check_kv(h, fn(h, cache.slot, fp, len(fp), at(out), written.value, C.byref(written)))
+    return out
 
 
 def restore_bytes(pool: KvPool, data, expected_fingerprint: Optional[str] = None) -> KvCache:
