@@ -386,14 +386,14 @@ bool attn_splitk_f32_appends(const PoolGeom &g, uint32_t group, uint32_t max_row
 
 // Fills splits / keys_per_split / block0 / ws0 (slot, rows, pos0, q_row0, kv_len, kv_lo are
 // set) and returns the number of partials. Every (item, KV head) is cut into equal runs of at
-// most T blocks, T the smallest run for which the batch is at most two workgroups per
+// most T blocks, T the smallest run for which the batch is at most groups_per_cu workgroups per
 // compute unit, and never shorter than one block per wavefront.
-uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads) {
+uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu) {
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
         (void)hipGetLastError();
-    const uint64_t capacity = uint64_t(2) * uint64_t(cus > 0 ? cus : 256);
+    const uint64_t capacity = groups_per_cu * uint64_t(cus > 0 ? cus : 256);
     const uint32_t group = q_heads / g.kv_heads;
     auto units_of = [&](const AttnItem &it) {
         return uint64_t(g.kv_heads) * ((uint64_t(it.rows) * group + 15) / 16);

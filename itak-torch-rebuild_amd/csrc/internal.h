@@ -473,8 +473,17 @@ hipError_t launch_attn_decode_f16(const AttnParams &p, const AttnBatch &b, uint3
 bool attn_splitk_f32_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
 // True when such a launch also appends the step's rows (k_new / v_new in its parameters).
 bool attn_splitk_f32_appends(const PoolGeom &g, uint32_t group, uint32_t max_rows);
-uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads);
+uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu = 2);
 hipError_t launch_attn_splitk_f32(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
+                                  hipStream_t stream);
+// f32-arithmetic MFMA split-K path for the other shapes (attn_splitk_any.hip): f16 and f32 pools,
+// any head_dim <= 256 that is a multiple of four, any group, implied query positions, tensors
+// 16-byte aligned. Planned by attn_splitk_f32_plan; partials are in log2 domain.
+bool attn_splitk_any_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
+// Workgroups of that kernel a compute unit holds.
+uint32_t attn_splitk_any_groups_per_cu(const PoolGeom &g);
+bool attn_splitk_any_appends(const PoolGeom &g, uint32_t group, uint32_t max_rows);
+hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream);
 // MFMA block path (speculative blocks and prefill chunks): same pools, any number of rows,
 // group dividing 16; K/V staged through LDS, split over the context when the launch would

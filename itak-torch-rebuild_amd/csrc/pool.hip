@@ -538,6 +538,22 @@ bool takes_splitk_f16(const itak_pool *pool, const PlanInput *in, uint32_t n, ui
            attn_splitk_f16_supports(pool->g, group, max_rows);  // g and gw differ in capacity only
 }
 
+// The f32-arithmetic matrix kernel takes what has no kernel of its own: f16 pools at other head dims
+// or with groups above 16, f32 pools at other head dims. Its 16-byte loads and stores ask for
+// tensors aligned to that (every row is a multiple of 16 bytes when head_dim is one of four
+// floats); others, odd head dims and explicit positions run on the general kernel.
+bool aligned16(const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+bool takes_splitk_any(const itak_pool *pool, const PlanInput *in, uint32_t n, uint64_t q_heads, const float *q_dev,
+                      const float *out_dev, const uint32_t *q_pos_dev) {
+    const uint32_t group = uint32_t(q_heads / pool->g.kv_heads);
+    uint32_t max_rows = 0;
+    for (uint32_t i = 0; i < n; ++i) max_rows = std::max(max_rows, in[i].rows);
+    return q_pos_dev == nullptr && aligned16(q_dev) && aligned16(out_dev) &&
+           !takes_splitk_f16(pool, in, n, q_heads, q_pos_dev) &&
+           !(pool->elem_f16 ? attn_prefill_f16_supports(pool->g, group) : attn_splitk_f32_supports(pool->g, group, max_rows)) &&
+           attn_splitk_any_supports(pool->g, group, max_rows);
+}
+
 // k_new / v_new non-null = the rows are not in the cache yet and the kernel appends them
 // (only valid when takes_splitk_f16 holds).
 itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, uint32_t n,
@@ -555,9 +571,10 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     // Decode steps and short blocks on f32 pools of head_dim 128: the f32 MFMA split-K kernel.
     const bool f32fast = !pool->elem_f16 && q_pos_dev == nullptr &&
                          attn_splitk_f32_supports(pool->g, group, max_rows);
+    const bool any = takes_splitk_any(pool, in, n, q_heads, q_dev, out_dev, q_pos_dev);
     const uint32_t rpb =
-        (mfma || prefill || f32fast) ? 0 : attn_generic_rows_per_block(group, pool->g.head_dim);
-    if (!mfma && !prefill && !f32fast && rpb == 0)
+        (mfma || prefill || f32fast || any) ? 0 : attn_generic_rows_per_block(group, pool->g.head_dim);
+    if (!mfma && !prefill && !f32fast && !any && rpb == 0)
         return unsupported(pool->err, "head_dim above 256 or GQA group too wide");
     const uint32_t tile = attn_generic_tile(pool->g.head_dim);
     constexpr uint64_t kTargetBlocks = 1024;  // about four workgroups per CU
@@ -589,8 +606,9 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads));
         } else if (prefill) {
             partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, k_new != nullptr);
-        } else if (f32fast) {
-            partials = attn_splitk_f32_plan(geom, b, uint32_t(q_heads));
+        } else if (f32fast || any) {
+            partials = attn_splitk_f32_plan(geom, b, uint32_t(q_heads),
+                                            any && max_rows * group <= 16 ? attn_splitk_any_groups_per_cu(geom) : 2);
         } else {
             b.rows_per_block = rpb;
             uint64_t key_work = 0;
@@ -672,8 +690,8 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
                       "fused_append=%d merge=%s",
                       ULL(layer), count, total_rows, ULL(q_heads), ULL(pool->g.kv_heads), ULL(view_len),
                       window, double(scale), double(softcap),
-                      mfma ? "splitk_f16" : prefill ? "prefill_f16" : f32fast ? "splitk_f32" : "generic",
-                      bl.total_blocks, splits, int(k_new != nullptr && (mfma || f32fast || prefill)),
+                      mfma ? "splitk_f16" : prefill ? "prefill_f16" : f32fast ? "splitk_f32" : any ? "splitk_any" : "generic",
+                      bl.total_blocks, splits, int(k_new != nullptr && (mfma || f32fast || any || prefill)),
                       partials == 0 ? "none" : on_die ? "on_die" : exchange_words ? "in_launch" : "launch");
         }
         AttnParams p{};
@@ -695,8 +713,8 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             p.kv_streams = layer_bytes * pool->layers.size() > (uint64_t(512) << 20) ? 1 : 0;  // twice the cache: well clear of it
         }
         p.spin_limit = pool->spin_limit;
-        p.k_new = (mfma || f32fast || prefill) ? k_new : nullptr;  // the caller passes them only to
-        p.v_new = (mfma || f32fast || prefill) ? v_new : nullptr;  // launches that append themselves
+        p.k_new = (mfma || f32fast || any || prefill) ? k_new : nullptr;  // the caller passes them only to
+        p.v_new = (mfma || f32fast || any || prefill) ? v_new : nullptr;  // launches that append themselves
         p.q_heads = uint32_t(q_heads);
         p.group = group;
         p.group_magic = (65536u + group - 1) / group;
@@ -727,12 +745,15 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         } else if (f32fast) {
             HIP_TRY(pool, launch_attn_splitk_f32(p, b, partials, pool->stream),
                     "launch f32 split-K attention");
+        } else if (any) {
+            HIP_TRY(pool, launch_attn_splitk_any(pool->elem_f16, p, b, partials, pool->stream),
+                    "launch split-K attention of any head_dim");
         } else {
             HIP_TRY(pool, launch_attn_generic(pool->elem_f16, p, b, partials, pool->stream),
                     "launch attention");
         }
         if (!exchange_words && !on_die)
-            HIP_TRY(pool, launch_attn_combine(p, b, partials, total_rows, (mfma || prefill || f32fast) ? 1 : 0,
+            HIP_TRY(pool, launch_attn_combine(p, b, partials, total_rows, (mfma || prefill || f32fast || any) ? 1 : 0,
                                               pool->stream, gate_folded ? gate : nullptr),
                     "launch split merge");
         if (gate && !gate_folded) {
@@ -2435,7 +2456,10 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
     const bool fuse =
         splitk || block_fuses ||
         (!pool->elem_f16 && !active.empty() &&
-         attn_splitk_f32_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows));
+         attn_splitk_f32_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows)) ||
+        (!active.empty() && aligned16(k_dev) && aligned16(v_dev) &&
+         takes_splitk_any(pool, active.data(), uint32_t(active.size()), num_q_heads, q_dev, out_dev, nullptr) &&
+         attn_splitk_any_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows));
     // The allocation-free form plans first and refuses, before anything changes, a step whose
     // launches need more workspace than the static array has.
     struct NoAllocScope {
