@@ -36,8 +36,10 @@
 // Bound: launch and memory latency on decode steps; on blocks the L2 that feeds a workgroup per 16
 // vectors (row-major: the f32 matrix pipe, 157 TFLOP/s).
 // The general VALU kernel, which these shapes took before, moves K and V through LDS as f32 and pays
-// an LDS read for every multiply-add: 8 slots of up to 1,500 rows at head_dim 80 took 124 us a layer
-// there (133 with append and merge).
+// an LDS read for every multiply-add. 32 Q / 8 KV heads, f16, us a layer, append and merge included:
+// head_dim 80, 8 slots of up to 1,500 rows 133 -> 13.4 (10.6 of it this kernel; 25.6 with its products
+// on the f32 pipe), 2 slots of 40 rows at 2,000 27.6, a 512-row chunk over 2,000 rows 76 (247 on the f32
+// pipe).
 //
 // Semantics: gqa_attention in crates/attention/src/attention.rs:104-215, softcap as
 // crates/torch-math/src/logits.rs:26-37. Partials are in the log2 domain.

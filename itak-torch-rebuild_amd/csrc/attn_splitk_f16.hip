@@ -437,12 +437,14 @@ __device__ __forceinline__ float split_lanes_sum(float v) {
 }
 // D = head_dim (64, 96, 128 or 256): a wavefront owns D/4 channels, i.e. D/16 chunks, in the next
 // power of two of lanes (at 96 two of eight sit idle), and the other lane bits are split lanes.
-template <int N, bool BASE2, bool GATE, int D = 128>
+// D = 0: any multiple of four, from the pool's geometry, in CL chunk lanes.
+template <int N, bool BASE2, bool GATE, int D = 128, int CL = 0>
 __device__ __forceinline__ void attn_combine128_body(const AttnParams &p, const AttnBatchT<N> &b,
                                                      uint32_t total_partials,
                                                      [[maybe_unused]] const float *gate) {
-    constexpr uint32_t kChunks = D / 16;                                   // per wavefront
-    constexpr uint32_t kChunkLanes = kChunks <= 4 ? 4 : kChunks <= 8 ? 8 : 16;
+    const uint32_t dim = D ? D : p.g.head_dim;
+    const uint32_t kChunks = (dim + 15) / 16;                              // per wavefront
+    constexpr uint32_t kChunkLanes = CL ? CL : D <= 64 ? 4 : D <= 128 ? 8 : 16;
     constexpr int SL = 64 / kChunkLanes;                                   // split lanes
     const uint32_t tid = threadIdx.x;
     ITAK_MARK_BEGIN
@@ -460,11 +462,12 @@ __device__ __forceinline__ void attn_combine128_body(const AttnParams &p, const 
     const uint64_t ps0 = item.ws0 + (uint64_t(row) * p.q_heads + head) * S;
     const uint32_t wave = tid >> 6, lane = tid & 63;
     const uint32_t cl = lane % kChunkLanes, sl = lane / kChunkLanes;  // chunk of the wavefront, split lane
-    const bool holds = cl < kChunks;                                   // (false only at head_dim 96)
-    const uint32_t c = wave * kChunks + min(cl, kChunks - 1);          // chunk of 4 channels
-    const float *ws_acc = p.ws + ps0 * D + c * 4;
-    const float2 *ws_ml = reinterpret_cast<const float2 *>(p.ws + uint64_t(total_partials) * D) + ps0;
-    const uint64_t at = (uint64_t(item.q_row0 + row) * p.q_heads + head) * D + c * 4;
+    // Chunk of 4 channels; lanes beyond the wavefront's chunks or head_dim read one that is there.
+    const bool holds = cl < kChunks && (D || wave * kChunks + cl < dim / 4);
+    const uint32_t c = D ? wave * kChunks + min(cl, kChunks - 1) : min(wave * kChunks + min(cl, kChunks - 1), dim / 4 - 1);
+    const float *ws_acc = p.ws + ps0 * dim + c * 4;
+    const float2 *ws_ml = reinterpret_cast<const float2 *>(p.ws + uint64_t(total_partials) * dim) + ps0;
+    const uint64_t at = (uint64_t(item.q_row0 + row) * p.q_heads + head) * dim + c * 4;
     // The gate of the lanes that write the output, fetched with the partials.
     [[maybe_unused]] float4 gt = make_float4(0.f, 0.f, 0.f, 0.f);
     if (GATE && sl == 0 && holds) gt = *reinterpret_cast<const float4 *>(gate + at);
@@ -478,7 +481,7 @@ __device__ __forceinline__ void attn_combine128_body(const AttnParams &p, const 
 #pragma unroll
         for (int u = 0; u < 8; ++u) {  // clamped, so the loads need no branch
             const uint32_t s = min(s0 + sl + u * SL, S - 1);
-            x[u] = *reinterpret_cast<const float4 *>(ws_acc + uint64_t(s) * D);
+            x[u] = *reinterpret_cast<const float4 *>(ws_acc + uint64_t(s) * dim);
             ml[u] = ws_ml[s];
         }
         // Nothing below may move above this line and no load below it: left to itself the
@@ -549,12 +552,12 @@ __global__ __launch_bounds__(256) void attn_combine128_gate_kernel(AttnParams p,
 }
 
 // The same merge at head dims 64, 96 and 256 (the partials of the block kernel and, at 64, of the
-// f32 kernel).
-template <int N, bool BASE2, bool GATE, int D>
+// f32 kernel), and (D = 0) at any other multiple of four.
+template <int N, bool BASE2, bool GATE, int D, int CL = 0>
 __global__ __launch_bounds__(256) void attn_combine_lanes_kernel(AttnParams p, AttnBatchT<N> b,
                                                                  uint32_t total_partials,
                                                                  const float *gate) {
-    attn_combine128_body<N, BASE2, GATE, D>(p, b, total_partials, gate);
+    attn_combine128_body<N, BASE2, GATE, D, CL>(p, b, total_partials, gate);
 }
 
 // The same merge for items of at most 16 splits, one wavefront per (row, Q head): lane =
@@ -697,6 +700,26 @@ hipError_t launch_attn_combine(const AttnParams &p, const AttnBatch &b, uint32_t
         else ITAK_LANES_D(256);
 #undef ITAK_LANES_D
 #undef ITAK_LANES
+        return hipGetLastError();
+    }
+    // The other head dims likewise (their partials are in the log2 domain): a merge of 256 outputs
+    // at head_dim 80 takes 3.3 us where the general kernel, with its two barriers and its walk
+    // through LDS at the end, takes 4.4.
+    if (base2 && p.g.head_dim % 4 == 0 && uint64_t(total_rows) * p.q_heads <= 4096) {
+        const dim3 grid(p.q_heads, total_rows);
+#define ITAK_LANES_ANY(G, CL)                                                                        \
+    ITAK_DISPATCH_BATCH(b.n, (attn_combine_lanes_kernel<N, true, G, 0, CL><<<grid, 256, 0, stream>>>( \
+                                 p, AttnBatchT<N>(b), total_partials, gate)))
+#define ITAK_LANES_CL(CL)                     \
+    do {                                      \
+        if (gate) ITAK_LANES_ANY(true, CL);   \
+        else ITAK_LANES_ANY(false, CL);       \
+    } while (0)
+        if (p.g.head_dim <= 64) ITAK_LANES_CL(4);
+        else if (p.g.head_dim <= 128) ITAK_LANES_CL(8);
+        else ITAK_LANES_CL(16);
+#undef ITAK_LANES_CL
+#undef ITAK_LANES_ANY
         return hipGetLastError();
     }
     ITAK_DISPATCH_BATCH(b.n, (attn_combine_kernel<N><<<total_rows * p.q_heads, kCombineThreads, 0,
