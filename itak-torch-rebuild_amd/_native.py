@@ -162,15 +162,15 @@ PROTOTYPES = {
     "itak_compute_cache_checkpoint": (_i32, [_P, _u32, _u64, C.POINTER(CheckpointRaw)]),
     "itak_compute_cache_rewind": (_i32, [_P, _u32, C.POINTER(CheckpointRaw), _u64]),
     "itak_compute_cache_release": (_i32, [_P, _u32, C.POINTER(CheckpointRaw)]),
-    "itak_attention_step_device": (_i32, [_P, _u64, C.POINTER(BatchItem), _u32, _P, _P, _P, _P,
+    "itak_attention_step_device": (_i32, [_P, _u64, _P, _u32, _P, _P, _P, _P,
                                           _u64, _f32, _f32]),
-    "itak_attention_step_device_noalloc": (_i32, [_P, _u64, C.POINTER(BatchItem), _u32, _P, _P, _P,
+    "itak_attention_step_device_noalloc": (_i32, [_P, _u64, _P, _u32, _P, _P, _P,
                                                   _P, _u64, _f32, _f32]),
-    "itak_attention_prep_step_device": (_i32, [_P, _u64, C.POINTER(BatchItem), _u32, _P, _P, _P, _P,
+    "itak_attention_prep_step_device": (_i32, [_P, _u64, _P, _u32, _P, _P, _P, _P,
                                                _P, _u64, _f32, _f32, C.POINTER(PrepParams)]),
-    "itak_attention_device": (_i32, [_P, _u64, C.POINTER(BatchItem), _u32, _P, _P, _u64, _f32,
+    "itak_attention_device": (_i32, [_P, _u64, _P, _u32, _P, _P, _u64, _f32,
                                      _f32]),
-    "itak_kv_append_device": (_i32, [_P, _u64, C.POINTER(BatchItem), _u32, _P, _P]),
+    "itak_kv_append_device": (_i32, [_P, _u64, _P, _u32, _P, _P]),
     "itak_kv_now_unix": (_u64, []),
     "itak_store_open": (_i32, [C.c_char_p, _u64, C.POINTER(_P)]),
     "itak_store_close": (None, [_P]),

@@ -462,9 +462,9 @@ hipError_t launch_attn_decode_f16(const AttnParams &p, const AttnBatch &b, uint3
 #define ITAK_LAUNCH_DECODE_QLO()                                                                   \
     do {                                                                                           \
         if (p.ring_blocks)                                                                         \
-            attn_decode_f16_kernel<N, true, true><<<b.total_blocks, kWaves * 64, 0, stream>>>(p, AttnBatchT<N>(b), total_partials); \
+            launch_kernel(attn_decode_f16_kernel<N, true, true>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<N>(b), total_partials); \
         else                                                                                       \
-            attn_decode_f16_kernel<N, false, true><<<b.total_blocks, kWaves * 64, 0, stream>>>(p, AttnBatchT<N>(b), total_partials); \
+            launch_kernel(attn_decode_f16_kernel<N, false, true>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<N>(b), total_partials); \
     } while (0)
         ITAK_DISPATCH_BATCH(b.n, ITAK_LAUNCH_DECODE_QLO());
 #undef ITAK_LAUNCH_DECODE_QLO
@@ -473,9 +473,9 @@ hipError_t launch_attn_decode_f16(const AttnParams &p, const AttnBatch &b, uint3
 #define ITAK_LAUNCH_DECODE()                                                                       \
     do {                                                                                           \
         if (p.ring_blocks)                                                                         \
-            attn_decode_f16_kernel<N, true><<<b.total_blocks, kWaves * 64, 0, stream>>>(p, AttnBatchT<N>(b), total_partials); \
+            launch_kernel(attn_decode_f16_kernel<N, true>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<N>(b), total_partials); \
         else                                                                                       \
-            attn_decode_f16_kernel<N, false><<<b.total_blocks, kWaves * 64, 0, stream>>>(p, AttnBatchT<N>(b), total_partials); \
+            launch_kernel(attn_decode_f16_kernel<N, false>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<N>(b), total_partials); \
     } while (0)
     ITAK_DISPATCH_BATCH(b.n, ITAK_LAUNCH_DECODE());
 #undef ITAK_LAUNCH_DECODE

@@ -321,7 +321,7 @@ hipError_t launch_attn_generic(int elem_f16, const AttnParams &p, const AttnBatc
             if (e != hipSuccess) return e;                                                       \
             granted = lds;                                                                       \
         }                                                                                        \
-        attn_generic_kernel<T, V, N><<<b.total_blocks, kThreads, lds, stream>>>(                 \
+        launch_kernel(attn_generic_kernel<T, V, N>, b.total_blocks, kThreads, lds, stream, \
             p, AttnBatchT<N>(b), total_partials);                                                \
     } while (0)
 #define ITAK_LAUNCH_TV()                 \

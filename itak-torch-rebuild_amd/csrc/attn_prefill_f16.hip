@@ -64,11 +64,7 @@ static uint32_t unit_block_count(const AttnItem &it, uint32_t rows_per_group, ui
 uint32_t attn_prefill_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t group, uint32_t q_heads,
                                uint32_t window, bool appends) {
     const uint32_t rows_per_group = uint32_t(tiles_for(b, group) * kWaves * 16) / padded_group(group);
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        (void)hipGetLastError();
-    const uint64_t per_cu = uint64_t(cus > 0 ? cus : 256);
+    const uint64_t per_cu = compute_units();
     uint64_t unit_blocks = 0;
     for (uint32_t i = 0; i < b.n; ++i) {
         const uint64_t units = uint64_t(g.kv_heads) * ((b.item[i].rows + rows_per_group - 1) / rows_per_group);

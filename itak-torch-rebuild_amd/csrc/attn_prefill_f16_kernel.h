@@ -778,8 +778,7 @@ hipError_t launch_prefill_ring(const AttnParams &p, const AttnBatch &b,
         reinterpret_cast<const void *>(&attn_prefill_f16_kernel<N, SOFTCAP, TILES, RING, STAGES, D, QLO>),
         hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (granted != hipSuccess) return granted;
-    attn_prefill_f16_kernel<N, SOFTCAP, TILES, RING, STAGES, D, QLO>
-        <<<b.total_blocks, kWaves * 64, lds, stream>>>(p, AttnBatchT<N>(b), total_partials);
+    launch_kernel(attn_prefill_f16_kernel<N, SOFTCAP, TILES, RING, STAGES, D, QLO>, b.total_blocks, kWaves * 64, lds, stream, p, AttnBatchT<N>(b), total_partials);
     return hipGetLastError();
 }
 

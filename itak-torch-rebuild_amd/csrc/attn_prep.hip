@@ -122,7 +122,7 @@ hipError_t launch_attn_prep(const PrepArgs &a, hipStream_t stream) {
     const uint64_t head_rows = uint64_t(a.total_rows) * (a.q_heads + a.kv_heads);
     if (head_rows == 0) return hipSuccess;
     const uint64_t blocks = (head_rows + kPrepWaves - 1) / kPrepWaves;
-    attn_prep_kernel<<<uint32_t(blocks), kPrepWaves * 64, 0, stream>>>(a);
+    launch_kernel(attn_prep_kernel, uint32_t(blocks), kPrepWaves * 64, 0, stream, a);
     return hipGetLastError();
 }
 
@@ -130,7 +130,7 @@ hipError_t launch_attn_gate(float *out, const float *gate, uint64_t count, hipSt
     if (count == 0) return hipSuccess;
     uint64_t blocks = (count + 255) / 256;
     if (blocks > 4096) blocks = 4096;
-    attn_gate_kernel<<<uint32_t(blocks), 256, 0, stream>>>(out, gate, count);
+    launch_kernel(attn_gate_kernel, uint32_t(blocks), 256, 0, stream, out, gate, count);
     return hipGetLastError();
 }
 

@@ -244,10 +244,10 @@ hipError_t launch_attn_splitk_f16(const AttnParams &p, const AttnBatch &b, uint3
         hipError_t e = grant_lds<NQ, W>(lds);                                             \
         if (e != hipSuccess) return e;                                                    \
         if (p.ring_blocks)                                                                \
-            attn_splitk_f16_kernel<NQ, W, N, true><<<b.total_blocks, W * 64, lds, stream>>>(  \
+            launch_kernel(attn_splitk_f16_kernel<NQ, W, N, true>, b.total_blocks, W * 64, lds, stream, \
                 p, AttnBatchT<N>(b), total_partials);                                     \
         else                                                                              \
-            attn_splitk_f16_kernel<NQ, W, N, false><<<b.total_blocks, W * 64, lds, stream>>>( \
+            launch_kernel(attn_splitk_f16_kernel<NQ, W, N, false>, b.total_blocks, W * 64, lds, stream, \
                 p, AttnBatchT<N>(b), total_partials);                                     \
     } while (0)
 #define ITAK_LAUNCH_PREP(NQ, W)                                                           \
@@ -256,12 +256,10 @@ hipError_t launch_attn_splitk_f16(const AttnParams &p, const AttnBatch &b, uint3
         hipError_t e = grant_lds<NQ, W, true>(lds);                                       \
         if (e != hipSuccess) return e;                                                    \
         if (p.ring_blocks)                                                                \
-            attn_splitk_f16_prep_kernel<NQ, W, N, true>                                   \
-                <<<b.total_blocks, W * 64, lds, stream>>>(p, AttnBatchT<N>(b), total_partials, \
+            launch_kernel(attn_splitk_f16_prep_kernel<NQ, W, N, true>, b.total_blocks, W * 64, lds, stream, p, AttnBatchT<N>(b), total_partials, \
                                                           *folded);                       \
         else                                                                              \
-            attn_splitk_f16_prep_kernel<NQ, W, N, false>                                  \
-                <<<b.total_blocks, W * 64, lds, stream>>>(p, AttnBatchT<N>(b), total_partials, \
+            launch_kernel(attn_splitk_f16_prep_kernel<NQ, W, N, false>, b.total_blocks, W * 64, lds, stream, p, AttnBatchT<N>(b), total_partials, \
                                                           *folded);                       \
     } while (0)
 #define ITAK_LAUNCH_NQ()                                  \
@@ -651,33 +649,25 @@ hipError_t launch_attn_combine(const AttnParams &p, const AttnBatch &b, uint32_t
     if (p.g.head_dim == 128 && most_splits <= 16 && uint64_t(total_rows) * p.q_heads >= 128) {
         const dim3 grid((p.q_heads + 3) / 4, total_rows);
         if (gate && base2)
-            ITAK_DISPATCH_BATCH(b.n, (attn_combine128_wave_kernel<N, true, true><<<grid, 256, 0, stream>>>(
-                                         p, AttnBatchT<N>(b), total_partials, gate)));
+            ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine128_wave_kernel<N, true, true>, grid, 256, 0, stream, p, AttnBatchT<N>(b), total_partials, gate)));
         else if (gate)
-            ITAK_DISPATCH_BATCH(b.n, (attn_combine128_wave_kernel<N, false, true><<<grid, 256, 0, stream>>>(
-                                         p, AttnBatchT<N>(b), total_partials, gate)));
+            ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine128_wave_kernel<N, false, true>, grid, 256, 0, stream, p, AttnBatchT<N>(b), total_partials, gate)));
         else if (base2)
-            ITAK_DISPATCH_BATCH(b.n, (attn_combine128_wave_kernel<N, true, false><<<grid, 256, 0, stream>>>(
-                                         p, AttnBatchT<N>(b), total_partials, nullptr)));
+            ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine128_wave_kernel<N, true, false>, grid, 256, 0, stream, p, AttnBatchT<N>(b), total_partials, nullptr)));
         else
-            ITAK_DISPATCH_BATCH(b.n, (attn_combine128_wave_kernel<N, false, false><<<grid, 256, 0, stream>>>(
-                                         p, AttnBatchT<N>(b), total_partials, nullptr)));
+            ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine128_wave_kernel<N, false, false>, grid, 256, 0, stream, p, AttnBatchT<N>(b), total_partials, nullptr)));
         return hipGetLastError();
     }
     if (p.g.head_dim == 128) {
         const dim3 grid(p.q_heads, total_rows);
         if (gate && base2)
-            ITAK_DISPATCH_BATCH(b.n, (attn_combine128_gate_kernel<N, true><<<grid, 256, 0, stream>>>(
-                                         p, AttnBatchT<N>(b), total_partials, gate)));
+            ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine128_gate_kernel<N, true>, grid, 256, 0, stream, p, AttnBatchT<N>(b), total_partials, gate)));
         else if (gate)
-            ITAK_DISPATCH_BATCH(b.n, (attn_combine128_gate_kernel<N, false><<<grid, 256, 0, stream>>>(
-                                         p, AttnBatchT<N>(b), total_partials, gate)));
+            ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine128_gate_kernel<N, false>, grid, 256, 0, stream, p, AttnBatchT<N>(b), total_partials, gate)));
         else if (base2)
-            ITAK_DISPATCH_BATCH(b.n, (attn_combine128_kernel<N, true><<<grid, 256, 0, stream>>>(
-                                         p, AttnBatchT<N>(b), total_partials)));
+            ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine128_kernel<N, true>, grid, 256, 0, stream, p, AttnBatchT<N>(b), total_partials)));
         else
-            ITAK_DISPATCH_BATCH(b.n, (attn_combine128_kernel<N, false><<<grid, 256, 0, stream>>>(
-                                         p, AttnBatchT<N>(b), total_partials)));
+            ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine128_kernel<N, false>, grid, 256, 0, stream, p, AttnBatchT<N>(b), total_partials)));
         return hipGetLastError();
     }
     // (A workgroup per output pays where the merge is a matter of latency; with thousands of
@@ -686,7 +676,7 @@ hipError_t launch_attn_combine(const AttnParams &p, const AttnBatch &b, uint32_t
         uint64_t(total_rows) * p.q_heads <= 4096) {
         const dim3 grid(p.q_heads, total_rows);
 #define ITAK_LANES(B2, G, D)                                                                  \
-    ITAK_DISPATCH_BATCH(b.n, (attn_combine_lanes_kernel<N, B2, G, D><<<grid, 256, 0, stream>>>( \
+    ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine_lanes_kernel<N, B2, G, D>, grid, 256, 0, stream, \
                                  p, AttnBatchT<N>(b), total_partials, gate)))
 #define ITAK_LANES_D(D)                                \
     do {                                               \
@@ -708,7 +698,7 @@ hipError_t launch_attn_combine(const AttnParams &p, const AttnBatch &b, uint32_t
     if (base2 && p.g.head_dim % 4 == 0 && uint64_t(total_rows) * p.q_heads <= 4096) {
         const dim3 grid(p.q_heads, total_rows);
 #define ITAK_LANES_ANY(G, CL)                                                                        \
-    ITAK_DISPATCH_BATCH(b.n, (attn_combine_lanes_kernel<N, true, G, 0, CL><<<grid, 256, 0, stream>>>( \
+    ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine_lanes_kernel<N, true, G, 0, CL>, grid, 256, 0, stream, \
                                  p, AttnBatchT<N>(b), total_partials, gate)))
 #define ITAK_LANES_CL(CL)                     \
     do {                                      \
@@ -722,8 +712,8 @@ hipError_t launch_attn_combine(const AttnParams &p, const AttnBatch &b, uint32_t
 #undef ITAK_LANES_ANY
         return hipGetLastError();
     }
-    ITAK_DISPATCH_BATCH(b.n, (attn_combine_kernel<N><<<total_rows * p.q_heads, kCombineThreads, 0,
-                                                      stream>>>(p, AttnBatchT<N>(b), total_partials,
+    ITAK_DISPATCH_BATCH(b.n, (launch_kernel(attn_combine_kernel<N>, total_rows * p.q_heads, kCombineThreads, 0,
+                                                      stream, p, AttnBatchT<N>(b), total_partials,
                                                                 base2, gate)));
     return hipGetLastError();
 }

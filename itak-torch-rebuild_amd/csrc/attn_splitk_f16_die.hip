@@ -135,7 +135,7 @@ bool die_layout_ok(int device) {
     bool ok = true;
     std::vector<uint32_t> host(kMost);
     for (uint32_t grid : {8u, 136u, uint32_t(cus), 1000u, kMost}) {
-        die_probe_kernel<<<grid, 64, 0, nullptr>>>(ids);
+        launch_kernel(die_probe_kernel, grid, 64, 0, nullptr, ids);
         if (hipStreamSynchronize(nullptr) != hipSuccess ||
             hipMemcpy(host.data(), ids, grid * sizeof(uint32_t), hipMemcpyDeviceToHost) != hipSuccess) {
             (void)hipGetLastError();
@@ -265,16 +265,16 @@ hipError_t launch_attn_splitk_f16_die(const AttnParams &p, const AttnBatch &b, c
         hipError_t e = grant_die_lds<NQ, W>(lds);                                                 \
         if (e != hipSuccess) return e;                                                            \
         if (prep && p.ring_blocks)                                                                \
-            attn_splitk_f16_die_prep_kernel<NQ, W, N, true><<<b.total_blocks, W * 64, lds, stream>>>( \
+            launch_kernel(attn_splitk_f16_die_prep_kernel<NQ, W, N, true>, b.total_blocks, W * 64, lds, stream, \
                 p, map, AttnBatchT<N>(b), total_partials, *folded);                               \
         else if (prep)                                                                            \
-            attn_splitk_f16_die_prep_kernel<NQ, W, N, false><<<b.total_blocks, W * 64, lds, stream>>>( \
+            launch_kernel(attn_splitk_f16_die_prep_kernel<NQ, W, N, false>, b.total_blocks, W * 64, lds, stream, \
                 p, map, AttnBatchT<N>(b), total_partials, *folded);                               \
         else if (p.ring_blocks)                                                                   \
-            attn_splitk_f16_die_kernel<NQ, W, N, true><<<b.total_blocks, W * 64, lds, stream>>>(  \
+            launch_kernel(attn_splitk_f16_die_kernel<NQ, W, N, true>, b.total_blocks, W * 64, lds, stream, \
                 p, map, AttnBatchT<N>(b), total_partials);                                        \
         else                                                                                      \
-            attn_splitk_f16_die_kernel<NQ, W, N, false><<<b.total_blocks, W * 64, lds, stream>>>( \
+            launch_kernel(attn_splitk_f16_die_kernel<NQ, W, N, false>, b.total_blocks, W * 64, lds, stream, \
                 p, map, AttnBatchT<N>(b), total_partials);                                        \
     } while (0)
 #define ITAK_LAUNCH_NQ()                      \

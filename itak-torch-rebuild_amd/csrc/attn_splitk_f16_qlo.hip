@@ -55,16 +55,16 @@ hipError_t launch_attn_splitk_f16_qlo(const AttnParams &p, const AttnBatch &b, u
         hipError_t e = grant_qlo_lds<NQ, W>(lds);                                                  \
         if (e != hipSuccess) return e;                                                             \
         if (prep && p.ring_blocks)                                                                 \
-            attn_splitk_f16_qlo_prep_kernel<NQ, W, N, true><<<b.total_blocks, W * 64, lds, stream>>>(  \
+            launch_kernel(attn_splitk_f16_qlo_prep_kernel<NQ, W, N, true>, b.total_blocks, W * 64, lds, stream, \
                 p, AttnBatchT<N>(b), total_partials, *folded);                                     \
         else if (prep)                                                                             \
-            attn_splitk_f16_qlo_prep_kernel<NQ, W, N, false><<<b.total_blocks, W * 64, lds, stream>>>( \
+            launch_kernel(attn_splitk_f16_qlo_prep_kernel<NQ, W, N, false>, b.total_blocks, W * 64, lds, stream, \
                 p, AttnBatchT<N>(b), total_partials, *folded);                                     \
         else if (p.ring_blocks)                                                                    \
-            attn_splitk_f16_qlo_kernel<NQ, W, N, true><<<b.total_blocks, W * 64, lds, stream>>>(   \
+            launch_kernel(attn_splitk_f16_qlo_kernel<NQ, W, N, true>, b.total_blocks, W * 64, lds, stream, \
                 p, AttnBatchT<N>(b), total_partials);                                              \
         else                                                                                       \
-            attn_splitk_f16_qlo_kernel<NQ, W, N, false><<<b.total_blocks, W * 64, lds, stream>>>(  \
+            launch_kernel(attn_splitk_f16_qlo_kernel<NQ, W, N, false>, b.total_blocks, W * 64, lds, stream, \
                 p, AttnBatchT<N>(b), total_partials);                                              \
     } while (0)
 #define ITAK_LAUNCH_NQ()                      \

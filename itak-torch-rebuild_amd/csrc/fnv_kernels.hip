@@ -210,11 +210,11 @@ hipError_t launch_fnv(const void *data, uint64_t bytes, void *scratch, unsigned 
     uint8_t *group_start = group_carry + groups;
     const unsigned char *b = static_cast<const unsigned char *>(data);
     for (uint32_t pair = 0; pair < 4; ++pair) {
-        fnv_round<<<groups, kThreads, 0, stream>>>(b, runs, pair, run_state, group_start, group_carry);
-        fnv_groups<<<1, kThreads, 0, stream>>>(groups, pair, group_carry, group_start, state);
+        launch_kernel(fnv_round, groups, kThreads, 0, stream, b, runs, pair, run_state, group_start, group_carry);
+        launch_kernel(fnv_groups, 1, kThreads, 0, stream, groups, pair, group_carry, group_start, state);
     }
-    fnv_walk<<<groups, kThreads, 0, stream>>>(b, runs, run_state, group_start, powers, group_sum);
-    fnv_join<<<1, kThreads, 0, stream>>>(runs, groups, powers, group_sum, state);
+    launch_kernel(fnv_walk, groups, kThreads, 0, stream, b, runs, run_state, group_start, powers, group_sum);
+    launch_kernel(fnv_join, 1, kThreads, 0, stream, runs, groups, powers, group_sum, state);
     return hipGetLastError();
 }
 

@@ -8,6 +8,28 @@
 
 namespace itak {
 
+// A kernel launch without the triple-chevron form's detour (the configuration pushed to and popped
+// from the runtime's per-thread stack): 1.95 us of host time instead of 2.45. Errors are the
+// runtime's last error, as after that form.
+template <typename... P>
+inline void launch_kernel_args(void (*kernel)(P...), dim3 grid, dim3 block, uint32_t lds, hipStream_t stream,
+                               const P &...args) {
+    void *at[] = {const_cast<void *>(static_cast<const void *>(&args))...};
+    (void)hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, at, lds, stream);
+}
+template <typename... P, typename... A>
+inline void launch_kernel(void (*kernel)(P...), dim3 grid, dim3 block, uint32_t lds, hipStream_t stream, const A &...args) {
+    static_assert(sizeof...(P) == sizeof...(A), "one argument per parameter");
+    launch_kernel_args<P...>(kernel, grid, block, lds, stream, static_cast<const P &>(args)...);
+}
+// A kernel without parameters.
+inline void launch_kernel(void (*kernel)(), dim3 grid, dim3 block, uint32_t lds, hipStream_t stream) {
+    (void)hipLaunchKernel(reinterpret_cast<const void *>(kernel), grid, block, nullptr, lds, stream);
+}
+
+// Compute units of the current device, asked of the runtime once per device.
+uint32_t compute_units();
+
 // Device layout of the KV pool, in elements of the storage type. One "plane" is the
 // rows of one (layer, slot, side, kv_head): capacity x head_dim elements, contiguous,
 // so a workgroup that streams one KV head reads one unbroken run of memory.

@@ -6,8 +6,26 @@
 #include "internal.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace itak {
+
+uint32_t compute_units() {
+    static std::atomic<uint32_t> known[64];
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    uint32_t n = known[dev].load(std::memory_order_relaxed);
+    if (n) return n;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) {
+        (void)hipGetLastError();
+        return 256;
+    }
+    known[dev].store(uint32_t(cus), std::memory_order_relaxed);
+    return uint32_t(cus);
+}
 
 __device__ __forceinline__ void store4(float *dst, const float4 &v) {
     *reinterpret_cast<float4 *>(dst) = v;
@@ -78,15 +96,15 @@ hipError_t launch_append(void *layer_base, int elem_f16, const PoolGeom &g, cons
     if (elem_f16) {
         auto *base = static_cast<uint16_t *>(layer_base);
         if (vec)
-            kv_append_kernel<uint16_t, 4><<<blocks, 256, 0, stream>>>(base, g, b, k_src, v_src);
+            launch_kernel(kv_append_kernel<uint16_t, 4>, blocks, 256, 0, stream, base, g, b, k_src, v_src);
         else
-            kv_append_kernel<uint16_t, 1><<<blocks, 256, 0, stream>>>(base, g, b, k_src, v_src);
+            launch_kernel(kv_append_kernel<uint16_t, 1>, blocks, 256, 0, stream, base, g, b, k_src, v_src);
     } else {
         auto *base = static_cast<float *>(layer_base);
         if (vec)
-            kv_append_kernel<float, 4><<<blocks, 256, 0, stream>>>(base, g, b, k_src, v_src);
+            launch_kernel(kv_append_kernel<float, 4>, blocks, 256, 0, stream, base, g, b, k_src, v_src);
         else
-            kv_append_kernel<float, 1><<<blocks, 256, 0, stream>>>(base, g, b, k_src, v_src);
+            launch_kernel(kv_append_kernel<float, 1>, blocks, 256, 0, stream, base, g, b, k_src, v_src);
     }
     return hipGetLastError();
 }
@@ -131,10 +149,10 @@ hipError_t launch_zero_rows(void *pool_base, int elem_f16, const PoolGeom &g, ui
         const uint32_t n = (layer_to - l < layers_per_launch) ? layer_to - l : layers_per_launch;
         dim3 grid(bx, b.n, n * planes_per_layer);
         if (elem_f16)
-            kv_zero_rows<uint16_t><<<grid, 256, 0, stream>>>(static_cast<uint16_t *>(pool_base), g,
+            launch_kernel(kv_zero_rows<uint16_t>, grid, 256, 0, stream, static_cast<uint16_t *>(pool_base), g,
                                                              l, b);
         else
-            kv_zero_rows<float><<<grid, 256, 0, stream>>>(static_cast<float *>(pool_base), g, l, b);
+            launch_kernel(kv_zero_rows<float>, grid, 256, 0, stream, static_cast<float *>(pool_base), g, l, b);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -286,14 +304,11 @@ hipError_t launch_restore(void *pool_base, int dst_f16, int src_f16, const PoolG
         if (bx > 2048) bx = 2048;
         dim3 grid(bx, 2, b.n);
         if (src_f16)
-            kv_restore_scalar<uint16_t, uint16_t><<<grid, 256, 0, stream>>>(
-                static_cast<uint16_t *>(pool_base), g, b);
+            launch_kernel(kv_restore_scalar<uint16_t, uint16_t>, grid, 256, 0, stream, static_cast<uint16_t *>(pool_base), g, b);
         else if (dst_f16)
-            kv_restore_scalar<float, uint16_t><<<grid, 256, 0, stream>>>(
-                static_cast<uint16_t *>(pool_base), g, b);
+            launch_kernel(kv_restore_scalar<float, uint16_t>, grid, 256, 0, stream, static_cast<uint16_t *>(pool_base), g, b);
         else
-            kv_restore_scalar<float, float><<<grid, 256, 0, stream>>>(
-                static_cast<float *>(pool_base), g, b);
+            launch_kernel(kv_restore_scalar<float, float>, grid, 256, 0, stream, static_cast<float *>(pool_base), g, b);
         return hipGetLastError();
     }
     if (g.v_block != 0) {  // blocked planes: keys and values of a block in one workgroup
@@ -303,13 +318,13 @@ hipError_t launch_restore(void *pool_base, int dst_f16, int src_f16, const PoolG
         const size_t lds = size_t(2) * kVBlock * (g.head_dim + 8) * sizeof(uint16_t);
         uint16_t *base = static_cast<uint16_t *>(pool_base);
         if (g.head_dim == 128 && src_f16)
-            kv_restore_blocked<uint16_t, 128><<<grid, 256, lds, stream>>>(base, g, b);
+            launch_kernel(kv_restore_blocked<uint16_t, 128>, grid, 256, lds, stream, base, g, b);
         else if (g.head_dim == 128)
-            kv_restore_blocked<float, 128><<<grid, 256, lds, stream>>>(base, g, b);
+            launch_kernel(kv_restore_blocked<float, 128>, grid, 256, lds, stream, base, g, b);
         else if (src_f16)
-            kv_restore_blocked<uint16_t, 0><<<grid, 256, lds, stream>>>(base, g, b);
+            launch_kernel(kv_restore_blocked<uint16_t, 0>, grid, 256, lds, stream, base, g, b);
         else
-            kv_restore_blocked<float, 0><<<grid, 256, lds, stream>>>(base, g, b);
+            launch_kernel(kv_restore_blocked<float, 0>, grid, 256, lds, stream, base, g, b);
         return hipGetLastError();
     }
     const uint64_t per_layer = uint64_t(b.max_rows) * g.kv_heads * (g.head_dim / vec);
@@ -317,13 +332,11 @@ hipError_t launch_restore(void *pool_base, int dst_f16, int src_f16, const PoolG
     if (bx > 2048) bx = 2048;
     dim3 grid(bx, 2, b.n);
     if (src_f16)
-        kv_restore_rows<uint16_t, uint16_t><<<grid, 256, 0, stream>>>(
-            static_cast<uint16_t *>(pool_base), g, b, 0);
+        launch_kernel(kv_restore_rows<uint16_t, uint16_t>, grid, 256, 0, stream, static_cast<uint16_t *>(pool_base), g, b, 0);
     else if (dst_f16)
-        kv_restore_rows<float, uint16_t><<<grid, 256, 0, stream>>>(
-            static_cast<uint16_t *>(pool_base), g, b, 0);
+        launch_kernel(kv_restore_rows<float, uint16_t>, grid, 256, 0, stream, static_cast<uint16_t *>(pool_base), g, b, 0);
     else
-        kv_restore_rows<float, float><<<grid, 256, 0, stream>>>(static_cast<float *>(pool_base), g,
+        launch_kernel(kv_restore_rows<float, float>, grid, 256, 0, stream, static_cast<float *>(pool_base), g,
                                                                b, 0);
     return hipGetLastError();
 }
@@ -406,10 +419,10 @@ hipError_t launch_read_runs(const void *base, const void *base_w, int elem_f16, 
 #define ITAK_RUNS(T, OUT)                                                                                  \
     do {                                                                                                   \
         if (by_eight)                                                                                      \
-            kv_read_runs<T, OUT, 8><<<grid, 256, 0, stream>>>(static_cast<const T *>(base),                \
+            launch_kernel(kv_read_runs<T, OUT, 8>, grid, 256, 0, stream, static_cast<const T *>(base),                \
                 static_cast<const T *>(base_w), g, gw, b, static_cast<OUT *>(out));                        \
         else                                                                                               \
-            kv_read_runs<T, OUT, 1><<<grid, 256, 0, stream>>>(static_cast<const T *>(base),                \
+            launch_kernel(kv_read_runs<T, OUT, 1>, grid, 256, 0, stream, static_cast<const T *>(base),                \
                 static_cast<const T *>(base_w), g, gw, b, static_cast<OUT *>(out));                        \
     } while (0)
     if (!elem_f16)
@@ -455,7 +468,7 @@ hipError_t launch_ring_rows(void *pool_base_w, int elem_f16, const PoolGeom &gw,
     if (bx > 1024) bx = 1024;
     dim3 grid(bx, 2, b.n);
 #define ITAK_RING_ROWS(T, TO)                                                                  \
-    kv_ring_rows_kernel<T, TO><<<grid, 256, 0, stream>>>(static_cast<T *>(pool_base_w), gw, b, \
+    launch_kernel(kv_ring_rows_kernel<T, TO>, grid, 256, 0, stream, static_cast<T *>(pool_base_w), gw, b, \
                                                          static_cast<T *>(saved))
     if (elem_f16) {
         if (to_ring) ITAK_RING_ROWS(uint16_t, true); else ITAK_RING_ROWS(uint16_t, false);
@@ -475,12 +488,10 @@ hipError_t launch_read_rows(const void *layer_base, int elem_f16, const PoolGeom
     if (bx > 4096) bx = 4096;
     dim3 grid(bx, 2, 1);
     if (elem_f16) {
-        kv_read_rows<uint16_t><<<grid, 256, 0, stream>>>(
-            static_cast<const uint16_t *>(layer_base), g, slot, first_row, rows, ring,
+        launch_kernel(kv_read_rows<uint16_t>, grid, 256, 0, stream, static_cast<const uint16_t *>(layer_base), g, slot, first_row, rows, ring,
             static_cast<uint16_t *>(keys_out), static_cast<uint16_t *>(values_out));
     } else {
-        kv_read_rows<float><<<grid, 256, 0, stream>>>(
-            static_cast<const float *>(layer_base), g, slot, first_row, rows, ring,
+        launch_kernel(kv_read_rows<float>, grid, 256, 0, stream, static_cast<const float *>(layer_base), g, slot, first_row, rows, ring,
             static_cast<float *>(keys_out), static_cast<float *>(values_out));
     }
     return hipGetLastError();
@@ -498,7 +509,7 @@ hipError_t launch_convert_f16(const float *src, uint16_t *dst, uint64_t count, h
     if (count == 0) return hipSuccess;
     uint64_t blocks = (count + 255) / 256;
     if (blocks > 65536) blocks = 65536;
-    convert_f32_to_f16<<<uint32_t(blocks), 256, 0, stream>>>(src, dst, count);
+    launch_kernel(convert_f32_to_f16, uint32_t(blocks), 256, 0, stream, src, dst, count);
     return hipGetLastError();
 }
 
@@ -521,12 +532,12 @@ __global__ void signal_done_kernel(uint32_t *pinned_word, uint32_t value) {
 hipError_t launch_stage_in(const void *pinned, void *dst, uint64_t bytes, hipStream_t stream) {
     const uint32_t n = uint32_t((bytes + 15) / 16);
     if (n == 0) return hipSuccess;
-    stage_in_kernel<<<(n + 255) / 256, 256, 0, stream>>>(static_cast<const uint4 *>(pinned),
+    launch_kernel(stage_in_kernel, (n + 255) / 256, 256, 0, stream, static_cast<const uint4 *>(pinned),
                                                          static_cast<uint4 *>(dst), n);
     return hipGetLastError();
 }
 hipError_t launch_signal_done(uint32_t *pinned_word, uint32_t value, hipStream_t stream) {
-    signal_done_kernel<<<1, 64, 0, stream>>>(pinned_word, value);
+    launch_kernel(signal_done_kernel, 1, 64, 0, stream, pinned_word, value);
     return hipGetLastError();
 }
 
@@ -543,7 +554,7 @@ hipError_t launch_fill_words(unsigned long long *dst, uint64_t count, unsigned l
     if (count == 0) return hipSuccess;
     uint64_t blocks = (count + 255) / 256;
     if (blocks > 4096) blocks = 4096;
-    fill_words_kernel<<<uint32_t(blocks), 256, 0, stream>>>(dst, count, value);
+    launch_kernel(fill_words_kernel, uint32_t(blocks), 256, 0, stream, dst, count, value);
     return hipGetLastError();
 }
 
@@ -586,7 +597,7 @@ hipError_t launch_probe_copy(const void *src, void *dst, uint64_t bytes, hipStre
     if (n == 0) return hipSuccess;
     uint64_t blocks = (n + 255) / 256;
     if (blocks > 16384) blocks = 16384;
-    probe_copy_kernel<<<uint32_t(blocks), 256, 0, stream>>>(static_cast<const uint4 *>(src),
+    launch_kernel(probe_copy_kernel, uint32_t(blocks), 256, 0, stream, static_cast<const uint4 *>(src),
                                                             static_cast<uint4 *>(dst), n);
     return hipGetLastError();
 }
@@ -596,12 +607,12 @@ hipError_t launch_probe_read(const void *src, uint64_t bytes, hipStream_t stream
     if (n == 0) return hipSuccess;
     uint64_t blocks = (n + 1023) / 1024;
     if (blocks > 8192) blocks = 8192;
-    probe_read_kernel<<<uint32_t(blocks), 256, 0, stream>>>(static_cast<const probe_u32x4 *>(src), n, nullptr);
+    launch_kernel(probe_read_kernel, uint32_t(blocks), 256, 0, stream, static_cast<const probe_u32x4 *>(src), n, nullptr);
     return hipGetLastError();
 }
 
 hipError_t launch_probe_empty(hipStream_t stream) {
-    probe_empty_kernel<<<1, 64, 0, stream>>>(nullptr);
+    launch_kernel(probe_empty_kernel, 1, 64, 0, stream, nullptr);
     return hipGetLastError();
 }
 
@@ -662,9 +673,9 @@ hipError_t launch_probe_mfma(bool random_operands, uint32_t iters, unsigned long
     const uint32_t grid = 2u * uint32_t(cus > 0 ? cus : 256);
     if (workgroups) *workgroups = grid;
     if (random_operands)
-        probe_mfma_kernel<true><<<grid, 256, 0, stream>>>(iters, clocks, nullptr);
+        launch_kernel(probe_mfma_kernel<true>, grid, 256, 0, stream, iters, clocks, nullptr);
     else
-        probe_mfma_kernel<false><<<grid, 256, 0, stream>>>(iters, clocks, nullptr);
+        launch_kernel(probe_mfma_kernel<false>, grid, 256, 0, stream, iters, clocks, nullptr);
     return hipGetLastError();
 }
 

@@ -112,6 +112,15 @@ struct RopeFreqTable {
     double *dev;
 };
 
+// One item's query rows against its slot; fills the split plan.
+struct PlanInput {
+    uint32_t slot;
+    uint32_t rows;
+    uint32_t pos0;
+    uint32_t kv_len;
+    uint32_t kv_lo;  // oldest position the item's queries may see
+};
+
 struct itak_pool {
     itak_pool_config cfg{};
     std::vector<RopeFreqTable> rope_tables;
@@ -170,9 +179,14 @@ struct itak_pool {
     // Pinned host memory for the host-pointer attention call: its small inputs are packed here
     // and go up in one copy; its kernels write the output here directly.
     unsigned char *hstage = nullptr;
+    unsigned char *hstage_dev = nullptr;  // the device's address of it
     uint64_t hstage_bytes = 0;
     // Pinned slots through which snapshot rows move between ordinary host memory and the device.
     HostRing ring;
+    // Plan of the step in progress, and the slots it has named (by the number of the step).
+    std::vector<PlanInput> plan, active;
+    std::vector<uint64_t> named;
+    uint64_t step_number = 0;
     uint32_t call_number = 0;  // what the last host-pointer call asked to be told when done
     mutable ErrorState err;
 };
@@ -448,11 +462,108 @@ itak_status ensure_hstage(itak_pool *pool, uint64_t bytes) {
     HIP_TRY(pool, hipHostMalloc(reinterpret_cast<void **>(&pool->hstage), want, hipHostMallocDefault),
             "allocate pinned staging");
     memset(pool->hstage, 0, want);  // the completion word of a call must not start out matching
+    void *mapped = nullptr;
+    HIP_TRY(pool, hipHostGetDevicePointer(&mapped, pool->hstage, 0), "map pinned staging");
+    pool->hstage_dev = static_cast<unsigned char *>(mapped);
     pool->hstage_bytes = want;
     return ITAK_OK;
 }
 
 uint64_t align_up(uint64_t x, uint64_t a) { return (x + a - 1) / a * a; }
+
+// ---- host-pointer attention calls ------------------------------------------------------
+// Such a call is dominated by its trips over the host link and by its launches, not by its
+// kernels. Its inputs are packed into pinned memory and read from there by the device, its output
+// is written into pinned memory by whichever kernel makes it, and the host watches for it there:
+// finding out from the runtime that a stream has drained costs several microseconds more.
+// Calls that move more than kHostPacked copy their arrays as they lie.
+constexpr uint64_t kHostPacked = 4ull << 20;
+// Up to here the host watches the output itself: every word of it is set beforehand to a pattern
+// that no arithmetic makes, and the output is there when the pattern is gone. (A NaN that came in
+// with a caller's row could carry it: such a call ends on the runtime's word.) Larger outputs are
+// announced by a one-thread launch; 2.4 us of host time and a launch behind the merge.
+constexpr uint64_t kHostWatched = 64ull << 10;
+constexpr uint32_t kNotYet = 0xffffa5c3u;
+// Inputs up to this size go up by a launch that reads them over the link (a copy-engine command
+// costs 7 us at 20 KB, the launch 3); above it the copy engine's rate wins.
+constexpr uint64_t kHostByLaunch = 256ull << 10;
+
+struct HostCall {
+    unsigned char *in = nullptr;       // where the host packs the inputs
+    unsigned char *in_dev = nullptr;   // the same memory as the device sees it
+    float *out_dev = nullptr;          // the output's place as the device sees it
+    uint64_t out_at = 0;               // and its offset in the pinned staging
+    uint64_t out_count = 0;            // floats
+};
+
+itak_status begin_host_call(itak_pool *pool, uint64_t in_bytes, uint64_t out_count, HostCall &c) {
+    // Layout: [completion word, 256 bytes] [inputs] [output]. The word sits at a fixed place, so it
+    // only ever holds call numbers, which only grow.
+    const uint64_t in_room = align_up(in_bytes, 256);
+    itak_status st = ensure_hstage(pool, kHostWord + in_room + out_count * 4);
+    if (st != ITAK_OK) return st;
+    c.in = pool->hstage + kHostWord;
+    c.in_dev = pool->hstage_dev + kHostWord;
+    c.out_at = kHostWord + in_room;
+    c.out_dev = reinterpret_cast<float *>(pool->hstage_dev + c.out_at);
+    c.out_count = out_count;
+    if (out_count * 4 <= kHostWatched)
+        std::fill_n(reinterpret_cast<uint32_t *>(pool->hstage + c.out_at), out_count, kNotYet);
+    return ITAK_OK;
+}
+
+// Everything of the call is on the stream: its output to `out`.
+itak_status finish_host_call(itak_pool *pool, const HostCall &c, float *out) {
+    const bool watched = c.out_count * 4 <= kHostWatched;
+    const uint32_t number = ++pool->call_number ? pool->call_number : ++pool->call_number;
+    if (!watched)
+        HIP_TRY(pool, launch_signal_done(reinterpret_cast<uint32_t *>(pool->hstage_dev), number, pool->stream),
+                "launch completion signal");
+    const unsigned char *from = pool->hstage + c.out_at;
+    unsigned char *to = reinterpret_cast<unsigned char *>(out);
+    const uint64_t bytes = c.out_count * 4;
+    timespec t0{};
+    clock_gettime(CLOCK_MONOTONIC, &t0);
+    // The host looks for 0.3 ms before it asks the runtime (which also reports a failed launch, and
+    // is what a call that takes longer falls back to).
+    auto look_until = [&](auto ready) {
+        for (uint32_t spin = 0;; ++spin) {
+            if (ready()) return true;
+            __builtin_ia32_pause();
+            if ((spin & 63u) != 63u) continue;
+            timespec t1{};
+            clock_gettime(CLOCK_MONOTONIC, &t1);
+            if ((t1.tv_sec - t0.tv_sec) * 1000000000ll + (t1.tv_nsec - t0.tv_nsec) > 300000) return false;
+        }
+    };
+    if (!watched) {
+        const volatile uint32_t *seen = reinterpret_cast<const volatile uint32_t *>(pool->hstage);
+        if (!look_until([&] { return __atomic_load_n(seen, __ATOMIC_ACQUIRE) == number; }))
+            HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after attention");
+        memcpy(out, from, bytes);
+        return ITAK_OK;
+    }
+    // A piece is copied first and looked at in the copy, so that what was looked at is what the
+    // caller gets.
+    for (uint64_t at = 0; at < bytes;) {
+        const uint64_t n = std::min<uint64_t>(512, bytes - at);
+        const bool arrived = look_until([&] {
+            asm volatile("" ::: "memory");
+            memcpy(to + at, from + at, n);
+            const uint32_t *w = reinterpret_cast<const uint32_t *>(to + at);
+            uint32_t missing = 0;
+            for (uint64_t i = 0; i < n / 4; ++i) missing |= w[i] == kNotYet;
+            return missing == 0;
+        });
+        if (!arrived) {
+            HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after attention");
+            memcpy(out, from, bytes);
+            return ITAK_OK;
+        }
+        at += n;
+    }
+    return ITAK_OK;
+}
 
 // The address of this device's copy of `scratch`, looked up on first use with the device
 // current; the exchange part is filled with the empty pattern then (a kernel on the null
@@ -508,15 +619,6 @@ hipError_t scratch_guard_leave(int device, hipStream_t stream) {
 struct WorkspaceNeed {
     uint64_t partial_floats = 0;   // split partials for a merge launch
     uint64_t exchange_words = 0;   // exchange words of launches that merge their own splits
-};
-
-// One item's query rows against its slot; fills the split plan.
-struct PlanInput {
-    uint32_t slot;
-    uint32_t rows;
-    uint32_t pos0;
-    uint32_t kv_len;
-    uint32_t kv_lo;  // oldest position the item's queries may see
 };
 
 // Builds the work list and launches the attention kernels. q/out are device pointers.
@@ -585,13 +687,15 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     uint32_t q_row0 = 0;
     for (uint32_t first = 0; first < n; first += kMaxBatchItems) {
         const uint32_t count = std::min<uint32_t>(kMaxBatchItems, n - first);
-        AttnBatch b{};
+        AttnBatch b;  // (cleared item by item: all 64 are three kilobytes)
         b.n = count;
+        b.total_blocks = b.rows_per_block = b.deep_ring = b.fold_units = 0;
         b.two_halves = prefill && pool->q_two_halves && pool->g.head_dim == 128 ? 1 : 0;
         uint32_t total_rows = 0;
         for (uint32_t i = 0; i < count; ++i) {
             const PlanInput &pi = in[first + i];
             AttnItem &it = b.item[i];
+            it = AttnItem{};
             it.slot = pi.slot;
             it.rows = pi.rows;
             it.pos0 = pi.pos0;
@@ -646,10 +750,12 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             exchange_words = attn_splitk_f16_plan_exchange(geom, b, uint32_t(q_heads));
         // Or on the units' compute dies, when the batch deals out evenly over them and is not
         // one the single-row decode kernel takes.
-        AttnBatch bd{};
-        DieMap dm{};
+        AttnBatch bd;
+        DieMap dm;
         uint32_t die_partials = 0;
         if (mfma && pool->die_merge && !exchange_words && !pool->q_two_halves) {
+            bd = AttnBatch{};
+            dm = DieMap{};
             AttnParams probe{};
             probe.g = geom;
             probe.group = group;
@@ -1490,11 +1596,14 @@ itak_status itak_kv_append_device(itak_pool *pool, uint64_t layer, const itak_ba
     if (layer >= pool->cfg.layer_count) return invalid_layer(pool->err, layer, pool->cfg.layer_count);
     if (item_count && (!items || !k_dev || !v_dev))
         return invalid_argument(pool->err, "items, k_dev or v_dev is null");
-    std::vector<uint8_t> seen(pool->slots.size(), 0);
+    std::vector<uint64_t> &named = pool->named;
+    named.resize(pool->slots.size(), 0);
+    const uint64_t number = ++pool->step_number;
     for (uint32_t i = 0; i < item_count; ++i) {
         Slot *s = find_slot(pool, items[i].slot);
         if (!s) return invalid_argument(pool->err, "slot is not in use");
-        if (seen[items[i].slot]++) return invalid_argument(pool->err, "slot listed twice in one step");
+        if (named[items[i].slot] == number) return invalid_argument(pool->err, "slot listed twice in one step");
+        named[items[i].slot] = number;
         uint64_t ok = 0;
         itak_status st = check_append_rows(pool, *s, layer, items[i].rows, &ok);
         if (st != ITAK_OK) return st;
@@ -2398,31 +2507,44 @@ itak_status itak_gqa_attention(itak_pool *pool, uint32_t slot, uint64_t layer, c
     bool consecutive = true;
     for (uint64_t i = 1; i < num_queries; ++i)
         consecutive = consecutive && query_positions[i] == query_positions[0] + i;
-    const uint64_t q_bytes = q_len * sizeof(float);
-    const uint64_t pos_bytes = align_up(num_queries * sizeof(uint32_t), 256);
-    itak_status st = ensure_stage(pool, 2 * align_up(q_bytes, 256) + pos_bytes);
+    const uint64_t q_bytes = align_up(q_len * sizeof(float), 256);
+    const uint64_t pos_bytes = consecutive ? 0 : align_up(num_queries * sizeof(uint32_t), 256);
+    itak_status st = ensure_stage(pool, 2 * q_bytes + pos_bytes);
     if (st != ITAK_OK) return st;
     float *qd = reinterpret_cast<float *>(pool->stage);
-    float *od = reinterpret_cast<float *>(pool->stage + align_up(q_bytes, 256));
-    uint32_t *pd = reinterpret_cast<uint32_t *>(pool->stage + 2 * align_up(q_bytes, 256));
-    HIP_TRY(pool, hipMemcpyAsync(qd, q, q_bytes, hipMemcpyHostToDevice, pool->stream), "upload q");
+    uint32_t *pd = reinterpret_cast<uint32_t *>(pool->stage + q_bytes);
+    float *od = reinterpret_cast<float *>(pool->stage + q_bytes + pos_bytes);
     std::vector<uint32_t> pos32;
     if (!consecutive) {
         pos32.resize(num_queries);
         for (uint64_t i = 0; i < num_queries; ++i)
             pos32[i] = uint32_t(std::min<uint64_t>(query_positions[i], 0xffffffffu));
-        HIP_TRY(pool,
-                hipMemcpyAsync(pd, pos32.data(), num_queries * 4, hipMemcpyHostToDevice,
-                               pool->stream),
-                "upload query positions");
+    }
+    const bool packed = 2 * q_bytes + pos_bytes <= kHostPacked;
+    HostCall call;
+    if (packed) {
+        st = begin_host_call(pool, q_bytes + pos_bytes, q_len, call);
+        if (st != ITAK_OK) return st;
+        memcpy(call.in, q, q_len * 4);
+        if (!consecutive) memcpy(call.in + q_bytes, pos32.data(), num_queries * 4);
+        if (q_bytes + pos_bytes <= kHostByLaunch)
+            HIP_TRY(pool, launch_stage_in(call.in_dev, qd, q_bytes + pos_bytes, pool->stream), "launch stage-in");
+        else
+            HIP_TRY(pool, hipMemcpyAsync(qd, call.in, q_bytes + pos_bytes, hipMemcpyHostToDevice, pool->stream), "upload q");
+    } else {
+        HIP_TRY(pool, hipMemcpyAsync(qd, q, q_len * 4, hipMemcpyHostToDevice, pool->stream), "upload q");
+        if (!consecutive)
+            HIP_TRY(pool, hipMemcpyAsync(pd, pos32.data(), num_queries * 4, hipMemcpyHostToDevice, pool->stream),
+                    "upload query positions");
     }
     PlanInput pi{slot, uint32_t(num_queries),
                  uint32_t(std::min<uint64_t>(query_positions[0], 0xffffffffu - num_queries)),
                  uint32_t(appended), uint32_t(oldest)};
-    st = run_attention(pool, layer, &pi, 1, qd, od, consecutive ? nullptr : pd, num_q_heads, scale,
+    st = run_attention(pool, layer, &pi, 1, qd, packed ? call.out_dev : od, consecutive ? nullptr : pd, num_q_heads, scale,
                        softcap);
     if (st != ITAK_OK) return st;
-    HIP_TRY(pool, hipMemcpyAsync(out, od, q_bytes, hipMemcpyDeviceToHost, pool->stream),
+    if (packed) return finish_host_call(pool, call, out);
+    HIP_TRY(pool, hipMemcpyAsync(out, od, q_len * 4, hipMemcpyDeviceToHost, pool->stream),
             "download attention output");
     HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after attention");
     return ITAK_OK;
@@ -2438,7 +2560,8 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
                                   bool no_alloc = false) {
     // Rows of zero-row items contribute nothing; q/k/v rows are numbered by walking the
     // items in order, so such items may simply be dropped.
-    std::vector<PlanInput> active;
+    std::vector<PlanInput> &active = pool->active;
+    active.clear();
     for (const PlanInput &p : plan)
         if (p.rows) active.push_back(p);
     uint32_t most_rows = 0;
@@ -2512,12 +2635,15 @@ static itak_status plan_step(itak_pool *pool, uint64_t layer, const itak_batch_i
     if (num_q_heads == 0) return zero_dimension(pool->err, "num_q_heads");
     if (num_q_heads % pool->g.kv_heads != 0)
         return non_divisible(pool->err, num_q_heads, pool->g.kv_heads);
-    std::vector<uint8_t> seen(pool->slots.size(), 0);
+    std::vector<uint64_t> &named = pool->named;
+    named.resize(pool->slots.size(), 0);
+    const uint64_t number = ++pool->step_number;
     plan.clear();
     for (uint32_t i = 0; i < item_count; ++i) {
         Slot *s = find_slot(pool, items[i].slot);
         if (!s) return invalid_argument(pool->err, "slot is not in use");
-        if (seen[items[i].slot]++) return invalid_argument(pool->err, "slot listed twice in one step");
+        if (named[items[i].slot] == number) return invalid_argument(pool->err, "slot listed twice in one step");
+        named[items[i].slot] = number;
         uint64_t ok = 0;
         itak_status st = check_append_rows(pool, *s, layer, items[i].rows, &ok);
         if (st != ITAK_OK) return st;
@@ -2543,7 +2669,7 @@ itak_status itak_attention_step_device(itak_pool *pool, uint64_t layer,
     if (item_count == 0) return ITAK_OK;
     if (!items || !q_dev || !k_dev || !v_dev || !out_dev)
         return invalid_argument(pool->err, "items or a device tensor is null");
-    std::vector<PlanInput> plan;
+    std::vector<PlanInput> &plan = pool->plan;
     itak_status st = plan_step(pool, layer, items, item_count, num_q_heads, plan);
     if (st != ITAK_OK) return st;
     if (std::isnan(scale)) scale = default_scale(pool->g.head_dim);
@@ -2560,7 +2686,7 @@ itak_status itak_attention_step_device_noalloc(itak_pool *pool, uint64_t layer,
     if (item_count == 0) return ITAK_OK;
     if (!items || !q_dev || !k_dev || !v_dev || !out_dev)
         return invalid_argument(pool->err, "items or a device tensor is null");
-    std::vector<PlanInput> plan;
+    std::vector<PlanInput> &plan = pool->plan;
     itak_status st = plan_step(pool, layer, items, item_count, num_q_heads, plan);
     if (st != ITAK_OK) return st;
     if (std::isnan(scale)) scale = default_scale(pool->g.head_dim);
@@ -2605,7 +2731,7 @@ itak_status itak_attention_prep_step_device(itak_pool *pool, uint64_t layer,
     } else if (D % 2 != 0) {
         return unsupported(pool->err, "attention preparation needs an even head_dim");
     }
-    std::vector<PlanInput> plan;
+    std::vector<PlanInput> &plan = pool->plan;
     itak_status st = plan_step(pool, layer, items, item_count, num_q_heads, plan);
     if (st != ITAK_OK) return st;
     uint64_t total_rows = 0;
@@ -2616,7 +2742,8 @@ itak_status itak_attention_prep_step_device(itak_pool *pool, uint64_t layer,
     // Steps the split-K kernel takes (decode, speculative blocks: up to 64 query vectors per KV
     // head) have Q and the new K rows prepared by that kernel and the gate applied by the
     // kernel that writes the output: no launch but the step's own two.
-    std::vector<PlanInput> active;
+    std::vector<PlanInput> &active = pool->active;  // step_on_device fills it again, with the same
+    active.clear();
     for (const PlanInput &p : plan)
         if (p.rows) active.push_back(p);
     const bool splitk = takes_splitk_f16(pool, active.data(), uint32_t(active.size()), num_q_heads,
@@ -2777,34 +2904,33 @@ itak_status itak_compute_attention(itak_pool *pool, uint32_t slot, uint64_t laye
     float *kd = reinterpret_cast<float *>(pool->stage + q_bytes);
     float *vd = reinterpret_cast<float *>(pool->stage + q_bytes + kv_bytes);
     float *od = reinterpret_cast<float *>(pool->stage + q_bytes + 2 * kv_bytes);
-    // A call is dominated by its trips over the host link, not by its kernels. Small inputs
-    // (a decode row, a speculative block) are packed into pinned memory and go up in one copy,
-    // and the kernel that writes the output writes it into pinned memory directly; large ones
-    // (a prefill chunk) are copied as they lie.
+    const float *q_src = qd, *k_src = kd, *v_src = vd;  // where the first kernel that reads them finds them
     const uint64_t in_bytes = q_bytes + 2 * kv_bytes;
-    const bool packed = in_bytes <= (1u << 20);
-    float *out_pinned = nullptr;
-    uint32_t *done_word = nullptr;  // in pinned memory, after the output
+    const bool packed = in_bytes + q_bytes <= kHostPacked;
+    HostCall call;
     if (packed) {
-        // Layout: [completion word, 256 bytes] [q | k | v] [output]. The word sits at a fixed
-        // place, so it only ever holds call numbers, which only grow.
-        st = ensure_hstage(pool, kHostWord + in_bytes + q_bytes);
+        st = begin_host_call(pool, in_bytes, q_len, call);
         if (st != ITAK_OK) return st;
-        unsigned char *hin = pool->hstage + kHostWord;
-        memcpy(hin, q, q_len * 4);
-        memcpy(hin + q_bytes, k, k_len * 4);
-        memcpy(hin + q_bytes + kv_bytes, v, v_len * 4);
-        void *mapped = nullptr;
-        HIP_TRY(pool, hipHostGetDevicePointer(&mapped, pool->hstage, 0), "map pinned staging");
-        unsigned char *pinned_dev = static_cast<unsigned char *>(mapped);
-        if (in_bytes <= (64u << 10))
-            HIP_TRY(pool, launch_stage_in(pinned_dev + kHostWord, qd, in_bytes, pool->stream),
-                    "launch stage-in");
-        else
-            HIP_TRY(pool, hipMemcpyAsync(qd, hin, in_bytes, hipMemcpyHostToDevice, pool->stream),
+        memcpy(call.in, q, q_len * 4);
+        memcpy(call.in + q_bytes, k, k_len * 4);
+        memcpy(call.in + q_bytes + kv_bytes, v, v_len * 4);
+        // Where everything is read once or nearly so, the kernels read it in pinned memory and the
+        // launch that would fetch it goes away: the rotation reads Q and K once, the workgroups that
+        // append the new rows read those, and every split of a KV head's keys its queries (four key
+        // blocks or more a split; 64 KB over the link is what the launch costs).
+        const uint64_t key_blocks = (appended + rows + 31) / 32;
+        const uint64_t q_reads = rotate ? 1 : std::max<uint64_t>((key_blocks + 3) / 4, 1);
+        const bool in_place = q_len * 4 * q_reads + 2 * k_len * 4 <= (64u << 10);
+        if (in_place) {
+            q_src = reinterpret_cast<const float *>(call.in_dev);
+            k_src = reinterpret_cast<const float *>(call.in_dev + q_bytes);
+            v_src = reinterpret_cast<const float *>(call.in_dev + q_bytes + kv_bytes);
+        } else if (in_bytes <= kHostByLaunch) {
+            HIP_TRY(pool, launch_stage_in(call.in_dev, qd, in_bytes, pool->stream), "launch stage-in");
+        } else {
+            HIP_TRY(pool, hipMemcpyAsync(qd, call.in, in_bytes, hipMemcpyHostToDevice, pool->stream),
                     "upload q, k, v");
-        out_pinned = reinterpret_cast<float *>(pinned_dev + kHostWord + in_bytes);
-        done_word = reinterpret_cast<uint32_t *>(pinned_dev);
+        }
     } else {
         HIP_TRY(pool, hipMemcpyAsync(kd, k, k_len * 4, hipMemcpyHostToDevice, pool->stream), "upload k");
         HIP_TRY(pool, hipMemcpyAsync(vd, v, v_len * 4, hipMemcpyHostToDevice, pool->stream), "upload v");
@@ -2816,16 +2942,18 @@ itak_status itak_compute_attention(itak_pool *pool, uint32_t slot, uint64_t laye
     // several blocks.
     const LayerInfo &L = pool->layers[layer];
     const uint64_t block_cap = L.windowed ? L.ring - L.window : std::max<uint64_t>(rows, 1);
-    // The rotation of a sliding-window layer (row i at position appended + i): in place on the
-    // staged rows, by the preparation launch, whose f64 angles, sines and cosines are the
+    // The rotation of a sliding-window layer (row i at position appended + i): by the preparation
+    // launch, whose f64 angles, sines and cosines are the
     // reference's (rope_interleaved.rs:103-114), so that the K rows this call stores are the
     // reference's rounded once. (The split-K kernel can rotate inside its own launch, with the
     // hardware's sine and cosine, within one f16 step of that; the device-resident step uses it,
     // where a launch counts. Here the call already copies its rows in and its output out.)
     auto rotate_block = [&](uint64_t done, uint64_t n, bool with_q) -> itak_status {
         PrepArgs a{};
-        a.q_in = a.q_out = qd + done * q_width;
-        a.k_in = a.k_out = kd + done * pool->row;
+        a.q_in = q_src + done * q_width;
+        a.q_out = qd + done * q_width;
+        a.k_in = k_src + done * pool->row;
+        a.k_out = kd + done * pool->row;
         a.rope_base = rope_freq_base_swa;
         a.rope_freq = rope_freq_table(pool, rope_freq_base_swa, pool->g.head_dim);
         a.interleaved = 1;
@@ -2845,7 +2973,7 @@ itak_status itak_compute_attention(itak_pool *pool, uint32_t slot, uint64_t laye
             const uint64_t n = std::min(block_cap, ok_rows - done);
             if (rotate && (st = rotate_block(done, n, false)) != ITAK_OK) return st;
             itak_batch_item item{slot, uint32_t(n)};
-            st = run_append(pool, layer, &item, 1, kd + done * pool->row, vd + done * pool->row);
+            st = run_append(pool, layer, &item, 1, (rotate ? kd : k_src) + done * pool->row, v_src + done * pool->row);
             if (st != ITAK_OK) return st;
         }
         HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after append");
@@ -2853,7 +2981,7 @@ itak_status itak_compute_attention(itak_pool *pool, uint32_t slot, uint64_t laye
         pool->err.info.code = ITAK_STEP_FAILED;
         return ITAK_STEP_FAILED;
     }
-    float *out_dev = out_pinned ? out_pinned : od;
+    float *out_dev = packed ? call.out_dev : od;
     for (uint64_t done = 0; done < rows; done += block_cap) {
         const uint64_t n = std::min(block_cap, rows - done);
         itak_batch_item item{slot, uint32_t(n)};
@@ -2862,40 +2990,16 @@ itak_status itak_compute_attention(itak_pool *pool, uint32_t slot, uint64_t laye
         std::vector<PlanInput> plan{
             PlanInput{slot, uint32_t(n), uint32_t(base), uint32_t(base + n), uint32_t(lo)}};
         if (rotate && (st = rotate_block(done, n, true)) != ITAK_OK) return st;
-        st = step_on_device(pool, layer, &item, 1, plan, qd + done * q_width, kd + done * pool->row,
-                            vd + done * pool->row, out_dev + done * q_width, num_q_heads,
+        st = step_on_device(pool, layer, &item, 1, plan, (rotate ? qd : q_src) + done * q_width,
+                            (rotate ? kd : k_src) + done * pool->row, v_src + done * pool->row, out_dev + done * q_width, num_q_heads,
                             default_scale(pool->g.head_dim),  // AttentionParams::new(), cpu.rs:584
                             softcap, nullptr);
         if (st != ITAK_OK) return st;
     }
-    if (!out_pinned) {
-        HIP_TRY(pool, hipMemcpyAsync(out, od, q_len * 4, hipMemcpyDeviceToHost, pool->stream),
-                "download attention output");
-        HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after attention");
-        return ITAK_OK;
-    }
-    // The last launch of the call writes the call's number where the host can see it; the host
-    // watches that word for a short while before it asks the runtime (which also reports a
-    // failed launch, and is what a call that takes longer falls back to).
-    const uint32_t number = ++pool->call_number ? pool->call_number : ++pool->call_number;
-    HIP_TRY(pool, launch_signal_done(done_word, number, pool->stream), "launch completion signal");
-    const volatile uint32_t *seen =
-        reinterpret_cast<const volatile uint32_t *>(pool->hstage);
-    timespec t0{};
-    clock_gettime(CLOCK_MONOTONIC, &t0);
-    bool arrived = false;
-    for (uint32_t spin = 0; !arrived; ++spin) {
-        arrived = __atomic_load_n(seen, __ATOMIC_ACQUIRE) == number;
-        if (arrived || (spin & 63u) != 63u) {
-            __builtin_ia32_pause();
-            continue;
-        }
-        timespec t1{};
-        clock_gettime(CLOCK_MONOTONIC, &t1);
-        if ((t1.tv_sec - t0.tv_sec) * 1000000000ll + (t1.tv_nsec - t0.tv_nsec) > 300000) break;
-    }
-    if (!arrived) HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after attention");
-    memcpy(out, pool->hstage + kHostWord + in_bytes, q_len * 4);
+    if (packed) return finish_host_call(pool, call, out);
+    HIP_TRY(pool, hipMemcpyAsync(out, od, q_len * 4, hipMemcpyDeviceToHost, pool->stream),
+            "download attention output");
+    HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after attention");
     return ITAK_OK;
 }
 
