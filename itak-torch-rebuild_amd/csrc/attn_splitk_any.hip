@@ -4,7 +4,7 @@
 // keep f32's precision, so that an f16 pool gives here what f32 arithmetic over its rows gives. A
 // short step's new rows are appended by the same launch.
 //
-// The shape of the work is attn_splitk_f32_kernel's (a workgroup of four wavefronts = item, KV
+// The shape of the work is attn_splitk_rows_kernel's (a workgroup of four wavefronts = item, KV
 // head, tile of 16 query vectors, run of 32-key blocks; a private online softmax per wavefront,
 // one merge through LDS) and its launches are planned by the same rule. What differs is the
 // operands. Which channel and which key an MFMA's k index stands for is free, and is chosen so that
@@ -23,12 +23,7 @@
 //     An infinite row times three halves of different signs, or of which one is zero, is NaN where
 //     the product is not: a wavefront whose sums come out not finite walks its keys again on the
 //     f32 pipe, query row by query row.
-//   row-major planes (f32; f16 at other multiples of 4): attn_splitk_any_kernel,
-//   v_mfma_f32_16x16x4_f32
-//     S^T tile t   four channels 16s + 4g .. + 3 of key 16t + i: four steps. Lane (j, g) receives
-//                  the scores of keys 16t + 4g + r.
-//     O^T (h, e)   four channels 64h + 4i .. + 3 of value row 16t + 4g + r; row i of output tile
-//                  (h, e) is channel 64h + 4i + e.
+//   row-major planes (f32; f16 at other multiples of 4): attn_splitk_rows_kernel.h
 //
 // DP is head_dim rounded up to a multiple of 32 (blocked) or 64 (row-major); pieces beyond head_dim
 // are read from the row's last valid piece and taken as zero.
@@ -43,8 +38,7 @@
 //
 // Semantics: gqa_attention in crates/attention/src/attention.rs:104-215, softcap as
 // crates/torch-math/src/logits.rs:26-37. Partials are in the log2 domain.
-#include "internal.h"
-#include "mfma_common.h"
+#include "attn_splitk_rows_kernel.h"
 
 #include <math.h>
 
@@ -54,321 +48,7 @@ namespace itak {
 
 namespace {
 
-constexpr int kWavesAny = 4;
-
-__device__ __forceinline__ float lanes4_max(float v) {  // over lanes l, l^16, l^32, l^48
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(c[0]), __uint_as_float(c[1]));
-}
-__device__ __forceinline__ float lanes4_sum(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(c[0]) + __uint_as_float(c[1]);
-}
-
-template <typename T>
-struct Piece4;  // four channels of a row-major row
-template <>
-struct Piece4<float> {
-    floatx4 v;
-    __device__ __forceinline__ void load(const float *p) { v = *reinterpret_cast<const floatx4 *>(p); }
-    __device__ __forceinline__ float at(int e) const { return v[e]; }
-    __device__ __forceinline__ void clear() { v = floatx4{0.f, 0.f, 0.f, 0.f}; }
-    __device__ __forceinline__ uint32_t not_finite() const {  // top bit set when one is
-        uint32_t s = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s |= (__float_as_uint(v[e]) & 0x7f800000u) + 0x00800000u;
-        return s & 0x80000000u;
-    }
-};
-template <>
-struct Piece4<uint16_t> {
-    half4 v;
-    __device__ __forceinline__ void load(const uint16_t *p) { v = *reinterpret_cast<const half4 *>(p); }
-    __device__ __forceinline__ float at(int e) const { return float(v[e]); }
-    __device__ __forceinline__ void clear() { v = half4{}; }
-    __device__ __forceinline__ uint32_t not_finite() const {
-        const uint2 x = __builtin_bit_cast(uint2, v);
-        return (((x.x & 0x7c007c00u) + 0x04000400u) | ((x.y & 0x7c007c00u) + 0x04000400u)) & 0x80008000u;
-    }
-};
-
-__device__ __forceinline__ uint16_t stored(float x, uint16_t) { return f32_to_f16_bits(x); }
-__device__ __forceinline__ float stored(float x, float) { return x; }
-
-// TT: 16-key tiles of a block whose rows are in registers at a time (1 where two would not fit).
-template <typename T, int DP, int TT, int N>
-__global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk_any_kernel(AttnParams p, AttnBatchT<N> b,
-                                                                         uint32_t total_partials) {
-    constexpr int kTiles = DP / 16;                 // output tiles
-    constexpr int kS = DP / 16;                     // steps of a key row per lane group
-    constexpr int kH = DP / 64;                     // pieces of a value row per lane
-    __shared__ float sm_m[kWavesAny][16], sm_l[kWavesAny][16];
-    __shared__ float sm_o[kWavesAny][kTiles][64][4];  // [wave][tile][lane][row of the lane]
-
-    const uint32_t tid = threadIdx.x;
-    const uint32_t wave = tid >> 6, lane = tid & 63;
-    const uint32_t g = lane >> 4, jl = lane & 15;
-    const uint32_t D = p.g.head_dim;
-
-    const AttnItem item = b.item[b.find_by_block(blockIdx.x)];
-    const uint32_t local = blockIdx.x - item.block0;
-    const uint32_t unit = local / item.splits, split = local % item.splits;
-    const uint32_t group = p.group, nvec = item.rows * group;
-    const uint32_t vtiles = (nvec + 15) / 16;
-    const uint32_t kv_head = unit % p.g.kv_heads, vtile = vtiles - 1 - unit / p.g.kv_heads;
-    // The rows this tile's vectors belong to bound the keys it walks.
-    const uint32_t row_first = (vtile * 16) / group;
-    const uint32_t row_last = min(item.rows - 1, (vtile * 16 + 15) / group);
-
-    const T *kplane = static_cast<const T *>(p.layer_base) + item.slot * p.g.slot_stride + kv_head * p.g.head_stride;
-    const T *vplane = kplane + p.g.side_stride;
-
-    const uint32_t ring_blocks = p.ring_blocks, ring = ring_blocks * kBlockKeys;
-    const uint32_t window = p.window, kv_lo = item.kv_lo;
-    const uint32_t nblocks = (min(item.pos0 + row_last + 1, item.kv_len) + kBlockKeys - 1) / kBlockKeys;
-    const uint32_t blocks_per_split = item.keys_per_split / kBlockKeys;
-    const uint32_t kb_begin = lowest_visible(item.pos0 + row_first, window, kv_lo) / kBlockKeys + split * blocks_per_split;
-    const uint32_t kb_end = min(nblocks, kb_begin + blocks_per_split);
-
-    // Fused append (p.k_new set): as in attn_splitk_f32_kernel, every workgroup whose blocks reach
-    // the new positions stores all of the item's rows of its KV head and meets at a barrier.
-    if (p.k_new != nullptr && kb_end * kBlockKeys > item.pos0) {
-        const uint32_t chunks = D / 4;
-        for (uint32_t f = tid; f < item.rows * 2 * chunks; f += kWavesAny * 64) {
-            const uint32_t r = f / (2 * chunks), rest = f % (2 * chunks);
-            const uint32_t side = rest >= chunks ? 1 : 0, c4 = (rest - side * chunks) * 4;
-            const float *src = (side ? p.v_new : p.k_new) +
-                               (uint64_t(item.q_row0 + r) * p.g.kv_heads + kv_head) * D + c4;
-            const floatx4 x = *reinterpret_cast<const floatx4 *>(src);
-            const uint32_t pos = item.pos0 + r, srow = ring ? pos % ring : pos;
-            T *plane = const_cast<T *>(side ? vplane : kplane);
-            T y[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] = stored(x[e], T{});
-            __builtin_memcpy(__builtin_assume_aligned(plane + uint64_t(srow) * D + c4, 4 * sizeof(T)), y, sizeof(y));
-        }
-        __syncthreads();
-    }
-
-    // This lane's query vector (column jl of the tile) and what its mask and its output need.
-    const uint32_t jv = vtile * 16 + jl;
-    const uint32_t j = min(jv, nvec - 1);
-    const uint32_t row = j / group, head = kv_head * group + j % group;
-    const uint32_t colpos = min(item.pos0 + row, item.kv_len - 1);
-    const uint32_t collo = lowest_visible(item.pos0 + row, window, kv_lo);
-    // [tile_lo, tile_hi): the positions some row of this tile sees.
-    const uint32_t tile_lo = lowest_visible(item.pos0 + row_first, window, kv_lo);
-    const uint32_t tile_hi = min(item.pos0 + row_last + 1, item.kv_len);
-    const uint32_t last_lo = lowest_visible(item.pos0 + row_last, window, kv_lo);
-    const uint32_t first_hi = min(item.pos0 + row_first, item.kv_len - 1) + 1;
-    const float softcap = p.softcap;
-    const float inv_cap = softcap > 0.0f ? 1.0f / softcap : 0.0f;
-    const float qscale = softcap > 0.0f ? p.scale : p.scale * kLog2e;
-
-    float qreg[kS][4];
-    {
-        const float *qp = p.q + (uint64_t(item.q_row0 + row) * p.q_heads + head) * D;
-#pragma unroll
-        for (int s = 0; s < kS; ++s) {
-            const uint32_t c = 16 * s + 4 * g;
-            const bool has = c < D && jv < nvec;
-            const floatx4 x = *reinterpret_cast<const floatx4 *>(qp + (c < D ? c : 0));
-#pragma unroll
-            for (int e = 0; e < 4; ++e) qreg[s][e] = has ? x[e] * qscale : 0.0f;
-        }
-    }
-
-    float m_run = -INFINITY, l_run = 0.0f;
-    floatx4 o[kTiles];
-#pragma unroll
-    for (int c = 0; c < kTiles; ++c) o[c] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    constexpr int kV = TT * 4 * kH;  // value pieces held
-    for (uint32_t kb = kb_begin + wave; kb < kb_end; kb += kWavesAny) {
-        const uint32_t sb = ring_blocks ? kb % ring_blocks : kb;  // storage block
-#pragma unroll 1
-        for (uint32_t t0 = 0; t0 < 2; t0 += TT) {
-            const uint32_t key0 = kb * kBlockKeys + 16 * t0;
-            if (TT == 1 && (key0 >= tile_hi || key0 + 16 <= tile_lo)) continue;
-            // ---- operands of the block's keys
-            Piece4<T> kreg[TT][kS];
-            Piece4<T> vreg[kV];
-            // Rows past the stored length are read from the last stored row (the plane may end there).
-            const uint32_t most = item.kv_len - 1 - min(item.kv_len - 1, key0);
-            const T *krow = kplane + uint64_t(sb * kBlockKeys + 16 * t0) * D;
-            const T *vrow = vplane + uint64_t(sb * kBlockKeys + 16 * t0) * D;
-            const bool beyond = key0 >= item.kv_len;  // the whole tile: read the block's first row instead
-            auto row_at = [&](uint32_t i) { return beyond ? 0u : min(i, most); };
-            if (beyond) krow -= uint64_t(16 * t0) * D, vrow -= uint64_t(16 * t0) * D;
-#pragma unroll
-            for (int t = 0; t < TT; ++t)
-#pragma unroll
-                for (int s = 0; s < kS; ++s)
-                    kreg[t][s].load(krow + row_at(16 * t + jl) * D + min(16u * s + 4 * g, D - 4));
-#pragma unroll
-            for (int t = 0; t < TT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int h = 0; h < kH; ++h)
-                        vreg[(t * 4 + r) * kH + h].load(vrow + row_at(16 * t + 4 * g + r) * D + min(64u * h + 4 * jl, D - 4));
-            auto key_of = [&](int t, int r) { return key0 + 16 * t + 4 * g + r; };
-
-            // ---- scores
-            float sc[TT][4];
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                floatx4 acc = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int s = 0; s < kS; ++s) {
-                    const bool has = 16u * s + 4 * g < D;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float a = kreg[t][s].at(e);
-                        // (Only the last four steps can lie beyond head_dim, and then not in all lanes.)
-                        if ((s + 1) * 16 > DP - 64) a = has ? a : 0.0f;
-                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a, qreg[s][e], acc, 0, 0, 0);
-                    }
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) sc[t][r] = acc[r];
-            }
-            const bool edge = key0 + 16 * TT > tile_hi || key0 < tile_lo;
-            float mx = -INFINITY;
-#pragma unroll
-            for (int t = 0; t < TT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t kp = key_of(t, r);
-                    float v = sc[t][r];
-                    if (softcap > 0.0f) v = softcap_log2(v, softcap, inv_cap);
-                    if (kp > colpos || kp < collo) v = -INFINITY;
-                    sc[t][r] = v;
-                    mx = fmaxf(mx, v);
-                }
-            // A row no query of the tile sees may hold anything, stale data or a value that is not
-            // finite: keep it out of P.V even as 0 * x.
-            if (edge) {
-#pragma unroll
-                    for (int t = 0; t < TT; ++t)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const uint32_t kp = key_of(t, r);
-                            if (kp >= tile_hi || kp < tile_lo) {
-#pragma unroll
-                                for (int h = 0; h < kH; ++h) vreg[(t * 4 + r) * kH + h].clear();
-                            }
-                        }
-            }
-            mx = lanes4_max(mx);
-            const float m_new = fmaxf(m_run, mx);
-            const bool dead = m_new == -INFINITY;
-            const float alpha = (dead || m_run == -INFINITY) ? (dead ? 1.0f : 0.0f) : fast_exp2(m_run - m_new);
-            float sum = 0.0f;
-#pragma unroll
-            for (int t = 0; t < TT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    // (Nothing finite in sight so far: -inf weighs zero against a reference of zero,
-                    // and a NaN score stays NaN and takes the row with it.)
-                    const float pe = fast_exp2(sc[t][r] - (dead ? 0.0f : m_new));
-                    sc[t][r] = pe;
-                    sum += pe;
-                }
-            l_run = l_run * alpha + sum;
-            m_run = m_new;
-#pragma unroll
-            for (int c = 0; c < kTiles; ++c) o[c] *= alpha;
-            auto value = [&](int t, int r, int c) -> float {
-                return vreg[(t * 4 + r) * kH + c / 4].at(c % 4);
-            };
-            // Rows that do not all see the same keys, and a value that is not finite: the product is
-            // taken once per query row of the tile with the keys it does not see cleared
-            // (attn_splitk_f32_kernel says why).
-            if (row_last > row_first && (key0 + 16 * TT > first_hi || key0 < last_lo)) {
-                uint32_t seen = 0;
-#pragma unroll
-                for (int i = 0; i < kV; ++i) seen |= vreg[i].not_finite();
-                seen = __builtin_amdgcn_ballot_w64(seen != 0) != 0 ? 1u : 0u;
-                if (seen) {
-#pragma unroll 1
-                    for (uint32_t rr = row_first; rr <= row_last; ++rr) {
-                        const uint32_t pos = min(item.pos0 + rr, item.kv_len - 1);
-                        const uint32_t lo = lowest_visible(item.pos0 + rr, window, kv_lo);
-                        const bool mine = row == rr;
-#pragma unroll
-                        for (int t = 0; t < TT; ++t)
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) {
-                                const uint32_t kp = key_of(t, r);
-                                const bool seen_by_row = kp <= pos && kp >= lo;
-#pragma unroll
-                                for (int c = 0; c < kTiles; ++c) {
-                                    const float a = seen_by_row ? value(t, r, c) : 0.0f;
-                                    const floatx4 zero = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-                                    const floatx4 part = __builtin_amdgcn_mfma_f32_16x16x4f32(a, sc[t][r], zero, 0, 0, 0);
-                                    if (mine) o[c] += part;
-                                    __builtin_amdgcn_sched_barrier(0);
-                                }
-                            }
-                    }
-                    continue;
-                }
-            }
-#pragma unroll
-            for (int t = 0; t < TT; ++t)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int c = 0; c < kTiles; ++c)
-                        o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(value(t, r, c), sc[t][r], o[c], 0, 0, 0);
-        }
-    }
-
-    // ---- merge the wavefronts through LDS
-    const float l_col = lanes4_sum(l_run);
-    if (g == 0) {
-        sm_m[wave][jl] = m_run;
-        sm_l[wave][jl] = l_col;
-    }
-#pragma unroll
-    for (int c = 0; c < kTiles; ++c) *reinterpret_cast<floatx4 *>(&sm_o[wave][c][lane][0]) = o[c];
-    __syncthreads();
-
-    float M = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kWavesAny; ++w) M = fmaxf(M, sm_m[w][jl]);
-    float L = 0.0f, wgt[kWavesAny];
-#pragma unroll
-    for (int w = 0; w < kWavesAny; ++w) {
-        const float mw = sm_m[w][jl];
-        wgt[w] = mw == -INFINITY ? 0.0f : fast_exp2(mw - M);
-        L = fmaf(sm_l[w][jl], wgt[w], L);
-    }
-    if (jv >= nvec) return;
-    const bool final_out = item.splits == 1;
-    const uint64_t ps = item.ws0 + (uint64_t(row) * p.q_heads + head) * item.splits + split;
-    float *dst = final_out ? p.out + (uint64_t(item.q_row0 + row) * p.q_heads + head) * D : p.ws + ps * D;
-    const float post = final_out ? 1.0f / L : 1.0f;
-    // Tile (h, e), register rr = channel 64h + 16g + 4rr + e: wavefront w finishes register w of all.
-#pragma unroll
-    for (int h = 0; h < kH; ++h) {
-        const uint32_t ch = 64 * h + 16 * g + 4 * wave;
-        floatx4 fin = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int w = 0; w < kWavesAny; ++w)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) fin[e] = fmaf(sm_o[w][4 * h + e][lane][wave], wgt[w], fin[e]);
-        fin *= post;
-        if (ch < D) *reinterpret_cast<floatx4 *>(dst + ch) = fin;
-    }
-    if (!final_out && wave == 0 && g == 0)
-        *reinterpret_cast<float2 *>(p.ws + uint64_t(total_partials) * D + ps * 2) = make_float2(M, L);
-}
+constexpr int kWavesAny = kWavesRows;
 
 // x = h[0] + h[1] + h[2] up to 2^-33 of the largest x the halves hold. A half that is not finite
 // has nothing left to say.
@@ -384,7 +64,7 @@ __device__ __forceinline__ void split3(float x, _Float16 &a, _Float16 &b, _Float
 constexpr float kWeightShift = 15.0f;
 
 template <int DP, int N>
-__global__ __launch_bounds__(kWavesAny * 64, DP <= 160 ? 2 : 1) void attn_splitk_halves_kernel(AttnParams p, AttnBatchT<N> b,
+__global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk_halves_kernel(AttnParams p, AttnBatchT<N> b,
                                                                                              uint32_t total_partials) {
     constexpr int kTiles = DP / 16;  // output tiles
     constexpr int kS = DP / 32;      // steps of a key row
@@ -428,19 +108,76 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 160 ? 2 : 1) void attn_splitk
     const float qscale = softcap > 0.0f ? p.scale : p.scale * kLog2e;
     const float *qp = p.q + (uint64_t(item.q_row0 + row) * p.q_heads + head) * D;
 
+    // Everything the first block needs is asked for before anything is waited for: the raw queries,
+    // then its keys and values; later blocks' keys are asked for when the scores have used up the
+    // operands of the block before, their values when its products have.
+    floatx4 x[kS][2];
+#pragma unroll
+    for (int s = 0; s < kS; ++s)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            x[s][h] = *reinterpret_cast<const floatx4 *>(qp + 8 * min(4u * s + g, chunks - 1) + 4 * h);
+
+    half8 k[2][kS], v[kTiles];
+    auto block_at = [&](uint32_t kb) { return uint64_t(ring_blocks ? kb % ring_blocks : kb) * (kVBlock * D); };
+    // Fused append (p.k_new set): the wavefront that owns a block stores the new rows in it and waits
+    // for the stores before it reads the block; nobody else reads these positions.
+    auto append_rows = [&](uint32_t kb) {
+        const uint32_t key0 = kb * kBlockKeys;
+        if (p.k_new == nullptr || key0 + kBlockKeys <= item.pos0) return;
+        uint16_t *kblk = kplane + block_at(kb), *vblk = vplane + block_at(kb);
+        const uint32_t from = key0 > item.pos0 ? key0 - item.pos0 : 0;
+        const uint32_t to = min(item.rows, key0 + kBlockKeys - item.pos0), quads = D / 4;
+        for (uint32_t f = lane; f < (to - from) * 2 * quads; f += 64) {
+            const uint32_t r = from + f / (2 * quads), rest = f % (2 * quads);
+            const uint32_t side = rest >= quads ? 1 : 0, c4 = (rest - side * quads) * 4;
+            const floatx4 y = *reinterpret_cast<const floatx4 *>(
+                (side ? p.v_new : p.k_new) + (uint64_t(item.q_row0 + r) * p.g.kv_heads + kv_head) * D + c4);
+            const uint32_t kk = (item.pos0 + r) % kBlockKeys;
+            uint16_t h[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[e] = f32_to_f16_bits(y[e]);
+            if (side) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) vblk[(c4 + e) * kVBlock + kk] = h[e];
+            } else {
+                const uint32_t t = (kk >> 2) & 1, i = (kk >> 3) * 4 + (kk & 3);
+                __builtin_memcpy(__builtin_assume_aligned(kblk + ((t * chunks + c4 / 8) * 16 + i) * 8 + c4 % 8, 8), h, 8);
+            }
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores have been acknowledged
+    };
+    auto load_keys = [&](uint32_t kb) {
+        const uint16_t *kblk = kplane + block_at(kb);
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int s = 0; s < kS; ++s)
+                k[t][s] = *reinterpret_cast<const half8 *>(kblk + ((t * chunks + min(4u * s + g, chunks - 1)) * 16 + jl) * 8);
+    };
+    auto load_values = [&](uint32_t kb) {
+        const uint16_t *vblk = vplane + block_at(kb);
+#pragma unroll
+        for (int c = 0; c < kTiles; ++c)
+            v[c] = *reinterpret_cast<const half8 *>(vblk + min(16u * c + jl, D - 1) * kVBlock + 8 * g);
+    };
+    uint32_t kb = kb_begin + wave;
+    if (kb < kb_end) {
+        append_rows(kb);
+        load_keys(kb);
+        load_values(kb);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
     // Q^T as three B operands: step s takes channels 8 (4s + g) .. + 7 of vector jl, times the power
     // of two that brings the vector's largest below 2^15; colscale takes it out of the scores again.
     half8 q[3][kS];
     float colscale;
     {
-        floatx4 x[kS][2];
         float most = 0.0f;
 #pragma unroll
         for (int s = 0; s < kS; ++s) {
-            const uint32_t c = 4 * s + g;
-            const bool has = c < chunks && jv < nvec;
-#pragma unroll
-            for (int h = 0; h < 2; ++h) x[s][h] = *reinterpret_cast<const floatx4 *>(qp + (c < chunks ? 8 * c + 4 * h : 0));
+            const bool has = 4u * s + g < chunks && jv < nvec;
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -502,44 +239,8 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 160 ? 2 : 1) void attn_splitk
         return alpha;
     };
 
-    for (uint32_t kb = kb_begin + wave; kb < kb_end; kb += kWavesAny) {
-        const uint32_t key0 = kb * kBlockKeys;
-        const uint64_t at = uint64_t(ring_blocks ? kb % ring_blocks : kb) * (kVBlock * D);
-        uint16_t *kblk = kplane + at, *vblk = vplane + at;
-        // Fused append (p.k_new set): the wavefront that owns a block stores the new rows in it and
-        // waits for the stores before it reads the block; nobody else reads these positions.
-        if (p.k_new != nullptr && key0 + kBlockKeys > item.pos0) {
-            const uint32_t from = key0 > item.pos0 ? key0 - item.pos0 : 0;
-            const uint32_t to = min(item.rows, key0 + kBlockKeys - item.pos0), quads = D / 4;
-            for (uint32_t f = lane; f < (to - from) * 2 * quads; f += 64) {
-                const uint32_t r = from + f / (2 * quads), rest = f % (2 * quads);
-                const uint32_t side = rest >= quads ? 1 : 0, c4 = (rest - side * quads) * 4;
-                const floatx4 x = *reinterpret_cast<const floatx4 *>(
-                    (side ? p.v_new : p.k_new) + (uint64_t(item.q_row0 + r) * p.g.kv_heads + kv_head) * D + c4);
-                const uint32_t kk = (item.pos0 + r) % kBlockKeys;
-                uint16_t h[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) h[e] = f32_to_f16_bits(x[e]);
-                if (side) {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) vblk[(c4 + e) * kVBlock + kk] = h[e];
-                } else {
-                    const uint32_t t = (kk >> 2) & 1, i = (kk >> 3) * 4 + (kk & 3);
-                    __builtin_memcpy(__builtin_assume_aligned(kblk + ((t * chunks + c4 / 8) * 16 + i) * 8 + c4 % 8, 8), h, 8);
-                }
-            }
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores have been acknowledged
-        }
-        half8 k[2][kS], v[kTiles];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int s = 0; s < kS; ++s)
-                k[t][s] = *reinterpret_cast<const half8 *>(kblk + ((t * chunks + min(4u * s + g, chunks - 1)) * 16 + jl) * 8);
-#pragma unroll
-        for (int c = 0; c < kTiles; ++c)
-            v[c] = *reinterpret_cast<const half8 *>(vblk + min(16u * c + jl, D - 1) * kVBlock + 8 * g);
-
+    for (; kb < kb_end; kb += kWavesAny) {
+        const uint32_t key0 = kb * kBlockKeys, next = kb + kWavesAny;
         float sc[2][4];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -553,6 +254,10 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 160 ? 2 : 1) void attn_splitk
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r) sc[t][r] = acc[r] * colscale;
+        }
+        if (next < kb_end) {
+            append_rows(next);
+            load_keys(next);
         }
         const float alpha = weigh(key0, sc);
         half8 w[3];
@@ -578,6 +283,7 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 160 ? 2 : 1) void attn_splitk
 #pragma unroll
             for (int h = 2; h >= 0; --h) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v[c], w[h], o[c], 0, 0, 0);
         }
+        if (next < kb_end) load_values(next);
     }
 
     float all = l_run;
@@ -679,7 +385,7 @@ bool attn_splitk_any_supports(const PoolGeom &g, uint32_t group, uint32_t max_ro
 }
 // By the registers of a wavefront: up to 168, up to 256, and more than that.
 uint32_t attn_splitk_any_groups_per_cu(const PoolGeom &g) {
-    if (g.v_block) return g.head_dim <= 96 ? 3 : g.head_dim <= 160 ? 2 : 1;
+    if (g.v_block) return g.head_dim <= 64 ? 3 : g.head_dim <= 128 ? 2 : 1;
     return g.head_dim <= 64 ? 3 : g.head_dim <= 128 ? 2 : 1;
 }
 // As for the f32 kernel: a step of up to 16 query vectors per KV head brings its rows along.
@@ -697,10 +403,10 @@ hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnB
     do {                                                                                          \
         if (b.n <= 8) {                                                                           \
             constexpr int N = 8;                                                                  \
-            __VA_ARGS__<<<grid, threads, 0, stream>>>(p, AttnBatchT<N>(b), total_partials);       \
+            launch_kernel(__VA_ARGS__, grid, threads, 0, stream, p, AttnBatchT<N>(b), total_partials);       \
         } else {                                                                                  \
             constexpr int N = 64;                                                                 \
-            __VA_ARGS__<<<grid, threads, 0, stream>>>(p, AttnBatchT<N>(b), total_partials);       \
+            launch_kernel(__VA_ARGS__, grid, threads, 0, stream, p, AttnBatchT<N>(b), total_partials);       \
         }                                                                                         \
     } while (0)
     if (elem_f16 && p.g.v_block) {
@@ -716,17 +422,17 @@ hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnB
         }
     } else if (elem_f16) {
         switch ((d + 63) / 64) {
-            case 1: ITAK_ANY(attn_splitk_any_kernel<uint16_t, 64, 2, N>); break;
-            case 2: ITAK_ANY(attn_splitk_any_kernel<uint16_t, 128, 2, N>); break;
-            case 3: ITAK_ANY(attn_splitk_any_kernel<uint16_t, 192, 2, N>); break;
-            default: ITAK_ANY(attn_splitk_any_kernel<uint16_t, 256, 2, N>); break;
+            case 1: ITAK_ANY(attn_splitk_rows_kernel<uint16_t, 64, false, 2, false, N>); break;
+            case 2: ITAK_ANY(attn_splitk_rows_kernel<uint16_t, 128, false, 2, false, N>); break;
+            case 3: ITAK_ANY(attn_splitk_rows_kernel<uint16_t, 192, false, 2, false, N>); break;
+            default: ITAK_ANY(attn_splitk_rows_kernel<uint16_t, 256, false, 2, false, N>); break;
         }
     } else {
         switch ((d + 63) / 64) {
-            case 1: ITAK_ANY(attn_splitk_any_kernel<float, 64, 2, N>); break;
-            case 2: ITAK_ANY(attn_splitk_any_kernel<float, 128, 2, N>); break;
-            case 3: ITAK_ANY(attn_splitk_any_kernel<float, 192, 1, N>); break;
-            default: ITAK_ANY(attn_splitk_any_kernel<float, 256, 1, N>); break;
+            case 1: ITAK_ANY(attn_splitk_rows_kernel<float, 64, false, 2, false, N>); break;
+            case 2: ITAK_ANY(attn_splitk_rows_kernel<float, 128, false, 2, false, N>); break;
+            case 3: ITAK_ANY(attn_splitk_rows_kernel<float, 192, false, 1, false, N>); break;
+            default: ITAK_ANY(attn_splitk_rows_kernel<float, 256, false, 1, false, N>); break;
         }
     }
 #undef ITAK_ANY
