@@ -64,7 +64,7 @@ static Variant pick_variant(const PoolGeom &g, const AttnBatch &b, uint32_t grou
     if (nvec > 16) return {2, 4, 2};
     // (Eight wavefronts for one-row steps only: that variant leaves out the exact treatment of
     // non-finite values that a step of several rows may need.)
-    return blocks >= 4096 && rows == 1 ? Variant{1, 8, 1} : Variant{1, 4, 0};
+    return b.whole_on_eight || (blocks >= 4096 && rows == 1) ? Variant{1, 8, 1} : Variant{1, 4, 0};
 }
 // The variant a planned batch takes: 0 = 16 vectors on four wavefronts, 1 = on eight, 2 = 32
 // vectors, 3 = 64 vectors.
@@ -150,17 +150,41 @@ static uint32_t variant_capacity(const Variant &v) {
     }
 }
 
+// Blocks up to which a batch's items stay whole: one workgroup per KV head walks the context, and
+// there is neither a partial nor a merge launch. A compute unit reads 16 KB of keys and values
+// (a block) in 0.25 us, a merge launch costs 3 us in a single-slot step; a wavefront's second block
+// costs half a microsecond. One-row steps take eight wavefronts from the fifth block on: up to 12
+// blocks, where the next wavefront's round begins to cost what the merge does, 18 for launches that
+// prepare their rows (their workgroups of one block each spend 2 us on that, and the whole form has
+// fewer of them), 24 from 64 workgroups on (the merge of many slots costs more). Longer steps have
+// four wavefronts only. One layer of 32 Q / 4 KV heads, us, split -> whole: 1 slot at 200 / 300 rows
+// 7.3 / 7.4 -> 5.1 / 5.4 (7.2 -> 7.2 at 400), 16 slots at 300 / 600 11.0 / 12.7 -> 8.7 / 11.1, with
+// preparation 1 slot at 200 / 500 9.2 / 9.3 -> 6.2 / 8.6; six rows at 200 10.7 -> 9.7.
+static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, bool one_row, bool prepares) {
+    if (!one_row) return 8;
+    if (g.kv_heads * b.n >= 64) return 24;
+    return prepares ? 18 : 12;
+}
+
 // Fills splits / keys_per_split / block0 / ws0 for a batch (the caller has set slot, rows,
 // pos0, q_row0, kv_len) and returns the number of partials the launch will write.
 // Every (item, KV head) is cut into equal runs of at most T blocks, T the smallest run for
 // which the whole batch fits the device in one wave of dispatch; a run is never shorter
 // than one block per wavefront.
-uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads) {
+uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares) {
+    uint32_t most = 0, most_rows = 0;
+    for (uint32_t i = 0; i < b.n; ++i) {
+        most = std::max(most, item_block_count(b.item[i]));
+        most_rows = std::max(most_rows, b.item[i].rows);
+    }
+    const bool whole = most <= whole_limit(g, b, most_rows == 1, prepares);
+    b.whole_on_eight = whole && most_rows == 1 && most > 4 ? 1 : 0;
     const Variant v = pick_variant(g, b, q_heads / g.kv_heads);
     const uint64_t capacity = variant_capacity(v);
     uint64_t blocks = 0;
     for (uint32_t i = 0; i < b.n; ++i) blocks += uint64_t(g.kv_heads) * item_block_count(b.item[i]);
     uint64_t T = std::max<uint64_t>((blocks + capacity - 1) / capacity, uint64_t(v.waves));
+    if (whole) T = std::max<uint64_t>(T, most);
     for (;; ++T) {
         uint64_t groups = 0;
         for (uint32_t i = 0; i < b.n; ++i) {

@@ -292,6 +292,7 @@ struct AttnBatch {
     uint32_t deep_ring;  // host side only: the block kernel's plan asks for its deeper LDS ring
     uint32_t fold_units; // host side only: the block kernel's plan for AttnParams::fold_units
     uint32_t two_halves; // host side only: the block kernel multiplies each query as two f16 halves
+    uint32_t whole_on_eight; // host side only: the split-K plan leaves every item whole on eight wavefronts
     AttnItem item[kMaxBatchItems];
 };
 // The kernel argument form of AttnBatch, sized to the batch: kernel arguments are
@@ -430,7 +431,8 @@ uint32_t attn_generic_tile(uint32_t head_dim);
 // MFMA split-K path: f16 pools with blocked value planes, head_dim 128, rows*group <= 64.
 // Partials are in log2 domain (combine with base2 = 1).
 bool attn_splitk_f16_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
-uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads);
+// (`prepares`: the launch prepares Q and the new K rows itself.)
+uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares = false);
 // After attn_splitk_f16_plan: whether the batch can merge its splits inside the split-K launch
 // (AttnParams::exchange). Returns the 64-bit words the exchange buffer must hold and re-bases
 // the items' ws0 on it, or 0 (items untouched) when the batch keeps the merge launch.
