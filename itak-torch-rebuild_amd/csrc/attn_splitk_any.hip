@@ -388,6 +388,10 @@ uint32_t attn_splitk_any_groups_per_cu(const PoolGeom &g) {
     if (g.v_block) return g.head_dim <= 64 ? 3 : g.head_dim <= 128 ? 2 : 1;
     return g.head_dim <= 64 ? 3 : g.head_dim <= 128 ? 2 : 1;
 }
+uint32_t attn_splitk_any_whole_blocks(const PoolGeom &g, int elem_f16) {
+    if (g.v_block) return g.head_dim <= 128 ? 12 : 8;
+    return elem_f16 || g.head_dim <= 64 ? 8 : 4;
+}
 // As for the f32 kernel: a step of up to 16 query vectors per KV head brings its rows along.
 bool attn_splitk_any_appends(const PoolGeom &g, uint32_t group, uint32_t max_rows) {
     return attn_splitk_any_supports(g, group, max_rows) && max_rows * group <= 16;

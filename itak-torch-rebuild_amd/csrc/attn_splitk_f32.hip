@@ -20,7 +20,7 @@ bool attn_splitk_f32_appends(const PoolGeom &g, uint32_t group, uint32_t max_row
 // set) and returns the number of partials. Every (item, KV head) is cut into equal runs of at
 // most T blocks, T the smallest run for which the batch is at most groups_per_cu workgroups per
 // compute unit, and never shorter than one block per wavefront.
-uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu) {
+uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu, uint32_t whole_blocks) {
     const uint64_t capacity = uint64_t(groups_per_cu) * compute_units();
     const uint32_t group = q_heads / g.kv_heads;
     auto units_of = [&](const AttnItem &it) {
@@ -29,6 +29,16 @@ uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads,
     uint64_t blocks = 0;
     for (uint32_t i = 0; i < b.n; ++i) blocks += units_of(b.item[i]) * item_block_count(b.item[i]);
     uint64_t T = std::max<uint64_t>((blocks + capacity - 1) / capacity, uint64_t(kWavesRows));
+    // A short step's short contexts stay whole (one tile of vectors per KV head): a merge launch costs
+    // 2 to 3 us, a wavefront's second 32-key block 1 us on the f32 pipe at head_dim 64, twice that at
+    // 128, half of it on the f16 pipe. One row at 200 positions, 1 slot: f32 at head_dim 64 8.1 -> 7.5
+    // us a layer (at 128 10.1 -> 10.2), f16 at 80 8.6 -> 6.5 and, at 300 positions, 8.4 -> 7.5.
+    uint32_t most = 0, most_vectors = 0;
+    for (uint32_t i = 0; i < b.n; ++i) {
+        most = std::max(most, item_block_count(b.item[i]));
+        most_vectors = std::max(most_vectors, b.item[i].rows * group);
+    }
+    if (most_vectors <= 16 && most <= whole_blocks) T = std::max<uint64_t>(T, most);
     for (;; ++T) {
         uint64_t groups = 0;
         for (uint32_t i = 0; i < b.n; ++i) {

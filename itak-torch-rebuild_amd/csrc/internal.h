@@ -497,7 +497,9 @@ hipError_t launch_attn_decode_f16(const AttnParams &p, const AttnBatch &b, uint3
 bool attn_splitk_f32_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
 // True when such a launch also appends the step's rows (k_new / v_new in its parameters).
 bool attn_splitk_f32_appends(const PoolGeom &g, uint32_t group, uint32_t max_rows);
-uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu = 2);
+// (`groups_per_cu` workgroups share a compute unit; contexts of `whole_blocks` blocks are not split.)
+uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu,
+                              uint32_t whole_blocks);
 hipError_t launch_attn_splitk_f32(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream);
 // f32-arithmetic MFMA split-K path for the other shapes (attn_splitk_any.hip): f16 and f32 pools,
@@ -506,6 +508,8 @@ hipError_t launch_attn_splitk_f32(const AttnParams &p, const AttnBatch &b, uint3
 bool attn_splitk_any_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
 // Workgroups of that kernel a compute unit holds.
 uint32_t attn_splitk_any_groups_per_cu(const PoolGeom &g);
+// Blocks up to which its short steps leave a context whole.
+uint32_t attn_splitk_any_whole_blocks(const PoolGeom &g, int elem_f16);
 bool attn_splitk_any_appends(const PoolGeom &g, uint32_t group, uint32_t max_rows);
 hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream);
