@@ -182,12 +182,25 @@ def debug_enabled() -> bool:
     return bool(N.load().itak_debug_enabled())
 
 
+_F32 = np.dtype(np.float32)
+_from_buffer, _addressof = C.c_char.from_buffer, C.addressof
+
+
 def _as_f32(x) -> np.ndarray:
+    if x.__class__ is np.ndarray and x.dtype is _F32 and x.flags.c_contiguous:
+        return x if x.ndim == 1 else x.reshape(-1)
     return np.ascontiguousarray(x, dtype=np.float32).reshape(-1)
 
 
 def _ptr(a: Optional[np.ndarray]):
-    return a.ctypes.data if a is not None and a.size else None
+    """Address of a contiguous array's data; None for none. (numpy's own `ctypes.data` builds two
+    objects for it, a microsecond an array on a call of twenty.)"""
+    if a is None or not a.size:
+        return None
+    try:
+        return _addressof(_from_buffer(a))
+    except TypeError:  # read-only memory is exported by the other way alone
+        return a.ctypes.data
 
 
 _ITEM_PACK = {}
@@ -532,10 +545,9 @@ class KvCache:
         return bool(out.value)
 
     def _bases(self, raw: N.CheckpointRaw) -> List[int]:
-        bases = np.empty(self.layer_count(), dtype=np.uint64)
-        _check(self._h, self._lib.itak_kv_checkpoint_bases(self._h, self.slot, C.byref(raw),
-                                                           _ptr(bases)))
-        return [int(b) for b in bases]
+        bases = (C.c_uint64 * len(self.pool.pattern))()
+        _check(self._h, self._lib.itak_kv_checkpoint_bases(self._h, self.slot, C.byref(raw), bases))
+        return list(bases)
 
     def checkpoint(self, max_round_tokens: int) -> Checkpoint:
         raw = N.CheckpointRaw()
@@ -608,13 +620,19 @@ def gqa_attention(q, num_queries: int, num_q_heads: int, query_positions: Sequen
                   view: CacheView, params: AttentionParams = AttentionParams()) -> np.ndarray:
     """attention::gqa_attention (attention.rs:104-215) on the device; flat f32 output."""
     q = _as_f32(q)
-    pos = np.asarray(query_positions, dtype=np.uint64).reshape(-1)
-    out = np.zeros(q.size, dtype=np.float32)
+    try:
+        pos = array("Q", query_positions)
+        pos_ptr, pos_size = pos.buffer_info()
+    except (TypeError, OverflowError):  # arrays of another type, several dimensions
+        pos = np.asarray(query_positions, dtype=np.uint64).reshape(-1)
+        pos_ptr, pos_size = _ptr(pos), pos.size
+    out = np.empty(q.size, dtype=_F32)  # every element is written, or the call raises
     c = view._c
-    _check(c._h, c._lib.itak_gqa_attention(
-        c._h, c.slot, view._layer, _ptr(q), q.size, num_queries, num_q_heads, _ptr(pos), pos.size,
-        math.nan if params.scale is None else float(params.scale), float(params.softcap),
-        _ptr(out)))
+    status = c._lib.itak_gqa_attention(
+        c._h, c.slot, view._layer, _ptr(q), q.size, num_queries, num_q_heads, pos_ptr if pos_size else None,
+        pos_size, _NAN if params.scale is None else float(params.scale), float(params.softcap), _ptr(out))
+    if status:
+        _raise_last(c._h)
     return out if num_queries else out[:0]
 
 
@@ -721,6 +739,8 @@ class HipCompute:
         except AttentionError as e:
             raise StepFailed(step, e.message or str(e)) from e
         self._shape = self._shape_of(cfg)
+        self._layers = list(cfg.layers)
+        self._widths = self._shape[1:]
 
     def attention(self, req: AttentionRequest, cache) -> np.ndarray:
         """Compute::attention (compute.rs:82, cpu.rs:506-655)."""
@@ -730,22 +750,26 @@ class HipCompute:
             raise StepFailed(step, f"key_length {cfg.key_length} != value_length "
                                    f"{cfg.value_length}: the KV cache stores keys and values at "
                                    "one head dimension")
-        if cfg.layer_kind(req.layer) != req.kind:
+        kind = cfg.layer_kind(req.layer)
+        if kind is not req.kind and kind != req.kind:
             raise StepFailed(step, f"request kind {req.kind} does not match the config's kind for "
                                    f"layer {req.layer}")
         q, k, v = _as_f32(req.q), _as_f32(req.k), _as_f32(req.v)
         if self._shape is None:
             self._build(cfg, step)
-        elif self._shape != self._shape_of(cfg):
+        elif ((self._layers != cfg.layers or self._widths != (cfg.kv_heads, cfg.key_length, cfg.value_length,
+                                                              cfg.sliding_window))
+              and self._shape != self._shape_of(cfg)):
             raise StepFailed(step, "this HipCompute already serves a model of a different shape; "
                                    "construct a fresh HipCompute per model (or reset this one) "
                                    "instead of retargeting it mid-sequence")
-        out = np.zeros(q.size, dtype=np.float32)
+        out = np.empty(q.size, dtype=_F32)  # every element is written, or the call raises
         c = self._cache
-        _check(c._h, c._lib.itak_compute_attention(
+        status = c._lib.itak_compute_attention(
             c._h, c.slot, req.layer, _ptr(q), q.size, _ptr(k), k.size, _ptr(v), v.size,
-            cfg.q_heads, cache.position(), self._softcap, cfg.rope_freq_base_swa, _ptr(out)),
-            step)
+            cfg.q_heads, cache.position(), self._softcap, cfg.rope_freq_base_swa, _ptr(out))
+        if status:
+            _raise_last(c._h, step)
         return out
 
     def _need_cache(self) -> KvCache:
