@@ -644,15 +644,31 @@ bool takes_splitk_f16(const itak_pool *pool, const PlanInput *in, uint32_t n, ui
 // or with groups above 16, f32 pools at other head dims. Its 16-byte loads and stores ask for
 // tensors aligned to that (every row is a multiple of 16 bytes when head_dim is one of four
 // floats); others, odd head dims and explicit positions run on the general kernel.
+// It also takes f16 steps of up to 16 query vectors per KV head at head dims 64, 96 and 256, where
+// the block kernel has nothing to share between its wavefronts: no LDS ring to fill before the first
+// product, runs down to one block per wavefront, short contexts left whole. 32 Q / 4 KV heads, us a
+// layer, block kernel -> this: one slot at 1,500 rows 9.5 -> 8.9, 11.3 -> 8.9, 15.8 -> 12.7 (head_dim
+// 64, 96, 256), 4 slots at 300 10.2 -> 7.2, 11.7 -> 8.1, 14.9 -> 13.3. At 256 a wavefront's operands
+// leave room for one workgroup per compute unit, so that launches of more than one block per wavefront
+// of the device and less than two run two rounds of blocks for little more than one round's work: those
+// stay with the block kernel (8 slots of 2,000 rows 21.8 against 23.5; of 3,000 rows 34.3 -> 28.5).
 bool aligned16(const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 bool takes_splitk_any(const itak_pool *pool, const PlanInput *in, uint32_t n, uint64_t q_heads, const float *q_dev,
                       const float *out_dev, const uint32_t *q_pos_dev) {
     const uint32_t group = uint32_t(q_heads / pool->g.kv_heads);
     uint32_t max_rows = 0;
-    for (uint32_t i = 0; i < n; ++i) max_rows = std::max(max_rows, in[i].rows);
+    uint64_t blocks = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        max_rows = std::max(max_rows, in[i].rows);
+        blocks += uint64_t(pool->g.kv_heads) * ((in[i].kv_len + 31) / 32 - in[i].kv_lo / 32);
+    }
+    const uint64_t round = 4 * uint64_t(compute_units());
+    const bool has_own = !pool->elem_f16 ? attn_splitk_f32_supports(pool->g, group, max_rows)
+                                         : attn_prefill_f16_supports(pool->g, group) &&
+                                               (pool->g.head_dim == 128 || max_rows * group > 16 ||
+                                                (pool->g.head_dim == 256 && blocks > round && blocks <= 2 * round));
     return q_pos_dev == nullptr && aligned16(q_dev) && aligned16(out_dev) &&
-           !takes_splitk_f16(pool, in, n, q_heads, q_pos_dev) &&
-           !(pool->elem_f16 ? attn_prefill_f16_supports(pool->g, group) : attn_splitk_f32_supports(pool->g, group, max_rows)) &&
+           !takes_splitk_f16(pool, in, n, q_heads, q_pos_dev) && !has_own &&
            attn_splitk_any_supports(pool->g, group, max_rows);
 }
 
@@ -668,12 +684,12 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     for (uint32_t i = 0; i < n; ++i) max_rows = std::max(max_rows, in[i].rows);
     const bool mfma = takes_splitk_f16(pool, in, n, q_heads, q_pos_dev);
     // Blocks of many rows (prefill chunks) on the same pools take the MFMA prefill kernel.
-    const bool prefill = !mfma && pool->elem_f16 && q_pos_dev == nullptr &&
+    const bool any = takes_splitk_any(pool, in, n, q_heads, q_dev, out_dev, q_pos_dev);
+    const bool prefill = !mfma && !any && pool->elem_f16 && q_pos_dev == nullptr &&
                          attn_prefill_f16_supports(pool->g, group);
     // Decode steps and short blocks on f32 pools of head_dim 128: the f32 MFMA split-K kernel.
     const bool f32fast = !pool->elem_f16 && q_pos_dev == nullptr &&
                          attn_splitk_f32_supports(pool->g, group, max_rows);
-    const bool any = takes_splitk_any(pool, in, n, q_heads, q_dev, out_dev, q_pos_dev);
     const uint32_t rpb =
         (mfma || prefill || f32fast || any) ? 0 : attn_generic_rows_per_block(group, pool->g.head_dim);
     if (!mfma && !prefill && !f32fast && !any && rpb == 0)
@@ -2572,17 +2588,18 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
     for (const PlanInput &p : active)
         most_blocks = std::max(most_blocks, (p.kv_len + 31) / 32 - p.kv_lo / 32);
     const bool splitk = takes_splitk_f16(pool, active.data(), uint32_t(active.size()), num_q_heads, nullptr);
+    const bool any = !active.empty() &&
+                     takes_splitk_any(pool, active.data(), uint32_t(active.size()), num_q_heads, q_dev, out_dev, nullptr);
     // (With the queries as two halves the block kernel runs its two-tile form, which brings no
     // rows along: the append is a launch of its own.)
     const bool block_fuses =
-        !splitk && pool->elem_f16 && !active.empty() && !(pool->q_two_halves && pool->g.head_dim == 128) &&
+        !splitk && !any && pool->elem_f16 && !active.empty() && !(pool->q_two_halves && pool->g.head_dim == 128) &&
         attn_prefill_f16_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows, most_blocks);
     const bool fuse =
         splitk || block_fuses ||
         (!pool->elem_f16 && !active.empty() &&
          attn_splitk_f32_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows)) ||
-        (!active.empty() && aligned16(k_dev) && aligned16(v_dev) &&
-         takes_splitk_any(pool, active.data(), uint32_t(active.size()), num_q_heads, q_dev, out_dev, nullptr) &&
+        (any && aligned16(k_dev) && aligned16(v_dev) &&
          attn_splitk_any_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows));
     // The allocation-free form plans first and refuses, before anything changes, a step whose
     // launches need more workspace than the static array has.

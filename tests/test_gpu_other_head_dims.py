@@ -104,3 +104,44 @@ def test_values_that_are_not_finite_reach_the_rows_that_see_them(elem, d, rows):
         fine = np.isfinite(want)
         assert (~fine).any() and rel_err(got[fine], want[fine]) <= 1e-5
         pool.close()
+
+
+# Head dims of the block kernel: steps of up to 16 query vectors run here too, to f32's precision.
+@pytest.mark.parametrize("window", [None, 100])
+@pytest.mark.parametrize("d,q_heads,kv_heads", [(64, 32, 4), (96, 8, 8), (256, 16, 1)])
+def test_short_steps_at_the_block_kernels_head_dims(d, q_heads, kv_heads, window):
+    P = pkg()
+    rng = np.random.default_rng(d)
+    kind = P.LayerKind.Global if window is None else P.LayerKind.windowed(window)
+    okind = oracle.LayerKind.Global if window is None else oracle.LayerKind.windowed(window)
+    pool = P.KvPool([kind], kv_heads, d, elem="f16", max_slots=2, capacity_rows=700)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    caches = [pool.acquire() for _ in range(2)]
+    refs = [oracle.KvCache.new([okind], kv_heads, d, store_f16=True) for _ in range(2)]
+    most = 16 // (q_heads // kv_heads)
+    for i, rows in enumerate(([most, 1], [1, 1], 300, [1, most], [1, 1], 300, [most, most], [1, 1])):
+        if isinstance(rows, int):  # a prompt, so that contexts are split too
+            k, v = normal(rng, rows, kv_heads * d), normal(rng, rows, kv_heads * d)
+            kd, vd = dev(k), dev(v)
+            for at in range(0, rows, 50):
+                pool.append_device(0, [(caches[0], 50)], kd[at:].data_ptr(), vd[at:].data_ptr())
+            for r in range(rows):
+                refs[0].append(0, k[r], v[r], refs[0].next_position(0))
+            continue
+        softcap = 30.0 if i % 3 == 2 else 0.0
+        total = sum(rows)
+        q = normal(rng, total, q_heads * d)
+        k, v = normal(rng, total, kv_heads * d), normal(rng, total, kv_heads * d)
+        qd, kd, vd = dev(q), dev(k), dev(v)
+        out = torch.empty_like(qd)
+        pool.attention_step_device(0, list(zip(caches, rows)), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(),
+                                   out.data_ptr(), q_heads, softcap=softcap)
+        torch.cuda.synchronize()
+        got, at = out.cpu().numpy(), 0
+        for s, r in enumerate(rows):
+            base = refs[s].next_position(0)
+            want = oracle.attention_step(refs[s], 0, q[at:at + r], k[at:at + r], v[at:at + r], q_heads, base,
+                                         oracle.AttentionParams(softcap=softcap), threads=8)
+            assert rel_err(got[at:at + r].reshape(-1), want) <= 1e-5, (rows, s, base)
+            at += r
+    pool.close()
