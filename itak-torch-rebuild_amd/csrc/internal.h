@@ -110,15 +110,15 @@ struct AppendBatch {
     uint32_t n;
     uint32_t total_rows;
     uint32_t ring;      // storage rows of a windowed layer's ring (position p lives in row p % ring); 0 = row p
-    // The launch moves total_rows source rows: rows [0, gap_at) and, when gap_rows != 0, the
-    // rows from gap_at + gap_rows on (the rows in between go another way).
-    uint32_t gap_at;
-    uint32_t gap_rows;
     uint32_t pad;
     AppendItem item[kMaxBatchItems];
 };
 hipError_t launch_append(void *layer_base, int elem_f16, const PoolGeom &g, const AppendBatch &b,
                          const float *k_src, const float *v_src, hipStream_t stream);
+// One item's run of rows into blocked f16 planes; sources aligned to 16 bytes, ring (a multiple of
+// 32, 0 = none) at least `rows` long.
+hipError_t launch_append_chunk(void *layer_base, const PoolGeom &g, uint32_t slot, uint32_t pos0, uint32_t rows,
+                               uint32_t ring, const float *k_src, const float *v_src, hipStream_t stream);
 
 // ---- zero fill of dropped rows (truncate scrub, slot reset) ------------------------
 struct ZeroItem {

@@ -54,8 +54,7 @@ __global__ __launch_bounds__(256) void kv_append_kernel(T *__restrict__ layer_ba
     const uint64_t per_row = 2ull * g.kv_heads * chunks;
     const uint64_t idx = blockIdx.x * 256ull + threadIdx.x;
     if (idx >= per_row * b.total_rows) return;
-    uint32_t row = uint32_t(idx / per_row);  // among the rows this launch moves, then in the source
-    if (b.gap_rows && row >= b.gap_at) row += b.gap_rows;
+    const uint32_t row = uint32_t(idx / per_row);
     uint32_t rem = uint32_t(idx % per_row);
     const uint32_t side = rem / (g.kv_heads * chunks);
     rem -= side * g.kv_heads * chunks;
@@ -290,6 +289,73 @@ __global__ __launch_bounds__(256) void kv_restore_blocked(uint16_t *__restrict__
         }
         __syncthreads();
     }
+}
+
+// A prompt chunk's rows into blocked planes, wherever the run starts and ends: a workgroup moves
+// one side of one (32-position block, kv head), source rows through LDS as in kv_restore_blocked. Only
+// the run's own rows are written: whole 16-byte value pieces where all eight keys of a piece belong to
+// the run, single halves at its two edges, so that on a ring the older rows beside it stay. One launch
+// where the run's head, body and tail were up to three; twice the workgroups of one per block, because
+// a chunk of a few hundred rows is bound by latency (load, barrier, store), not by bytes.
+// grid = (blocks the run touches, kv heads, 2 sides).
+template <int HD>
+__global__ __launch_bounds__(256) void kv_append_chunk(uint16_t *__restrict__ layer_base, PoolGeom g, uint32_t slot,
+                                                       uint32_t pos0, uint32_t rows, uint32_t ring_blocks,
+                                                       const float *__restrict__ k_src, const float *__restrict__ v_src) {
+    extern __shared__ uint16_t tile[];  // [32][head_dim + 8]
+    const uint32_t head = blockIdx.y, side = blockIdx.z;
+    const uint32_t D = HD ? uint32_t(HD) : g.head_dim, stride = D + 8, chunks = D / 4;
+    const uint32_t kb = pos0 / kVBlock + blockIdx.x;
+    const uint32_t from = max(pos0, kb * kVBlock) - kb * kVBlock;
+    const uint32_t to = min(pos0 + rows - kb * kVBlock, kVBlock);  // this block's rows [from, to)
+    const float *src = (side ? v_src : k_src) + (int64_t(kb) * kVBlock - int64_t(pos0)) * int64_t(g.kv_heads * D) + head * D;
+    uint16_t *blk = layer_base + slot * g.slot_stride + side * g.side_stride + head * g.head_stride +
+                    uint64_t(ring_blocks ? kb % ring_blocks : kb) * (kVBlock * D);
+    for (uint32_t i = from * chunks + threadIdx.x; i < to * chunks; i += 256) {
+        const uint32_t r = i / chunks, c = (i % chunks) * 4;
+        typedef float f4v __attribute__((ext_vector_type(4)));
+        const f4v q = __builtin_nontemporal_load(reinterpret_cast<const f4v *>(src + int64_t(r) * (g.kv_heads * D) + c));
+        store4(tile + r * stride + c, make_float4(q[0], q[1], q[2], q[3]));
+    }
+    __syncthreads();
+    if (side == 0) {
+        for (uint32_t piece = threadIdx.x; piece < kVBlock * (D / 8); piece += 256) {
+            const uint32_t i = piece % 16, tc = piece / 16, c = tc % (D / 8), t = tc / (D / 8);
+            const uint32_t key = (i >> 2) * 8 + t * 4 + (i & 3);
+            if (key >= from && key < to)
+                *reinterpret_cast<uint4 *>(blk + uint64_t(piece) * 8) = *reinterpret_cast<const uint4 *>(tile + key * stride + c * 8);
+        }
+        return;
+    }
+    for (uint32_t i = threadIdx.x; i < D * (kVBlock / 8); i += 256) {
+        const uint32_t d = i / (kVBlock / 8), r8 = (i % (kVBlock / 8)) * 8;
+        if (r8 + 8 <= from || r8 >= to) continue;
+        uint16_t v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = tile[(r8 + e) * stride + d];
+        uint16_t *dst = blk + d * kVBlock + r8;
+        if (r8 >= from && r8 + 8 <= to) {
+            *reinterpret_cast<uint4 *>(dst) = make_uint4(v[0] | (uint32_t(v[1]) << 16), v[2] | (uint32_t(v[3]) << 16),
+                                                         v[4] | (uint32_t(v[5]) << 16), v[6] | (uint32_t(v[7]) << 16));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (r8 + e >= from && r8 + e < to) dst[e] = v[e];
+        }
+    }
+}
+
+hipError_t launch_append_chunk(void *layer_base, const PoolGeom &g, uint32_t slot, uint32_t pos0, uint32_t rows,
+                               uint32_t ring, const float *k_src, const float *v_src, hipStream_t stream) {
+    if (rows == 0) return hipSuccess;
+    const dim3 grid((pos0 % kVBlock + rows + kVBlock - 1) / kVBlock, g.kv_heads, 2);
+    const size_t lds = size_t(kVBlock) * (g.head_dim + 8) * sizeof(uint16_t);
+    uint16_t *base = static_cast<uint16_t *>(layer_base);
+    if (g.head_dim == 128)
+        launch_kernel(kv_append_chunk<128>, grid, 256, lds, stream, base, g, slot, pos0, rows, ring / kVBlock, k_src, v_src);
+    else
+        launch_kernel(kv_append_chunk<0>, grid, 256, lds, stream, base, g, slot, pos0, rows, ring / kVBlock, k_src, v_src);
+    return hipGetLastError();
 }
 
 // Element-wise fallback for head dims or alignments the vector paths cannot take.
