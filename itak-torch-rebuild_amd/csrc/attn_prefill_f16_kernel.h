@@ -69,7 +69,7 @@ __host__ __device__ inline uint32_t padded_group(uint32_t group) {
 }
 // New rows a launch that appends its own rows carries at most: sixteen 16-byte pieces a thread.
 constexpr int fuse_rows(int d) { return d <= 128 ? 64 : 16; }
-constexpr uint32_t kOneTileBlocks = 520;  // key blocks up to which blocks of <= 512 vectors take one tile
+constexpr uint32_t kFuseBlocks = 520;  // key blocks up to which short blocks append in the launch
 
 __device__ __forceinline__ float column_max4(float v) {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -88,8 +88,7 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
 // The direct-to-LDS load is issued from inline assembly: the compiler then neither tracks it
 // (it would make every LDS read wait for all of them) nor needs to, because the only consumer
 // is ordered by the explicit s_waitcnt vmcnt + s_barrier at the top of each iteration.
-constexpr int kStages = 4;      // blocks of the LDS ring: three in flight while one is read
-constexpr int kDeepStages = 8;  // for short runs of blocks, one workgroup per compute unit
+constexpr int kStages = 4;  // blocks of the LDS ring: three in flight while one is read
 
 __device__ __forceinline__ void lds_dma16(const void *src, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
@@ -111,7 +110,7 @@ __device__ __forceinline__ void wait_vmcnt() {
 // halves, q = hi + lo with hi = f16(q) and lo = f16(q - hi), and every score is K.hi + K.lo: the
 // queries' rounding to f16, which is relative to each channel and so grows with the scores,
 // leaves the scores. Half as many score products again on a kernel the matrix pipe bounds.
-template <int N, bool SOFTCAP, int kTiles, bool RING, int STAGES, int D, bool QLO = false>
+template <int N, bool SOFTCAP, int kTiles, bool RING, int D, bool QLO = false>
 __global__ __launch_bounds__(kWaves * 64, D <= 128 ? 2 : 1) void attn_prefill_f16_kernel(
     AttnParams p, AttnBatchT<N> b, uint32_t total_partials) {
     constexpr int kD = D;
@@ -232,7 +231,7 @@ __global__ __launch_bounds__(kWaves * 64, D <= 128 ? 2 : 1) void attn_prefill_f1
         // number of loads in flight stays the same in every iteration.
         const uint64_t off = uint64_t(RING ? next_sb : min(kb, max(nblocks, 1u) - 1)) * kBlockVec;
         if (RING && kb + 1 < nblocks) next_sb = next_sb + 1 == ring_blocks ? 0 : next_sb + 1;
-        const uint32_t dst = dma_base + (kb % STAGES) * kStageBytes;
+        const uint32_t dst = dma_base + (kb % kStages) * kStageBytes;
 #pragma unroll
         for (int i = 0; i < kPieces; ++i) {
             const uint32_t ii = i == kPieces - 1 ? last_piece : uint32_t(i);
@@ -306,10 +305,10 @@ __global__ __launch_bounds__(kWaves * 64, D <= 128 ? 2 : 1) void attn_prefill_f1
                          : "v"(qp[qt] + (s >> 1) * 32 + (s & 1) * 4)                            \
                          : "memory");
 #define ITAK_RING_FILL                                                                          \
-    _Pragma("unroll") for (int ahead = 0; ahead < STAGES - 1; ++ahead) issue_block(kb_begin + ahead);
+    _Pragma("unroll") for (int ahead = 0; ahead < kStages - 1; ++ahead) issue_block(kb_begin + ahead);
 // Everything older than the ring's loads has landed. The registers named after the wait pass
 // through an (empty) statement behind it, so that nothing that reads them is scheduled ahead.
-#define ITAK_WAIT_BEHIND_RING asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLoads * (STAGES - 1)) : "memory");
+#define ITAK_WAIT_BEHIND_RING asm volatile("s_waitcnt vmcnt(%0)" : : "n"(kLoads * (kStages - 1)) : "memory");
 #define ITAK_Q_ARRIVED(qraw)                                                                    \
     _Pragma("unroll") for (int qt = 0; qt < kTiles; ++qt)                                       \
         _Pragma("unroll") for (int s = 0; s < 2 * kSteps; ++s) asm volatile("" : "+v"(qraw[qt][s]));
@@ -451,22 +450,22 @@ __global__ __launch_bounds__(kWaves * 64, D <= 128 ? 2 : 1) void attn_prefill_f1
     }
 
     for (uint32_t kb = kb_begin; kb < nblocks; ++kb) {
-        // This thread's pieces of block kb have landed (the loads of the next STAGES - 2 blocks
+        // This thread's pieces of block kb have landed (the loads of the next kStages - 2 blocks
         // may still fly); after the barrier everybody's have, and everybody is done with
         // block kb - 1, whose stage the loads for block kb + 3 may now overwrite.
-        wait_vmcnt<kLoads * (STAGES - 2)>();
+        wait_vmcnt<kLoads * (kStages - 2)>();
         if (kb == kb_begin) { ITAK_MARK(7) }
         __builtin_amdgcn_s_barrier();
         if (kb == kb_begin) { ITAK_MARK(8) }
-        issue_block(kb + STAGES - 1);
-        const uint16_t *lds_k = lds_ring + (kb % STAGES) * (kStageBytes / 2);
+        issue_block(kb + kStages - 1);
+        const uint16_t *lds_k = lds_ring + (kb % kStages) * (kStageBytes / 2);
         const uint16_t *lds_v = lds_k + kBlockElems;
         if constexpr (kCanFuse) {
             if (patches && (kb + 1) * kBlockKeys > item.pos0) {
                 // The block holds new positions: what the loads brought for them is whatever
                 // the planes held (the storing workgroup may or may not have got there yet);
                 // the rows themselves go over it, in the stage's layouts.
-                uint16_t *sk = lds_ring + (kb % STAGES) * (kStageBytes / 2), *sv = sk + kBlockElems;
+                uint16_t *sk = lds_ring + (kb % kStages) * (kStageBytes / 2), *sv = sk + kBlockElems;
 #pragma unroll
                 for (int u = 0; u < kFusePieces; ++u) {
                     const uint32_t r = nrow + uint32_t(kRowsPerPass) * u;
@@ -770,28 +769,16 @@ __global__ __launch_bounds__(kWaves * 64, D <= 128 ? 2 : 1) void attn_prefill_f1
     ITAK_MARK_END
 }
 
-template <int N, bool SOFTCAP, int TILES, bool RING, int STAGES, int D, bool QLO = false>
-hipError_t launch_prefill_ring(const AttnParams &p, const AttnBatch &b,
+template <int N, bool SOFTCAP, int TILES, bool RING, int D, bool QLO = false>
+hipError_t launch_prefill(const AttnParams &p, const AttnBatch &b,
                                       uint32_t total_partials, hipStream_t stream) {
-    constexpr size_t lds = size_t(STAGES) * stage_bytes(D);
+    constexpr size_t lds = size_t(kStages) * stage_bytes(D);
     static const hipError_t granted = hipFuncSetAttribute(
-        reinterpret_cast<const void *>(&attn_prefill_f16_kernel<N, SOFTCAP, TILES, RING, STAGES, D, QLO>),
+        reinterpret_cast<const void *>(&attn_prefill_f16_kernel<N, SOFTCAP, TILES, RING, D, QLO>),
         hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (granted != hipSuccess) return granted;
-    launch_kernel(attn_prefill_f16_kernel<N, SOFTCAP, TILES, RING, STAGES, D, QLO>, b.total_blocks, kWaves * 64, lds, stream, p, AttnBatchT<N>(b), total_partials);
+    launch_kernel(attn_prefill_f16_kernel<N, SOFTCAP, TILES, RING, D, QLO>, b.total_blocks, kWaves * 64, lds, stream, p, AttnBatchT<N>(b), total_partials);
     return hipGetLastError();
-}
-
-template <int N, bool SOFTCAP, int TILES, bool RING, int D, bool QLO = false>
-hipError_t launch_prefill(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
-                                 hipStream_t stream) {
-    if constexpr (D <= 128) {
-        if (b.deep_ring)
-            return launch_prefill_ring<N, SOFTCAP, TILES, RING, kDeepStages, D, QLO>(p, b, total_partials, stream);
-    } else if (b.deep_ring) {
-        return hipErrorInvalidValue;
-    }
-    return launch_prefill_ring<N, SOFTCAP, TILES, RING, kStages, D, QLO>(p, b, total_partials, stream);
 }
 
 // Softcap, ring and tile count chosen for one head_dim. BY_CLASS: an instantiation per batch

@@ -289,7 +289,7 @@ struct AttnBatch {
     uint32_t n;
     uint32_t total_blocks;
     uint32_t rows_per_block;
-    uint32_t deep_ring;  // host side only: the block kernel's plan asks for its deeper LDS ring
+    uint32_t tiles;      // host side only: column tiles per wavefront in the block kernel's plan
     uint32_t fold_units; // host side only: the block kernel's plan for AttnParams::fold_units
     uint32_t two_halves; // host side only: the block kernel multiplies each query as two f16 halves
     uint32_t whole_on_eight; // host side only: the split-K plan leaves every item whole on eight wavefronts

@@ -705,7 +705,7 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         const uint32_t count = std::min<uint32_t>(kMaxBatchItems, n - first);
         AttnBatch b;  // (cleared item by item: all 64 are three kilobytes)
         b.n = count;
-        b.total_blocks = b.rows_per_block = b.deep_ring = b.fold_units = b.whole_on_eight = 0;
+        b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = 0;
         b.two_halves = prefill && pool->q_two_halves && pool->g.head_dim == 128 ? 1 : 0;
         uint32_t total_rows = 0;
         for (uint32_t i = 0; i < count; ++i) {
