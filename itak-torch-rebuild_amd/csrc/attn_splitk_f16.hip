@@ -60,6 +60,7 @@ static Variant pick_variant(const PoolGeom &g, const AttnBatch &b, uint32_t grou
         rows = std::max(rows, b.item[i].rows);
         blocks += uint64_t(g.kv_heads) * item_block_count(b.item[i]);
     }
+    if (b.tiled) return {1, int(b.tiled), b.tiled == 8 ? 1 : 0};
     if (nvec > 32) return {4, 4, 3};
     if (nvec > 16) return {2, 4, 2};
     // (Eight wavefronts for one-row steps only: that variant leaves out the exact treatment of
@@ -97,6 +98,31 @@ static hipError_t grant_lds(size_t lds) {
             e = hipFuncSetAttribute(kernels[k], hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e == hipSuccess) granted = lds;
     return e;
+}
+template <int W>
+static hipError_t grant_tiled_lds(size_t lds) {
+    if (lds <= 64 * 1024) return hipSuccess;
+    static const hipError_t granted = [](size_t bytes) {
+        const void *kernels[] = {
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_kernel<W, 1, false>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_kernel<W, 8, false>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_kernel<W, 64, false>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_kernel<W, 1, true>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_kernel<W, 8, true>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_kernel<W, 64, true>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_prep_kernel<W, 1, false>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_prep_kernel<W, 8, false>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_prep_kernel<W, 64, false>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_prep_kernel<W, 1, true>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_prep_kernel<W, 8, true>),
+            reinterpret_cast<const void *>(&attn_splitk_f16_tiled_prep_kernel<W, 64, true>)};
+        for (const void *k : kernels) {
+            const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes));
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }(lds);
+    return granted;
 }
 // Workgroups of a variant the device holds at once (registers and LDS decide), asked of the
 // runtime once per variant: the smallest figure over every instantiation a launch of the
@@ -150,48 +176,86 @@ static uint32_t variant_capacity(const Variant &v) {
     }
 }
 
-// Blocks up to which a batch's items stay whole: one workgroup per KV head walks the context, and
-// there is neither a partial nor a merge launch. A compute unit reads 16 KB of keys and values
-// (a block) in 0.25 us, a merge launch costs 3 us in a single-slot step; a wavefront's second block
-// costs half a microsecond. One-row steps take eight wavefronts from the fifth block on: up to 12
-// blocks, where the next wavefront's round begins to cost what the merge does, 18 for launches that
-// prepare their rows (their workgroups of one block each spend 2 us on that, and the whole form has
-// fewer of them), 24 from 64 workgroups on (the merge of many slots costs more). Longer steps have
-// four wavefronts only. One layer of 32 Q / 4 KV heads, us, split -> whole: 1 slot at 200 / 300 rows
+// Blocks up to which a batch's items stay whole: one workgroup per KV head (and 16 query vectors) walks
+// the context, and there is neither a partial nor a merge launch. A compute unit reads 16 KB of keys and
+// values (a block) in 0.25 us, a merge launch costs 3 us in a single-slot step; a wavefront's second block
+// costs half a microsecond. Eight wavefronts from the fifth block on. One-row steps: up to 12 blocks,
+// where the next wavefront's round begins to cost what the merge does, 18 for launches that prepare
+// their rows (their workgroups of one block each spend 2 us on that, and the whole form has fewer of
+// them), 24 from 64 workgroups on (the merge of many slots costs more). Steps of several rows, whose merge
+// is larger, up to 16, 24 from 128 workgroups on (up to 8 blocks in the forms that take a unit's vectors
+// together). One layer of 32 Q / 4 KV heads, us, split -> whole: 1 slot at 200 / 300 rows
 // 7.3 / 7.4 -> 5.1 / 5.4 (7.2 -> 7.2 at 400), 16 slots at 300 / 600 11.0 / 12.7 -> 8.7 / 11.1, with
-// preparation 1 slot at 200 / 500 9.2 / 9.3 -> 6.2 / 8.6; six rows at 200 10.7 -> 9.7.
-static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, bool one_row, bool prepares) {
-    if (!one_row) return 8;
+// preparation 1 slot at 200 / 500 9.2 / 9.3 -> 6.2 / 8.6; seven rows at 150 / 350 / 500 8.6 / 8.9 / 8.9 ->
+// 6.8 / 7.2 / 7.8, 8 slots of them at 700 13.8 -> 13.1.
+static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows, uint32_t tiles, bool prepares,
+                            bool may_tile) {
+    if (rows > 1) return !may_tile ? 8 : g.kv_heads * b.n * tiles >= 128 ? 24 : 16;
     if (g.kv_heads * b.n >= 64) return 24;
     return prepares ? 18 : 12;
 }
 
+// The tiled form gives every 16 query vectors of a unit (item, KV head) workgroups of their own, with one
+// set of operand registers a wavefront instead of two (165 registers, three wavefronts a SIMD): no
+// accumulators of 32 or 64 vectors to merge over the wavefronts (128 KB of LDS at 64), nothing rescaled
+// in accumulation registers, and a step of a few blocks spreads over more of the device. The unit's keys
+// and values are read once per tile, out of one L2: where a launch is bound by what it reads, the forms of
+// two and four tiles a wavefront are the better ones. Four tiles: up to 9 blocks per compute unit, 7 where
+// 16 units and more leave those forms at most 16 splits to merge; two tiles: up to 20. One tile always
+// (one workgroup per compute unit, of eight wavefronts from 16 blocks on: twice as many, with
+// half the run, lost everywhere to the larger merge). 32 Q / 4 KV heads, us a layer, before -> tiled: seven
+// rows at 1,000 / 4,096 / 16,384 11.4 / 12.5 / 18.3 -> 9.0 / 9.8 / 16.9, four rows 9.5 / 9.9 / 15.5 ->
+// 8.4 / 8.8 / 13.1, 8 slots of four rows at 2,000 16.5 -> 14.6; one row at 16,384 12.3 -> 11.6.
+static bool takes_tiles(const PoolGeom &g, const AttnBatch &b, uint32_t tiles, uint64_t blocks, uint64_t cus) {
+    return tiles == 1 || blocks <= (tiles == 2 ? 20 : g.kv_heads * b.n < 16 ? 9 : 7) * cus;
+}
+
 // Fills splits / keys_per_split / block0 / ws0 for a batch (the caller has set slot, rows,
 // pos0, q_row0, kv_len) and returns the number of partials the launch will write.
-// Every (item, KV head) is cut into equal runs of at most T blocks, T the smallest run for
-// which the whole batch fits the device in one wave of dispatch; a run is never shorter
-// than one block per wavefront.
-uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares) {
+// Every unit is cut into equal runs of at most T blocks, T the smallest run for which the whole
+// batch fits the device in one wave of dispatch; a run is never shorter than one block per wavefront.
+// may_tile = false keeps the forms that the exchange inside the launch and the queries as two
+// halves are written for.
+uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares, bool may_tile) {
+    const uint32_t group = q_heads / g.kv_heads;
     uint32_t most = 0, most_rows = 0;
-    for (uint32_t i = 0; i < b.n; ++i) {
-        most = std::max(most, item_block_count(b.item[i]));
-        most_rows = std::max(most_rows, b.item[i].rows);
-    }
-    const bool whole = most <= whole_limit(g, b, most_rows == 1, prepares);
-    b.whole_on_eight = whole && most_rows == 1 && most > 4 ? 1 : 0;
-    const Variant v = pick_variant(g, b, q_heads / g.kv_heads);
-    const uint64_t capacity = variant_capacity(v);
     uint64_t blocks = 0;
-    for (uint32_t i = 0; i < b.n; ++i) blocks += uint64_t(g.kv_heads) * item_block_count(b.item[i]);
-    uint64_t T = std::max<uint64_t>((blocks + capacity - 1) / capacity, uint64_t(v.waves));
-    if (whole) T = std::max<uint64_t>(T, most);
-    for (;; ++T) {
+    for (uint32_t i = 0; i < b.n; ++i) {
+        const uint32_t nb = item_block_count(b.item[i]);
+        most = std::max(most, nb);
+        most_rows = std::max(most_rows, b.item[i].rows);
+        blocks += uint64_t(g.kv_heads) * nb;
+    }
+    const uint64_t cus = compute_units();
+    const uint32_t tiles = (most_rows * group + 15) / 16;
+    const bool may = may_tile && takes_tiles(g, b, tiles, blocks, cus);
+    const bool whole = most <= whole_limit(g, b, most_rows, tiles, prepares, may);
+    b.whole_on_eight = whole && most > 4 && (may || most_rows == 1) ? 1 : 0;
+    // (A whole one-row step has no second tile and hardly a second block: the form with two sets of
+    // operands, whose next block is under way before the first is multiplied, is 0.4 us faster.)
+    b.tiled = !may || (whole && most_rows == 1) ? 0
+              : (whole ? b.whole_on_eight != 0 : tiles == 1 && blocks >= 16 * cus) ? 8 : 4;
+    auto units_of = [&](const AttnItem &it) { return g.kv_heads * (b.tiled ? (it.rows * group + 15) / 16 : 1u); };
+    auto groups_at = [&](uint32_t run) {
         uint64_t groups = 0;
-        for (uint32_t i = 0; i < b.n; ++i) {
-            const uint64_t nb = item_block_count(b.item[i]);
-            groups += uint64_t(g.kv_heads) * std::max<uint64_t>((nb + T - 1) / T, 1);
-        }
-        if (groups <= capacity || T >= blocks) break;
+        for (uint32_t i = 0; i < b.n; ++i)
+            groups += uint64_t(units_of(b.item[i])) * std::max((item_block_count(b.item[i]) + run - 1) / run, 1u);
+        return groups;
+    };
+    const Variant v = pick_variant(g, b, group);
+    const uint64_t capacity = b.tiled ? cus : variant_capacity(v);
+    blocks = 0;
+    for (uint32_t i = 0; i < b.n; ++i) blocks += uint64_t(units_of(b.item[i])) * item_block_count(b.item[i]);
+    uint32_t T = std::max(uint32_t((blocks + capacity - 1) / capacity), uint32_t(v.waves));
+    if (whole) {
+        T = std::max(T, most);
+    } else if (b.tiled == 4 && most_rows == 1 && !prepares && most <= 96 && groups_at(4) <= 2 * cus) {
+        // Runs of four blocks are the one-row kernel's (attn_decode_f16.hip), of which a compute unit
+        // holds several: up to two each, while no merge has more than 24 splits (4 slots at 2,048
+        // rows 11.0 -> 10.5, 8 KV heads 8 slots at 1,000 12.9 -> 12.5; one slot at 8,192, 65 splits: 8.5 -> 9.8).
+        T = 4;
+    } else if (groups_at(most ? most : 1) < capacity) {
+        while (T < most && groups_at(T) > capacity) ++T;
     }
     uint32_t block0 = 0, ws0 = 0;
     for (uint32_t i = 0; i < b.n; ++i) {
@@ -205,7 +269,7 @@ uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads,
             it.splits > 1 ? uint32_t(((uint64_t(1) << 32) + it.splits - 1) / it.splits) : 0;
         it.block0 = block0;
         it.ws0 = ws0;
-        block0 += g.kv_heads * it.splits;
+        block0 += units_of(it) * it.splits;
         if (it.splits > 1) ws0 += it.rows * q_heads * it.splits;
     }
     b.total_blocks = block0;
@@ -262,6 +326,29 @@ hipError_t launch_attn_splitk_f16(const AttnParams &p, const AttnBatch &b, uint3
     if (!prep && v.index == 0 && attn_decode_f16_takes(p, b))
         return launch_attn_decode_f16(p, b, total_partials, stream, q_two_halves);
     if (q_two_halves) return launch_attn_splitk_f16_qlo(p, b, total_partials, stream, folded);
+    if (b.tiled) {
+#define ITAK_LAUNCH_TILED(W)                                                                                       \
+    do {                                                                                                           \
+        const size_t lds = variant_lds(1, W);                                                                      \
+        hipError_t e = grant_tiled_lds<W>(lds);                                                                    \
+        if (e != hipSuccess) return e;                                                                             \
+        if (prep && p.ring_blocks)                                                                                 \
+            launch_kernel(attn_splitk_f16_tiled_prep_kernel<W, N, true>, b.total_blocks, W * 64, lds, stream, p, AttnBatchT<N>(b), total_partials, *folded); \
+        else if (prep)                                                                                             \
+            launch_kernel(attn_splitk_f16_tiled_prep_kernel<W, N, false>, b.total_blocks, W * 64, lds, stream, p, AttnBatchT<N>(b), total_partials, *folded); \
+        else if (p.ring_blocks)                                                                                    \
+            launch_kernel(attn_splitk_f16_tiled_kernel<W, N, true>, b.total_blocks, W * 64, lds, stream, p, AttnBatchT<N>(b), total_partials); \
+        else                                                                                                       \
+            launch_kernel(attn_splitk_f16_tiled_kernel<W, N, false>, b.total_blocks, W * 64, lds, stream, p, AttnBatchT<N>(b), total_partials); \
+    } while (0)
+        if (b.tiled == 8) {
+            ITAK_DISPATCH_BATCH(b.n, ITAK_LAUNCH_TILED(8));
+        } else {
+            ITAK_DISPATCH_BATCH(b.n, ITAK_LAUNCH_TILED(4));
+        }
+#undef ITAK_LAUNCH_TILED
+        return hipGetLastError();
+    }
 #define ITAK_LAUNCH(NQ, W)                                                                \
     do {                                                                                  \
         const size_t lds = variant_lds(NQ, W);                                            \

@@ -38,9 +38,8 @@ __device__ __forceinline__ uint32_t storage_block(uint32_t kb, uint32_t ring_blo
     return ring_blocks ? kb % ring_blocks : kb;
 }
 
-__device__ __forceinline__ void load_block(BlockOperands &b, const uint16_t *kplane,
-                                           const uint16_t *vplane, uint32_t kb, uint32_t g,
-                                           uint32_t i) {
+__device__ __forceinline__ void load_block_keys(BlockOperands &b, const uint16_t *kplane, uint32_t kb, uint32_t g,
+                                                uint32_t i) {
     // Key rows of MFMA tile t are interleaved so that the lane group g ends up holding
     // scores of the 8 consecutive keys g*8 .. g*8+7: row i of tile t is key
     // (i/4)*8 + t*4 + i%4 of the block. The blocked key plane stores the 16-byte piece
@@ -52,10 +51,18 @@ __device__ __forceinline__ void load_block(BlockOperands &b, const uint16_t *kpl
 #pragma unroll
         for (int s = 0; s < 4; ++s)
             b.k[t][s] = ITAK_KV_LOAD(reinterpret_cast<const half8 *>(kb_base + ((t * 16 + s * 4) * 16) * 8));
+}
+__device__ __forceinline__ void load_block_values(BlockOperands &b, const uint16_t *vplane, uint32_t kb, uint32_t g,
+                                                  uint32_t i) {
     const uint16_t *vb = vplane + uint64_t(kb) * (kBlockKeys * kD) + i * kBlockKeys + g * 8;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt)
         b.v[dt] = ITAK_KV_LOAD(reinterpret_cast<const half8 *>(vb + dt * 16 * kBlockKeys));
+}
+__device__ __forceinline__ void load_block(BlockOperands &b, const uint16_t *kplane, const uint16_t *vplane, uint32_t kb,
+                                           uint32_t g, uint32_t i) {
+    load_block_keys(b, kplane, kb, g, i);
+    load_block_values(b, vplane, kb, g, i);
 }
 
 // Fused append. The workgroup that owns the blocks holding the new positions
@@ -65,8 +72,7 @@ __device__ __forceinline__ void load_block(BlockOperands &b, const uint16_t *kpl
 // nothing depends on the stores within the launch.
 constexpr int kNewStride = kD + 8;  // LDS row stride of the staged new rows (halves)
 
-__device__ __forceinline__ void patch_new_rows(BlockOperands &b, const _Float16 *sm_newk,
-                                               const _Float16 *sm_newv, uint32_t kb, uint32_t g,
+__device__ __forceinline__ void patch_new_keys(BlockOperands &b, const _Float16 *sm_newk, uint32_t kb, uint32_t g,
                                                uint32_t i, uint32_t pos0, uint32_t kv_len) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -77,6 +83,9 @@ __device__ __forceinline__ void patch_new_rows(BlockOperands &b, const _Float16 
             for (int s = 0; s < 4; ++s) b.k[t][s] = *reinterpret_cast<const half8 *>(src + s * 32);
         }
     }
+}
+__device__ __forceinline__ void patch_new_values(BlockOperands &b, const _Float16 *sm_newv, uint32_t kb, uint32_t g,
+                                                 uint32_t i, uint32_t pos0, uint32_t kv_len) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         const uint32_t key = kb * kBlockKeys + g * 8 + e;
@@ -86,6 +95,11 @@ __device__ __forceinline__ void patch_new_rows(BlockOperands &b, const _Float16 
             for (int dt = 0; dt < 8; ++dt) b.v[dt][e] = src[dt * 16];
         }
     }
+}
+__device__ __forceinline__ void patch_new_rows(BlockOperands &b, const _Float16 *sm_newk, const _Float16 *sm_newv,
+                                               uint32_t kb, uint32_t g, uint32_t i, uint32_t pos0, uint32_t kv_len) {
+    patch_new_keys(b, sm_newk, kb, g, i, pos0, kv_len);
+    patch_new_values(b, sm_newv, kb, g, i, pos0, kv_len);
 }
 
 // Reductions over the four lanes that share a query-vector column (lanes l, l^16, l^32,
@@ -109,7 +123,8 @@ __device__ __forceinline__ float column_sum(float v) {
 // What the exact treatment of non-finite value rows needs to know of the item's query rows.
 struct RowSpan {
     uint32_t pos0;    // position of the item's first query row (not clamped)
-    uint32_t rows;
+    uint32_t row_first, row_end;  // the rows of the workgroup's vectors
+    uint32_t vec0;    // and the first of those
     uint32_t window;  // 0 on a global layer
     uint32_t kv_lo;
     uint32_t magic;   // j / group == (j * magic) >> 16
@@ -130,9 +145,9 @@ template <bool RING>
 __device__ __forceinline__ void accumulate_by_row(floatx4 (&o)[8], const BlockOperands &b, half8 pb,
                                                   uint32_t qt, uint32_t key_base, uint32_t jl,
                                                   uint32_t kv_len, const RowSpan &span) {
-    const uint32_t my_row = ((qt * 16 + jl) * span.magic) >> 16;
+    const uint32_t my_row = ((span.vec0 + qt * 16 + jl) * span.magic) >> 16;
 #pragma unroll 1
-    for (uint32_t r = 0; r < span.rows; ++r) {
+    for (uint32_t r = span.row_first; r < span.row_end; ++r) {
         const uint32_t pos = min(span.pos0 + r, kv_len - 1);
         const uint32_t lo = RING ? lowest_visible(span.pos0 + r, span.window, span.kv_lo) : 0u;
         const uint32_t end = min(pos + 1 - min(pos + 1, key_base), 8u);   // this lane's keys up to pos
@@ -197,7 +212,7 @@ __device__ __forceinline__ void process_block(WaveState<NQ> &st, BlockOperands &
         if (!low_edge && span.appends) return span.new_not_finite;
         return any_not_finite(b.v);
     };
-    const bool by_row = BYROW && span.rows > 1 && need_mask && (NQ <= 2 || !tail) && suspect();
+    const bool by_row = BYROW && span.row_end - span.row_first > 1 && need_mask && (NQ <= 2 || !tail) && suspect();
 #pragma unroll
     for (int qt = 0; qt < NQ; ++qt) {
         half8 qb[4];
@@ -302,7 +317,7 @@ __device__ __forceinline__ void process_block(WaveState<NQ> &st, BlockOperands &
         if (tail) zero_tail();
         // (The values are looked at after the tail is cleared: what lies past the stored rows
         // is nobody's to see.)
-        const bool by_row_late = by_row || (BYROW && span.rows > 1 && need_mask && tail && suspect());
+        const bool by_row_late = by_row || (BYROW && span.row_end - span.row_first > 1 && need_mask && tail && suspect());
         if constexpr (!FIRST) {
 #pragma unroll
             for (int qt = 0; qt < NQ; ++qt)
@@ -525,7 +540,9 @@ __device__ __forceinline__ void die_merge(const AttnParams &p, const AttnItem &i
     }
 }
 
-template <int NQ, int WAVES, int N, bool RING, bool PREP, bool DIE, bool QLO = false>
+// TILED: a step of more than 16 query vectors per KV head as so many workgroups of 16 vectors each
+// (attn_splitk_f16.hip says when).
+template <int NQ, int WAVES, int N, bool RING, bool PREP, bool DIE, bool QLO = false, bool TILED = false>
 __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const AttnBatchT<N> &b,
                                                      uint32_t total_partials,
                                                      [[maybe_unused]] const FoldedParams &fold,
@@ -570,6 +587,7 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
     // i % 8, and die d serves KV head d % heads of the items of bin d / heads, one after the
     // other along the die's own index i / 8.
     uint32_t item_at = 0, kv_head = 0, split = 0;
+    uint32_t vec0 = 0;  // first query vector of this workgroup
     if constexpr (DIE) {
         const uint32_t die = blockIdx.x & (kDieCount - 1), idx = blockIdx.x >> 3;
         const uint32_t bin = die >> dm.shift;
@@ -597,10 +615,24 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
     if constexpr (DIE) {
         split = blockIdx.x / kDieCount - item.block0;
     } else {
-        const uint32_t local = blockIdx.x - item.block0;
+        uint32_t local = blockIdx.x - item.block0;
+        if constexpr (TILED) {
+            // Eight units (KV head, split) after eight others, and within the eight a tile after the
+            // other: workgroup i runs on compute die i mod 8, so the tiles of a unit, which read the
+            // same keys and values, find them in one L2.
+            const uint32_t tiles = (nvec + 15) / 16, units = p.g.kv_heads * item.splits;
+            const uint32_t eight = local / (8 * tiles), in = local - eight * 8 * tiles;
+            const uint32_t held = min(8u, units - eight * 8);
+            vec0 = in / held;
+            local = eight * 8 + in - vec0 * held;
+            vec0 *= 16;
+        }
         kv_head = item.splits > 1 ? __umulhi(local, item.splits_magic) : local;
         split = local - kv_head * item.splits;
     }
+    // The rows of this workgroup's vectors.
+    const uint32_t row_first = TILED ? (vec0 * magic) >> 16 : 0;
+    const uint32_t row_last = TILED ? (min(vec0 + 15, nvec - 1) * magic) >> 16 : item.rows - 1;
     // DIE: first partial of this (item, KV head) unit, partial (split, vector j) at
     // unit_ps0 + split * nvec + j; units start on multiples of 16 partials, so that no cache
     // line of the (m, l) pairs is shared between units.
@@ -650,7 +682,7 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
 #pragma unroll
     for (int u = 0; u < QL; ++u) {
         const uint32_t f = tid + u * WAVES * 64;
-        const uint32_t j = min(f >> 5, nvec - 1), c4 = (f & 31) * 4;
+        const uint32_t j = min(vec0 + (f >> 5), nvec - 1), c4 = (f & 31) * 4;
         const uint32_t row = (j * magic) >> 16, head = kv_head * group + (j - row * group);
         qld[u] = *reinterpret_cast<const float4 *>(
             p.q + (uint64_t(item.q_row0 + row) * p.q_heads + head) * kD + c4);
@@ -662,6 +694,20 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
     if constexpr (PREP) {
         if (fold.prep_q_weight) wq = *reinterpret_cast<const float4 *>(fold.prep_q_weight + pc4);
         if (fold.prep_k_weight) wk = *reinterpret_cast<const float4 *>(fold.prep_k_weight + pc4);
+    }
+    // And its pairs' frequencies. First pair index of this lane: interleaved pairs are (2i, 2i+1);
+    // half-split pair i joins channels i and i + rot/2. (Asked for ahead of the keys and values: loads
+    // return in order, and the rotation must not wait for those.)
+    [[maybe_unused]] double freq[4] = {0.0, 0.0, 0.0, 0.0};
+    const uint32_t prot = PREP ? fold.prep_rot : 0;
+    const bool pinter = PREP && fold.prep_interleaved != 0;
+    const int trig_pairs = pinter ? 2 : 4;
+    [[maybe_unused]] const uint32_t pair0 = pinter ? pc4 >> 1 : (pc4 < prot >> 1 ? pc4 : pc4 - (prot >> 1));
+    if constexpr (PREP) {
+        if (prot && fold.prep_freq) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) freq[i] = fold.prep_freq[min(pair0 + i, (prot >> 1) - 1)];
+        }
     }
 
     // ---- 3. the wavefront's first block (a wavefront without one loads the split's first
@@ -675,11 +721,13 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
 
     // ---- 4. in the shadow of the loads: what the mask and the epilogue need per column.
     uint32_t colpos[NQ], collo[NQ], colout[NQ], colps[NQ];
-    const uint32_t lo_min = lowest_visible(item.pos0, window, kv_lo);
-    const uint32_t lo_max = lowest_visible(item.pos0 + item.rows - 1, window, kv_lo);
+    const uint32_t lo_min = lowest_visible(item.pos0 + row_first, window, kv_lo);
+    const uint32_t lo_max = lowest_visible(item.pos0 + row_last, window, kv_lo);
+    const uint32_t first_pos = min(item.pos0 + row_first, item.kv_len - 1);
+    const uint32_t seen_end = TILED ? min(item.pos0 + row_last + 1, item.kv_len) : item.kv_len;
 #pragma unroll
     for (int qt = 0; qt < NQ; ++qt) {
-        const uint32_t j = qt * 16 + jl;
+        const uint32_t j = vec0 + qt * 16 + jl;
         const uint32_t row = (j * magic) >> 16, head = kv_head * group + (j - row * group);
         // A query ahead of the stored rows sees them all: for the mask its position is the
         // last stored one (its window still follows from where it really stands).
@@ -695,20 +743,12 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
     // PREP: this lane's pairs and their rotation at the step's first position, still in the
     // shadow of the loads (nothing here depends on what they bring).
     [[maybe_unused]] PrepTrig trig0;
-    [[maybe_unused]] double freq[4] = {0.0, 0.0, 0.0, 0.0};
-    [[maybe_unused]] int trig_pairs = 0;
-    const uint32_t prot = PREP ? fold.prep_rot : 0;
-    const bool pinter = PREP && fold.prep_interleaved != 0;
     if constexpr (PREP) {
         if (prot) {
-            const uint32_t half = prot >> 1;
-            // First pair index of this lane: interleaved pairs are (2i, 2i+1); half-split pair i
-            // joins channels i and i + rot/2.
-            const uint32_t pair0 = pinter ? pc4 >> 1 : (pc4 < half ? pc4 : pc4 - half);
-            trig_pairs = pinter ? 2 : 4;
+            if (!fold.prep_freq)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (i < trig_pairs) freq[i] = exp2(double(pair0 + i) * fold.prep_freq_step);
+                for (int i = 0; i < 4; ++i)
+                    if (i < trig_pairs) freq[i] = exp2(double(pair0 + i) * fold.prep_freq_step);
             prep_trig(trig0, double(item.pos0), freq, trig_pairs);
         }
     }
@@ -721,7 +761,7 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
         const uint32_t j = f >> 5, c4 = (f & 31) * 4;
         float4 a = qld[u];
         if constexpr (PREP) {
-            const uint32_t jr = min(j, nvec - 1), row = (jr * magic) >> 16;
+            const uint32_t jr = min(vec0 + j, nvec - 1), row = (jr * magic) >> 16;
             PrepTrig t = trig0;
             if (prot && row != 0) prep_trig(t, double(item.pos0 + row), freq, trig_pairs);
             a = prep_chunk(a, fold.prep_q_weight != nullptr, wq, fold.prep_eps, c4, lane, prot, pinter, t);
@@ -729,12 +769,12 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
         const float4 as = make_float4(a.x * qscale, a.y * qscale, a.z * qscale, a.w * qscale);
         half4 h{static_cast<_Float16>(as.x), static_cast<_Float16>(as.y),
                 static_cast<_Float16>(as.z), static_cast<_Float16>(as.w)};
-        if (j >= nvec) h = half4{0, 0, 0, 0};
+        if (vec0 + j >= nvec) h = half4{0, 0, 0, 0};
         *reinterpret_cast<half4 *>(sm_q + j * kQStride + c4) = h;
         if constexpr (QLO) {  // what the rounding to f16 dropped, as a second f16
             half4 l{static_cast<_Float16>(as.x - float(h[0])), static_cast<_Float16>(as.y - float(h[1])),
                     static_cast<_Float16>(as.z - float(h[2])), static_cast<_Float16>(as.w - float(h[3]))};
-            if (j >= nvec) l = half4{0, 0, 0, 0};
+            if (vec0 + j >= nvec) l = half4{0, 0, 0, 0};
             *reinterpret_cast<half4 *>(sm_q_lo + j * kQStride + c4) = l;
         }
     }
@@ -763,6 +803,7 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
             const uint32_t key = item.pos0 + r, kin = key % kBlockKeys;
             const uint64_t blk =
                 uint64_t(storage_block(key / kBlockKeys, ring_blocks)) * (kBlockKeys * kD);
+            if (TILED && vec0 != 0) continue;  // the first tile's workgroup stores
             if (side == 0) {
                 const uint32_t kt = (kin >> 2) & 1, ki = (kin >> 3) * 4 + (kin & 3);
                 *reinterpret_cast<uint2 *>(kplane + blk + ((kt * 16 + (c4 >> 3)) * 16 + ki) * 8 +
@@ -800,7 +841,8 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
     // operand sets, so the next block's loads fly while the current one is multiplied; with
     // 64 vectors the accumulators take that room and the other wavefronts hide the latency.
     WaveState<NQ> st;
-    const RowSpan span{item.pos0, item.rows, window, kv_lo, magic, fused, new_not_finite};
+    const RowSpan span{item.pos0, row_first, row_last + 1, vec0, window, kv_lo, magic, fused, new_not_finite};
+    if constexpr (!TILED) {
 #define ITAK_BLOCK(FIRST, BUF, KB)                                                               \
     do {                                                                                         \
         if (fused && ((KB) + 1) * kBlockKeys > item.pos0)                                        \
@@ -811,17 +853,17 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
         if constexpr (NQ > 2) { /* (no room for two copies beside 128 accumulators; the one copy  \
            costs the 7-row verify block 3 %: 23.7 -> 24.5 us per layer, same box) */             \
             process_block<NQ, FIRST, RING, true, QLO>(st, BUF, qreg, sm_q, sm_q_lo, KB, g, jl, colpos, \
-                                 collo, min(item.pos0, item.kv_len - 1), item.kv_len, lo_min,    \
+                                 collo, first_pos, seen_end, lo_min,    \
                                  lo_max, softcap, inv_cap, span);                                \
-        } else if (WAVES != 8 && item.rows > 1 &&                                                \
-            (((KB) + 1) * kBlockKeys > min(item.pos0, item.kv_len - 1) + 1 ||                    \
+        } else if (WAVES != 8 && row_last > row_first &&                                         \
+            (((KB) + 1) * kBlockKeys > first_pos + 1 ||                                          \
              (RING && (KB) * kBlockKeys < lo_max)))                                              \
             process_block<NQ, FIRST, RING, WAVES != 8, QLO>(st, BUF, qreg, sm_q, sm_q_lo, KB, g, jl, colpos, \
-                                 collo, min(item.pos0, item.kv_len - 1), item.kv_len, lo_min,    \
+                                 collo, first_pos, seen_end, lo_min,    \
                                  lo_max, softcap, inv_cap, span);                                \
         else                                                                                     \
             process_block<NQ, FIRST, RING, false, QLO>(st, BUF, qreg, sm_q, sm_q_lo, KB, g, jl, colpos, collo, \
-                                 min(item.pos0, item.kv_len - 1), item.kv_len, lo_min, lo_max,   \
+                                 first_pos, seen_end, lo_min, lo_max,   \
                                  softcap, inv_cap, span);                                        \
     } while (0)
     if (has_block) {
@@ -858,6 +900,79 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
         }
     }
 #undef ITAK_BLOCK
+    } else {
+        // One set of operand registers: the next block's keys are asked for when the scores have used
+        // this one's, its values when the products have. That leaves the registers for three wavefronts
+        // a SIMD, whose loads fly together; a second set (above) takes a whole SIMD for one.
+        st.m[0] = -INFINITY;
+        st.l[0] = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) st.o[0][dt] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (; kb < kb_end; kb += WAVES) {
+            const uint32_t key_base = kb * kBlockKeys + g * 8, next = kb + WAVES;
+            const bool holds_new = fused && (kb + 1) * kBlockKeys > item.pos0;
+            if (holds_new) patch_new_keys(buf_a, sm_newk, kb, g, jl, item.pos0, item.kv_len);
+            float sc[8];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                floatx4 s = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(buf_a.k[t][k], qreg[k], s, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sc[t * 4 + r] = s[r];
+            }
+            if (next < kb_end) load_block_keys(buf_a, kplane, storage_block(next, ring_blocks), g, jl);
+            if (softcap > 0.0f) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) sc[e] = softcap_log2(sc[e], softcap, inv_cap);
+            }
+            const bool low_edge = RING && kb * kBlockKeys < lo_max;
+            const bool need_mask = (kb + 1) * kBlockKeys > first_pos + 1 || low_edge;
+            if (need_mask) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (key_base + e > colpos[0] || (RING && key_base + e < collo[0])) sc[e] = -INFINITY;
+            }
+            float mx = sc[0];
+#pragma unroll
+            for (int e = 1; e < 8; ++e) mx = fmaxf(mx, sc[e]);
+            mx = column_max(mx);
+            const float m_new = fmaxf(st.m[0], mx);
+            const bool dead = m_new == -INFINITY;  // (see process_block)
+            const float m_ref = dead ? 0.0f : m_new;
+            float sum = 0.0f;
+            half8 pb;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float pe = fast_exp2(sc[e] - m_ref);
+                sum += pe;
+                pb[e] = static_cast<_Float16>(pe);
+            }
+            const float alpha = dead ? 1.0f : fast_exp2(st.m[0] - m_new);
+            st.l[0] = st.l[0] * alpha + sum;
+            st.m[0] = m_new;
+            if (holds_new) patch_new_values(buf_a, sm_newv, kb, g, jl, item.pos0, item.kv_len);
+            if ((kb + 1) * kBlockKeys > seen_end || (RING && kb * kBlockKeys < lo_min)) {
+                const uint32_t end = min(seen_end - min(seen_end, key_base), 8u);
+                const uint32_t first = RING ? min(lo_min - min(lo_min, key_base), 8u) : 0u;
+                const u32x4 keep = first_halves(end) & ~first_halves(first);
+#pragma unroll
+                for (int dt = 0; dt < 8; ++dt) buf_a.v[dt] = keep_halves(buf_a.v[dt], keep);
+            }
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) st.o[0][dt] *= alpha;
+            if (need_mask && row_last > row_first &&
+                __builtin_expect(!low_edge && fused ? new_not_finite : any_not_finite(buf_a.v), false)) {
+                accumulate_by_row<RING>(st.o[0], buf_a, pb, 0, key_base, jl, seen_end, span);
+#pragma unroll
+                for (int dt = 0; dt < 8; ++dt) buf_a.v[dt] = half8{0, 0, 0, 0, 0, 0, 0, 0};
+            }
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt)
+                st.o[0][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(buf_a.v[dt], pb, st.o[0][dt], 0, 0, 0);
+            if (next < kb_end) load_block_values(buf_a, vplane, storage_block(next, ring_blocks), g, jl);
+        }
+    }
 
     // ---- merge the wavefronts through LDS ------------------------------------------------
     ITAK_MARK(6)
@@ -887,7 +1002,7 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
     if (exchanges) xg.init(p.ws, item, kv_head, split, nvec);
 #pragma unroll
     for (int qt = 0; qt < NQ; ++qt) {
-        const uint32_t j = qt * 16 + jl;
+        const uint32_t j = vec0 + qt * 16 + jl;
         floatx4 ow[kDtPerWave][WAVES];
         float mw[WAVES], lw[WAVES];
 #pragma unroll
@@ -988,6 +1103,17 @@ __global__ __launch_bounds__(WAVES * 64) void attn_splitk_f16_prep_kernel(AttnPa
                                                                           uint32_t total_partials,
                                                                           FoldedParams f) {
     attn_splitk_f16_body<NQ, WAVES, N, RING, true, false>(p, b, total_partials, f, DieMap{});
+}
+// The form of 16-vector tiles.
+template <int WAVES, int N, bool RING>
+__global__ __launch_bounds__(WAVES * 64) void attn_splitk_f16_tiled_kernel(AttnParams p, AttnBatchT<N> b,
+                                                                           uint32_t total_partials) {
+    attn_splitk_f16_body<1, WAVES, N, RING, false, false, false, true>(p, b, total_partials, FoldedParams{}, DieMap{});
+}
+template <int WAVES, int N, bool RING>
+__global__ __launch_bounds__(WAVES * 64) void attn_splitk_f16_tiled_prep_kernel(AttnParams p, AttnBatchT<N> b,
+                                                                                uint32_t total_partials, FoldedParams f) {
+    attn_splitk_f16_body<1, WAVES, N, RING, true, false, false, true>(p, b, total_partials, f, DieMap{});
 }
 // The same with the queries as two halves (ITAK_POOL_Q_TWO_HALVES).
 template <int NQ, int WAVES, int N, bool RING>

@@ -292,6 +292,7 @@ struct AttnBatch {
     uint32_t tiles;      // host side only: column tiles per wavefront in the block kernel's plan
     uint32_t fold_units; // host side only: the block kernel's plan for AttnParams::fold_units
     uint32_t two_halves; // host side only: the block kernel multiplies each query as two f16 halves
+    uint32_t tiled; // host side only: the split-K plan gives every 16 query vectors their own workgroups
     uint32_t whole_on_eight; // host side only: the split-K plan leaves every item whole on eight wavefronts
     AttnItem item[kMaxBatchItems];
 };
@@ -399,7 +400,8 @@ struct FoldedParams {
     float prep_eps;
     const float *prep_q_weight; // [head_dim] or null: no norm
     const float *prep_k_weight;
-    double prep_freq_step;      // pair i turns at position * 2^(i * prep_freq_step) radians
+    double prep_freq_step;      // pair i turns at position * 2^(i * prep_freq_step) radians,
+    const double *prep_freq;    // which is prep_freq[i] where the host could make the table
 };
 // sigmoid for the writers of f16-KV attention output, whose bar is 2e-3: one exponential
 // and one reciprocal instruction, a few ulp, the same limits at both ends (0 and 1) as the
@@ -432,7 +434,7 @@ uint32_t attn_generic_tile(uint32_t head_dim);
 // Partials are in log2 domain (combine with base2 = 1).
 bool attn_splitk_f16_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
 // (`prepares`: the launch prepares Q and the new K rows itself.)
-uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares = false);
+uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares = false, bool may_tile = false);
 // After attn_splitk_f16_plan: whether the batch can merge its splits inside the split-K launch
 // (AttnParams::exchange). Returns the 64-bit words the exchange buffer must hold and re-bases
 // the items' ws0 on it, or 0 (items untouched) when the batch keeps the merge launch.

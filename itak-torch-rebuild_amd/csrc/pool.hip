@@ -705,7 +705,7 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         const uint32_t count = std::min<uint32_t>(kMaxBatchItems, n - first);
         AttnBatch b;  // (cleared item by item: all 64 are three kilobytes)
         b.n = count;
-        b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = 0;
+        b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.tiled = 0;
         b.two_halves = prefill && pool->q_two_halves && pool->g.head_dim == 128 ? 1 : 0;
         uint32_t total_rows = 0;
         for (uint32_t i = 0; i < count; ++i) {
@@ -723,7 +723,8 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         }
         uint32_t partials = 0;
         if (mfma) {
-            partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads), folded && folded->prep_on);
+            partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads), folded && folded->prep_on,
+                                            !pool->q_two_halves && !pool->merge_in_launch);
         } else if (prefill) {
             partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, k_new != nullptr);
         } else if (f32fast || any) {
@@ -2716,6 +2717,7 @@ itak_status itak_attention_prep_step_device(itak_pool *pool, uint64_t layer,
         folded.prep_q_weight = prep->q_norm_weight;
         folded.prep_k_weight = prep->k_norm_weight;
         // Pair i turns at position * base^(-2i/rot) = position * 2^(i * step).
+        folded.prep_freq = rotate ? rope_freq_table(pool, prep->rope_base, rotary) : nullptr;
         folded.prep_freq_step = rotate ? -2.0 * std::log2(double(prep->rope_base)) / double(rotary) : 0.0;
         return step_on_device(pool, layer, items, item_count, plan, q_dev, k_dev, v_dev, out_dev,
                               num_q_heads, scale, softcap, &folded);
