@@ -4,7 +4,7 @@
 // keep f32's precision, so that an f16 pool gives here what f32 arithmetic over its rows gives. A
 // short step's new rows are appended by the same launch.
 //
-// The shape of the work is attn_splitk_rows_kernel's (a workgroup of four wavefronts = item, KV
+// The shape of the work is attn_splitk_rows_kernel's (a workgroup of four or eight wavefronts = item, KV
 // head, tile of 16 query vectors, run of 32-key blocks; a private online softmax per wavefront,
 // one merge through LDS) and its launches are planned by the same rule. What differs is the
 // operands. Which channel and which key an MFMA's k index stands for is free, and is chosen so that
@@ -48,7 +48,6 @@ namespace itak {
 
 namespace {
 
-constexpr int kWavesAny = kWavesRows;
 
 // x = h[0] + h[1] + h[2] up to 2^-33 of the largest x the halves hold. A half that is not finite
 // has nothing left to say.
@@ -63,13 +62,13 @@ __device__ __forceinline__ void split3(float x, _Float16 &a, _Float16 &b, _Float
 // outputs carry them too, and lose them in the division.
 constexpr float kWeightShift = 15.0f;
 
-template <int DP, int N>
-__global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk_halves_kernel(AttnParams p, AttnBatchT<N> b,
-                                                                                             uint32_t total_partials) {
+template <int DP, int W, int N>
+__global__ __launch_bounds__(W * 64, DP <= 128 ? 8 / W : 1) void attn_splitk_halves_kernel(AttnParams p, AttnBatchT<N> b,
+                                                                                          uint32_t total_partials) {
     constexpr int kTiles = DP / 16;  // output tiles
     constexpr int kS = DP / 32;      // steps of a key row
-    __shared__ float sm_m[kWavesAny][16], sm_l[kWavesAny][16];
-    __shared__ float sm_o[kWavesAny][kTiles][64][4];  // [wave][tile][lane][row of the lane]
+    __shared__ float sm_m[W][16], sm_l[W][16];
+    __shared__ float sm_o[W][kTiles][64][4];  // [wave][tile][lane][row of the lane]
 
     const uint32_t tid = threadIdx.x;
     const uint32_t wave = tid >> 6, lane = tid & 63;
@@ -124,16 +123,20 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk
     // for the stores before it reads the block; nobody else reads these positions.
     auto append_rows = [&](uint32_t kb) {
         const uint32_t key0 = kb * kBlockKeys;
-        if (p.k_new == nullptr || key0 + kBlockKeys <= item.pos0) return;
+        if (p.k_new == nullptr || key0 + kBlockKeys <= item.pos0 || key0 >= item.pos0 + item.rows) return;
         uint16_t *kblk = kplane + block_at(kb), *vblk = vplane + block_at(kb);
         const uint32_t from = key0 > item.pos0 ? key0 - item.pos0 : 0;
         const uint32_t to = min(item.rows, key0 + kBlockKeys - item.pos0), quads = D / 4;
-        for (uint32_t f = lane; f < (to - from) * 2 * quads; f += 64) {
+        const uint32_t pieces = (to - from) * 2 * quads;
+        auto fetch = [&](uint32_t f, uint32_t &side, uint32_t &kk, uint32_t &c4) {
             const uint32_t r = from + f / (2 * quads), rest = f % (2 * quads);
-            const uint32_t side = rest >= quads ? 1 : 0, c4 = (rest - side * quads) * 4;
-            const floatx4 y = *reinterpret_cast<const floatx4 *>(
+            side = rest >= quads ? 1 : 0;
+            c4 = (rest - side * quads) * 4;
+            kk = (item.pos0 + r) % kBlockKeys;
+            return *reinterpret_cast<const floatx4 *>(
                 (side ? p.v_new : p.k_new) + (uint64_t(item.q_row0 + r) * p.g.kv_heads + kv_head) * D + c4);
-            const uint32_t kk = (item.pos0 + r) % kBlockKeys;
+        };
+        auto place = [&](const floatx4 &y, uint32_t side, uint32_t kk, uint32_t c4) {
             uint16_t h[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) h[e] = f32_to_f16_bits(y[e]);
@@ -144,6 +147,20 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk
                 const uint32_t t = (kk >> 2) & 1, i = (kk >> 3) * 4 + (kk & 3);
                 __builtin_memcpy(__builtin_assume_aligned(kblk + ((t * chunks + c4 / 8) * 16 + i) * 8 + c4 % 8, 8), h, 8);
             }
+        };
+        uint32_t f0 = 0;
+        for (; f0 + 256 <= pieces; f0 += 256) {  // several rows: four pieces a lane under way at a time
+            floatx4 y[4];
+            uint32_t side[4], kk[4], c4[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) y[u] = fetch(f0 + 64 * u + lane, side[u], kk[u], c4[u]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) place(y[u], side[u], kk[u], c4[u]);
+        }
+        for (uint32_t f = f0 + lane; f < pieces; f += 64) {
+            uint32_t side, kk, c4;
+            const floatx4 y = fetch(f, side, kk, c4);
+            place(y, side, kk, c4);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores have been acknowledged
     };
@@ -162,10 +179,13 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk
             v[c] = *reinterpret_cast<const half8 *>(vblk + min(16u * c + jl, D - 1) * kVBlock + 8 * g);
     };
     uint32_t kb = kb_begin + wave;
-    if (kb < kb_end) {
-        append_rows(kb);
-        load_keys(kb);
-        load_values(kb);
+    if (kb < kb_end) append_rows(kb);
+    {
+        // (A wavefront without a block loads one and ignores it: behind a branch the wait for the queries
+        // would be a wait for every load.)
+        const uint32_t some = min(kb, (item.kv_len - 1) / kBlockKeys);
+        load_keys(some);
+        load_values(some);
     }
     __builtin_amdgcn_sched_barrier(0);
 
@@ -239,8 +259,8 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk
         return alpha;
     };
 
-    for (; kb < kb_end; kb += kWavesAny) {
-        const uint32_t key0 = kb * kBlockKeys, next = kb + kWavesAny;
+    for (; kb < kb_end; kb += W) {
+        const uint32_t key0 = kb * kBlockKeys, next = kb + W;
         float sc[2][4];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -301,7 +321,7 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk
             l_run = 0.0f;
             floatx4 out = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-            for (uint32_t kb = kb_begin + wave; kb < kb_end; kb += kWavesAny) {
+            for (uint32_t kb = kb_begin + wave; kb < kb_end; kb += W) {
                 const uint32_t key0 = kb * kBlockKeys;
                 const uint64_t at = uint64_t(ring_blocks ? kb % ring_blocks : kb) * (kVBlock * D);
                 floatx4 acc[2] = {};
@@ -353,10 +373,10 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk
 
     float M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < kWavesAny; ++w) M = fmaxf(M, sm_m[w][jl]);
-    float L = 0.0f, wgt[kWavesAny];
+    for (int w = 0; w < W; ++w) M = fmaxf(M, sm_m[w][jl]);
+    float L = 0.0f, wgt[W];
 #pragma unroll
-    for (int w = 0; w < kWavesAny; ++w) {
+    for (int w = 0; w < W; ++w) {
         const float mw = sm_m[w][jl];
         wgt[w] = mw == -INFINITY ? 0.0f : fast_exp2(mw - M);
         L = fmaf(sm_l[w][jl], wgt[w], L);
@@ -367,10 +387,10 @@ __global__ __launch_bounds__(kWavesAny * 64, DP <= 128 ? 2 : 1) void attn_splitk
     float *dst = final_out ? p.out + (uint64_t(item.q_row0 + row) * p.q_heads + head) * D : p.ws + ps * D;
     const float post = final_out ? 1.0f / L : 1.0f;
     // Tile c, lane (jl, g), register rr = channel 16c + 4g + rr: wavefront w finishes tiles w, w + 4, ..
-    for (uint32_t c = wave; 16 * c < D; c += kWavesAny) {
+    for (uint32_t c = wave; 16 * c < D; c += W) {
         floatx4 fin = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int w = 0; w < kWavesAny; ++w) fin += *reinterpret_cast<const floatx4 *>(&sm_o[w][c][lane][0]) * wgt[w];
+        for (int w = 0; w < W; ++w) fin += *reinterpret_cast<const floatx4 *>(&sm_o[w][c][lane][0]) * wgt[w];
         fin *= post;
         *reinterpret_cast<floatx4 *>(dst + 16 * c + 4 * g) = fin;
     }
@@ -388,57 +408,81 @@ uint32_t attn_splitk_any_groups_per_cu(const PoolGeom &g) {
     if (g.v_block) return g.head_dim <= 64 ? 3 : g.head_dim <= 128 ? 2 : 1;
     return g.head_dim <= 64 ? 3 : g.head_dim <= 128 ? 2 : 1;
 }
-uint32_t attn_splitk_any_whole_blocks(const PoolGeom &g, int elem_f16) {
-    if (g.v_block) return g.head_dim <= 128 ? 12 : 8;
-    return elem_f16 || g.head_dim <= 64 ? 8 : 4;
-}
-// As for the f32 kernel: a step of up to 16 query vectors per KV head brings its rows along.
-bool attn_splitk_any_appends(const PoolGeom &g, uint32_t group, uint32_t max_rows) {
-    return attn_splitk_any_supports(g, group, max_rows) && max_rows * group <= 16;
+// f32 steps bring their rows along (attn_splitk_rows_kernel.h: they are read where they are). So do
+// f16 steps of up to 16 query vectors per KV head, and of a few rows more, of which every tile's workgroups
+// that reach the new positions store all: 3 us of launch saved, a microsecond spent for eight rows
+// (scattered stores of two bytes; head_dim 80, 32 Q / 8 KV heads, six rows at 450 12.5 -> 9.7 us a layer;
+// twenty rows 9.9 -> 11.0).
+bool attn_splitk_any_appends(const PoolGeom &g, int elem_f16, uint32_t group, uint32_t max_rows) {
+    return attn_splitk_any_supports(g, group, max_rows) && (!elem_f16 || max_rows * group <= 16 || max_rows <= 8);
 }
 
 hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream) {
     if (b.total_blocks == 0) return hipSuccess;
     const uint32_t d = p.g.head_dim;
-    const dim3 grid(b.total_blocks), threads(kWavesAny * 64);
     // (Batches of one item take the eight-item argument block: 0.1 us on a launch of 5.)
-#define ITAK_ANY(...)                                                                             \
+#define ITAK_ANY(W, ...)                                                                          \
     do {                                                                                          \
         if (b.n <= 8) {                                                                           \
             constexpr int N = 8;                                                                  \
-            launch_kernel(__VA_ARGS__, grid, threads, 0, stream, p, AttnBatchT<N>(b), total_partials);       \
+            launch_kernel(__VA_ARGS__, b.total_blocks, W * 64, 0, stream, p, AttnBatchT<N>(b), total_partials); \
         } else {                                                                                  \
             constexpr int N = 64;                                                                 \
-            launch_kernel(__VA_ARGS__, grid, threads, 0, stream, p, AttnBatchT<N>(b), total_partials);       \
+            launch_kernel(__VA_ARGS__, b.total_blocks, W * 64, 0, stream, p, AttnBatchT<N>(b), total_partials); \
         }                                                                                         \
+    } while (0)
+#define ITAK_HALVES(DP)                                                        \
+    do {                                                                       \
+        if constexpr (DP <= 128) {                                             \
+            if (b.on_eight) {                                                  \
+                ITAK_ANY(8, attn_splitk_halves_kernel<DP, 8, N>);              \
+                break;                                                         \
+            }                                                                  \
+        }                                                                      \
+        ITAK_ANY(4, attn_splitk_halves_kernel<DP, 4, N>);                      \
+    } while (0)
+#define ITAK_ROWS(T, DP, TT)                                                   \
+    do {                                                                       \
+        if constexpr (DP <= 128) {                                             \
+            if (b.on_eight) {                                                  \
+                ITAK_ANY(8, attn_splitk_rows_kernel<T, DP, false, 1, false, 8, true, N>); \
+                break;                                                         \
+            }                                                                  \
+        }                                                                      \
+        if (b.half_blocks)                                                     \
+            ITAK_ANY(4, attn_splitk_rows_kernel<T, DP, false, 1, false, 4, true, N>); \
+        else                                                                   \
+            ITAK_ANY(4, attn_splitk_rows_kernel<T, DP, false, TT, false, 4, false, N>); \
     } while (0)
     if (elem_f16 && p.g.v_block) {
         switch ((d + 31) / 32) {
-            case 1: ITAK_ANY(attn_splitk_halves_kernel<32, N>); break;
-            case 2: ITAK_ANY(attn_splitk_halves_kernel<64, N>); break;
-            case 3: ITAK_ANY(attn_splitk_halves_kernel<96, N>); break;
-            case 4: ITAK_ANY(attn_splitk_halves_kernel<128, N>); break;
-            case 5: ITAK_ANY(attn_splitk_halves_kernel<160, N>); break;
-            case 6: ITAK_ANY(attn_splitk_halves_kernel<192, N>); break;
-            case 7: ITAK_ANY(attn_splitk_halves_kernel<224, N>); break;
-            default: ITAK_ANY(attn_splitk_halves_kernel<256, N>); break;
+            case 1: ITAK_HALVES(32); break;
+            case 2: ITAK_HALVES(64); break;
+            case 3: ITAK_HALVES(96); break;
+            case 4: ITAK_HALVES(128); break;
+            case 5: ITAK_HALVES(160); break;
+            case 6: ITAK_HALVES(192); break;
+            case 7: ITAK_HALVES(224); break;
+            default: ITAK_HALVES(256); break;
         }
     } else if (elem_f16) {
         switch ((d + 63) / 64) {
-            case 1: ITAK_ANY(attn_splitk_rows_kernel<uint16_t, 64, false, 2, false, N>); break;
-            case 2: ITAK_ANY(attn_splitk_rows_kernel<uint16_t, 128, false, 2, false, N>); break;
-            case 3: ITAK_ANY(attn_splitk_rows_kernel<uint16_t, 192, false, 2, false, N>); break;
-            default: ITAK_ANY(attn_splitk_rows_kernel<uint16_t, 256, false, 2, false, N>); break;
+            case 1: ITAK_ROWS(uint16_t, 64, 2); break;
+            case 2: ITAK_ROWS(uint16_t, 128, 2); break;
+            case 3: ITAK_ROWS(uint16_t, 192, 2); break;
+            default: ITAK_ROWS(uint16_t, 256, 2); break;
         }
     } else {
         switch ((d + 63) / 64) {
-            case 1: ITAK_ANY(attn_splitk_rows_kernel<float, 64, false, 2, false, N>); break;
-            case 2: ITAK_ANY(attn_splitk_rows_kernel<float, 128, false, 2, false, N>); break;
-            case 3: ITAK_ANY(attn_splitk_rows_kernel<float, 192, false, 1, false, N>); break;
-            default: ITAK_ANY(attn_splitk_rows_kernel<float, 256, false, 1, false, N>); break;
+            case 1: ITAK_ROWS(float, 64, 1); break;
+            case 2: ITAK_ROWS(float, 128, 1); break;
+            case 3: ITAK_ROWS(float, 192, 1); break;
+            default: ITAK_ROWS(float, 256, 1); break;
         }
     }
+#undef ITAK_ROWS
+#undef ITAK_HALVES
 #undef ITAK_ANY
     return hipGetLastError();
 }

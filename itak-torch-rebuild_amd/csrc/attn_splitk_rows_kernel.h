@@ -3,11 +3,11 @@
 // out: the 1e-5 bar of f32 pools holds), K and V read straight from their planes, no LDS in the
 // loop. Instantiated in attn_splitk_f32.hip (f32, head_dim 64 and 128) and attn_splitk_any.hip.
 //
-// One workgroup of four wavefronts owns (item, KV head, tile of 16 query vectors, split = a run of
+// One workgroup of four or eight wavefronts owns (item, KV head, tile of 16 query vectors, split = a run of
 // 32-key blocks), a query vector being one row of one Q head of the group; a block of more than 16
 // vectors is several tiles, each walking the keys its own rows see (tiles of later rows first: they
 // have the longest runs). Each wavefront walks its own blocks with a private online softmax, the
-// four merge once through LDS. The MFMA takes one float per lane and operand: A[i][k] from lane
+// wavefronts merge once through LDS. The MFMA takes one float per lane and operand: A[i][k] from lane
 // i + 16k, B[k][j] from lane j + 16k, and returns rows 4g .. 4g+3 of column j to lane j + 16g. A dot
 // product does not care in which order its terms are taken, so the channels (for K.Q^T) and the
 // keys (for V^T.P^T) are assigned to the MFMA's k index in whatever order lets every lane fetch four
@@ -41,12 +41,12 @@
 
 #include "internal.h"
 #include "mfma_common.h"
+#include "split_exchange.h"
 
 namespace itak {
 
 namespace {
 
-constexpr int kWavesRows = 4;
 
 __device__ __forceinline__ float lanes4_max(float v) {  // over lanes l, l^16, l^32, l^48
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -99,15 +99,19 @@ struct Piece4<uint16_t> {
 
 // DP: head_dim rounded up to a multiple of 64 (pieces beyond head_dim are read from the row's last
 // and taken as zero); EXACT: it is head_dim. TT: 16-key tiles whose rows are in registers at a time
-// (1 where two would not fit).
-template <typename T, int DP, bool EXACT, int TT, bool STREAM, int N>
-__global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_splitk_rows_kernel(AttnParams p, AttnBatchT<N> b,
-                                                                                            uint32_t total_partials) {
+// (1 where two would not fit). W: wavefronts. HALF: they take half a block each, in turn.
+template <typename T, int DP, bool EXACT, int TT, bool STREAM, int W, bool kHalf, int N>
+__global__ __launch_bounds__(W * 64, DP <= 128 && W == 4 ? 2 : 1) void attn_splitk_rows_kernel(AttnParams p, AttnBatchT<N> b,
+                                                                                             uint32_t total_partials) {
+    static_assert(!kHalf || TT == 1, "half a block is one tile");
     constexpr int kTiles = DP / 16;  // output tiles (h, e)
     constexpr int kS = DP / 16;      // pieces of a key row per lane group
     constexpr int kH = DP / 64;      // pieces of a value row per lane
-    __shared__ float sm_m[kWavesRows][16], sm_l[kWavesRows][16];
-    __shared__ float sm_o[kWavesRows][kTiles][64][4];  // [wave][tile][lane][row of the lane]
+    __shared__ float sm_m[W][16], sm_l[W][16];
+    __shared__ floatx4 sm_q[DP * 4];
+    // [wave][tile][row of the lane][lane]: written and read a float a lane without bank conflicts (with the
+    // lane's four rows side by side the merge's reads were four-way conflicts, 0.4 us of a one-row step).
+    __shared__ float sm_o[W][kTiles][4][64];
 
     const uint32_t tid = threadIdx.x;
     const uint32_t wave = tid >> 6, lane = tid & 63;
@@ -147,25 +151,60 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
     const float qscale = softcap > 0.0f ? p.scale : p.scale * kLog2e;
     const float *qp = p.q + (uint64_t(item.q_row0 + row) * p.q_heads + head) * D;
 
-    // Q^T as B operands: step (s, e) takes channel 16s + 4g + e of vector jl.
-    floatx4 q[kS];
+    // Channels of a lane's pieces. Only those of the last 64 can lie beyond head_dim.
+    auto key_piece = [&](int s) { return EXACT || 16 * (s + 1) <= DP - 64 ? 16u * s + 4 * g : min(16u * s + 4 * g, D - 4); };
+    auto value_piece = [&](int h) { return EXACT || h + 1 < kH ? 64u * h + 4 * jl : min(64u * h + 4 * jl, D - 4); };
+
+    // Q^T as B operands: step (s, e) takes channel 16s + 4g + e of vector jl. The tile's vectors are read
+    // once and handed round through LDS, piece (s, g, vector) at (4s + g) * 16 + vector: read by every
+    // wavefront they are a third of what a compute unit's load path moves for a block.
+    constexpr int kQ = (DP * 4 + W * 64 - 1) / (W * 64);  // pieces a thread stages
+    floatx4 q_raw[kQ];
 #pragma unroll
-    for (int s = 0; s < kS; ++s) q[s] = *reinterpret_cast<const floatx4 *>(qp + (EXACT ? 16 * s + 4 * g : min(16u * s + 4 * g, D - 4)));
+    for (int u = 0; u < kQ; ++u) {
+        const uint32_t f = min(tid + u * W * 64, DP * 4u - 1), c4 = (f / 16) * 4, vj = min(vtile * 16 + f % 16, nvec - 1);
+        const uint32_t r = vj / group, hd = kv_head * group + vj - r * group;
+        q_raw[u] = *reinterpret_cast<const floatx4 *>(p.q + (uint64_t(item.q_row0 + r) * p.q_heads + hd) * D +
+                                                      (EXACT ? c4 : min(c4, D - 4)));
+    }
 
     // A step of the walk: TT tiles of block kb, from tile t0.
     Piece4<T> k[TT][kS], v[TT][4][kH];
-    // Storage row of key row i of the step. Rows past the stored length are read from the last
-    // stored row instead (the plane may end there) and masked.
+    // Fused append (p.k_new set). f32 rows: whoever reads a new position reads it where the caller left
+    // it, so nothing waits for a store, and the workgroups of the last tile of vectors, which between
+    // them walk every block, copy the rows to the planes when they are done. (Every step takes its rows'
+    // addresses through the same selects: as a path of its own, which only the last block's wavefront
+    // ran, cold, it cost a one-row launch 0.8 us.) f16 rows: the wavefront that owns
+    // a block stores the new rows in it and waits for the stores before it reads the block (where several
+    // tiles' workgroups walk the block, each stores the same rows and reads its own).
+    constexpr bool kInPlace = sizeof(T) == 4;
+    const bool fused = p.k_new != nullptr;
+    const uint32_t fresh_from = kInPlace && fused ? item.pos0 : 0xffffffffu;
+    const uint32_t new_stride = p.g.kv_heads * D;
+    const uint64_t new_at = uint64_t(item.q_row0) * new_stride + kv_head * D;
+    // Row i of the step: its storage row, and where its data is. Rows past the stored length are read
+    // from the last stored row instead (the plane may end there) and masked.
+    auto step_pos = [&](uint32_t kb, uint32_t t0, uint32_t i) { return min(kb * kBlockKeys + 16 * t0 + i, item.kv_len - 1); };
     auto step_row = [&](uint32_t kb, uint32_t t0, uint32_t i) {
-        const uint32_t pos = min(kb * kBlockKeys + 16 * t0 + i, item.kv_len - 1);
-        return (ring_blocks ? kb % ring_blocks : kb) * kBlockKeys + pos - kb * kBlockKeys;
+        return (ring_blocks ? kb % ring_blocks : kb) * kBlockKeys + step_pos(kb, t0, i) - kb * kBlockKeys;
+    };
+    auto row_at = [&](const T *plane, const float *fresh, uint32_t kb, uint32_t t0, uint32_t i) -> const T * {
+        if constexpr (kInPlace) {
+            const uint32_t pos = step_pos(kb, t0, i);
+            const bool is_new = pos >= fresh_from;
+            const uint32_t row = is_new ? pos - item.pos0 : step_row(kb, t0, i);
+            return (is_new ? fresh + new_at : plane) + uint64_t(row) * (is_new ? new_stride : D);
+        } else {
+            return plane + uint64_t(step_row(kb, t0, i)) * D;
+        }
     };
     auto load_keys = [&](uint32_t kb, uint32_t t0) {
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
-            const T *kr = kplane + uint64_t(step_row(kb, t0, 16 * t + jl)) * D;
+            const T *kr = row_at(kplane, p.k_new, kb, t0, 16 * t + jl);
 #pragma unroll
-            for (int s = 0; s < kS; ++s) k[t][s].template load<STREAM>(kr + (EXACT ? 16 * s + 4 * g : min(16u * s + 4 * g, D - 4)));
+            for (int s = 0; s < kS; ++s) k[t][s].template load<STREAM>(kr + key_piece(s));
+            if (kInPlace) __builtin_amdgcn_sched_barrier(0);  // (all rows' addresses at once would not fit)
         }
     };
     auto load_values = [&](uint32_t kb, uint32_t t0) {
@@ -173,18 +212,45 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
         for (int t = 0; t < TT; ++t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const T *vr = vplane + uint64_t(step_row(kb, t0, 16 * t + 4 * g + r)) * D;
+                const T *vr = row_at(vplane, p.v_new, kb, t0, 16 * t + 4 * g + r);
 #pragma unroll
-                for (int h = 0; h < kH; ++h) v[t][r][h].template load<STREAM>(vr + (EXACT ? 64 * h + 4 * jl : min(64u * h + 4 * jl, D - 4)));
+                for (int h = 0; h < kH; ++h) v[t][r][h].template load<STREAM>(vr + value_piece(h));
+                if (kInPlace) __builtin_amdgcn_sched_barrier(0);
             }
     };
-    // Fused append (p.k_new set): the wavefront that owns a block stores the new rows in it and waits
-    // for the stores before it reads the block; nobody else reads these positions.
-    auto append_rows = [&](uint32_t kb) {
-        const uint32_t key0 = kb * kBlockKeys;
-        if (p.k_new == nullptr || key0 + kBlockKeys <= item.pos0) return;
+    // The rows this workgroup copies: those of its blocks. A thread's first piece is asked for now and
+    // stored at the end.
+    const uint32_t own_from = max(item.pos0, kb_begin * kBlockKeys), own_to = min(item.kv_len, kb_end * kBlockKeys);
+    const uint32_t quads = D / 4;
+    const uint32_t own_pieces = kInPlace && fused && vtile == vtiles - 1 && own_to > own_from ? (own_to - own_from) * 2 * quads : 0;
+    auto own_piece = [&](uint32_t f, const float *&src, T *&dst) {
+        const uint32_t pos = own_from + f / (2 * quads), rest = f % (2 * quads), side = rest >= quads ? 1 : 0;
+        const uint32_t c4 = (rest - side * quads) * 4;
+        src = (side ? p.v_new : p.k_new) + new_at + uint64_t(pos - item.pos0) * new_stride + c4;
+        dst = (side ? vplane : kplane) + uint64_t(ring_blocks ? pos % (ring_blocks * kBlockKeys) : pos) * D + c4;
+    };
+    floatx4 own = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (tid < own_pieces) {
+        const float *src;
+        T *dst;
+        own_piece(tid, src, dst);
+        own = *reinterpret_cast<const floatx4 *>(src);
+    }
+    auto store_own = [&] {
+        for (uint32_t f = tid; f < own_pieces; f += W * 64) {
+            const float *src;
+            T *dst;
+            own_piece(f, src, dst);
+            if (f != tid) own = *reinterpret_cast<const floatx4 *>(src);
+            Piece4<T>::store(dst, own);
+        }
+    };
+    auto append_rows = [&](uint32_t kb, uint32_t t0) {
+        if constexpr (!kInPlace) {
+        const uint32_t key0 = kb * kBlockKeys + (kHalf ? 16 * t0 : 0), keys = kHalf ? 16 : kBlockKeys;
+        if (!fused || key0 + keys <= item.pos0 || key0 >= item.pos0 + item.rows) return;
         const uint32_t from = key0 > item.pos0 ? key0 - item.pos0 : 0;
-        const uint32_t to = min(item.rows, key0 + kBlockKeys - item.pos0), quads = D / 4;
+        const uint32_t to = min(item.rows, key0 + keys - item.pos0), quads = D / 4;
         for (uint32_t f = lane; f < (to - from) * 2 * quads; f += 64) {
             const uint32_t r = from + f / (2 * quads), rest = f % (2 * quads);
             const uint32_t side = rest >= quads ? 1 : 0, c4 = (rest - side * quads) * 4;
@@ -194,20 +260,41 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
             Piece4<T>::store((side ? vplane : kplane) + uint64_t(srow) * D + c4, y);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores have been acknowledged
+        }
     };
-    uint32_t kb = kb_begin + wave, t0 = 0;
-    if (kb < kb_end) {
-        append_rows(kb);
-        load_keys(kb, 0);
-        load_values(kb, 0);
+    auto advance = [&](uint32_t &kb, uint32_t &t0) {
+        if constexpr (kHalf) {
+            kb += W / 2;
+        } else {
+            t0 += TT;
+            if (t0 == 2) {
+                t0 = 0;
+                kb += W;
+            }
+        }
+    };
+    uint32_t kb = kb_begin + (kHalf ? wave / 2 : wave), t0 = kHalf ? wave & 1 : 0;
+    if (kb < kb_end) append_rows(kb, t0);
+    {
+        // (A wavefront without a block loads one and ignores it: behind a branch the wait for the queries
+        // would be a wait for every load, and the barrier below the slowest wavefront's.)
+        const uint32_t some = min(kb, (item.kv_len - 1) / kBlockKeys);
+        load_keys(some, t0);
+        load_values(some, t0);
     }
     __builtin_amdgcn_sched_barrier(0);
 
 #pragma unroll
-    for (int s = 0; s < kS; ++s) {
-        if (jv >= nvec || (!EXACT && 16u * s + 4 * g >= D)) q[s] = floatx4{0.f, 0.f, 0.f, 0.f};
-        q[s] *= qscale;
+    for (int u = 0; u < kQ; ++u) {
+        const uint32_t f = tid + u * W * 64;
+        floatx4 x = q_raw[u] * qscale;
+        if (vtile * 16 + f % 16 >= nvec || (!EXACT && (f / 16) * 4 >= D)) x = floatx4{0.f, 0.f, 0.f, 0.f};
+        if (f < DP * 4u) sm_q[f] = x;
     }
+    lds_barrier();
+    floatx4 q[kS];
+#pragma unroll
+    for (int s = 0; s < kS; ++s) q[s] = sm_q[s * 64 + lane];
 
     float m_run = -INFINITY, l_run = 0.0f;
     floatx4 o[kTiles];
@@ -252,11 +339,8 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
 
     while (kb < kb_end) {
         const uint32_t key0 = kb * kBlockKeys + 16 * t0;
-        uint32_t next_kb = kb, next_t0 = t0 + TT;
-        if (next_t0 == 2) {
-            next_t0 = 0;
-            next_kb += kWavesRows;
-        }
+        uint32_t next_kb = kb, next_t0 = t0;
+        advance(next_kb, next_t0);
         float sc[TT][4];
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
@@ -272,7 +356,7 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
             for (int r = 0; r < 4; ++r) sc[t][r] = acc[r];
         }
         if (next_kb < kb_end) {
-            if (next_t0 == 0) append_rows(next_kb);
+            if (kHalf || next_t0 == 0) append_rows(next_kb, next_t0);
             load_keys(next_kb, next_t0);
         }
         const float alpha = weigh(key0, sc);
@@ -310,7 +394,8 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
     for (int c = 0; c < kTiles; ++c) {
         // (Output rows beyond head_dim hold whatever the clamped pieces gave.)
         all += (o[c][0] + o[c][1]) + (o[c][2] + o[c][3]);
-        *reinterpret_cast<floatx4 *>(&sm_o[wave][c][lane][0]) = o[c];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sm_o[wave][c][r][lane] = o[c][r];
     }
     if (__builtin_amdgcn_ballot_w64(!(fabsf(all) < INFINITY)) != 0) {
 #pragma unroll 1
@@ -320,9 +405,9 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
             l_run = 0.0f;
             floatx4 out = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 1
-            for (uint32_t sb = kb_begin + wave; sb < kb_end; sb += kWavesRows)
+            for (uint32_t sb = kb_begin + (kHalf ? wave / 2 : wave); sb < kb_end; sb += kHalf ? W / 2 : W)
 #pragma unroll 1
-                for (uint32_t st = 0; st < 2; st += TT) {
+                for (uint32_t st = kHalf ? wave & 1 : 0; st < 2; st += kHalf ? 2 : TT) {
                     const uint32_t key0 = sb * kBlockKeys + 16 * st;
                     floatx4 acc[TT] = {};
 #pragma unroll 1
@@ -331,7 +416,7 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
 #pragma unroll
                         for (int t = 0; t < TT; ++t)
                             acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                Piece4<T>::one(kplane + uint64_t(step_row(sb, st, 16 * t + jl)) * D + ch), qv, acc[t], 0, 0, 0);
+                                Piece4<T>::one(row_at(kplane, p.k_new, sb, st, 16 * t + jl) + ch), qv, acc[t], 0, 0, 0);
                     }
                     float sc[TT][4];
 #pragma unroll
@@ -344,7 +429,7 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
                     for (int t = 0; t < TT; ++t)
 #pragma unroll
                         for (int r = 0; r < 4; ++r)
-                            x[t][r] = Piece4<T>::one(vplane + uint64_t(step_row(sb, st, 16 * t + 4 * g + r)) * D + ch_out);
+                            x[t][r] = Piece4<T>::one(row_at(vplane, p.v_new, sb, st, 16 * t + 4 * g + r) + ch_out);
 #pragma unroll 1
                     for (uint32_t rr = row_first; rr <= row_last; ++rr) {
                         const uint32_t pos = min(item.pos0 + rr, item.kv_len - 1);
@@ -361,7 +446,8 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
                         if (row == rr) out += part;
                     }
                 }
-            *reinterpret_cast<floatx4 *>(&sm_o[wave][c][lane][0]) = out;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sm_o[wave][c][r][lane] = out[r];
         }
     }
 
@@ -375,28 +461,30 @@ __global__ __launch_bounds__(kWavesRows * 64, DP <= 128 ? 2 : 1) void attn_split
 
     float M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < kWavesRows; ++w) M = fmaxf(M, sm_m[w][jl]);
-    float L = 0.0f, wgt[kWavesRows];
+    for (int w = 0; w < W; ++w) M = fmaxf(M, sm_m[w][jl]);
+    float L = 0.0f, wgt[W];
 #pragma unroll
-    for (int w = 0; w < kWavesRows; ++w) {
+    for (int w = 0; w < W; ++w) {
         const float mw = sm_m[w][jl];
         wgt[w] = mw == -INFINITY ? 0.0f : fast_exp2(mw - M);
         L = fmaf(sm_l[w][jl], wgt[w], L);
     }
+    store_own();
     if (jv >= nvec) return;
     const bool final_out = item.splits == 1;
     const uint64_t ps = item.ws0 + (uint64_t(row) * p.q_heads + head) * item.splits + split;
     float *dst = final_out ? p.out + (uint64_t(item.q_row0 + row) * p.q_heads + head) * D : p.ws + ps * D;
     const float post = final_out ? 1.0f / L : 1.0f;
-    // Tile (h, e), register rr = channel 64h + 16g + 4rr + e: wavefront w finishes register w of all.
-#pragma unroll
-    for (int h = 0; h < kH; ++h) {
-        const uint32_t ch = 64 * h + 16 * g + 4 * wave;
+    // Tile (h, e), register rr = channel 64h + 16g + 4rr + e: wavefront w finishes register w % 4 of
+    // every (of eight: every second) h.
+    const uint32_t rr = wave % 4;
+    for (int h = wave / 4; h < kH; h += W / 4) {
+        const uint32_t ch = 64 * h + 16 * g + 4 * rr;
         floatx4 fin = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int w = 0; w < kWavesRows; ++w)
+        for (int w = 0; w < W; ++w)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) fin[e] = fmaf(sm_o[w][4 * h + e][lane][wave], wgt[w], fin[e]);
+            for (int e = 0; e < 4; ++e) fin[e] = fmaf(sm_o[w][4 * h + e][rr][lane], wgt[w], fin[e]);
         fin *= post;
         if (EXACT || ch < D) *reinterpret_cast<floatx4 *>(dst + ch) = fin;
     }

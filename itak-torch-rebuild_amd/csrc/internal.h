@@ -292,6 +292,8 @@ struct AttnBatch {
     uint32_t tiles;      // host side only: column tiles per wavefront in the block kernel's plan
     uint32_t fold_units; // host side only: the block kernel's plan for AttnParams::fold_units
     uint32_t two_halves; // host side only: the block kernel multiplies each query as two f16 halves
+    uint32_t on_eight; // host side only: the rows and halves kernels run on eight wavefronts
+    uint32_t half_blocks; // host side only: the rows kernel's wavefronts take half a block each
     uint32_t tiled; // host side only: the split-K plan gives every 16 query vectors their own workgroups
     uint32_t whole_on_eight; // host side only: the split-K plan leaves every item whole on eight wavefronts
     AttnItem item[kMaxBatchItems];
@@ -497,11 +499,8 @@ hipError_t launch_attn_decode_f16(const AttnParams &p, const AttnBatch &b, uint3
 // f32 MFMA split-K path: f32 pools (row-major planes), head_dim 128, rows*group <= 16, implied
 // query positions. Partials are in log2 domain (combine with base2 = 1).
 bool attn_splitk_f32_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
-// True when such a launch also appends the step's rows (k_new / v_new in its parameters).
-bool attn_splitk_f32_appends(const PoolGeom &g, uint32_t group, uint32_t max_rows);
-// (`groups_per_cu` workgroups share a compute unit; contexts of `whole_blocks` blocks are not split.)
-uint32_t attn_splitk_f32_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu,
-                              uint32_t whole_blocks);
+// (`groups_per_cu` workgroups of four wavefronts share a compute unit.)
+uint32_t attn_splitk_f32_plan(const PoolGeom &g, int elem_f16, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu);
 hipError_t launch_attn_splitk_f32(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream);
 // f32-arithmetic MFMA split-K path for the other shapes (attn_splitk_any.hip): f16 and f32 pools,
@@ -510,9 +509,9 @@ hipError_t launch_attn_splitk_f32(const AttnParams &p, const AttnBatch &b, uint3
 bool attn_splitk_any_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
 // Workgroups of that kernel a compute unit holds.
 uint32_t attn_splitk_any_groups_per_cu(const PoolGeom &g);
-// Blocks up to which its short steps leave a context whole.
-uint32_t attn_splitk_any_whole_blocks(const PoolGeom &g, int elem_f16);
-bool attn_splitk_any_appends(const PoolGeom &g, uint32_t group, uint32_t max_rows);
+// True when such a launch also appends the step's rows (k_new / v_new in its parameters); launches of
+// the f32 kernel always do.
+bool attn_splitk_any_appends(const PoolGeom &g, int elem_f16, uint32_t group, uint32_t max_rows);
 hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream);
 // MFMA block path (speculative blocks and prefill chunks): same pools, any number of rows,

@@ -705,7 +705,7 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         const uint32_t count = std::min<uint32_t>(kMaxBatchItems, n - first);
         AttnBatch b;  // (cleared item by item: all 64 are three kilobytes)
         b.n = count;
-        b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.tiled = 0;
+        b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.tiled = b.on_eight = b.half_blocks = 0;
         b.two_halves = prefill && pool->q_two_halves && pool->g.head_dim == 128 ? 1 : 0;
         uint32_t total_rows = 0;
         for (uint32_t i = 0; i < count; ++i) {
@@ -728,9 +728,8 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         } else if (prefill) {
             partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, k_new != nullptr);
         } else if (f32fast || any) {
-            partials = attn_splitk_f32_plan(geom, b, uint32_t(q_heads),
-                                            any && max_rows * group <= 16 ? attn_splitk_any_groups_per_cu(geom) : 2,
-                                            attn_splitk_any_whole_blocks(geom, pool->elem_f16));
+            partials = attn_splitk_f32_plan(geom, pool->elem_f16, b, uint32_t(q_heads),
+                                            any && max_rows * group <= 16 ? attn_splitk_any_groups_per_cu(geom) : 2);
         } else {
             b.rows_per_block = rpb;
             uint64_t key_work = 0;
@@ -2537,9 +2536,9 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
     const bool fuse =
         splitk || block_fuses ||
         (!pool->elem_f16 && !active.empty() &&
-         attn_splitk_f32_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows)) ||
+         attn_splitk_f32_supports(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows)) ||
         (any && aligned16(k_dev) && aligned16(v_dev) &&
-         attn_splitk_any_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows));
+         attn_splitk_any_appends(pool->g, pool->elem_f16, uint32_t(num_q_heads / pool->g.kv_heads), most_rows));
     // The allocation-free form plans first and refuses, before anything changes, a step whose
     // launches need more workspace than the static array has.
     struct NoAllocScope {

@@ -145,3 +145,46 @@ def test_short_steps_at_the_block_kernels_head_dims(d, q_heads, kv_heads, window
             assert rel_err(got[at:at + r].reshape(-1), want) <= 1e-5, (rows, s, base)
             at += r
     pool.close()
+
+
+# Row-major and blocked planes on four and eight wavefronts, whole and split, rows brought along by every
+# tile of a step: contexts at the ends of rounds of four, eight, sixteen and twenty-four blocks.
+@pytest.mark.parametrize("elem,d,q_heads,kv_heads", [("f32", 64, 32, 4), ("f32", 128, 8, 8), ("f32", 100, 9, 3), ("f16", 80, 32, 8),
+                                                     ("f16", 72, 8, 1), ("f16", 112, 40, 2)])
+@pytest.mark.parametrize("ctx", [10, 60, 127, 250, 500, 760, 1500])
+def test_rounds_of_wavefronts(elem, d, q_heads, kv_heads, ctx):
+    P = pkg()
+    rng = np.random.default_rng(d + ctx)
+    pool = P.KvPool([P.LayerKind.Global], kv_heads, d, elem=elem, max_slots=2, capacity_rows=1600)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    caches = [pool.acquire() for _ in range(2)]
+    refs = [oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, d, store_f16=elem == "f16") for _ in range(2)]
+    for cache, ref, n in zip(caches, refs, (ctx, ctx // 3)):
+        k, v = normal(rng, n, kv_heads * d), normal(rng, n, kv_heads * d)
+        kd, vd = dev(k), dev(v)
+        pool.append_device(0, [(cache, n)], kd.data_ptr(), vd.data_ptr())
+        for i in range(n):
+            ref.append(0, k[i], v[i], i)
+    kept = []
+    for rows in ((1, 1), (8, 3), (1, 16)):
+        total = sum(rows)
+        q = normal(rng, total, q_heads * d)
+        k, v = normal(rng, total, kv_heads * d), normal(rng, total, kv_heads * d)
+        qd, kd, vd = dev(q), dev(k), dev(v)
+        out = torch.empty_like(qd)
+        pool.attention_step_device(0, list(zip(caches, rows)), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), q_heads)
+        torch.cuda.synchronize()
+        got, at = out.cpu().numpy(), 0
+        for s, r in enumerate(rows):
+            want = oracle.attention_step(refs[s], 0, q[at:at + r], k[at:at + r], v[at:at + r], q_heads,
+                                         refs[s].next_position(0), threads=8)
+            assert rel_err(got[at:at + r].reshape(-1), want) <= 1e-5, (rows, s)
+            kept.append((s, refs[s].next_position(0) - r, k[at:at + r], v[at:at + r]))
+            at += r
+    store = (lambda x: oracle.f32_to_f16_array(x)) if elem == "f16" else (lambda x: x)
+    for s, base, k, v in kept:  # what the launches appended
+        for r in range(len(k)):
+            _, gk, gv = caches[s].read_rows(0, base + r, 1)
+            assert np.array_equal(gk.reshape(-1), store(k[r]).reshape(-1)), (s, base, r)
+            assert np.array_equal(gv.reshape(-1), store(v[r]).reshape(-1)), (s, base, r)
+    pool.close()
