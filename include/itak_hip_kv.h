@@ -284,8 +284,11 @@ itak_status itak_pool_create(const itak_pool_config *config, itak_pool **out);
 void itak_pool_destroy(itak_pool *pool);
 
 /* Stream every later call on this pool enqueues on (a hipStream_t; NULL = the
-   null stream). The pool never creates streams of its own and does not wait for the
-   previous stream: ordering between the two is the caller's to arrange. The stream
+   null stream). The pool never creates streams of its own and does not wait for what
+   device-pointer calls enqueued on the previous stream: ordering between the two is the
+   caller's to arrange. (It does wait for what a host-pointer call left there: such a call
+   returns when its output is whole, which its last launch may outlast by a moment. Not while
+   one of the two streams is being captured.) The stream
    may be one that is being captured into a HIP graph, provided the pool's scratch
    buffers are already large enough (run the same step once uncaptured first). */
 itak_status itak_pool_set_stream(itak_pool *pool, void *hip_stream);

@@ -5,6 +5,7 @@
 #include "../../include/itak_hip_kv.h"
 #include "internal.h"
 #include "host_ring.h"
+#include "host_turns.h"
 #include "itkv.h"
 
 #include <sys/mman.h>
@@ -180,7 +181,8 @@ struct itak_pool {
     // and go up in one copy; its kernels write the output here directly.
     unsigned char *hstage = nullptr;
     unsigned char *hstage_dev = nullptr;  // the device's address of it
-    uint64_t hstage_bytes = 0;
+    uint64_t hstage_half = 0;             // bytes of each of its two halves (host_turns.h)
+    HostTurns turns;
     // Pinned slots through which snapshot rows move between ordinary host memory and the device.
     HostRing ring;
     // Plan of the step in progress, and the slots it has named (by the number of the step).
@@ -451,25 +453,38 @@ itak_status ensure_prep(itak_pool *pool, uint64_t floats) {
     return ITAK_OK;
 }
 
+uint64_t align_up(uint64_t x, uint64_t a) { return (x + a - 1) / a * a; }
+
 constexpr uint64_t kHostWord = 256;  // bytes at the head of the pinned staging kept for the completion word
-itak_status ensure_hstage(itak_pool *pool, uint64_t bytes) {
-    if (bytes <= pool->hstage_bytes) return ITAK_OK;
+itak_status ensure_hstage(itak_pool *pool, uint64_t half_bytes) {
+    if (half_bytes <= pool->hstage_half) return ITAK_OK;
     HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize before growing pinned staging");
+    pool->turns.drained();
     if (pool->hstage) HIP_TRY(pool, hipHostFree(pool->hstage), "free pinned staging");
     pool->hstage = nullptr;
-    pool->hstage_bytes = 0;
-    const uint64_t want = std::max<uint64_t>(bytes + bytes / 2, 1u << 18);
-    HIP_TRY(pool, hipHostMalloc(reinterpret_cast<void **>(&pool->hstage), want, hipHostMallocDefault),
+    pool->hstage_half = 0;
+    const uint64_t half = align_up(std::max<uint64_t>(half_bytes + half_bytes / 2, 1u << 18), 256);
+    HIP_TRY(pool, hipHostMalloc(reinterpret_cast<void **>(&pool->hstage), kHostWord + 2 * half, hipHostMallocDefault),
             "allocate pinned staging");
-    memset(pool->hstage, 0, want);  // the completion word of a call must not start out matching
+    memset(pool->hstage, 0, kHostWord);  // the completion word of a call must not start out matching
     void *mapped = nullptr;
     HIP_TRY(pool, hipHostGetDevicePointer(&mapped, pool->hstage, 0), "map pinned staging");
     pool->hstage_dev = static_cast<unsigned char *>(mapped);
-    pool->hstage_bytes = want;
+    pool->hstage_half = half;
     return ITAK_OK;
 }
 
-uint64_t align_up(uint64_t x, uint64_t a) { return (x + a - 1) / a * a; }
+hipStream_t stream_of(const HostTurns &turns) { return static_cast<hipStream_t>(const_cast<void *>(turns.stream())); }
+
+// Waits until nothing of earlier host-pointer calls runs, on whichever stream they ran.
+itak_status drain_host_calls(itak_pool *pool) {
+    if (hipStreamSynchronize(stream_of(pool->turns)) != hipSuccess) {
+        (void)hipGetLastError();  // (the caller has destroyed that stream)
+        HIP_TRY(pool, hipDeviceSynchronize(), "wait for an earlier call's launches");
+    }
+    pool->turns.drained();
+    return ITAK_OK;
+}
 
 // ---- host-pointer attention calls ------------------------------------------------------
 // Such a call is dominated by its trips over the host link and by its launches, not by its
@@ -497,14 +512,17 @@ struct HostCall {
 };
 
 itak_status begin_host_call(itak_pool *pool, uint64_t in_bytes, uint64_t out_count, HostCall &c) {
-    // Layout: [completion word, 256 bytes] [inputs] [output]. The word sits at a fixed place, so it
-    // only ever holds call numbers, which only grow.
+    // Layout: [completion word, 256 bytes] [inputs, output] [inputs, output], the halves in turn. The
+    // word sits at a fixed place, so it only ever holds call numbers, which only grow.
     const uint64_t in_room = align_up(in_bytes, 256);
-    itak_status st = ensure_hstage(pool, kHostWord + in_room + out_count * 4);
+    itak_status st = ITAK_OK;
+    if (pool->turns.must_drain(pool->stream)) st = drain_host_calls(pool);
+    if (st == ITAK_OK) st = ensure_hstage(pool, in_room + out_count * 4);
     if (st != ITAK_OK) return st;
-    c.in = pool->hstage + kHostWord;
-    c.in_dev = pool->hstage_dev + kHostWord;
-    c.out_at = kHostWord + in_room;
+    const uint64_t at = kHostWord + pool->turns.begin(pool->stream) * pool->hstage_half;
+    c.in = pool->hstage + at;
+    c.in_dev = pool->hstage_dev + at;
+    c.out_at = at + in_room;
     c.out_dev = reinterpret_cast<float *>(pool->hstage_dev + c.out_at);
     c.out_count = out_count;
     if (out_count * 4 <= kHostWatched)
@@ -540,6 +558,7 @@ itak_status finish_host_call(itak_pool *pool, const HostCall &c, float *out) {
         const volatile uint32_t *seen = reinterpret_cast<const volatile uint32_t *>(pool->hstage);
         if (!look_until([&] { return __atomic_load_n(seen, __ATOMIC_ACQUIRE) == number; }))
             HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after attention");
+        pool->turns.drained();
         memcpy(out, from, bytes);
         return ITAK_OK;
     }
@@ -557,11 +576,13 @@ itak_status finish_host_call(itak_pool *pool, const HostCall &c, float *out) {
         });
         if (!arrived) {
             HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after attention");
+            pool->turns.drained();
             memcpy(out, from, bytes);
             return ITAK_OK;
         }
         at += n;
     }
+    pool->turns.seen();
     return ITAK_OK;
 }
 
@@ -1345,7 +1366,26 @@ void itak_pool_destroy(itak_pool *pool) {
 
 itak_status itak_pool_set_stream(itak_pool *pool, void *hip_stream) {
     if (!pool) return ITAK_INVALID_ARGUMENT;
-    pool->stream = static_cast<hipStream_t>(hip_stream);
+    const hipStream_t next = static_cast<hipStream_t>(hip_stream);
+    if (next != pool->stream && pool->turns.running()) {
+        // A host-pointer call has returned on the arrival of its output, and its last launch may still be
+        // storing rows: what the new stream is given must find them. Not where one of the two streams is
+        // being captured (a wait would spoil the capture): nothing captured runs before its first replay,
+        // and the next host-pointer call waits in any case.
+        const hipStream_t tail = stream_of(pool->turns);
+        auto idle = [](hipStream_t s) {
+            hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+            return hipStreamIsCapturing(s, &status) == hipSuccess && status == hipStreamCaptureStatusNone;
+        };
+        if (idle(tail) && idle(next)) {
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (some other stream of this thread may be captured)
+            const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+            if (hipStreamSynchronize(tail) == hipSuccess) pool->turns.drained();
+            if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        }
+        (void)hipGetLastError();
+    }
+    pool->stream = next;
     return ITAK_OK;
 }
 
@@ -2934,6 +2974,7 @@ itak_status itak_compute_attention(itak_pool *pool, uint32_t slot, uint64_t laye
             if (st != ITAK_OK) return st;
         }
         HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after append");
+        pool->turns.drained();
         pool->err = saved;
         pool->err.info.code = ITAK_STEP_FAILED;
         return ITAK_STEP_FAILED;
