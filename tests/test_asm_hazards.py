@@ -18,9 +18,11 @@ import pytest
 from helpers import ROOT
 
 CSRC = os.path.join(ROOT, "itak-torch-rebuild_amd", "csrc")
-# The files that instantiate the kernel (attn_prefill_f16_kernel.h), and how many instantiations
-# each must at least show.
-SOURCES = {"attn_prefill_f16.hip": 48, "attn_prefill_f16_dims.hip": 72}
+# The files that instantiate the kernel (attn_prefill_f16_kernel.h), and how many instantiations each
+# must at least show: softcap or none, ring or none, times 3 batch sizes and 1 or 2 tiles at head_dim 128;
+# times 2 batch sizes and 1 or 2 tiles at three other head dims; times 2 batch sizes with the queries as
+# two halves.
+SOURCES = {"attn_prefill_f16.hip": 24, "attn_prefill_f16_dims.hip": 48, "attn_prefill_f16_qlo.hip": 8}
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 
