@@ -456,6 +456,11 @@ itak_status ensure_prep(itak_pool *pool, uint64_t floats) {
 uint64_t align_up(uint64_t x, uint64_t a) { return (x + a - 1) / a * a; }
 
 constexpr uint64_t kHostWord = 256;  // bytes at the head of the pinned staging kept for the completion word
+constexpr uint64_t kHostHalf = 1u << 19;  // smallest half of the rest
+// Making and freeing pinned memory takes some 45 us, as much as a small call, which a program with a pool
+// for every sequence would pay for each. A pool that closes leaves a staging of the smallest size for the
+// next one: at most one a device (a megabyte), kept until the process ends.
+std::atomic<unsigned char *> g_spare_hstage[kMaxDevices];
 itak_status ensure_hstage(itak_pool *pool, uint64_t half_bytes) {
     if (half_bytes <= pool->hstage_half) return ITAK_OK;
     HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize before growing pinned staging");
@@ -463,9 +468,11 @@ itak_status ensure_hstage(itak_pool *pool, uint64_t half_bytes) {
     if (pool->hstage) HIP_TRY(pool, hipHostFree(pool->hstage), "free pinned staging");
     pool->hstage = nullptr;
     pool->hstage_half = 0;
-    const uint64_t half = align_up(std::max<uint64_t>(half_bytes + half_bytes / 2, 1u << 18), 256);
-    HIP_TRY(pool, hipHostMalloc(reinterpret_cast<void **>(&pool->hstage), kHostWord + 2 * half, hipHostMallocDefault),
-            "allocate pinned staging");
+    const uint64_t half = align_up(std::max<uint64_t>(half_bytes + half_bytes / 2, kHostHalf), 256);
+    if (half == kHostHalf) pool->hstage = g_spare_hstage[pool->cfg.device].exchange(nullptr);
+    if (!pool->hstage)
+        HIP_TRY(pool, hipHostMalloc(reinterpret_cast<void **>(&pool->hstage), kHostWord + 2 * half, hipHostMallocDefault),
+                "allocate pinned staging");
     memset(pool->hstage, 0, kHostWord);  // the completion word of a call must not start out matching
     void *mapped = nullptr;
     HIP_TRY(pool, hipHostGetDevicePointer(&mapped, pool->hstage, 0), "map pinned staging");
@@ -484,6 +491,17 @@ itak_status drain_host_calls(itak_pool *pool) {
     }
     pool->turns.drained();
     return ITAK_OK;
+}
+
+// The staging of a pool that closes; nothing else uses it once the host-pointer calls' launches have ended.
+void release_hstage(itak_pool *pool) {
+    const bool quiet = !pool->turns.running() || drain_host_calls(pool) == ITAK_OK;
+    unsigned char *none = nullptr;
+    if (pool->hstage && !(quiet && pool->hstage_half == kHostHalf &&
+                          g_spare_hstage[pool->cfg.device].compare_exchange_strong(none, pool->hstage)))
+        (void)hipHostFree(pool->hstage);
+    pool->hstage = nullptr;
+    pool->hstage_half = 0;
 }
 
 // ---- host-pointer attention calls ------------------------------------------------------
@@ -1359,7 +1377,7 @@ void itak_pool_destroy(itak_pool *pool) {
         if (t.dev) (void)hipFree(t.dev);
     for (void *buf : pool->ring_saved)
         if (buf) (void)hipFree(buf);
-    if (pool->hstage) (void)hipHostFree(pool->hstage);
+    release_hstage(pool);
     pool->ring.close();
     delete pool;
 }

@@ -4,9 +4,11 @@ into and when launches must have ended first.
 
 On the CPU: the class itself under random calls, failures and changes of stream, against a device that
 keeps every launch running for as long as it may. On the GPU: calls whose stored rows are fetched behind
-the output, back to back, and a change of stream right after a call; rows bit for bit."""
+the output, back to back, and a change of stream right after a call; rows bit for bit. And caches with
+a pool of their own, in turn and from several threads, which leave their staging to each other."""
 import os
 import subprocess
+import threading
 
 import numpy as np
 import pytest
@@ -105,3 +107,38 @@ def test_rows_fetched_behind_the_output_are_the_calls_own(rows):
         assert np.asarray(got).tobytes() == want.tobytes()
     pool.synchronize()
     pool.close()
+
+
+@pytest.mark.gpu
+def test_caches_of_their_own_in_turn_and_from_threads():
+    P = pkg()
+    q_heads, kv_heads, d = 8, 2, 64
+    failed = []
+
+    def sequences(seed, count):
+        try:
+            rng = np.random.default_rng(seed)
+            for i in range(count):
+                n, nq = int(rng.integers(20, 200)), int(rng.integers(1, 400 if i == 2 else 12))  # (one staging outgrows the rest)
+                nq = min(nq, n)
+                k, v, q = (normal(rng, n, kv_heads * d), normal(rng, n, kv_heads * d), normal(rng, nq, q_heads * d))
+                cache = P.KvCache.new([P.LayerKind.Global], kv_heads, d, elem="f32", capacity_rows=256)
+                ref = oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, d)
+                cache.restore_bulk(0, 0, k, v)
+                ref.restore_bulk(0, 0, k, v)
+                at = list(range(n - nq, n))
+                for _ in range(2):
+                    got = P.gqa_attention(q, nq, q_heads, at, cache.view(0), P.AttentionParams())
+                    want = oracle.gqa_attention(q, nq, q_heads, at, ref.view(0), oracle.AttentionParams())
+                    assert rel_err(np.asarray(got).reshape(-1), np.asarray(want).reshape(-1)) <= 1e-5, (seed, i)
+                cache.pool.close()
+        except BaseException as e:  # noqa: B036 - reported by the main thread
+            failed.append((seed, repr(e)))
+
+    sequences(0, 6)
+    threads = [threading.Thread(target=sequences, args=(seed, 8)) for seed in range(1, 5)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
