@@ -116,7 +116,17 @@ __global__ __launch_bounds__(256) void attn_gate_kernel(float *__restrict__ out,
         out[i] = out[i] * sigmoid_ref(gate[i]);
 }
 
+__global__ __launch_bounds__(kFillDoubles) void fill_doubles_kernel(double *__restrict__ dst, FillDoubles a) {
+    if (threadIdx.x < a.n) dst[threadIdx.x] = a.v[threadIdx.x];
+}
+
 }  // namespace
+
+hipError_t launch_fill_doubles(double *dst, const FillDoubles &a, hipStream_t stream) {
+    if (a.n == 0) return hipSuccess;
+    launch_kernel(fill_doubles_kernel, 1, kFillDoubles, 0, stream, dst, a);
+    return hipGetLastError();
+}
 
 hipError_t launch_attn_prep(const PrepArgs &a, hipStream_t stream) {
     const uint64_t head_rows = uint64_t(a.total_rows) * (a.q_heads + a.kv_heads);

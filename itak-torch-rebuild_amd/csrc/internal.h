@@ -253,6 +253,13 @@ struct PrepArgs {
     uint32_t pos0[kMaxBatchItems];   // position of that row
 };
 hipError_t launch_attn_prep(const PrepArgs &a, hipStream_t stream);
+// dst[0 .. n) = v, which travels as the launch's argument.
+constexpr uint32_t kFillDoubles = 64;
+struct FillDoubles {
+    uint32_t n;
+    double v[kFillDoubles];
+};
+hipError_t launch_fill_doubles(double *dst, const FillDoubles &a, hipStream_t stream);
 // out[i] *= sigmoid(gate[i]) (CpuCompute::attn_gate, cpu.rs:657-673).
 hipError_t launch_attn_gate(float *out, const float *gate, uint64_t count, hipStream_t stream);
 

@@ -106,11 +106,11 @@ std::atomic<uint64_t> g_next_cache_id{1};  // cache.rs:32
 
 }  // namespace
 
-// rope_base^(-2i/rotary_dim), i < rotary_dim/2, computed on the host and kept on the device.
+// rope_base^(-2i/rotary_dim), i < rotary_dim/2, computed on the host and kept on the device, table after
+// table behind the pool's planes.
 struct RopeFreqTable {
     float base;
     uint32_t rotary;
-    double *dev;
 };
 
 // One item's query rows against its slot; fills the split plan.
@@ -125,6 +125,8 @@ struct PlanInput {
 struct itak_pool {
     itak_pool_config cfg{};
     std::vector<RopeFreqTable> rope_tables;
+    double *rope_dev = nullptr;      // room for rope_tables_max tables of head_dim / 2
+    uint32_t rope_tables_max = 0;
     // Global layers and windowed layers are two groups of planes with their own row capacity:
     // `g` (capacity_rows per plane) and `gw` (the longest ring per plane). Within a group the
     // layers are consecutive, so the kernels that walk several layers take (group base,
@@ -374,31 +376,35 @@ itak_status ensure_stage(itak_pool *pool, uint64_t bytes) {
     return ITAK_OK;
 }
 
-// The rotation frequencies of (base, rotary_dim) in device memory, made on first use: the same
-// expression, in the same f64 libm, as rope.rs:99-116 and rope_interleaved.rs:103-114 evaluate
-// on the host. Null when the table does not exist yet and cannot be made now (the stream is
-// being captured, or the allocation failed): the preparation kernel then takes the powers itself.
+// The rotation frequencies of (base, rotary_dim) in device memory: the same expression, in the same f64
+// libm, as rope.rs:99-116 and rope_interleaved.rs:103-114 evaluate on the host. Made on first use by a
+// launch that carries them as its argument, ahead of the step on its stream: nothing is allocated and
+// nothing waits (as an allocation and a copy of its own it made a preparing decode step's first call
+// 31.6 us instead of 22.6; taking the powers in the kernel 19.5). Null when there is no room for another table, or none yet and the stream is being
+// captured: the preparation kernel then takes the powers itself.
 const double *rope_freq_table(itak_pool *pool, float base, uint32_t rotary) {
     if (!(base > 1.0f) || rotary < 2) return nullptr;
-    for (const RopeFreqTable &t : pool->rope_tables)
-        if (t.base == base && t.rotary == rotary) return t.dev;
+    const uint64_t width = pool->g.head_dim / 2;
+    for (size_t i = 0; i < pool->rope_tables.size(); ++i)
+        if (pool->rope_tables[i].base == base && pool->rope_tables[i].rotary == rotary) return pool->rope_dev + i * width;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(pool->stream, &status) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }
-    if (status != hipStreamCaptureStatusNone || pool->rope_tables.size() >= 64) return nullptr;
-    std::vector<double> host(rotary / 2);
-    for (uint32_t i = 0; i < rotary / 2; ++i)
-        host[i] = std::pow(double(base), -double(2 * i) / double(rotary));
-    double *dev = nullptr;
-    if (hipMalloc(reinterpret_cast<void **>(&dev), host.size() * sizeof(double)) != hipSuccess ||
-        hipMemcpy(dev, host.data(), host.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
-        (void)hipGetLastError();
-        if (dev) (void)hipFree(dev);
-        return nullptr;
+    if (status != hipStreamCaptureStatusNone || pool->rope_tables.size() >= pool->rope_tables_max) return nullptr;
+    double *dev = pool->rope_dev + pool->rope_tables.size() * width;
+    for (uint32_t first = 0; first < rotary / 2; first += kFillDoubles) {
+        FillDoubles a;
+        a.n = std::min<uint32_t>(kFillDoubles, rotary / 2 - first);
+        for (uint32_t i = 0; i < a.n; ++i)
+            a.v[i] = std::pow(double(base), -double(2 * (first + i)) / double(rotary));
+        if (launch_fill_doubles(dev + first, a, pool->stream) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
     }
-    pool->rope_tables.push_back(RopeFreqTable{base, rotary, dev});
+    pool->rope_tables.push_back(RopeFreqTable{base, rotary});
     return dev;
 }
 
@@ -1317,12 +1323,22 @@ itak_status itak_pool_create(const itak_pool_config *config, itak_pool **out) {
     pool->gw = gw;
     pool->rows_limit = config->capacity_rows;
     pool->bytes = bytes;
-    he = hipMalloc(reinterpret_cast<void **>(&pool->base), bytes);
+    // Rotation frequencies: 64 tables (bases and rotated widths) at the head dims that can attend.
+    pool->rope_tables_max = uint32_t(std::clamp<uint64_t>(16384 / config->head_dim, 4, 64));
+    uint64_t planes = 0, all = 0;
+    if (__builtin_add_overflow(bytes, uint64_t(255), &planes) ||
+        __builtin_add_overflow(planes &= ~uint64_t(255),
+                               pool->rope_tables_max * (config->head_dim / 2) * sizeof(double), &all)) {
+        delete pool;
+        return size_overflow(e, "global layer storage");
+    }
+    he = hipMalloc(reinterpret_cast<void **>(&pool->base), all);
     if (he != hipSuccess) {
         delete pool;
         return hip_error(e, he, "allocate KV pool");
     }
     pool->base_w = pool->base + bytes_g;
+    pool->rope_dev = reinterpret_cast<double *>(pool->base + planes);
     // Fresh storage is all zero bytes, as the reference's ring storage is
     // (cache.rs:139) and as the scrub guarantee needs.
     he = hipMemset(pool->base, 0, bytes);
@@ -1373,8 +1389,6 @@ void itak_pool_destroy(itak_pool *pool) {
     if (pool->prep) (void)hipFree(pool->prep);
     if (pool->xws) (void)hipFree(pool->xws);
     if (pool->die_words) (void)hipFree(pool->die_words);
-    for (const RopeFreqTable &t : pool->rope_tables)
-        if (t.dev) (void)hipFree(t.dev);
     for (void *buf : pool->ring_saved)
         if (buf) (void)hipFree(buf);
     release_hstage(pool);
