@@ -111,6 +111,9 @@ std::atomic<uint64_t> g_next_cache_id{1};  // cache.rs:32
 struct RopeFreqTable {
     float base;
     uint32_t rotary;
+    bool made;                   // by an eager launch: whatever runs later finds it
+    unsigned long long capture;  // the capture that holds a launch that makes it, and on which stream
+    hipStream_t stream;
 };
 
 // One item's query rows against its slot; fills the split plan.
@@ -380,20 +383,27 @@ itak_status ensure_stage(itak_pool *pool, uint64_t bytes) {
 // libm, as rope.rs:99-116 and rope_interleaved.rs:103-114 evaluate on the host. Made on first use by a
 // launch that carries them as its argument, ahead of the step on its stream: nothing is allocated and
 // nothing waits (as an allocation and a copy of its own it made a preparing decode step's first call
-// 31.6 us instead of 22.6; taking the powers in the kernel 19.5). Null when there is no room for another table, or none yet and the stream is being
-// captured: the preparation kernel then takes the powers itself.
+// 31.6 us instead of 22.6; taking the powers in the kernel 19.5). A first use inside a capture is captured
+// with the step, whose replays then make the table themselves, always the same; for everything outside
+// that graph it has yet to be made. Null when there is no room for another table: the preparation kernel
+// then takes the powers itself.
 const double *rope_freq_table(itak_pool *pool, float base, uint32_t rotary) {
     if (!(base > 1.0f) || rotary < 2) return nullptr;
-    const uint64_t width = pool->g.head_dim / 2;
-    for (size_t i = 0; i < pool->rope_tables.size(); ++i)
-        if (pool->rope_tables[i].base == base && pool->rope_tables[i].rotary == rotary) return pool->rope_dev + i * width;
+    size_t at = 0;
+    while (at < pool->rope_tables.size() && !(pool->rope_tables[at].base == base && pool->rope_tables[at].rotary == rotary)) ++at;
+    double *dev = pool->rope_dev + at * (pool->g.head_dim / 2);
+    if (at < pool->rope_tables.size() && pool->rope_tables[at].made) return dev;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(pool->stream, &status) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
+    unsigned long long capture = 0;
+    bool known = hipStreamGetCaptureInfo(pool->stream, &status, &capture) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    const bool captured = known && status == hipStreamCaptureStatusActive;
+    if (at == pool->rope_tables.size()) {
+        if (at == pool->rope_tables_max) return nullptr;
+        pool->rope_tables.push_back(RopeFreqTable{base, rotary, false, 0, nullptr});
     }
-    if (status != hipStreamCaptureStatusNone || pool->rope_tables.size() >= pool->rope_tables_max) return nullptr;
-    double *dev = pool->rope_dev + pool->rope_tables.size() * width;
+    RopeFreqTable &table = pool->rope_tables[at];
+    if (captured && table.capture == capture && table.stream == pool->stream) return dev;
     for (uint32_t first = 0; first < rotary / 2; first += kFillDoubles) {
         FillDoubles a;
         a.n = std::min<uint32_t>(kFillDoubles, rotary / 2 - first);
@@ -404,7 +414,9 @@ const double *rope_freq_table(itak_pool *pool, float base, uint32_t rotary) {
             return nullptr;
         }
     }
-    pool->rope_tables.push_back(RopeFreqTable{base, rotary});
+    table.made = known && status == hipStreamCaptureStatusNone;
+    table.capture = captured ? capture : 0;
+    table.stream = pool->stream;
     return dev;
 }
 

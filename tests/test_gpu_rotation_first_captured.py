@@ -1,0 +1,72 @@
+"""The first rotation of a pool may be captured into a graph: the rows it stores and the outputs are those
+of an eager first rotation, bit for bit, at every replay and of an eager step afterwards. At positions of
+a million a frequency that differs in its last bit shows in the stored f32 rows."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import normal, pkg
+from test_gpu_graph_replay import capture
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("elem,d,rows,rotary", [
+    ("f32", 128, 128, 0),   # the preparation launch
+    ("f32", 256, 40, 0),    # a table of two launches
+    ("f32", 96, 64, 40),    # part of the head turns
+    ("f16", 64, 128, 0),    # rounded rows
+    ("f16", 128, 1, 0),     # prepared inside the attention launch
+    ("f16", 128, 7, 64),
+])
+def test_a_first_rotation_inside_a_capture_equals_an_eager_one(elem, d, rows, rotary):
+    P = pkg()
+    rng = np.random.default_rng(d + rows)
+    q_heads, kv_heads, layers, window, base = 16, 4, 3, max(64, rows), 1e6
+    row, held = kv_heads * d, 1_000_000
+    stream = torch.cuda.current_stream()
+    q, k, v = (torch.from_numpy(normal(rng, layers, rows, w)).cuda() for w in (q_heads * d, row, row))
+    k0, v0 = normal(rng, window, row), normal(rng, window, row)
+
+    def make():
+        pool = P.KvPool([P.LayerKind.windowed(window)] * layers, kv_heads, d, elem=elem, ring_headroom=rows)
+        pool.set_stream(stream.cuda_stream)
+        cache = pool.acquire()
+        for layer in range(layers):
+            cache.restore_bulk(layer, held - window, k0, v0)
+        out = torch.empty_like(q)
+
+        def step(rope_base=base):
+            for layer in range(layers):
+                pool.attention_prep_step_device(
+                    layer, [(cache, rows)], q[layer].data_ptr(), k[layer].data_ptr(), v[layer].data_ptr(),
+                    out[layer].data_ptr(), q_heads, rope_base=rope_base, rotary_dim=rotary if rope_base else 0)
+
+        def result():
+            torch.cuda.synchronize()
+            kept = [np.asarray(x).tobytes() for layer in range(layers) for x in cache.view(layer).rows()[1:]]
+            return out.cpu().numpy().tobytes(), kept
+
+        step(rope_base=0.0)  # the pool's scratch reaches its size; nothing has turned yet
+        torch.cuda.synchronize()
+        pool.truncate([cache], [held])
+        return pool, cache, out, step, result
+
+    eager_pool, _, _, step, result = make()
+    step()
+    want = result()
+
+    pool, cache, out, step, result = make()
+    graph = capture(pool, stream, step)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        assert result() == want
+    pool.truncate([cache], [held])
+    out.fill_(float("nan"))
+    step()  # the pool's first eager rotation
+    assert result() == want
+    graph.replay()
+    assert result() == want
+    pool.close()
+    eager_pool.close()
