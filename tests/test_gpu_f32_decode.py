@@ -1,7 +1,8 @@
-"""Steps on f32 pools of head_dim 128 (the reference's own storage type) run on the f32 MFMA
-kernel: decode rows, verify blocks and prefill chunks as tiles of 16 query vectors; other head
-dims stay on the generic kernel. Both are held to the oracle within 1e-5 relative to the largest
-output magnitude, the f32 bar."""
+"""Steps on f32 pools (the reference's own storage type) run on the f32 MFMA kernel: decode rows, verify
+blocks and prefill chunks as tiles of 16 query vectors, at head_dim 64 and 128 in instantiations of their
+own, at other multiples of four in the padded ones. Head dims that are no multiple of four, explicit
+positions and tensors off 16-byte alignment stay on the generic kernel. All are held to the oracle within
+1e-5 relative to the largest output magnitude, the f32 bar."""
 import numpy as np
 import pytest
 import torch
@@ -100,13 +101,69 @@ def test_blocks_of_any_length_run_as_tiles_of_sixteen_vectors(ctxs, rows, q_head
 
 
 @pytest.mark.parametrize("ctxs,rows,q_heads,kv_heads,window", [
-    ([512], 1, 32, 4, None),                 # configs[0]: the reference's CPU-runnable case
+    ([512], 1, 32, 4, None),                 # the reference's CPU-runnable case
     ([0, 31, 1000], 1, 8, 2, None), ([700], 2, 32, 4, None), ([300, 64], 8, 32, 4, None),
     ([0], 200, 16, 4, None), ([900], 1, 32, 4, 256), ([600], 30, 8, 8, 128)])
 def test_head_dim_64_runs_on_the_same_kernel(ctxs, rows, q_heads, kv_heads, window):
     run(ctxs, rows=rows, q_heads=q_heads, kv_heads=kv_heads, window=window, steps=3, seed=rows + 64, d=64)
 
 
-def test_other_head_dims_keep_the_generic_kernel():
+def test_other_head_dims_run_padded():
     run([300], rows=1, q_heads=8, kv_heads=2, d=96, seed=11)
     run([300], rows=3, q_heads=4, kv_heads=2, d=256, seed=12)
+
+
+@pytest.fixture
+def kernels(capfd):
+    """The kernels of the attention launches since the last look, from the diagnostic channel."""
+    lib = P()._native.load()
+    lib.itak_set_debug_enabled(1)
+    capfd.readouterr()
+    yield lambda: [w[7:] for w in capfd.readouterr().err.split() if w.startswith("kernel=")]
+    lib.itak_set_debug_enabled(0)
+
+
+@pytest.mark.parametrize("elem,d", [("f32", 33), ("f32", 50), ("f16", 50), ("f16", 7)])
+def test_head_dims_that_are_no_multiple_of_four_run_on_the_generic_kernel(kernels, elem, d):
+    if elem == "f32":
+        run([300, 70], rows=1, q_heads=6, kv_heads=2, d=d, seed=13)
+        run([100], rows=20, q_heads=6, kv_heads=2, d=d, window=64, seed=14)
+    else:
+        rng = np.random.default_rng(d)
+        k, v, q = (normal(rng, 90, w) for w in (2 * d, 2 * d, 6 * d))
+        pool = P().KvPool(1, 2, d, elem=elem, capacity_rows=96)
+        cache, ref = pool.acquire(), oracle.KvCache.new([oracle.LayerKind.Global], 2, d, store_f16=True)
+        qd, kd, vd = (torch.from_numpy(x).cuda() for x in (q, k, v))
+        out = torch.empty_like(qd)
+        pool.attention_step_device(0, [(cache, 90)], qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), 6)
+        pool.synchronize()
+        want = oracle.attention_step(ref, 0, q, k, v, 6, 0, oracle.AttentionParams(), threads=8)
+        assert rel_err(out.cpu().numpy().reshape(-1), want) <= 1e-5
+        pool.close()
+    seen = kernels()
+    assert seen and set(seen) == {"generic"}, seen
+
+
+def test_explicit_positions_and_unaligned_tensors_run_on_the_generic_kernel(kernels):
+    rng = np.random.default_rng(15)
+    q_heads, kv_heads, d, n = 8, 2, 96, 200
+    k, v, q = (normal(rng, n, w) for w in (kv_heads * d, kv_heads * d, q_heads * d))
+    pool = P().KvPool(1, kv_heads, d, elem="f32", capacity_rows=n + 8)
+    cache, ref = pool.acquire(), oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, d)
+    cache.restore_bulk(0, 0, k, v)
+    ref.restore_bulk(0, 0, k, v)
+    at = [199, 3, 77]
+    kernels()
+    got = P().gqa_attention(q[:3], 3, q_heads, at, cache.view(0), P().AttentionParams())
+    assert kernels() == ["generic"]
+    want = oracle.gqa_attention(q[:3], 3, q_heads, at, ref.view(0), oracle.AttentionParams())
+    assert rel_err(np.asarray(got).reshape(-1), np.asarray(want).reshape(-1)) <= 1e-5
+    # A step whose tensors start four bytes into a line: new rows first, then the general kernel.
+    kept = [torch.from_numpy(np.concatenate([[0], x[:2].reshape(-1)]).astype(np.float32)).cuda() for x in (q, k, v, q)]
+    ptrs = [t.data_ptr() + 4 for t in kept]
+    pool.attention_step_device(0, [(cache, 2)], *ptrs, q_heads)
+    pool.synchronize()
+    assert kernels() == ["generic"]
+    want = oracle.attention_step(ref, 0, q[:2], k[:2], v[:2], q_heads, n, oracle.AttentionParams(), threads=8)
+    assert rel_err(kept[3].cpu().numpy()[1:], want) <= 1e-5
+    pool.close()
