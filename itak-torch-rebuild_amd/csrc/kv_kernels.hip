@@ -377,6 +377,7 @@ __global__ __launch_bounds__(256) void kv_restore_scalar(D *__restrict__ pool_ba
     }
 }
 
+constexpr uint32_t kBlockLdsMaxDim = 496;  // 2 * 32 * (496 + 8) * 2 bytes = 63 KB
 hipError_t launch_restore(void *pool_base, int dst_f16, int src_f16, const PoolGeom &g,
                           const RestoreBatch &b, hipStream_t stream) {
     if (b.n == 0 || b.max_rows == 0) return hipSuccess;
@@ -388,7 +389,8 @@ hipError_t launch_restore(void *pool_base, int dst_f16, int src_f16, const PoolG
     }
     const uint32_t vec = src_f16 ? 8 : 4;
     const bool use_vec = aligned && (g.head_dim % vec == 0);
-    if (!use_vec || (g.v_block != 0 && !block_aligned)) {
+    // (A block's rows of both sides have to fit the LDS a launch may ask for.)
+    if (!use_vec || (g.v_block != 0 && (!block_aligned || g.head_dim > kBlockLdsMaxDim))) {
         const uint64_t per_layer = uint64_t(b.max_rows) * g.kv_heads * g.head_dim;
         uint32_t bx = uint32_t((per_layer + 255) / 256);
         if (bx > 2048) bx = 2048;

@@ -955,9 +955,10 @@ itak_status run_append(itak_pool *pool, uint64_t layer, const itak_batch_item *i
                        const float *k_dev, const float *v_dev) {
     const LayerInfo &L = pool->layers[layer];
     const PoolGeom &geom = geom_of(pool, layer);
-    // A long run of one slot's rows into blocked planes (a prefill chunk) moves by blocks.
+    // A long run of one slot's rows into blocked planes (a prefill chunk) moves by blocks. (At the head
+    // dims that can attend; a block's rows of wider heads outgrow the LDS a launch may ask for.)
     constexpr uint32_t kChunkRows = 64;
-    if (n == 1 && pool->elem_f16 && geom.v_block != 0 && items[0].rows >= kChunkRows && aligned16(k_dev) && aligned16(v_dev) &&
+    if (n == 1 && pool->elem_f16 && geom.v_block != 0 && geom.head_dim <= 256 && items[0].rows >= kChunkRows && aligned16(k_dev) && aligned16(v_dev) &&
         (!L.windowed || (L.ring % kVBlock == 0 && items[0].rows <= L.ring))) {
         const uint32_t slot = items[0].slot, rows = items[0].rows;
         HIP_TRY(pool, launch_append_chunk(layer_base(pool, layer), geom, slot, uint32_t(pool->slots[slot].appended[layer]), rows,

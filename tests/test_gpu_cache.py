@@ -146,6 +146,27 @@ def test_chunk_append_is_bit_exact_and_leaves_its_neighbours_alone(start, rows):
     pool.close()
 
 
+@pytest.mark.parametrize("head_dim", [256, 272, 496, 512, 1008, 1040])
+def test_wide_heads_append_and_restore_by_whatever_moves_them(head_dim):
+    # Up to 256 a chunk moves by blocks, up to 496 a restore does (a block's rows fit the LDS a launch may
+    # ask for); wider heads go row by row.
+    import torch
+    rng = np.random.default_rng(head_dim)
+    n = 70
+    k, v = normal(rng, n, 2 * head_dim), normal(rng, n, 2 * head_dim)
+    kd, vd = torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda()
+    pool = P().KvPool(1, 2, head_dim, elem="f16", max_slots=2, capacity_rows=96)
+    appended, restored = pool.acquire(), pool.acquire()
+    pool.append_device(0, [(appended, n)], kd.data_ptr(), vd.data_ptr())
+    restored.restore_bulk_ptr(0, 0, kd.data_ptr(), vd.data_ptr(), k.size, src_f16=False)
+    pool.synchronize()
+    for cache in (appended, restored):
+        _, gk, gv = cache.read_rows(0, 0, n)
+        assert np.array_equal(gk.reshape(n, -1), oracle.f32_to_f16_array(k))
+        assert np.array_equal(gv.reshape(n, -1), oracle.f32_to_f16_array(v))
+    pool.close()
+
+
 def test_f32_to_f16_conversion_matches_the_oracle_on_every_rounding_class():
     import torch
 
