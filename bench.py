@@ -161,8 +161,7 @@ def cache_maintenance(args, pkg, torch, dev, stream, timed):
             "data": "synthetic",
             "config": {"workload": "append of a 2048-row chunk per layer into a 30720-row f16 cache, "
                                    "8 layers cycled, HIP graph replay", "layers_per_step": layers},
-            "roofline": {"bound": "hbm", "kernel": "kv_append_kernel (rows up to the block boundary) + "
-                                                   "kv_restore_blocked (chunk append, per layer)", "achieved": round(gbs, 2),
+            "roofline": {"bound": "hbm", "kernel": "kv_append_chunk (one launch per layer)", "achieved": round(gbs, 2),
                          "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
                          "traffic": None, "us_per_launch": round(step_s / layers * 1e6, 3),
                          "bytes_per_launch": bytes_layer},
@@ -979,7 +978,8 @@ def run_workload(args, pkg, torch, np, dev, stream, timed):
         lean = args.kv == "f16" and rows == 1 and wl in ("decode", "hybrid")
         roofline = {
             "bound": "hbm",
-            "kernel": (("attn_decode_f16_kernel" if lean else f"attn_splitk_{args.kv}_kernel") +
+            "kernel": (("attn_decode_f16_kernel" if lean else
+                        "attn_splitk_rows_kernel" if args.kv == "f32" else "attn_splitk_f16_kernel") +
                        (" (splits merged inside the launch)" if args.merge_in_launch else
                         " (each unit's splits merged on its compute die by the unit's last "
                         "workgroup: one launch per layer)" if merge_form == "on_die" else
