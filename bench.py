@@ -46,11 +46,11 @@ MFMA_F16_PEAK_TFLOPS = 2500.0
 # known size: (bytes, the summary under profiles/ that holds the run and the scaling factors).
 # They are not measured by this run: `traffic_source` says where each came from.
 PROFILE_TRAFFIC = {
-    ("decode", "f16"): (9_805_775, "profiles/attn_decode_f16_ctx4096_traffic.md"),
-    ("ragged", "f16"): (216_797_776, "profiles/attn_splitk_f16_ragged16_traffic.md"),
+    ("decode", "f16"): (9_805_777, "profiles/attn_decode_f16_ctx4096_traffic.md"),
+    ("ragged", "f16"): (216_737_831, "profiles/attn_splitk_f16_ragged16_traffic.md"),
     ("prefill", "f16"): (201_442_441, "profiles/attn_prefill_f16_chunk2048_prefix30720_traffic.md"),
-    ("verify", "f16"): (87_437_369, "profiles/attn_splitk_f16_verify_traffic.md"),
-    ("decode", "f32"): (18_240_825, "profiles/attn_splitk_f32_decode_ctx4096_traffic.md"),
+    ("verify", "f16"): (87_447_720, "profiles/attn_splitk_f16_verify_traffic.md"),
+    ("decode", "f32"): (18_267_848, "profiles/attn_splitk_f32_decode_ctx4096_traffic.md"),
 }
 
 
@@ -979,7 +979,9 @@ def run_workload(args, pkg, torch, np, dev, stream, timed):
         roofline = {
             "bound": "hbm",
             "kernel": (("attn_decode_f16_kernel" if lean else
-                        "attn_splitk_rows_kernel" if args.kv == "f32" else "attn_splitk_f16_kernel") +
+                        "attn_splitk_rows_kernel" if args.kv == "f32" else
+                        "attn_splitk_f16_tiled_kernel" if wl == "ragged" and merge_form == "launch" else
+                        "attn_splitk_f16_kernel") +
                        (" (splits merged inside the launch)" if args.merge_in_launch else
                         " (each unit's splits merged on its compute die by the unit's last "
                         "workgroup: one launch per layer)" if merge_form == "on_die" else
