@@ -203,10 +203,16 @@ static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows
 // two and four tiles a wavefront are the better ones. Four tiles: up to 9 blocks per compute unit, 7 where
 // 16 units and more leave those forms at most 16 splits to merge; two tiles: up to 20. One tile always
 // (one workgroup per compute unit, of eight wavefronts from 16 blocks on: twice as many, with
-// half the run, lost everywhere to the larger merge). 32 Q / 4 KV heads, us a layer, before -> tiled: seven
+// half the run, lost everywhere to the larger merge), but for one-row steps that prepare their rows: up to
+// five blocks per compute unit a wavefront has one or two, and the form with two sets of operands asks for
+// the second before the rotation waits (32 Q / 4 KV heads at 700 / 2,048 / 4,096, tiled -> not, 8.9 / 9.1 /
+// 9.7 -> 8.8 / 9.0 / 9.5; 8 KV heads 9.3 / 9.6 / 10.1 -> 9.1 / 9.4 / 9.8; at 16,384 and 8,192 12.7 and 11.6
+// against 12.9 and 11.9). 32 Q / 4 KV heads, us a layer, before -> tiled: seven
 // rows at 1,000 / 4,096 / 16,384 11.4 / 12.5 / 18.3 -> 9.0 / 9.8 / 16.9, four rows 9.5 / 9.9 / 15.5 ->
 // 8.4 / 8.8 / 13.1, 8 slots of four rows at 2,000 16.5 -> 14.6; one row at 16,384 12.3 -> 11.6.
-static bool takes_tiles(const PoolGeom &g, const AttnBatch &b, uint32_t tiles, uint64_t blocks, uint64_t cus) {
+static bool takes_tiles(const PoolGeom &g, const AttnBatch &b, uint32_t tiles, uint64_t blocks, uint64_t cus,
+                        bool prepares_one) {
+    if (prepares_one && blocks <= 5 * cus) return false;
     return tiles == 1 || blocks <= (tiles == 2 ? 20 : g.kv_heads * b.n < 16 ? 9 : 7) * cus;
 }
 
@@ -228,7 +234,7 @@ uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads,
     }
     const uint64_t cus = compute_units();
     const uint32_t tiles = (most_rows * group + 15) / 16;
-    const bool may = may_tile && takes_tiles(g, b, tiles, blocks, cus);
+    const bool may = may_tile && takes_tiles(g, b, tiles, blocks, cus, prepares && most_rows == 1);
     const bool whole = most <= whole_limit(g, b, most_rows, tiles, prepares, may);
     b.whole_on_eight = whole && most > 4 && (may || most_rows == 1) ? 1 : 0;
     // (A whole one-row step has no second tile and hardly a second block: the form with two sets of
