@@ -412,9 +412,10 @@ uint32_t attn_splitk_any_groups_per_cu(const PoolGeom &g) {
 // f16 steps of up to 16 query vectors per KV head, and of a few rows more, of which every tile's workgroups
 // that reach the new positions store all: 3 us of launch saved, a microsecond spent for eight rows
 // (scattered stores of two bytes; head_dim 80, 32 Q / 8 KV heads, six rows at 450 12.5 -> 9.7 us a layer;
-// twenty rows 9.9 -> 11.0).
+// twenty rows 9.9 -> 11.0). More than eight rows of wide heads are too many for the one wavefront that owns
+// their block: head_dim 256, 8 Q / 8 KV heads, sixteen rows at 400 / 1,100 21.0 / 22.9 -> 15.6 / 16.7.
 bool attn_splitk_any_appends(const PoolGeom &g, int elem_f16, uint32_t group, uint32_t max_rows) {
-    return attn_splitk_any_supports(g, group, max_rows) && (!elem_f16 || max_rows * group <= 16 || max_rows <= 8);
+    return attn_splitk_any_supports(g, group, max_rows) && (!elem_f16 || max_rows <= 8 || (max_rows * group <= 16 && max_rows * g.head_dim <= 2048));
 }
 
 hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
