@@ -227,7 +227,7 @@ __global__ __launch_bounds__(W * 64, DP <= 128 && W == 4 ? 2 : 1) void attn_spli
     const uint32_t own_to = min(item.rows, (vtile * 16 + 16 + group - 1) / group);
     const uint32_t quads = D / 4;
     const uint32_t own_pieces = kInPlace && fused && own_to > own_from ? (own_to - own_from) * 2 * quads : 0;
-    const uint32_t own_first = split * (W * 64) + tid;
+    const uint32_t own_first = (item.splits - 1 - split) * (W * 64) + tid;  // (the last split's run is the shortest)
     auto own_piece = [&](uint32_t f, const float *&src, T *&dst) {
         const uint32_t r = own_from + f / (2 * quads), rest = f % (2 * quads), side = rest >= quads ? 1 : 0;
         const uint32_t pos = item.pos0 + r, c4 = (rest - side * quads) * 4;
