@@ -2,6 +2,8 @@
 // instantiations (attn_prefill_f16_kernel.h has the kernel).
 #include "attn_prefill_f16_kernel.h"
 
+#include <cmath>
+
 // Timeline marks of attn_prefill_f16_kernel: 0 first instruction, 1 addresses known, 2 first
 // blocks and Q requested, 3 Q converted (it has arrived), 4 first block multiplied, 5 last block
 // multiplied, 6 output or partials issued, 11 all done; of the first block: 7 its loads have
@@ -38,26 +40,44 @@ static uint32_t unit_block_count(const AttnItem &it, uint32_t rows_per_group, ui
 // cheapest. A wavefront holds one or two 16-vector tiles (`tiles`), so a workgroup 64 or 128 vectors,
 // and every (row tile, KV head) unit's context is cut into equal runs.
 //
-// The walk. Alone on its compute unit a workgroup takes kAlone a block: with three blocks in flight
+// The walk. Alone on its compute unit a workgroup takes `alone` a block: with three blocks in flight
 // one tile waits for memory, two for the chain of their products. Two to a compute unit share it,
-// kShared a block of each: less than twice as much, since the waiting overlaps. More workgroups than
-// the device holds at once queue behind one another, the longest first. Splits cost a second launch
-// (kMerge) and their partials, written and read again at kPartialRate.
+// `shared` a block of each: less than twice as much, since the waiting overlaps (at head_dim 256 there is
+// room for one, and the second comes after it). More workgroups than the device holds at once queue
+// behind one another, the longest first. Splits cost a second launch (`merge`) and their partials, written
+// and read again at `rate`.
 //
-// Fitted on 9 to 1,200 rows over contexts of 0 to 30,000 at 1, 4 and 8 KV heads, global and windowed,
-// with every count of tiles and splits timed for each: the pick is 1.4 % behind the best of them on
-// average; the rules by size it replaces, which also had an eight-stage ring for launches of one
-// workgroup per compute unit (never the best of a shape), were 7 % behind.
+// Head_dim 128: fitted on 9 to 1,200 rows over contexts of 0 to 30,000 at 1, 4 and 8 KV heads, global and
+// windowed, with every count of tiles and splits timed for each: the pick is 1.4 % behind the best of
+// them on average; the rules by size it replaces, which also had an eight-stage ring for launches of one
+// workgroup per compute unit (never the best of a shape), were 7 % behind. The other head dims have
+// figures of their own, fitted the same way on 4 to 200 rows, 1 to 16 slots and contexts of 90 to 9,000, with
+// what the launch reads as a second bound: a block does not take half the time at half the head_dim, and a
+// merge launch is another kernel there, with less of a rate. With the figures of 128 scaled by the head_dim,
+// windows and contexts of a few hundred positions stayed whole and runs at 256 were never shorter than eight
+// blocks: 5 to 14 % behind the best plan, up to 65; with their own 1.2 to 2 %, up to 23. Us a layer: head_dim
+// 256, four rows at 400 20.3 -> 12.5; head_dim 96, four rows on a window of 512 14.0 -> 10.4; head_dim 64, 5
+// slots of seven rows at 1,100 17.1 -> 14.1. (The other way: head_dim 64, 16 slots of seven at 1,100 17.8 ->
+// 20.9.)
 struct PlanCost {
-    static constexpr float kAlone[2] = {0.345f, 0.56f}, kShared[2] = {0.6f, 0.83f};
-    static constexpr float kMerge = 4.5f, kPartialRate = 2.5e6f;  // bytes a microsecond
+    float alone[2], shared[2], merge;
+    float rate;              // bytes a microsecond
+    float hidden, read_rate; // what a launch reads once, beside that part of its walk (0 = not priced)
 };
+static const PlanCost &plan_cost(uint32_t head_dim) {
+    static constexpr PlanCost k64 = {{0.30f, 0.43f}, {0.47f, 0.78f}, 4.1f, 1.25e6f, 0.14f, 16.2e6f};
+    static constexpr PlanCost k96 = {{0.41f, 0.56f}, {0.58f, 0.67f}, 4.2f, 1.14e6f, 0.16f, 8.0e6f};
+    static constexpr PlanCost k128 = {{0.345f, 0.56f}, {0.6f, 0.83f}, 4.5f, 2.5e6f, 0.0f, 0.0f};
+    static constexpr PlanCost k256 = {{0.70f, 1.20f}, {2.79f, 4.74f}, 4.7f, 5.8e6f, 0.38f, 5.2e6f};
+    return head_dim <= 64 ? k64 : head_dim <= 96 ? k96 : head_dim <= 128 ? k128 : k256;
+}
 
 struct Shape {
     uint64_t groups = 0;         // workgroups
     uint64_t blocks = 0;         // blocks all of them walk
     float longest = 0.0f;        // and one of them at most
     uint64_t partial_bytes = 0;
+    uint64_t read_bytes = 0;     // keys and values, once
 };
 // An item's blocks per unit and its units, for the tiles at hand.
 struct ItemWork {
@@ -73,22 +93,22 @@ static Shape shape_of(const PoolGeom &g, const AttnBatch &b, const ItemWork *wor
         // (A causal row tile ends where its rows do.)
         s.blocks += uint64_t(units) * (nb - (window ? 0 : std::min(rows / 64, nb / 2)));
         // (The workgroups that convert and place new rows walk that much less, see below.)
-        s.longest = std::max(s.longest, float(nb + (appends ? rows / 8 + 1 : 0)) / float(splits));
+        const float run = float(nb + (appends ? rows / 8 + 1 : 0)) / float(splits);
+        s.longest = std::max(s.longest, g.head_dim == 128 ? run : std::ceil(run));  // (as each was fitted)
+        s.read_bytes += uint64_t(g.kv_heads) * nb * stage_bytes(int(g.head_dim));
         if (splits > 1) s.partial_bytes += uint64_t(rows) * q_heads * splits * (g.head_dim + 2) * 4;
     }
     return s;
 }
-static float cost_of(const PoolGeom &g, const Shape &s, int tiles, uint64_t per_cu) {
-    const float wide = float(g.head_dim) / 128.0f;
-    const float alone = PlanCost::kAlone[tiles - 1] * wide;
-    // (head_dim 256 leaves room for one workgroup per compute unit.)
-    const float shared = g.head_dim > 128 ? 2 * alone : PlanCost::kShared[tiles - 1] * wide;
+static float cost_of(const PlanCost &cost, const Shape &s, int tiles, uint64_t per_cu) {
+    const float alone = cost.alone[tiles - 1], shared = cost.shared[tiles - 1];
     float walk = s.longest * alone;
     if (s.groups > 2 * per_cu)
         walk = std::max(walk, 0.5f * walk + float(s.blocks) / float(2 * per_cu) * shared);
     else if (s.groups > per_cu)
         walk = std::max(walk, 0.27f * walk + 0.73f * float(s.blocks) / float(s.groups) * shared);
-    return walk + (s.partial_bytes ? PlanCost::kMerge + float(s.partial_bytes) / PlanCost::kPartialRate : 0.0f);
+    if (cost.read_rate > 0.0f) walk = std::max(walk, cost.hidden * walk + float(s.read_bytes) / cost.read_rate);
+    return walk + (s.partial_bytes ? cost.merge + float(s.partial_bytes) / cost.rate : 0.0f);
 }
 
 // Fills splits / keys_per_split / block0 / ws0 and the tiles for a batch (slot, rows, pos0, q_row0,
@@ -118,11 +138,14 @@ uint32_t attn_prefill_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t group, 
         for (uint32_t c = 0; c < sizeof(kCounts); c += b.n > 8 && c ? 2 : 1) {
             const uint32_t run = std::max((most + kCounts[c] - 1) / kCounts[c], 1u);
             if (run == before) continue;
-            // (A run asks for three blocks more than it walks, at head_dim 256 of 32 KiB each: 4 slots of one
-            // row over 1,500, 8 KV heads, in runs of six 22.8 us, of eight 17.8.)
-            if (c && run < (g.head_dim > 128 ? 8u : 2u)) break;
+            // (A run asks for three blocks more than it walks, at head_dim 256 of 32 KiB each. One-row steps there
+            // are many short units and mind: 4 slots over 1,500, 8 KV heads, in runs of six 22.8 us, of eight 17.8.
+            // Steps of several rows do not: one slot of four rows at 400, 4 KV heads, 20.4 -> 12.5 with runs of two.)
+            if (c && run < (g.head_dim > 128 && nvec <= 16 ? 8u : 2u)) break;
             before = run;
-            const float cost = cost_of(g, shape_of(g, b, work, q_heads, window, run, appends), tiles, per_cu);
+            const Shape shape = shape_of(g, b, work, q_heads, window, run, appends);
+            if (b.partial_limit && shape.partial_bytes > b.partial_limit) break;  // (the whole contexts come first and have none)
+            const float cost = cost_of(plan_cost(g.head_dim), shape, tiles, per_cu);
             if (cost < least) {
                 least = cost;
                 T = run;

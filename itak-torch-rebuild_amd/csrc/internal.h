@@ -303,6 +303,7 @@ struct AttnBatch {
     uint32_t half_blocks; // host side only: the rows kernel's wavefronts take half a block each
     uint32_t tiled; // host side only: the split-K plan gives every 16 query vectors their own workgroups
     uint32_t whole_on_eight; // host side only: the split-K plan leaves every item whole on eight wavefronts
+    uint64_t partial_limit;  // host side only: bytes of partials the block kernel's plan may take (0 = any)
     AttnItem item[kMaxBatchItems];
 };
 // The kernel argument form of AttnBatch, sized to the batch: kernel arguments are

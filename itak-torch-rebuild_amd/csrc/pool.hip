@@ -764,6 +764,9 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         b.n = count;
         b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.tiled = b.on_eight = b.half_blocks = 0;
         b.two_halves = prefill && pool->q_two_halves && pool->g.head_dim == 128 ? 1 : 0;
+        // (At head_dim 128 a step whose best plan outgrows the static workspace is refused; at the others it
+        // takes the best that fits.)
+        b.partial_limit = (need_only || pool->no_alloc_call) && pool->g.head_dim != 128 ? kScratchBytes - kScratchExchangeBytes : 0;
         uint32_t total_rows = 0;
         for (uint32_t i = 0; i < count; ++i) {
             const PlanInput &pi = in[first + i];

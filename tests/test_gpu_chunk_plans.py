@@ -74,3 +74,39 @@ def test_chunks_against_the_oracle(rows, ctx, q_heads, kv_heads, window):
     want = oracle.attention_step(ref, 0, q, k[ctx:], v[ctx:], q_heads, ctx, threads=8)
     assert max_abs(out.cpu().numpy().reshape(-1), want) <= 2e-3
     pool.close()
+
+
+# The block kernel at its other head dims, whose plans are priced by figures of their own: few and many rows,
+# short runs and long ones, one and several items. The allocation-free call takes the best plan its workspace
+# holds.
+@pytest.mark.parametrize("window", [None, 200])
+@pytest.mark.parametrize("q_heads,kv_heads", [(32, 4), (8, 1), (6, 3)])
+@pytest.mark.parametrize("rows,ctx", [(9, 40), (7, 420), (17, 600), (40, 1500), (130, 300), (60, 3900)])
+@pytest.mark.parametrize("d", [64, 96, 256])
+def test_blocks_at_the_other_head_dims(d, rows, ctx, q_heads, kv_heads, window):
+    P = pkg()
+    kind = P.LayerKind.Global if window is None else P.LayerKind.windowed(window)
+    okind = oracle.LayerKind.Global if window is None else oracle.LayerKind.windowed(window)
+    rng = np.random.default_rng(rows + ctx + d)
+    contexts, width = (ctx, ctx // 5), kv_heads * d
+    refs = [oracle.KvCache.new([okind], kv_heads, d, store_f16=True) for _ in contexts]
+    pools = [P.KvPool([kind], kv_heads, d, elem="f16", max_slots=2, capacity_rows=ctx + rows, ring_headroom=max(64, rows))
+             for _ in range(2)]
+    caches = [[pool.acquire() for _ in contexts] for pool in pools]
+    for s, n in enumerate(contexts):
+        first = 0 if window is None else max(0, n - window)
+        k, v = normal(rng, n - first, width), normal(rng, n - first, width)
+        for cache in (caches[0][s], caches[1][s], refs[s]):
+            cache.restore_bulk(0, first, k, v)
+    q, k, v = (normal(rng, 2 * rows, w) for w in (q_heads * d, width, width))
+    qd, kd, vd = dev(q), dev(k), dev(v)
+    want = np.concatenate([np.asarray(oracle.attention_step(refs[s], 0, q[s * rows:][:rows], k[s * rows:][:rows],
+                                                            v[s * rows:][:rows], q_heads, contexts[s], threads=8)).reshape(-1)
+                           for s in range(2)])
+    for pool, held, step in zip(pools, caches, ("attention_step_device", "attention_step_device_noalloc")):
+        pool.set_stream(torch.cuda.current_stream().cuda_stream)
+        out = torch.full_like(qd, float("nan"))
+        getattr(pool, step)(0, [(c, rows) for c in held], qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), q_heads)
+        torch.cuda.synchronize()
+        assert max_abs(out.cpu().numpy().reshape(-1), want) <= 2e-3, step
+        pool.close()
