@@ -105,9 +105,13 @@ enum {
    is NaN the whole output row. One difference is left on f16 pools: a softmax weight below about
    2^-24 of its row's largest (a scaled score 17 below the row's maximum) is zero as an f16
    operand, and zero times an infinite value is NaN where the reference has an infinity.
-   Matrix-pipe kernels exist for f16 pools at head_dim 64, 96, 128 and 256 with up to 16 Q heads per
-   KV head and for f32 pools at head_dim 64 and 128; every other shape (any head_dim up to 256)
-   runs on a general kernel that is correct and one to two orders of magnitude slower. */
+   Every head_dim up to 256 that is a multiple of four runs on the matrix pipe. f16 pools have
+   kernels of their own at 64, 96, 128 and 256 with up to 16 Q heads per KV head (above); at 64, 96
+   and 256 the steps of up to 16 query vectors per KV head, and at other head dims and wider groups
+   every step, hold f32's precision over the stored rows (queries and weights enter as three f16
+   each, or the f32 pipe is used). What is left (head dims that are no multiple of four, explicit query
+   positions that do not follow one another, tensors that do not start on 16 bytes) runs on a
+   general kernel that is correct and one to two orders of magnitude slower. */
 enum { ITAK_ELEM_F32 = 0, ITAK_ELEM_F16 = 1 };
 
 /* Layer kinds (attention::LayerKind, cache.rs:36-48). */
@@ -436,9 +440,12 @@ itak_status itak_kv_capture_itkv_f16(itak_pool *pool, uint32_t slot, const char 
 /* KvSnapshot::from_bytes followed by restore_checked (snapshot.rs:351-371) into a fresh
    slot (either format version; f16 rows go into an f16 pool as they are and are refused by
    an f32 pool): the snapshot's geometry must be the pool's, and, when expected_fingerprint is not
-   NULL, its fingerprint the expected one. The rows are gathered from `bytes` in place when
-   the device can read them there (pinned host or device memory, 4-byte aligned payload),
-   otherwise staged. An f32 snapshot into an f16 pool converts exactly as append does. */
+   NULL, its fingerprint the expected one. A payload of 128 KB and more goes to a device buffer of
+   its own size for the length of the call, is summed there (version 1; version 2 by host threads
+   meanwhile) and gathered from there once the sum is known good; where that buffer cannot be had,
+   and below that size, the host sums, and the rows are gathered from `bytes` in place when the device
+   can read them there (pinned memory, 4-byte aligned payload), otherwise staged. An f32 snapshot into
+   an f16 pool converts exactly as append does. */
 itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *bytes, uint64_t len,
                                  const char *expected_fingerprint,
                                  uint64_t expected_fingerprint_len);

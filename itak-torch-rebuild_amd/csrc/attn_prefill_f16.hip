@@ -56,8 +56,8 @@ static uint32_t unit_block_count(const AttnItem &it, uint32_t rows_per_group, ui
 // merge launch is another kernel there, with less of a rate. With the figures of 128 scaled by the head_dim,
 // windows and contexts of a few hundred positions stayed whole and runs at 256 were never shorter than eight
 // blocks: 5 to 14 % behind the best plan, up to 65; with their own 1.2 to 2 %, up to 23. Us a layer: head_dim
-// 256, four rows at 400 20.3 -> 12.5; head_dim 96, four rows on a window of 512 14.0 -> 10.4; head_dim 64, 5
-// slots of seven rows at 1,100 17.1 -> 14.1. (The other way: head_dim 64, 16 slots of seven at 1,100 17.8 ->
+// 256, four rows at 400 20.3 -> 12.5; head_dim 96, four rows on a window of 512 14.0 -> 10.1; head_dim 64, 5
+// slots of seven rows at 1,100 17.1 -> 14.0. (The other way: head_dim 64, 16 slots of seven at 1,100 17.8 ->
 // 20.9.)
 struct PlanCost {
     float alone[2], shared[2], merge;

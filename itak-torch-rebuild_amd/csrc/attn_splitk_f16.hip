@@ -187,7 +187,9 @@ static uint32_t variant_capacity(const Variant &v) {
 // together). One layer of 32 Q / 4 KV heads, us, split -> whole: 1 slot at 200 / 300 rows
 // 7.3 / 7.4 -> 5.1 / 5.4 (7.2 -> 7.2 at 400), 16 slots at 300 / 600 11.0 / 12.7 -> 8.7 / 11.1, with
 // preparation 1 slot at 200 / 500 9.2 / 9.3 -> 6.2 / 8.6; seven rows at 150 / 350 / 500 8.6 / 8.9 / 8.9 ->
-// 6.8 / 7.2 / 7.8, 8 slots of them at 700 13.8 -> 13.1.
+// 6.8 / 7.2 / 7.8, 8 slots of them at 700 13.8 -> 13.1. Checked at 4, 8 and 1 KV heads and groups of 1 to 8 with
+// every shape forced either way: within 5 % of the better but for a few just past a line (16 slots of one
+// row at 900, 8 KV heads, split 19.1, whole 16.5).
 static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows, uint32_t tiles, bool prepares,
                             bool may_tile) {
     if (rows > 1) return !may_tile ? 8 : g.kv_heads * b.n * tiles >= 128 ? 24 : 16;
