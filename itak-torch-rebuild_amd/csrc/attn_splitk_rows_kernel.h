@@ -223,11 +223,12 @@ __global__ __launch_bounds__(W * 64, DP <= 128 && W == 4 ? 2 : 1) void attn_spli
     };
     // The rows this workgroup copies (see above). A thread's first piece is asked for now and stored at
     // the end.
-    const uint32_t own_from = (vtile * 16 + group - 1) / group;
-    const uint32_t own_to = min(item.rows, (vtile * 16 + 16 + group - 1) / group);
+    const uint32_t own_from = row_first + (row_first * group < vtile * 16 ? 1 : 0), own_to = row_last + 1;
     const uint32_t quads = D / 4;
-    const uint32_t own_pieces = kInPlace && fused && own_to > own_from ? (own_to - own_from) * 2 * quads : 0;
-    const uint32_t own_first = (item.splits - 1 - split) * (W * 64) + tid;  // (the last split's run is the shortest)
+    const uint32_t own_base = (item.splits - 1 - split) * (W * 64);  // (the last split's run is the shortest)
+    const uint32_t own_rows = kInPlace && fused && own_to > own_from ? own_to - own_from : 0;
+    const uint32_t own_pieces = own_base < own_rows * 2 * quads ? own_rows * 2 * quads : 0;
+    const uint32_t own_first = own_base + tid;
     auto own_piece = [&](uint32_t f, const float *&src, T *&dst) {
         const uint32_t r = own_from + f / (2 * quads), rest = f % (2 * quads), side = rest >= quads ? 1 : 0;
         const uint32_t pos = item.pos0 + r, c4 = (rest - side * quads) * 4;
