@@ -146,6 +146,31 @@ def test_chunk_append_is_bit_exact_and_leaves_its_neighbours_alone(start, rows):
     pool.close()
 
 
+@pytest.mark.parametrize("head_dim,start,rows", [(128, 0, 1023), (128, 0, 1024), (128, 37, 1025), (80, 3, 1639),
+                                                 (80, 0, 1638), (256, 5, 512)])
+def test_runs_that_no_cache_holds_are_stored_alike(head_dim, start, rows):
+    # From 4 MB of f16 rows on a run is stored with the streaming hint: either side of that size, from aligned and
+    # unaligned positions, every byte is the host conversion's and nothing beside the run is touched.
+    import torch
+
+    width = 8 * head_dim
+    rng = np.random.default_rng(head_dim + start + rows)
+    n = start + rows
+    k, v = normal(rng, n, width), normal(rng, n, width)
+    kd, vd = torch.from_numpy(k).cuda(), torch.from_numpy(v).cuda()
+    pool = P().KvPool(1, 8, head_dim, elem="f16", capacity_rows=n + 70)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    cache = pool.acquire()
+    for first, last in ((0, start), (start, n)):
+        if last > first:
+            pool.append_device(0, [(cache, last - first)], kd[first:].data_ptr(), vd[first:].data_ptr())
+    gk, gv = cache.read_raw(0)
+    assert np.array_equal(gk[:n].reshape(n, width), oracle.f32_to_f16_array(k))
+    assert np.array_equal(gv[:n].reshape(n, width), oracle.f32_to_f16_array(v))
+    assert not gk[n:].any() and not gv[n:].any()
+    pool.close()
+
+
 @pytest.mark.parametrize("head_dim", [256, 272, 496, 512, 1008, 1040])
 def test_wide_heads_append_and_restore_by_whatever_moves_them(head_dim):
     # Up to 256 a chunk moves by blocks, up to 496 a restore does (a block's rows fit the LDS a launch may
