@@ -405,7 +405,6 @@ bool attn_splitk_any_supports(const PoolGeom &g, uint32_t group, uint32_t max_ro
 }
 // By the registers of a wavefront: up to 168, up to 256, and more than that.
 uint32_t attn_splitk_any_groups_per_cu(const PoolGeom &g) {
-    if (g.v_block) return g.head_dim <= 64 ? 3 : g.head_dim <= 128 ? 2 : 1;
     return g.head_dim <= 64 ? 3 : g.head_dim <= 128 ? 2 : 1;
 }
 // f32 steps bring their rows along (attn_splitk_rows_kernel.h: they are read where they are). So do
