@@ -107,7 +107,7 @@ std::atomic<uint64_t> g_next_cache_id{1};  // cache.rs:32
 }  // namespace
 
 // rope_base^(-2i/rotary_dim), i < rotary_dim/2, computed on the host and kept on the device, table after
-// table behind the pool's planes.
+// table behind the pool's planes (or in an allocation of their own).
 struct RopeFreqTable {
     float base;
     uint32_t rotary;
@@ -129,6 +129,7 @@ struct itak_pool {
     itak_pool_config cfg{};
     std::vector<RopeFreqTable> rope_tables;
     double *rope_dev = nullptr;      // room for rope_tables_max tables of head_dim / 2
+    bool rope_apart = false;         // in an allocation of their own
     uint32_t rope_tables_max = 0;
     // Global layers and windowed layers are two groups of planes with their own row capacity:
     // `g` (capacity_rows per plane) and `gw` (the longest ring per plane). Within a group the
@@ -1341,20 +1342,24 @@ itak_status itak_pool_create(const itak_pool_config *config, itak_pool **out) {
     pool->bytes = bytes;
     // Rotation frequencies: 64 tables (bases and rotated widths) at the head dims that can attend.
     pool->rope_tables_max = uint32_t(std::clamp<uint64_t>(16384 / config->head_dim, 4, 64));
+    const uint64_t tables = pool->rope_tables_max * (config->head_dim / 2) * sizeof(double);
     uint64_t planes = 0, all = 0;
     if (__builtin_add_overflow(bytes, uint64_t(255), &planes) ||
-        __builtin_add_overflow(planes &= ~uint64_t(255),
-                               pool->rope_tables_max * (config->head_dim / 2) * sizeof(double), &all)) {
+        __builtin_add_overflow(planes &= ~uint64_t(255), tables, &all)) {
         delete pool;
         return size_overflow(e, "global layer storage");
     }
-    he = hipMalloc(reinterpret_cast<void **>(&pool->base), all);
+    // They lie behind the planes, unless that takes the planes over the 64 MB up to which the runtime keeps
+    // freed memory: 8 layers x 4 KV heads x 4,096 positions, exactly 64 MB, made and freed in 19 + 37 us, with the
+    // tables behind them 41 + 270, beside them 20 + 41.
+    constexpr uint64_t kKeptByRuntime = 64ull << 20;
+    pool->rope_apart = planes <= kKeptByRuntime && all > kKeptByRuntime;
+    he = hipMalloc(reinterpret_cast<void **>(&pool->base), pool->rope_apart ? bytes : all);
     if (he != hipSuccess) {
         delete pool;
         return hip_error(e, he, "allocate KV pool");
     }
     pool->base_w = pool->base + bytes_g;
-    pool->rope_dev = reinterpret_cast<double *>(pool->base + planes);
     // Fresh storage is all zero bytes, as the reference's ring storage is
     // (cache.rs:139) and as the scrub guarantee needs.
     he = hipMemset(pool->base, 0, bytes);
@@ -1387,6 +1392,12 @@ itak_status itak_pool_create(const itak_pool_config *config, itak_pool **out) {
         delete pool;
         return hip_error(e, he, "look up the static split workspace");
     }
+    pool->rope_dev = reinterpret_cast<double *>(pool->base + planes);
+    if (pool->rope_apart && hipMalloc(reinterpret_cast<void **>(&pool->rope_dev), tables) != hipSuccess) {
+        (void)hipGetLastError();
+        pool->rope_dev = nullptr;
+        pool->rope_tables_max = 0;  // (the preparation kernel then takes the powers itself)
+    }
     ITAK_DIAG("kv pool built layers=%u kv_heads=%llu head_dim=%llu elem=%s slots=%u capacity_rows=%llu "
               "device_bytes=%llu",
               config->layer_count, ULL(config->num_kv_heads), ULL(config->head_dim),
@@ -1400,6 +1411,7 @@ void itak_pool_destroy(itak_pool *pool) {
     if (!pool) return;
     (void)hipStreamSynchronize(pool->stream);
     if (pool->base) (void)hipFree(pool->base);
+    if (pool->rope_apart && pool->rope_dev) (void)hipFree(pool->rope_dev);
     if (pool->stage) (void)hipFree(pool->stage);
     if (pool->ws) (void)hipFree(pool->ws);
     if (pool->prep) (void)hipFree(pool->prep);

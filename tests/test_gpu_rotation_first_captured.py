@@ -70,3 +70,29 @@ def test_a_first_rotation_inside_a_capture_equals_an_eager_one(elem, d, rows, ro
     assert result() == want
     pool.close()
     eager_pool.close()
+
+
+def test_frequencies_beside_a_pool_of_64_megabytes():
+    # 128 rings of 128 rows are 64 MB exactly, and the frequencies lie in an allocation of their own; with a layer
+    # less or more they lie behind the planes. What is stored and returned is the same.
+    P = pkg()
+    rng = np.random.default_rng(64)
+    q_heads, kv_heads, d, rows, held = 8, 4, 128, 40, 1_000_000
+    q, k, v = (torch.from_numpy(normal(rng, rows, h * d)).cuda() for h in (q_heads, kv_heads, kv_heads))
+    k0, v0 = normal(rng, 64, kv_heads * d), normal(rng, 64, kv_heads * d)
+    got = []
+    for layers in (127, 128, 129):
+        pool = P.KvPool([P.LayerKind.windowed(64)] * layers, kv_heads, d, elem="f32", ring_headroom=64)
+        pool.set_stream(torch.cuda.current_stream().cuda_stream)
+        cache, out = pool.acquire(), torch.empty_like(q)
+        for layer in (0, layers - 1):
+            cache.restore_bulk(layer, held - 64, k0, v0)
+            for base in (1e6, 1e4):  # two tables
+                pool.attention_prep_step_device(layer, [(cache, rows)], q.data_ptr(), k.data_ptr(), v.data_ptr(),
+                                                out.data_ptr(), q_heads, rope_base=base)
+                torch.cuda.synchronize()
+                got.append((layers, layer > 0, base, out.cpu().numpy().tobytes(),
+                            [np.asarray(x).tobytes() for x in cache.view(layer).rows()[1:]]))
+        pool.close()
+    assert all(a[1:] == b[1:] for a, b in zip(got[:4], got[4:8]))
+    assert all(a[1:] == b[1:] for a, b in zip(got[:4], got[8:]))
