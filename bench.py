@@ -925,8 +925,7 @@ def run_workload(args, pkg, torch, np, dev, stream, timed):
         value = flops_layer * layers / step_s / 1e12
         roofline = {
             "bound": "mfma",
-            "kernel": "attn_prefill_f16_kernel (one tile per wavefront, appends the chunk's rows) + "
-                      "attn_combine128_wave_kernel",
+            "kernel": "attn_tiles_f16_kernel (appends the chunk's rows) + attn_combine128_wave_kernel",
             "achieved": round(value, 2),
             "peak": MFMA_F16_PEAK_TFLOPS,
             "unit": "TFLOP/s",
@@ -935,7 +934,7 @@ def run_workload(args, pkg, torch, np, dev, stream, timed):
             "us_per_launch": round(step_s / layers * 1e6, 2),
             "flops_per_launch": flops_layer,
             "timed": "one layer of the timed step (HIP graph replay of all layers): append + "
-                     "attention in the block kernel's launch, then the merge launch",
+                     "attention in one launch, then the merge launch",
             "attention_only_us_per_launch": round(attn_s * 1e6, 2),
         }
     elif wl.startswith("prefill"):

@@ -154,6 +154,7 @@ uint32_t attn_prefill_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t group, 
         }
     }
     const uint32_t rows_per_group = b.tiles * kWaves * 16 / gp;
+    b.plan_cost = least;
     b.fold_units = 0;
     uint32_t block0 = 0, ws0 = 0;
     for (uint32_t i = 0; i < b.n; ++i) {

@@ -77,13 +77,6 @@ __device__ __forceinline__ float column_max4(float v) {
     const auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(c[0]), __uint_as_float(c[1]));
 }
-// The largest of three, none of them a signalling NaN (scores and -inf): one instruction, no
-// quieting of the inputs.
-__device__ __forceinline__ float max3(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
 
 // The direct-to-LDS load is issued from inline assembly: the compiler then neither tracks it
 // (it would make every LDS read wait for all of them) nor needs to, because the only consumer

@@ -303,6 +303,10 @@ struct AttnBatch {
     uint32_t half_blocks; // host side only: the rows kernel's wavefronts take half a block each
     uint32_t tiled; // host side only: the split-K plan gives every 16 query vectors their own workgroups
     uint32_t whole_on_eight; // host side only: the split-K plan leaves every item whole on eight wavefronts
+    uint32_t tile_sets;  // host side only: the tiles kernel's plan, sets of 16 query vectors a tile
+    uint32_t tile_waves; // and wavefronts a workgroup
+    uint32_t tile_exact; // and whether the softmax keeps the exact running maximum
+    float plan_cost;     // host side only: what the block kernel's planner expects of its plan, us without the launch
     uint64_t partial_limit;  // host side only: bytes of partials the block kernel's plan may take (0 = any)
     AttnItem item[kMaxBatchItems];
 };
@@ -541,6 +545,25 @@ hipError_t launch_attn_prefill_f16_qlo(const AttnParams &p, const AttnBatch &b, 
                                        hipStream_t stream);
 hipError_t launch_attn_prefill_f16_dims(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                         bool one, hipStream_t stream);
+// Tiles of 16 or 32 query vectors whose wavefronts split the keys (attn_tiles_f16.hip): blocks of some
+// rows on the same pools at head_dim 128, new rows brought along or appended before. The batch's plan
+// says which form; `gate` multiplies the rows of items with one split.
+struct TilesPlan {
+    uint32_t sets = 0;   // of 16 query vectors a tile; 0 = the launch is another kernel's
+    uint32_t waves = 0;
+    uint32_t run = 0;    // blocks a split walks at most
+    bool appends = false; // the launch brings the step's rows along
+    bool exact = false;   // the softmax keeps the exact running maximum
+};
+bool attn_tiles_f16_supports(const PoolGeom &g, uint32_t group, uint32_t most_rows);
+// The cheapest form for a batch (slot, rows, pos0, kv_len, kv_lo set) and its cost in us. `brings_rows`: the
+// step's rows are not in the cache yet (appended by the launch where the form can, else before it); `few_rows`: a
+// step the split-K kernel takes as well.
+float attn_tiles_f16_choose(const PoolGeom &g, const AttnBatch &b, uint32_t q_heads, uint32_t window, bool brings_rows,
+                            bool few_rows, uint64_t partial_limit, TilesPlan &plan);
+uint32_t attn_tiles_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, const TilesPlan &plan);
+hipError_t launch_attn_tiles_f16(const AttnParams &p, const AttnBatch &b, uint32_t total_partials, const float *gate,
+                                 hipStream_t stream);
 // Merge of split partials; total_rows = query rows of the batch. With `gate` the merged rows
 // are multiplied by sigmoid(gate) as they are written (items with one split are not touched:
 // their writer was the attention kernel).

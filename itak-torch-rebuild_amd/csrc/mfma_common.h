@@ -19,6 +19,14 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// The largest of three, none of them a signalling NaN (scores and -inf): one instruction, no
+// quieting of the inputs.
+__device__ __forceinline__ float max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 // A mask over the eight halves of an operand register group (a lane's eight keys of a value
 // piece) that keeps the first n. Element-wise conditional stores into such a vector compile to
 // a permute and a shift per half under execution masks, hundreds of instructions on a path that

@@ -730,27 +730,113 @@ bool takes_splitk_any(const itak_pool *pool, const PlanInput *in, uint32_t n, ui
            attn_splitk_any_supports(pool->g, group, max_rows);
 }
 
+// Clears a batch's plan and names its items' places; q rows counted from q_row0. Returns their rows.
+uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t q_row0) {
+    b.n = count;  // (cleared item by item: all 64 are three kilobytes)
+    b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.tiled = b.on_eight = b.half_blocks = 0;
+    b.two_halves = b.tile_sets = b.tile_waves = b.tile_exact = 0;
+    b.plan_cost = 0.0f;
+    b.partial_limit = 0;
+    uint32_t rows = 0;
+    for (uint32_t i = 0; i < count; ++i) {
+        AttnItem &it = b.item[i];
+        it = AttnItem{};
+        it.slot = in[i].slot;
+        it.rows = in[i].rows;
+        it.pos0 = in[i].pos0;
+        it.q_row0 = q_row0 + rows;
+        it.kv_len = in[i].kv_len;
+        it.kv_lo = in[i].kv_lo;
+        rows += in[i].rows;
+    }
+    return rows;
+}
+
+// Steps on f16 pools at head_dim 128 that the tiles kernel (attn_tiles_f16.hip) takes from the split-K kernel
+// and the block kernel, and in which form.
+//
+// Against the block kernel the two planners' costs decide; `kBlockLaunch` and `kBlockAppends` put that
+// kernel's walk and merge on the tiles' scale (medians over the shapes the tiles' figures were fitted on). The pick is
+// 1.4 % behind the better of the two kernels there and in two of 549 shapes slower than the block
+// kernel by more than 2 %. 32 Q / 4 KV heads, us a layer, block kernel -> tiles: 61 rows on 0 / 300 / 1,000 12.4 / 17.9 /
+// 19.1 -> 7.5 / 8.9 / 12.3, on a window of 2,048 18.8 -> 15.9; 24 rows on 4,099 18.4 -> 14.1; 128 rows on 1,000
+// 24.5 -> 13.8; 512 rows on 0 20.1 -> 17.1. The block kernel keeps many rows on long contexts (192 rows on 12,000:
+// 62.5 against 73.3).
+//
+// Against the split-K kernel, whose 16-vector steps are the better ones throughout (the rows come in through
+// LDS, the loads stream): steps of more vectors while the keys are at most one and a half blocks per compute
+// unit and the launch is its longest chain (7 rows at 300 9.7 -> 8.3, at 1,000 9.6 -> 8.6, 8 slots at 300 10.4 -> 9.7;
+// 160 shapes there 9 % faster on average, 7 % slower at worst). Beyond, each tile's pass over the keys shows
+// (keys that are not in the last-level cache: 4 slots of four rows at 8,192 20.4 against 21.7).
+TilesPlan choose_tiles(const itak_pool *pool, uint64_t layer, const PlanInput *in, uint32_t n, uint64_t q_heads,
+                       bool prepares, bool brings_rows, bool no_alloc) {
+    TilesPlan plan;
+    const uint32_t group = uint32_t(q_heads / pool->g.kv_heads);
+    uint32_t max_rows = 0;
+    uint64_t blocks = 0;
+    for (uint32_t i = 0; i < n; ++i) {
+        max_rows = std::max(max_rows, in[i].rows);
+        blocks += uint64_t(pool->g.kv_heads) * ((in[i].kv_len + 31) / 32 - in[i].kv_lo / 32);
+    }
+    if (!pool->elem_f16 || pool->q_two_halves || n == 0 || n > uint32_t(kMaxBatchItems) ||
+        !attn_tiles_f16_supports(pool->g, group, max_rows))
+        return plan;
+    const bool splitk = takes_splitk_f16(pool, in, n, q_heads, nullptr);
+    if (splitk && (prepares || pool->merge_in_launch || pool->die_merge || max_rows * group <= 16 ||
+                   2 * blocks > 3 * uint64_t(compute_units())))
+        return plan;
+    const PoolGeom &geom = geom_of(pool, layer);
+    const uint32_t window = uint32_t(std::min<uint64_t>(pool->layers[layer].window, 0xffffffffu));
+    const uint64_t limit = no_alloc ? kScratchBytes - kScratchExchangeBytes : 0;
+    AttnBatch b;
+    start_batch(b, in, n, 0);
+    TilesPlan form;
+    const float cost = attn_tiles_f16_choose(geom, b, uint32_t(q_heads), window, brings_rows, splitk, limit, form);
+    if (form.sets == 0) return plan;
+    uint64_t partials = 0;
+    if (splitk) {
+        if (no_alloc) partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads), false, true);
+    } else {
+        constexpr float kBlockLaunch = 6.8f, kBlockAppends = 6.4f;
+        uint32_t most_blocks = 0;
+        for (uint32_t i = 0; i < n; ++i) most_blocks = std::max(most_blocks, item_block_count(b.item[i]));
+        const bool appends = brings_rows && attn_prefill_f16_appends(pool->g, group, max_rows, most_blocks);
+        partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, appends);
+        if (cost >= b.plan_cost + kBlockLaunch + (brings_rows && !appends ? kBlockAppends : 0.0f)) return plan;
+    }
+    // (The allocation-free call refuses what it refused: a step whose partials outgrow its workspace.)
+    if (limit && partials * (pool->g.head_dim + 2) * sizeof(float) > limit) return plan;
+    return form;
+}
+
 // k_new / v_new non-null = the rows are not in the cache yet and the kernel appends them
 // (only valid when takes_splitk_f16 holds).
 itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, uint32_t n,
                           const float *q_dev, float *out_dev, const uint32_t *q_pos_dev,
                           uint64_t q_heads, float scale, float softcap,
                           const float *k_new = nullptr, const float *v_new = nullptr,
-                          const FoldedParams *folded = nullptr, WorkspaceNeed *need_only = nullptr) {
+                          const FoldedParams *folded = nullptr, WorkspaceNeed *need_only = nullptr,
+                          const TilesPlan *chosen = nullptr) {
     const uint32_t group = uint32_t(q_heads / pool->g.kv_heads);
     uint32_t max_rows = 0;
     for (uint32_t i = 0; i < n; ++i) max_rows = std::max(max_rows, in[i].rows);
-    const bool mfma = takes_splitk_f16(pool, in, n, q_heads, q_pos_dev);
+    // (A step has asked already, since who appends hangs on it.)
+    const TilesPlan form = chosen ? *chosen
+                           : q_pos_dev ? TilesPlan{}
+                                       : choose_tiles(pool, layer, in, n, q_heads, folded && folded->prep_on, false,
+                                                      need_only || pool->no_alloc_call);
+    const bool tiles = form.sets != 0;
+    const bool mfma = !tiles && takes_splitk_f16(pool, in, n, q_heads, q_pos_dev);
     // Blocks of many rows (prefill chunks) on the same pools take the MFMA prefill kernel.
     const bool any = takes_splitk_any(pool, in, n, q_heads, q_dev, out_dev, q_pos_dev);
-    const bool prefill = !mfma && !any && pool->elem_f16 && q_pos_dev == nullptr &&
+    const bool prefill = !tiles && !mfma && !any && pool->elem_f16 && q_pos_dev == nullptr &&
                          attn_prefill_f16_supports(pool->g, group);
     // Decode steps and short blocks on f32 pools of head_dim 128: the f32 MFMA split-K kernel.
     const bool f32fast = !pool->elem_f16 && q_pos_dev == nullptr &&
                          attn_splitk_f32_supports(pool->g, group, max_rows);
     const uint32_t rpb =
-        (mfma || prefill || f32fast || any) ? 0 : attn_generic_rows_per_block(group, pool->g.head_dim);
-    if (!mfma && !prefill && !f32fast && !any && rpb == 0)
+        (tiles || mfma || prefill || f32fast || any) ? 0 : attn_generic_rows_per_block(group, pool->g.head_dim);
+    if (!tiles && !mfma && !prefill && !f32fast && !any && rpb == 0)
         return unsupported(pool->err, "head_dim above 256 or GQA group too wide");
     const uint32_t tile = attn_generic_tile(pool->g.head_dim);
     constexpr uint64_t kTargetBlocks = 1024;  // about four workgroups per CU
@@ -761,29 +847,17 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     uint32_t q_row0 = 0;
     for (uint32_t first = 0; first < n; first += kMaxBatchItems) {
         const uint32_t count = std::min<uint32_t>(kMaxBatchItems, n - first);
-        AttnBatch b;  // (cleared item by item: all 64 are three kilobytes)
-        b.n = count;
-        b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.tiled = b.on_eight = b.half_blocks = 0;
+        AttnBatch b;
+        const uint32_t total_rows = start_batch(b, in + first, count, q_row0);
+        q_row0 += total_rows;
         b.two_halves = prefill && pool->q_two_halves && pool->g.head_dim == 128 ? 1 : 0;
         // (At head_dim 128 a step whose best plan outgrows the static workspace is refused; at the others it
         // takes the best that fits.)
         b.partial_limit = (need_only || pool->no_alloc_call) && pool->g.head_dim != 128 ? kScratchBytes - kScratchExchangeBytes : 0;
-        uint32_t total_rows = 0;
-        for (uint32_t i = 0; i < count; ++i) {
-            const PlanInput &pi = in[first + i];
-            AttnItem &it = b.item[i];
-            it = AttnItem{};
-            it.slot = pi.slot;
-            it.rows = pi.rows;
-            it.pos0 = pi.pos0;
-            it.q_row0 = q_row0;
-            it.kv_len = pi.kv_len;
-            it.kv_lo = pi.kv_lo;
-            q_row0 += pi.rows;
-            total_rows += pi.rows;
-        }
         uint32_t partials = 0;
-        if (mfma) {
+        if (tiles) {
+            partials = attn_tiles_f16_plan(geom, b, uint32_t(q_heads), form);
+        } else if (mfma) {
             partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads), folded && folded->prep_on,
                                             !pool->q_two_halves && !pool->merge_in_launch);
         } else if (prefill) {
@@ -856,8 +930,10 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             ws = reinterpret_cast<float *>(exchange_words ? pool->scratch_dev
                                                           : pool->scratch_dev + kScratchExchangeBytes);
         } else {
-            itak_status st = exchange_words ? ensure_exchange(pool, exchange_words)
-                                            : ensure_workspace(pool, partial_floats);
+            // (A chunk's windowed and global layers are split differently; the first one's partials leave
+            // room for the others': growing costs a wait and an allocation, 600 us in the middle of a forward.)
+            const uint64_t floats = tiles && !form.exact && partials ? std::max<uint64_t>(partial_floats, 1u << 21) : partial_floats;
+            itak_status st = exchange_words ? ensure_exchange(pool, exchange_words) : ensure_workspace(pool, floats);
             if (st != ITAK_OK) return st;
             ws = exchange_words ? reinterpret_cast<float *>(pool->xws) : pool->ws;
         }
@@ -874,8 +950,8 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
                       "fused_append=%d merge=%s",
                       ULL(layer), count, total_rows, ULL(q_heads), ULL(pool->g.kv_heads), ULL(view_len),
                       window, double(scale), double(softcap),
-                      mfma ? "splitk_f16" : prefill ? "prefill_f16" : f32fast ? "splitk_f32" : any ? "splitk_any" : "generic",
-                      bl.total_blocks, splits, int(k_new != nullptr && (mfma || f32fast || any || prefill)),
+                      tiles ? "tiles_f16" : mfma ? "splitk_f16" : prefill ? "prefill_f16" : f32fast ? "splitk_f32" : any ? "splitk_any" : "generic",
+                      bl.total_blocks, splits, int(k_new != nullptr && (tiles || mfma || f32fast || any || prefill)),
                       partials == 0 ? "none" : on_die ? "on_die" : exchange_words ? "in_launch" : "launch");
         }
         AttnParams p{};
@@ -897,8 +973,8 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             p.kv_streams = layer_bytes * pool->layers.size() > (uint64_t(512) << 20) ? 1 : 0;  // twice the cache: well clear of it
         }
         p.spin_limit = pool->spin_limit;
-        p.k_new = (mfma || f32fast || any || prefill) ? k_new : nullptr;  // the caller passes them only to
-        p.v_new = (mfma || f32fast || any || prefill) ? v_new : nullptr;  // launches that append themselves
+        p.k_new = (tiles || mfma || f32fast || any || prefill) ? k_new : nullptr;  // the caller passes them only to
+        p.v_new = (tiles || mfma || f32fast || any || prefill) ? v_new : nullptr;  // launches that append themselves
         p.q_heads = uint32_t(q_heads);
         p.group = group;
         p.group_magic = (65536u + group - 1) / group;
@@ -909,7 +985,7 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         // variants can; otherwise a launch of its own over the chunk's rows.
         bool merged_only = mfma || prefill;
         for (uint32_t i = 0; i < count; ++i) merged_only = merged_only && bl.item[i].splits > 1;
-        const bool gate_folded = gate && (prepares || (mfma && merged_only));
+        const bool gate_folded = gate && (prepares || tiles || (mfma && merged_only));
         if (on_die) {
             dm.tickets = pool->die_words;
             dm.faults = pool->die_words + kDieTicketBytes / sizeof(uint32_t);
@@ -923,6 +999,8 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
                     launch_attn_splitk_f16(p, b, partials, max_rows, pool->stream,
                                            prepares ? folded : nullptr, pool->q_two_halves),
                     "launch split-K attention");
+        } else if (tiles) {
+            HIP_TRY(pool, launch_attn_tiles_f16(p, b, partials, gate, pool->stream), "launch tiles of attention");
         } else if (prefill) {
             HIP_TRY(pool, launch_attn_prefill_f16(p, b, partials, pool->stream),
                     "launch block attention");
@@ -937,7 +1015,7 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
                     "launch attention");
         }
         if (!exchange_words && !on_die)
-            HIP_TRY(pool, launch_attn_combine(p, b, partials, total_rows, (mfma || prefill || f32fast || any) ? 1 : 0,
+            HIP_TRY(pool, launch_attn_combine(p, b, partials, total_rows, (tiles || mfma || prefill || f32fast || any) ? 1 : 0,
                                               pool->stream, gate_folded ? gate : nullptr),
                     "launch split merge");
         if (gate && !gate_folded) {
@@ -2628,13 +2706,15 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
     const bool splitk = takes_splitk_f16(pool, active.data(), uint32_t(active.size()), num_q_heads, nullptr);
     const bool any = !active.empty() &&
                      takes_splitk_any(pool, active.data(), uint32_t(active.size()), num_q_heads, q_dev, out_dev, nullptr);
+    const TilesPlan tiles = choose_tiles(pool, layer, active.data(), uint32_t(active.size()), num_q_heads,
+                                         folded && folded->prep_on, true, no_alloc);
     // (With the queries as two halves the block kernel runs its two-tile form, which brings no
     // rows along: the append is a launch of its own.)
     const bool block_fuses =
         !splitk && !any && pool->elem_f16 && !active.empty() && !(pool->q_two_halves && pool->g.head_dim == 128) &&
         attn_prefill_f16_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows, most_blocks);
     const bool fuse =
-        splitk || block_fuses ||
+        tiles.sets ? tiles.appends : splitk || block_fuses ||
         (!pool->elem_f16 && !active.empty() &&
          attn_splitk_f32_supports(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows)) ||
         (any && aligned16(k_dev) && aligned16(v_dev) &&
@@ -2650,7 +2730,7 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
         WorkspaceNeed need;
         itak_status st = run_attention(pool, layer, active.data(), uint32_t(active.size()), q_dev, out_dev,
                                        nullptr, num_q_heads, scale, softcap, nullptr, nullptr, folded,
-                                       &need);
+                                       &need, &tiles);
         if (st != ITAK_OK) return st;
         const uint64_t partial_bytes = need.partial_floats * sizeof(float);
         const uint64_t exchange_bytes = need.exchange_words * 8;
@@ -2675,12 +2755,12 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
         for (uint32_t i = 0; i < item_count; ++i)
             advance(pool->slots[items[i].slot], layer, items[i].rows);
         return run_attention(pool, layer, active.data(), uint32_t(active.size()), q_dev, out_dev,
-                             nullptr, num_q_heads, scale, softcap, k_dev, v_dev, folded);
+                             nullptr, num_q_heads, scale, softcap, k_dev, v_dev, folded, nullptr, &tiles);
     }
     itak_status st = run_append(pool, layer, items, item_count, k_dev, v_dev);
     if (st != ITAK_OK) return st;
     return run_attention(pool, layer, active.data(), uint32_t(active.size()), q_dev, out_dev,
-                         nullptr, num_q_heads, scale, softcap, nullptr, nullptr, folded);
+                         nullptr, num_q_heads, scale, softcap, nullptr, nullptr, folded, nullptr, &tiles);
 }
 
 // Validates one batched step and returns the per-item plan (positions before the append).
