@@ -4,7 +4,13 @@
 // (8 to 10 GB/s on this host, less where the destination's pages are touched for the first time),
 // and the link carries 55 GB/s. Here up to eight host threads fill or empty the slots while the
 // copy engine works on others, in the order of the stream. 4 MiB a slot: a copy command costs
-// microseconds and 4 MiB take 75 on the link; eight slots keep eight threads busy.
+// ten microseconds and 4 MiB take 75 on the link; eight slots keep eight threads busy. A thread takes a few
+// hundred microseconds over 4 MiB, though, so an upload begins and a download ends with smaller chunks.
+//
+// Rows that are f32 outside and f16 values inside cross the link as halves: the host threads widen them
+// as they empty a slot (f16 to f32 is exact), or narrow them as they fill one where every value of the chunk
+// is an f16's, and the device narrows or widens on its side. The link then carries half the bytes, and
+// what the threads read and write is a quarter less.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -37,10 +43,19 @@ struct RingSpan {
 hipError_t ring_upload(HostRing &ring, const std::vector<RingSpan> &spans, hipStream_t stream,
                        const std::function<hipError_t(uint64_t)> &after = nullptr);
 
+// f32 values at `src` to device memory, as halves at halves + at / 2 (16-byte aligned) while every value is an
+// f16's, else as they are at floats + at: `after(n, from, to)` is called like ring_upload's, with the bytes [from, to)
+// (of the f32 values) that have arrived as halves since the last call, all others among them as floats.
+hipError_t ring_upload_narrow(HostRing &ring, const void *src, uint64_t bytes, void *floats, void *halves, hipStream_t stream,
+                              const std::function<hipError_t(uint64_t, uint64_t, uint64_t)> &after);
+// Whether this host converts halves in its vector units (both calls that do need it).
+bool host_has_f16();
+
 // `bytes` bytes to host memory at `out`, chunk by chunk: `source(at, n, &p)` enqueues whatever
 // makes bytes [at, at + n) on the stream and says where they lie in device memory; `at` goes up in
-// steps of kRingChunk. Returns when the bytes are in place.
-hipError_t ring_download(HostRing &ring, void *out, uint64_t bytes, hipStream_t stream,
+// steps of at most kRingChunk, and no step crosses a multiple of it. `widen`: the device holds halves, and f32
+// values are wanted (`at`, `n` and `bytes` count those). Returns when the bytes are in place.
+hipError_t ring_download(HostRing &ring, void *out, uint64_t bytes, hipStream_t stream, bool widen,
                          const std::function<hipError_t(uint64_t, uint64_t, const void **)> &source);
 
 }  // namespace itak

@@ -9,6 +9,10 @@
 
 #include "itkv.h"
 
+#if !defined(__HIP_DEVICE_COMPILE__)
+#include <immintrin.h>
+#endif
+
 namespace itak {
 
 hipError_t HostRing::open(uint64_t slots) {
@@ -35,11 +39,73 @@ void HostRing::close() {
 
 namespace {
 
+// n bytes of f32 values from n / 2 bytes of halves, and back: false where some value is no f16's (a NaN
+// counts as none: its payload would have to survive two conversions on either side).
+#if !defined(__HIP_DEVICE_COMPILE__)
+// (Streaming stores are no faster here: the pages are fresh, and the kernel has just cleared them.)
+__attribute__((target("avx,f16c"))) void widen_halves(unsigned char *out, const unsigned char *in, uint64_t n) {
+    uint64_t at = 0;
+    for (; at + 32 <= n; at += 32)
+        _mm256_storeu_ps(reinterpret_cast<float *>(out + at),
+                         _mm256_cvtph_ps(_mm_loadu_si128(reinterpret_cast<const __m128i *>(in + at / 2))));
+    for (; at < n; at += 4) {
+        uint16_t h;
+        memcpy(&h, in + at / 2, 2);
+        const float f = _mm_cvtss_f32(_mm_cvtph_ps(_mm_cvtsi32_si128(h)));
+        memcpy(out + at, &f, 4);
+    }
+}
+__attribute__((target("avx,f16c"))) bool narrow_floats(unsigned char *out, const unsigned char *in, uint64_t n) {
+    __m256 differ = _mm256_setzero_ps();
+    uint64_t at = 0;
+    for (; at + 32 <= n; at += 32) {
+        const __m256 f = _mm256_loadu_ps(reinterpret_cast<const float *>(in + at));
+        const __m128i h = _mm256_cvtps_ph(f, _MM_FROUND_TO_NEAREST_INT);
+        _mm_storeu_si128(reinterpret_cast<__m128i *>(out + at / 2), h);
+        // (Zero equals minus zero and an f16's sign is kept, so equal values are equal bits; unordered differs.)
+        differ = _mm256_or_ps(differ, _mm256_cmp_ps(f, _mm256_cvtph_ps(h), _CMP_NEQ_UQ));
+    }
+    bool exact = _mm256_movemask_ps(differ) == 0;
+    for (; at < n; at += 4) {
+        float f;
+        memcpy(&f, in + at, 4);
+        const uint16_t h = uint16_t(_mm_cvtsi128_si32(_mm_cvtps_ph(_mm_set_ss(f), _MM_FROUND_TO_NEAREST_INT)));
+        memcpy(out + at / 2, &h, 2);
+        const float back = _mm_cvtss_f32(_mm_cvtph_ps(_mm_cvtsi32_si128(h)));
+        exact = exact && f == back;
+    }
+    return exact;
+}
+bool has_f16c() {
+    __builtin_cpu_init();
+    return __builtin_cpu_supports("avx") && __builtin_cpu_supports("f16c");
+}
+#else
+void widen_halves(unsigned char *, const unsigned char *, uint64_t) {}
+bool narrow_floats(unsigned char *, const unsigned char *, uint64_t) { return false; }
+bool has_f16c() { return false; }
+#endif
+
+// Part of a transfer that goes through one slot: bytes [at, at + bytes) of it.
 struct Chunk {
     const unsigned char *src;
     unsigned char *dst;
     uint64_t bytes;
+    uint64_t at;
 };
+
+// A run of `bytes` bytes cut into chunks of kRingChunk, the first (`ramp_up`) or last one in four and its neighbour
+// in two. fn(at, n) for each in order.
+template <class F>
+void cut(uint64_t bytes, bool ramp_up, F fn) {
+    const uint64_t unit = kRingChunk, whole = (bytes + unit - 1) / unit;
+    for (uint64_t c = 0; c < whole; ++c) {
+        const uint64_t from_end = ramp_up ? c : whole - 1 - c;
+        const uint64_t part = unit / (from_end == 0 ? 4 : from_end == 1 ? 2 : 1);
+        const uint64_t end = std::min(bytes, (c + 1) * unit);
+        for (uint64_t at = c * unit; at < end; at += part) fn(at, std::min(part, end - at));
+    }
+}
 
 // What the threads of one transfer share. Chunk c uses slot c % kRingSlots; thread w of `workers`
 // has the chunks w, w + workers, ..
@@ -91,58 +157,124 @@ hipError_t run_transfer(Transfer &t, uint64_t chunks, Work work, Drive drive) {
     return hipError_t(t.error.load());
 }
 
-}  // namespace
-
-hipError_t ring_upload(HostRing &ring, const std::vector<RingSpan> &spans, hipStream_t stream,
-                       const std::function<hipError_t(uint64_t)> &after) {
-    std::vector<Chunk> chunks;
-    for (const RingSpan &s : spans)
-        for (uint64_t at = 0; at < s.bytes; at += kRingChunk)
-            chunks.push_back(Chunk{static_cast<const unsigned char *>(s.src) + at, static_cast<unsigned char *>(s.dst) + at,
-                                   std::min(kRingChunk, s.bytes - at)});
-    if (chunks.empty()) return hipSuccess;
-    if (hipError_t e = ring.open(chunks.size()); e != hipSuccess) return e;
+// The upload of `chunks`: fill_slot(c, slot memory) on the helpers, send(c, slot memory) on this thread, in order.
+template <class Fill, class Send>
+hipError_t run_upload(HostRing &ring, uint64_t chunks, hipStream_t stream, Fill fill_slot, Send send) {
+    if (chunks == 0) return hipSuccess;
+    if (hipError_t e = ring.open(chunks); e != hipSuccess) return e;
     Transfer t;
     auto fill = [&](uint64_t first, uint64_t step) {
-        for (uint64_t c = first; c < chunks.size(); c += step) {
+        for (uint64_t c = first; c < chunks; c += step) {
             const uint32_t slot = c % kRingSlots;
             if (c >= kRingSlots) {
                 if (!t.wait([&] { return t.enqueued.load(std::memory_order_acquire) > c - kRingSlots; })) return;
                 if (hipError_t e = hipEventSynchronize(ring.moved[slot]); e != hipSuccess) return t.fail(e);
             }
-            memcpy(ring.slot[slot], chunks[c].src, chunks[c].bytes);
+            fill_slot(c, ring.slot[slot]);
             t.host_done[slot].store(c + 1, std::memory_order_release);
         }
     };
     auto drive = [&] {
-        uint64_t sent = 0;
-        for (uint64_t c = 0; c < chunks.size(); ++c) {
+        for (uint64_t c = 0; c < chunks; ++c) {
             const uint32_t slot = c % kRingSlots;
             if (!t.wait([&] { return t.host_done[slot].load(std::memory_order_acquire) == c + 1; })) return;
-            hipError_t e = hipMemcpyAsync(chunks[c].dst, ring.slot[slot], chunks[c].bytes,
-                                          hipMemcpyHostToDevice, stream);
-            if (e == hipSuccess) e = hipEventRecord(ring.moved[slot], stream);
-            sent += chunks[c].bytes;
-            if (e == hipSuccess) t.enqueued.store(c + 1, std::memory_order_release);
-            if (e == hipSuccess && after) e = after(sent);
+            hipError_t e = send(c, ring.slot[slot], ring.moved[slot], t.enqueued);
             if (e != hipSuccess) return t.fail(e);
         }
     };
-    if (chunks.size() == 1) {  // nothing to overlap
+    if (chunks == 1) {  // nothing to overlap
         fill(0, 1);
         drive();
         return hipError_t(t.error.load());
     }
-    return run_transfer(t, chunks.size(), fill, drive);
+    return run_transfer(t, chunks, fill, drive);
 }
 
-hipError_t ring_download(HostRing &ring, void *out, uint64_t bytes, hipStream_t stream,
+}  // namespace
+
+bool host_has_f16() {
+    static const bool has = has_f16c();
+    return has;
+}
+
+hipError_t ring_upload(HostRing &ring, const std::vector<RingSpan> &spans, hipStream_t stream,
+                       const std::function<hipError_t(uint64_t)> &after) {
+    std::vector<Chunk> chunks;
+    for (size_t i = 0; i < spans.size(); ++i) {
+        const RingSpan &s = spans[i];
+        const auto add = [&](uint64_t at, uint64_t n) {
+            chunks.push_back(Chunk{static_cast<const unsigned char *>(s.src) + at, static_cast<unsigned char *>(s.dst) + at, n, at});
+        };
+        if (i == 0)
+            cut(s.bytes, true, add);
+        else
+            for (uint64_t at = 0; at < s.bytes; at += kRingChunk) add(at, std::min(kRingChunk, s.bytes - at));
+    }
+    uint64_t sent = 0;
+    return run_upload(
+        ring, chunks.size(), stream, [&](uint64_t c, unsigned char *slot) { memcpy(slot, chunks[c].src, chunks[c].bytes); },
+        [&](uint64_t c, unsigned char *slot, hipEvent_t moved, std::atomic<uint64_t> &enqueued) {
+            hipError_t e = hipMemcpyAsync(chunks[c].dst, slot, chunks[c].bytes, hipMemcpyHostToDevice, stream);
+            if (e == hipSuccess) e = hipEventRecord(moved, stream);
+            sent += chunks[c].bytes;
+            if (e == hipSuccess) enqueued.store(c + 1, std::memory_order_release);
+            return e == hipSuccess && after ? after(sent) : e;
+        });
+}
+
+hipError_t ring_upload_narrow(HostRing &ring, const void *src, uint64_t bytes, void *floats, void *halves, hipStream_t stream,
+                              const std::function<hipError_t(uint64_t, uint64_t, uint64_t)> &after) {
+    std::vector<Chunk> chunks;
+    cut(bytes, true, [&](uint64_t at, uint64_t n) {
+        chunks.push_back(Chunk{static_cast<const unsigned char *>(src) + at, static_cast<unsigned char *>(floats) + at, n, at});
+    });
+    // One chunk with a value that is no f16's says what the rest holds: they are not tried any more.
+    std::atomic<bool> worth_it{true};
+    std::vector<unsigned char> narrowed(chunks.size(), 0);
+    uint64_t from = 0, to = 0;  // arrived as halves and not reported
+    return run_upload(
+        ring, chunks.size(), stream,
+        [&](uint64_t c, unsigned char *slot) {
+            if (worth_it.load(std::memory_order_relaxed)) {
+                if (narrow_floats(slot, chunks[c].src, chunks[c].bytes)) {
+                    narrowed[c] = 1;
+                    return;
+                }
+                worth_it.store(false, std::memory_order_relaxed);
+            }
+            memcpy(slot, chunks[c].src, chunks[c].bytes);
+        },
+        [&](uint64_t c, unsigned char *slot, hipEvent_t moved, std::atomic<uint64_t> &enqueued) {
+            const Chunk &k = chunks[c];
+            void *dst = narrowed[c] ? static_cast<unsigned char *>(halves) + k.at / 2 : k.dst;
+            hipError_t e = hipMemcpyAsync(dst, slot, narrowed[c] ? k.bytes / 2 : k.bytes, hipMemcpyHostToDevice, stream);
+            if (e == hipSuccess) e = hipEventRecord(moved, stream);
+            if (e != hipSuccess) return e;
+            enqueued.store(c + 1, std::memory_order_release);
+            if (narrowed[c] && to == k.at) {
+                to = k.at + k.bytes;
+            } else if (narrowed[c]) {  // behind a chunk that came as floats: what lay before it goes first
+                if (to > from) e = after(k.at, from, to);
+                from = k.at, to = k.at + k.bytes;
+            }
+            if (e != hipSuccess) return e;
+            const uint64_t end = k.at + k.bytes;
+            if (end < bytes && end % (kRingChunk * kRingSlots) != 0) return hipSuccess;
+            e = after(end, from, to);
+            from = to = end;
+            return e;
+        });
+}
+
+hipError_t ring_download(HostRing &ring, void *out, uint64_t bytes, hipStream_t stream, bool widen,
                          const std::function<hipError_t(uint64_t, uint64_t, const void **)> &source) {
     if (bytes == 0) return hipSuccess;
-    const uint64_t chunks = (bytes + kRingChunk - 1) / kRingChunk;
+    std::vector<Chunk> list;
+    cut(bytes, false, [&](uint64_t at, uint64_t n) {
+        list.push_back(Chunk{nullptr, static_cast<unsigned char *>(out) + at, n, at});
+    });
+    const uint64_t chunks = list.size();
     if (hipError_t e = ring.open(chunks); e != hipSuccess) return e;
-    unsigned char *to = static_cast<unsigned char *>(out);
-    auto size_of = [&](uint64_t c) { return std::min(kRingChunk, bytes - c * kRingChunk); };
     Transfer t;
     auto drive = [&] {
         for (uint64_t c = 0; c < chunks; ++c) {
@@ -151,9 +283,9 @@ hipError_t ring_download(HostRing &ring, void *out, uint64_t bytes, hipStream_t 
                 !t.wait([&] { return t.host_done[slot].load(std::memory_order_acquire) == c - kRingSlots + 1; }))
                 return;
             const void *from = nullptr;
-            hipError_t e = source(c * kRingChunk, size_of(c), &from);
+            hipError_t e = source(list[c].at, list[c].bytes, &from);
             if (e == hipSuccess)
-                e = hipMemcpyAsync(ring.slot[slot], from, size_of(c), hipMemcpyDeviceToHost, stream);
+                e = hipMemcpyAsync(ring.slot[slot], from, widen ? list[c].bytes / 2 : list[c].bytes, hipMemcpyDeviceToHost, stream);
             if (e == hipSuccess) e = hipEventRecord(ring.moved[slot], stream);
             if (e != hipSuccess) return t.fail(e);
             t.enqueued.store(c + 1, std::memory_order_release);
@@ -164,7 +296,10 @@ hipError_t ring_download(HostRing &ring, void *out, uint64_t bytes, hipStream_t 
             const uint32_t slot = c % kRingSlots;
             if (!t.wait([&] { return t.enqueued.load(std::memory_order_acquire) > c; })) return;
             if (hipError_t e = hipEventSynchronize(ring.moved[slot]); e != hipSuccess) return t.fail(e);
-            memcpy(to + c * kRingChunk, ring.slot[slot], size_of(c));
+            if (widen)
+                widen_halves(list[c].dst, ring.slot[slot], list[c].bytes);
+            else
+                memcpy(list[c].dst, ring.slot[slot], list[c].bytes);
             t.host_done[slot].store(c + 1, std::memory_order_release);
         }
     };

@@ -214,6 +214,8 @@ hipError_t launch_ring_rows(void *pool_base_w, int elem_f16, const PoolGeom &gw,
                             const RingRowsBatch &b, void *saved, bool to_ring, hipStream_t stream);
 
 hipError_t launch_convert_f16(const float *src, uint16_t *dst, uint64_t count, hipStream_t stream);
+// The other way: `count` halves at src (16-byte aligned, like dst) as f32.
+hipError_t launch_widen_f16(const uint16_t *src, float *dst, uint64_t count, hipStream_t stream);
 // Host-pointer calls: `bytes` (rounded up to 16) from pinned host memory into device memory by
 // a kernel, and a word in pinned host memory set to `value` once everything before it on the
 // stream has finished.

@@ -615,6 +615,26 @@ hipError_t launch_convert_f16(const float *src, uint16_t *dst, uint64_t count, h
     return hipGetLastError();
 }
 
+// Halves that came over the host link as f32 rows again: 16 bytes in, 32 out a thread and turn; bound by HBM.
+__global__ __launch_bounds__(256) void widen_f16_to_f32(const uint16_t *__restrict__ src, float *__restrict__ dst,
+                                                        uint64_t count) {
+    typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+    typedef float float8_t __attribute__((ext_vector_type(8)));
+    const uint64_t step = uint64_t(gridDim.x) * 256, pieces = count / 8;
+    for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < pieces; i += step) {
+        const half8_t h = *reinterpret_cast<const half8_t *>(src + i * 8);
+        *reinterpret_cast<float8_t *>(dst + i * 8) = __builtin_convertvector(h, float8_t);
+    }
+    const uint64_t last = pieces * 8 + threadIdx.x;
+    if (blockIdx.x == 0 && last < count) dst[last] = float(__builtin_bit_cast(_Float16, src[last]));
+}
+hipError_t launch_widen_f16(const uint16_t *src, float *dst, uint64_t count, hipStream_t stream) {
+    if (count == 0) return hipSuccess;
+    const uint64_t blocks = std::min<uint64_t>((count / 8 + 255) / 256, 4096);
+    launch_kernel(widen_f16_to_f32, uint32_t(std::max<uint64_t>(blocks, 1)), 256, 0, stream, src, dst, count);
+    return hipGetLastError();
+}
+
 // ------------------------------------------------- host-pointer call: in and done
 // The small inputs of a host-pointer call lie packed in pinned host memory. One launch reads
 // them over the host link into device memory (a copy engine's command costs more than this

@@ -247,3 +247,54 @@ def test_f16_snapshots_stay_with_f16_pools_and_go_through_the_store(tmp_path):
         P().KvSnapshot.from_bytes(bytes(bad))
     assert e.value.variant in ("InconsistentSnapshot", "ChecksumMismatch")
     f32_pool.close(); f16_pool.close()
+
+
+# Version 1 of an f16 pool crosses the link as halves. Every half there is goes out as the f32 value it is
+# (as the small captures, whose rows the device widens, have it), the sum holds, and comes back. Sizes
+# around the chunks of the ring and the pieces that are summed at a time.
+def test_every_half_through_a_version_1_snapshot():
+    kv_heads, d, tokens = 4, 128, 256
+    pool = P().KvPool(2, kv_heads, d, elem="f16", max_slots=3, capacity_rows=tokens)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    cache, few = pool.acquire(), pool.acquire()
+    halves = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.float16)
+    k = halves.repeat(2).view(tokens, kv_heads * d).contiguous().cuda()
+    v = k.flip(0).contiguous()
+    cache.restore_snapshot_ptrs(tokens, cache.snapshot_layer_table([(0, tokens, k.data_ptr(), v.data_ptr())] * 2), src_f16=True)
+    torch.cuda.synchronize()
+    data = P().capture_bytes(cache, "m")
+    got = np.frombuffer(data[-8 - 4 * tokens * kv_heads * d * 4:-8], dtype="<u4").reshape(4, -1)
+    want = k.cpu().reshape(-1).numpy()
+    for side, rows in ((0, want), (1, v.cpu().reshape(-1).numpy())):
+        number = ~np.isnan(rows)
+        assert np.array_equal(got[side][number], rows[number].astype(np.float32).view("<u4"))
+        assert np.isnan(got[side][~number].view("<f4")).all()
+    restored = P().restore_bytes(pool, data, "m")  # (the sum, which the device took of its own f32 rows, holds)
+    for layer in range(2):
+        for a, b in zip(cache.read_raw(layer), restored.read_raw(layer)):
+            a, b = np.asarray(a).view(np.float16), np.asarray(b).view(np.float16)
+            number = ~np.isnan(a)
+            assert np.array_equal(a[number].view(np.uint16), b[number].view(np.uint16)) and np.isnan(b[~number]).all()
+    pool.close()
+
+
+@pytest.mark.parametrize("layers,tokens", [(1, 33), (2, 511), (2, 512), (2, 513), (4, 2048), (4, 2051), (5, 3333)])
+@pytest.mark.parametrize("exact", ["all", "first layer", "none"])
+def test_version_1_of_f16_pools_at_the_rings_edges(layers, tokens, exact):
+    kv_heads, d = 4, 128
+    pool, cache, ref = fill(layers, kv_heads, d, tokens, "f16", seed=tokens, capacity=tokens)
+    data = P().capture_bytes(cache, "edge")
+    assert data == okv.KvSnapshot.capture(ref, "edge").to_bytes()
+    if exact != "all":  # rows that are no halves: a snapshot of an f32 cache
+        rng = np.random.default_rng(1)
+        ref = oracle.KvCache.new([oracle.LayerKind.Global] * layers, kv_heads, d)
+        for layer in range(layers):
+            k, v = normal(rng, tokens, kv_heads * d), normal(rng, tokens, kv_heads * d)
+            if exact == "first layer" and layer == 0:
+                k, v = k.astype(np.float16).astype(np.float32), v.astype(np.float16).astype(np.float32)
+            ref.restore_bulk(layer, 0, k, v)
+        data = okv.KvSnapshot.capture(ref, "edge").to_bytes()
+        ref = okv.KvSnapshot.from_bytes(data).restore(store_f16=True)
+    again = P().restore_bytes(pool, data, "edge")
+    assert P().capture_bytes(again, "edge") == okv.KvSnapshot.capture(ref, "edge").to_bytes()
+    pool.close()
