@@ -25,6 +25,7 @@
 // crates/wgpu-compute/src/kernels/k1_q4k_gemv.rs:285-329; softcap as in attn_splitk_f16.hip.
 #include "internal.h"
 #include "mfma_common.h"
+#include "prep_fold.h"
 #include "split_exchange.h"
 #include "timeline.h"
 
@@ -75,9 +76,14 @@ __device__ __forceinline__ half8 to_half8_rne(float4 a, float4 b) {
 
 // QLO: the queries as two f16 halves, q = hi + lo, scores K.hi + K.lo (attn_splitk_f16_qlo.hip
 // says why).
-template <int N, bool RING, bool QLO = false>
-__global__ __launch_bounds__(kWaves * 64) void attn_decode_f16_kernel(AttnParams p, AttnBatchT<N> b,
-                                                                       uint32_t total_partials) {
+// PREP: Q and the new K row are normed and rotated on their way in (prep_fold.h), and the gate applied where
+// this launch writes the output. One position serves both, so the rotation is worked out once, in
+// the shadow of the loads. 32 Q / 4 KV heads, us a layer, the split-K
+// kernel's preparing form -> this one: 700 / 4,096 positions 8.8 / 9.2 -> 7.5 / 8.1, a window of 2,048 10.4 -> 9.1; 8 KV
+// heads at 2,000 9.1 -> 8.1.
+template <int N, bool RING, bool QLO, bool PREP>
+__device__ __forceinline__ void attn_decode_f16_body(const AttnParams &p, const AttnBatchT<N> &b, uint32_t total_partials,
+                                                     [[maybe_unused]] const FoldedParams &fold) {
     __shared__ float sm_m[kWaves * 16];
     __shared__ float sm_l[kWaves * 16];
     __shared__ __attribute__((aligned(16))) float sm_o[kWaves * 8 * 64 * 4];
@@ -101,6 +107,9 @@ __global__ __launch_bounds__(kWaves * 64) void attn_decode_f16_kernel(AttnParams
                      "s"(b.item[0].kv_len), "s"(b.item[0].splits), "s"(b.item[0].keys_per_split),
                      "s"(b.item[0].block0), "s"(b.item[0].ws0), "s"(b.item[0].splits_magic),
                      "s"(b.item[0].kv_lo), "s"(p.window), "s"(p.ring_blocks));
+    if (N == 1 && PREP)
+        asm volatile("" ::"s"(fold.prep_q_weight), "s"(fold.prep_k_weight), "s"(fold.prep_eps), "s"(fold.prep_rot),
+                     "s"(fold.prep_interleaved), "s"(fold.prep_freq_step), "s"(fold.prep_freq), "s"(fold.gate));
     const AttnItem item = b.item[b.find_by_block(blockIdx.x)];
     const uint32_t local = blockIdx.x - item.block0;
     // Workgroups reach the device in the order of their index and the launch ends with its
@@ -160,6 +169,22 @@ __global__ __launch_bounds__(kWaves * 64) void attn_decode_f16_kernel(AttnParams
         const float *src = (lane < 32 ? p.k_new : p.v_new) + uint64_t(item.q_row0) * row_width + kv_head * kD;
         nraw = *reinterpret_cast<const float4 *>(src + (lane & 31) * 4);
     }
+    // PREP: the norm weights and the frequencies of this lane's four channels, asked for ahead of the keys.
+    // Interleaved pairs are (2i, 2i+1); half-split pair i joins channels i and i + rot/2.
+    const uint32_t pc4 = (tid & 31u) * 4, prot = PREP ? fold.prep_rot : 0;
+    const bool pinter = PREP && fold.prep_interleaved != 0;
+    const int trig_pairs = pinter ? 2 : 4;
+    [[maybe_unused]] const uint32_t pair0 = pinter ? pc4 >> 1 : (pc4 < prot >> 1 ? pc4 : pc4 - (prot >> 1));
+    [[maybe_unused]] float4 wq = make_float4(1.f, 1.f, 1.f, 1.f), wk = wq;
+    [[maybe_unused]] double freq[4] = {0.0, 0.0, 0.0, 0.0};
+    if constexpr (PREP) {
+        if (fold.prep_q_weight) wq = *reinterpret_cast<const float4 *>(fold.prep_q_weight + pc4);
+        if (fold.prep_k_weight) wk = *reinterpret_cast<const float4 *>(fold.prep_k_weight + pc4);
+        if (prot && fold.prep_freq) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) freq[i] = fold.prep_freq[min(pair0 + i, (prot >> 1) - 1)];
+        }
+    }
     // Key rows of MFMA tile t are interleaved so that lane group g ends up holding the scores of
     // the 8 consecutive keys g*8 .. g*8+7 (the layout of internal.h).
     half8 bk[2][4], bv[8];
@@ -178,10 +203,24 @@ __global__ __launch_bounds__(kWaves * 64) void attn_decode_f16_kernel(AttnParams
     }
     ITAK_MARK(2)
 
+    [[maybe_unused]] PrepTrig trig;
+    if constexpr (PREP) {
+        if (prot) {
+            if (!fold.prep_freq)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (i < trig_pairs) freq[i] = exp2(double(pair0 + i) * fold.prep_freq_step);
+            prep_trig(trig, double(pos), freq, trig_pairs);
+        }
+    }
     // ---- Q^T as f16 through LDS while the block is in flight.
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const uint32_t f = tid + u * kWaves * 64, j = f >> 5, c4 = (f & 31) * 4;
+        if constexpr (PREP) {
+            if (u == 0 || group > 8)  // (up to eight heads a group, the second half is padding)
+                qraw[u] = prep_chunk(qraw[u], fold.prep_q_weight != nullptr, wq, fold.prep_eps, c4, lane, prot, pinter, trig);
+        }
         half4 h{static_cast<_Float16>(qraw[u].x), static_cast<_Float16>(qraw[u].y),
                 static_cast<_Float16>(qraw[u].z), static_cast<_Float16>(qraw[u].w)};
         if (j >= group) h = half4{0, 0, 0, 0};
@@ -196,6 +235,10 @@ __global__ __launch_bounds__(kWaves * 64) void attn_decode_f16_kernel(AttnParams
     uint2 packed{0u, 0u};
     if (owns_new && wave == 0) {
         const uint32_t c4 = (lane & 31) * 4;
+        if constexpr (PREP) {  // (the upper half's row is the values', which stay as they are)
+            const float4 k = prep_chunk(nraw, fold.prep_k_weight != nullptr, wk, fold.prep_eps, c4, lane, prot, pinter, trig);
+            if (lane < 32) nraw = k;
+        }
         const uint32_t h0 = f32_to_f16_bits(nraw.x), h1 = f32_to_f16_bits(nraw.y);
         const uint32_t h2 = f32_to_f16_bits(nraw.z), h3 = f32_to_f16_bits(nraw.w);
         packed = uint2{h0 | (h1 << 16), h2 | (h3 << 16)};
@@ -367,8 +410,15 @@ __global__ __launch_bounds__(kWaves * 64) void attn_decode_f16_kernel(AttnParams
             float *dst = p.out + (uint64_t(item.q_row0) * p.q_heads + kv_head * group + jl) * kD;
             const float inv = __builtin_amdgcn_rcpf(L);
 #pragma unroll
-            for (int x = 0; x < 2; ++x)
-                *reinterpret_cast<floatx4 *>(dst + (wave * 2 + x) * 16 + g * 4) = acc[x] * inv;
+            for (int x = 0; x < 2; ++x) {
+                floatx4 y = acc[x] * inv;
+                if (PREP && fold.gate) {
+                    const float4 gt = *reinterpret_cast<const float4 *>(fold.gate + (dst - p.out) + (wave * 2 + x) * 16 + g * 4);
+                    y = floatx4{y[0] * sigmoid_fast(gt.x), y[1] * sigmoid_fast(gt.y), y[2] * sigmoid_fast(gt.z),
+                                y[3] * sigmoid_fast(gt.w)};
+                }
+                *reinterpret_cast<floatx4 *>(dst + (wave * 2 + x) * 16 + g * 4) = y;
+            }
         }
         store_new_row();
         ITAK_MARK_END
@@ -406,6 +456,16 @@ __global__ __launch_bounds__(kWaves * 64) void attn_decode_f16_kernel(AttnParams
     tm_[7] = gathered_at;
 #endif
     ITAK_MARK_END
+}
+template <int N, bool RING, bool QLO = false>
+__global__ __launch_bounds__(kWaves * 64) void attn_decode_f16_kernel(AttnParams p, AttnBatchT<N> b,
+                                                                       uint32_t total_partials) {
+    attn_decode_f16_body<N, RING, QLO, false>(p, b, total_partials, FoldedParams{});
+}
+template <int N, bool RING>
+__global__ __launch_bounds__(kWaves * 64) void attn_decode_f16_prep_kernel(AttnParams p, AttnBatchT<N> b,
+                                                                            uint32_t total_partials, FoldedParams f) {
+    attn_decode_f16_body<N, RING, false, true>(p, b, total_partials, f);
 }
 
 }  // namespace
@@ -456,8 +516,20 @@ uint32_t attn_decode_f16_resident_groups() {
 }
 
 hipError_t launch_attn_decode_f16(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
-                                  hipStream_t stream, bool q_two_halves) {
+                                  hipStream_t stream, bool q_two_halves, const FoldedParams *prepares) {
     if (b.total_blocks == 0) return hipSuccess;
+    if (prepares) {
+#define ITAK_LAUNCH_DECODE_PREP()                                                                  \
+    do {                                                                                           \
+        if (p.ring_blocks)                                                                         \
+            launch_kernel(attn_decode_f16_prep_kernel<N, true>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<N>(b), total_partials, *prepares); \
+        else                                                                                       \
+            launch_kernel(attn_decode_f16_prep_kernel<N, false>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<N>(b), total_partials, *prepares); \
+    } while (0)
+        ITAK_DISPATCH_BATCH(b.n, ITAK_LAUNCH_DECODE_PREP());
+#undef ITAK_LAUNCH_DECODE_PREP
+        return hipGetLastError();
+    }
     if (q_two_halves) {
 #define ITAK_LAUNCH_DECODE_QLO()                                                                   \
     do {                                                                                           \

@@ -180,21 +180,18 @@ static uint32_t variant_capacity(const Variant &v) {
 // the context, and there is neither a partial nor a merge launch. A compute unit reads 16 KB of keys and
 // values (a block) in 0.25 us, a merge launch costs 3 us in a single-slot step; a wavefront's second block
 // costs half a microsecond. Eight wavefronts from the fifth block on. One-row steps: up to 12 blocks,
-// where the next wavefront's round begins to cost what the merge does, 18 for launches that prepare
-// their rows (their workgroups of one block each spend 2 us on that, and the whole form has fewer of
-// them), 24 from 64 workgroups on (the merge of many slots costs more). Steps of several rows, whose merge
+// where the next wavefront's round begins to cost what the merge does (launches that prepare their rows as well:
+// 1 slot at 250 / 320 / 400 split 7.4 / 7.3 / 7.3, whole 6.5 / 7.4 / 8.4), 24 from 64 workgroups on (the merge of many
+// slots costs more). Steps of several rows, whose merge
 // is larger, up to 16, 24 from 128 workgroups on (up to 8 blocks in the forms that take a unit's vectors
 // together). One layer of 32 Q / 4 KV heads, us, split -> whole: 1 slot at 200 / 300 rows
-// 7.3 / 7.4 -> 5.1 / 5.4 (7.2 -> 7.2 at 400), 16 slots at 300 / 600 11.0 / 12.7 -> 8.7 / 11.1, with
-// preparation 1 slot at 200 / 500 9.2 / 9.3 -> 6.2 / 8.6; seven rows at 150 / 350 / 500 8.6 / 8.9 / 8.9 ->
+// 7.3 / 7.4 -> 5.1 / 5.4 (7.2 -> 7.2 at 400), 16 slots at 300 / 600 11.0 / 12.7 -> 8.7 / 11.1; seven rows at 150 / 350 / 500 8.6 / 8.9 / 8.9 ->
 // 6.8 / 7.2 / 7.8, 8 slots of them at 700 13.8 -> 13.1. Checked at 4, 8 and 1 KV heads and groups of 1 to 8 with
 // every shape forced either way: within 5 % of the better but for a few just past a line (16 slots of one
 // row at 900, 8 KV heads, split 19.1, whole 16.5).
-static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows, uint32_t tiles, bool prepares,
-                            bool may_tile) {
+static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows, uint32_t tiles, bool may_tile) {
     if (rows > 1) return !may_tile ? 8 : g.kv_heads * b.n * tiles >= 128 ? 24 : 16;
-    if (g.kv_heads * b.n >= 64) return 24;
-    return prepares ? 18 : 12;
+    return g.kv_heads * b.n >= 64 ? 24 : 12;
 }
 
 // The tiled form gives every 16 query vectors of a unit (item, KV head) workgroups of their own, with one
@@ -206,10 +203,9 @@ static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows
 // 16 units and more leave those forms at most 16 splits to merge; two tiles: up to 20. One tile always
 // (one workgroup per compute unit, of eight wavefronts from 16 blocks on: twice as many, with
 // half the run, lost everywhere to the larger merge), but for one-row steps that prepare their rows: up to
-// five blocks per compute unit a wavefront has one or two, and the form with two sets of operands asks for
-// the second before the rotation waits (32 Q / 4 KV heads at 700 / 2,048 / 4,096, tiled -> not, 8.9 / 9.1 /
-// 9.7 -> 8.8 / 9.0 / 9.5; 8 KV heads 9.3 / 9.6 / 10.1 -> 9.1 / 9.4 / 9.8; at 16,384 and 8,192 12.7 and 11.6
-// against 12.9 and 11.9). 32 Q / 4 KV heads, us a layer, before -> tiled: seven
+// five blocks per compute unit their wavefronts have one block each and the one-row kernel takes them (4 slots of
+// 4 KV heads at 1,800 and 3,000, 3.6 and 5.9 blocks, tiled 10.3 and 12.0, one-row 10.3 and 12.2; 2 slots of 8 KV
+// heads at 5,000 13.5 and 13.9). 32 Q / 4 KV heads, us a layer, before -> tiled: seven
 // rows at 1,000 / 4,096 / 16,384 11.4 / 12.5 / 18.3 -> 9.0 / 9.8 / 16.9, four rows 9.5 / 9.9 / 15.5 ->
 // 8.4 / 8.8 / 13.1, 8 slots of four rows at 2,000 16.5 -> 14.6; one row at 16,384 12.3 -> 11.6.
 static bool takes_tiles(const PoolGeom &g, const AttnBatch &b, uint32_t tiles, uint64_t blocks, uint64_t cus,
@@ -237,7 +233,7 @@ uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads,
     const uint64_t cus = compute_units();
     const uint32_t tiles = (most_rows * group + 15) / 16;
     const bool may = may_tile && takes_tiles(g, b, tiles, blocks, cus, prepares && most_rows == 1);
-    const bool whole = most <= whole_limit(g, b, most_rows, tiles, prepares, may);
+    const bool whole = most <= whole_limit(g, b, most_rows, tiles, may);
     b.whole_on_eight = whole && most > 4 && (may || most_rows == 1) ? 1 : 0;
     // (A whole one-row step has no second tile and hardly a second block: the form with two sets of
     // operands, whose next block is under way before the first is multiplied, is 0.4 us faster.)
@@ -331,8 +327,8 @@ hipError_t launch_attn_splitk_f16(const AttnParams &p, const AttnBatch &b, uint3
     if (b.total_blocks == 0) return hipSuccess;
     const Variant v = pick_variant(p.g, b, p.group);
     const bool prep = folded && folded->prep_on;
-    if (!prep && v.index == 0 && attn_decode_f16_takes(p, b))
-        return launch_attn_decode_f16(p, b, total_partials, stream, q_two_halves);
+    if (v.index == 0 && (!prep || (!q_two_halves && !p.exchange)) && attn_decode_f16_takes(p, b))
+        return launch_attn_decode_f16(p, b, total_partials, stream, q_two_halves, prep ? folded : nullptr);
     if (q_two_halves) return launch_attn_splitk_f16_qlo(p, b, total_partials, stream, folded);
     if (b.tiled) {
 #define ITAK_LAUNCH_TILED(W)                                                                                       \

@@ -508,8 +508,9 @@ bool attn_decode_f16_takes(const AttnParams &p, const AttnBatch &b);
 // Workgroups of that kernel the device holds at once (the smallest figure over its
 // instantiations, asked of the runtime once).
 uint32_t attn_decode_f16_resident_groups();
+// `prepares`: Q and the new K rows are prepared by the launch (not with q_two_halves or an exchange).
 hipError_t launch_attn_decode_f16(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
-                                  hipStream_t stream, bool q_two_halves = false);
+                                  hipStream_t stream, bool q_two_halves = false, const FoldedParams *prepares = nullptr);
 // f32 MFMA split-K path: f32 pools (row-major planes), head_dim 128, rows*group <= 16, implied
 // query positions. Partials are in log2 domain (combine with base2 = 1).
 bool attn_splitk_f32_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);

@@ -274,3 +274,16 @@ def test_bad_preparation_parameters_are_refused_by_name():
         assert text in str(e.value)
     assert cache.next_position(0) == 0  # nothing was appended by a refused step
     pool.close()
+
+
+# The one-row kernel's preparing form: contexts left whole (the launch gates) and split (the merge does), the
+# new row first and last in its block, groups up to 16 and of one head, both rotations, part of a row turned,
+# a window whose ring wraps, no norm, no rotation.
+@pytest.mark.parametrize("interleaved", [True, False])
+@pytest.mark.parametrize("q_heads,kv_heads,ctx,norm,rope_base,rotary,gate,window", [
+    (32, 4, 0, True, 1e6, 0, True, None), (32, 4, 31, True, 1e4, 0, True, None), (16, 1, 96, True, 1e6, 64, True, None),
+    (8, 8, 127, False, 1e6, 0, True, None), (32, 4, 703, True, 1e6, 0, True, None), (10, 1, 800, True, 0.0, 0, True, None),
+    (8, 8, 1600, True, 1e4, 32, False, None), (32, 8, 640, False, 1e6, 0, True, None), (24, 8, 1500, True, 1e6, 0, True, 600)])
+def test_one_row_steps_prepared_in_the_launch(q_heads, kv_heads, ctx, norm, rope_base, rotary, gate, window, interleaved):
+    run_case("f16", q_heads, kv_heads, 128, ctx=ctx, rows=1, norm=norm, rope_base=rope_base, interleaved=interleaved,
+             rotary=rotary, gate=gate, seed=ctx, window=window)
