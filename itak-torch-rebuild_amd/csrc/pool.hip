@@ -864,7 +864,8 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, k_new != nullptr);
         } else if (f32fast || any) {
             partials = attn_splitk_f32_plan(geom, pool->elem_f16, b, uint32_t(q_heads),
-                                            any && max_rows * group <= 16 ? attn_splitk_any_groups_per_cu(geom) : 2);
+                                            any && max_rows * group <= 16 ? attn_splitk_any_groups_per_cu(geom) : 2,
+                                            need_only || pool->no_alloc_call ? kScratchBytes - kScratchExchangeBytes : 0);
         } else {
             b.rows_per_block = rpb;
             uint64_t key_work = 0;

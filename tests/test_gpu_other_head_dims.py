@@ -188,3 +188,43 @@ def test_rounds_of_wavefronts(elem, d, q_heads, kv_heads, ctx):
             assert np.array_equal(gk.reshape(-1), store(k[r]).reshape(-1)), (s, base, r)
             assert np.array_equal(gv.reshape(-1), store(v[r]).reshape(-1)), (s, base, r)
     pool.close()
+
+
+# Blocks of several tiles, cut by the estimates: contexts left whole that the even fill had split, fewer and
+# more splits than it, halves of blocks, eight wavefronts; contexts of one length, nearly so, and apart
+# (which keep the even fill). `most` = the splits that the launch may have.
+@pytest.mark.parametrize("elem,d,q_heads,kv_heads,rows,ctxs,most", [
+    ("f16", 192, 32, 4, 38, (198, 198, 198), 1), ("f16", 240, 8, 1, 33, (1206, 1190), 64), ("f16", 144, 8, 8, 25, (610,), 64),
+    ("f16", 80, 32, 4, 13, (911,) * 7, 1), ("f16", 48, 6, 2, 9, (333, 320), 64), ("f16", 112, 32, 4, 9, (700, 90), 64),
+    ("f32", 64, 32, 4, 12, (845, 840, 833, 845, 845, 845, 845, 831), 1), ("f32", 64, 24, 8, 3, (1500, 30), 64),
+    ("f32", 128, 32, 4, 19, (635,) * 6, 1), ("f32", 128, 8, 1, 15, (1900, 1891), 64), ("f32", 128, 32, 4, 3, (614,) * 7, 64),
+])
+def test_blocks_of_several_tiles(elem, d, q_heads, kv_heads, rows, ctxs, most, capfd):
+    P = pkg()
+    rng = np.random.default_rng(d + rows)
+    pool = P.KvPool([P.LayerKind.Global], kv_heads, d, elem=elem, max_slots=len(ctxs), capacity_rows=max(ctxs) + rows + 8)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    caches = [pool.acquire() for _ in ctxs]
+    refs = [oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, d, store_f16=elem == "f16") for _ in ctxs]
+    for cache, ref, n in zip(caches, refs, ctxs):
+        k, v = normal(rng, n, kv_heads * d), normal(rng, n, kv_heads * d)
+        cache.restore_bulk(0, 0, k, v)
+        ref.restore_bulk(0, 0, k, v)
+    total = rows * len(ctxs)
+    q, k, v = normal(rng, total, q_heads * d), normal(rng, total, kv_heads * d), normal(rng, total, kv_heads * d)
+    qd, kd, vd = dev(q), dev(k), dev(v)
+    out = torch.full_like(qd, float("nan"))
+    lib = P._native.load()
+    capfd.readouterr()
+    lib.itak_set_debug_enabled(1)
+    pool.attention_step_device(0, [(c, rows) for c in caches], qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), q_heads)
+    lib.itak_set_debug_enabled(0)
+    torch.cuda.synchronize()
+    splits = [int(w[7:]) for w in capfd.readouterr().err.split() if w.startswith("splits=")]
+    assert len(splits) == 1 and 1 <= splits[0] <= most
+    got = out.cpu().numpy()
+    for s, ref in enumerate(refs):
+        at = slice(s * rows, (s + 1) * rows)
+        want = oracle.attention_step(ref, 0, q[at], k[at], v[at], q_heads, ctxs[s], threads=8)
+        assert rel_err(got[at].reshape(-1), want) <= 1e-5, s
+    pool.close()
