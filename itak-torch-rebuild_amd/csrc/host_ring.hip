@@ -56,23 +56,26 @@ __attribute__((target("avx,f16c"))) void widen_halves(unsigned char *out, const 
     }
 }
 __attribute__((target("avx,f16c"))) bool narrow_floats(unsigned char *out, const unsigned char *in, uint64_t n) {
-    __m256 differ = _mm256_setzero_ps();
+    __m256 differ = _mm256_setzero_ps(), unordered = _mm256_setzero_ps();
     uint64_t at = 0;
     for (; at + 32 <= n; at += 32) {
         const __m256 f = _mm256_loadu_ps(reinterpret_cast<const float *>(in + at));
         const __m128i h = _mm256_cvtps_ph(f, _MM_FROUND_TO_NEAREST_INT);
         _mm_storeu_si128(reinterpret_cast<__m128i *>(out + at / 2), h);
-        // (Zero equals minus zero and an f16's sign is kept, so equal values are equal bits; unordered differs.)
-        differ = _mm256_or_ps(differ, _mm256_cmp_ps(f, _mm256_cvtph_ps(h), _CMP_NEQ_UQ));
+        // (Bits, not values: a thread that takes subnormal f32 values as zero, as torch.set_flush_denormal asks for, would
+        // find them equal to the zeros they become.)
+        differ = _mm256_or_ps(differ, _mm256_xor_ps(f, _mm256_cvtph_ps(h)));
+        unordered = _mm256_or_ps(unordered, _mm256_cmp_ps(f, f, _CMP_UNORD_Q));
     }
-    bool exact = _mm256_movemask_ps(differ) == 0;
+    const __m256i bits = _mm256_castps_si256(differ);
+    bool exact = _mm256_testz_si256(bits, bits) && _mm256_movemask_ps(unordered) == 0;
     for (; at < n; at += 4) {
         float f;
         memcpy(&f, in + at, 4);
         const uint16_t h = uint16_t(_mm_cvtsi128_si32(_mm_cvtps_ph(_mm_set_ss(f), _MM_FROUND_TO_NEAREST_INT)));
         memcpy(out + at / 2, &h, 2);
         const float back = _mm_cvtss_f32(_mm_cvtph_ps(_mm_cvtsi32_si128(h)));
-        exact = exact && f == back;
+        exact = exact && f == f && memcmp(&f, &back, 4) == 0;
     }
     return exact;
 }

@@ -298,3 +298,28 @@ def test_version_1_of_f16_pools_at_the_rings_edges(layers, tokens, exact):
     again = P().restore_bytes(pool, data, "edge")
     assert P().capture_bytes(again, "edge") == okv.KvSnapshot.capture(ref, "edge").to_bytes()
     pool.close()
+
+
+# Subnormal f32 values are no halves, also for a thread that takes them as zero: the sum is over the file's bits.
+def test_version_1_with_subnormals_loads_while_the_caller_flushes_them():
+    kv_heads, d, tokens = 4, 128, 600
+    rng = np.random.default_rng(3)
+    ref = oracle.KvCache.new([oracle.LayerKind.Global] * 2, kv_heads, d)
+    for layer in range(2):
+        k, v = (normal(rng, tokens, kv_heads * d).astype(np.float16).astype(np.float32) for _ in range(2))
+        k.view(np.uint32)[::7, ::3] = 0x80000123  # -4e-43
+        ref.restore_bulk(layer, 0, k, v)
+    data = okv.KvSnapshot.capture(ref, "m").to_bytes()
+    pool = P().KvPool(2, kv_heads, d, elem="f16", max_slots=2, capacity_rows=tokens)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    plain = P().restore_bytes(pool, data, "m")
+    flushes = torch.set_flush_denormal(True)
+    try:
+        flushed = P().restore_bytes(pool, data, "m")
+    finally:
+        torch.set_flush_denormal(False)
+    assert flushes
+    for layer in range(2):
+        for a, b in zip(plain.read_raw(layer), flushed.read_raw(layer)):
+            assert np.array_equal(np.asarray(a).view(np.uint16), np.asarray(b).view(np.uint16))
+    pool.close()
