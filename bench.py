@@ -729,7 +729,7 @@ def run_workload(args, pkg, torch, np, dev, stream, timed):
         layers, slots, rows, lengths = 16, 1, 64, [4096]
         name = ("the reference's own prefill chunk (crates/wgpu-compute/src/session.rs:186-195): 64 rows "
                 "appended and attended causally at context 4096, 30B-class heads, f16 KV, 16 layers "
-                "cycled; the block kernel splits the context, appends the rows itself and a merge "
+                "cycled; the tiles kernel splits the context, appends the rows itself and a merge "
                 "launch follows")
     elif wl == "hybrid":
         layers, slots, rows, lengths = 8, 1, 1, [32768]
@@ -911,7 +911,7 @@ def run_workload(args, pkg, torch, np, dev, stream, timed):
             "us_per_layer": round(prep_s / layers * 1e6, 3),
             "added_us_per_layer": round((prep_s - step_s) / layers * 1e6, 3),
             "launches_added_per_layer": 0 if folded else 1,
-            "what": ("RMSNorm + RoPE of Q and of the new K row inside the split-K kernel, the gate "
+            "what": ("RMSNorm + RoPE of Q and of the new K row inside the attention kernel, the gate "
                      "in the kernel that writes the output: the step's own two launches"
                      if folded else
                      "attn_prep_kernel (RMSNorm + RoPE of Q and K, one launch) before the fused "
