@@ -89,6 +89,32 @@ def test_against_the_oracle(kernels, ctxs, rows, q_heads, kv_heads, window, soft
     pool.close()
 
 
+# Rings of one and two blocks, where two position blocks of a step are the same storage block: its old rows
+# are read beside the new ones' stores, and each row is in one place only.
+@pytest.mark.parametrize("ctx,rows,window,headroom", [(20, 20, 1, 31), (7, 30, 2, 30), (300, 31, 1, 31), (20, 40, 20, 40),
+                                                      (95, 34, 30, 34), (1000, 61, 3, 61), (63, 9, 16, 40)])
+def test_rings_of_one_and_two_blocks(kernels, ctx, rows, window, headroom):
+    q_heads, kv_heads = 32, 4
+    P = pkg()
+    rng = np.random.default_rng(ctx)
+    pool = P.KvPool([P.LayerKind.windowed(window)], kv_heads, D, elem="f16", capacity_rows=ctx + 3 * rows, ring_headroom=headroom)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    cache = pool.acquire()
+    ref = oracle.KvCache.new([oracle.LayerKind.windowed(window)], kv_heads, D, store_f16=True)
+    first = max(0, ctx - window)
+    k, v = normal(rng, ctx - first, kv_heads * D), normal(rng, ctx - first, kv_heads * D)
+    cache.restore_bulk(0, first, k, v)
+    ref.restore_bulk(0, first, k, v)
+    for at in (ctx, ctx + rows, ctx + 2 * rows):
+        q, k, v = (normal(rng, rows, w * D) for w in (q_heads, kv_heads, kv_heads))
+        kernels()
+        got = step(pool, [cache], rows, q, k, v, q_heads)
+        assert kernels() == ["tiles_f16"]
+        want = oracle.attention_step(ref, 0, q, k, v, q_heads, at, threads=8)
+        assert max_abs(got.reshape(-1), np.asarray(want).reshape(-1)) <= 2e-3
+    pool.close()
+
+
 # The stored planes, raw, are what the row kernel writes: no byte beside the new rows', NaNs canonical.
 @pytest.mark.parametrize("ctx,rows,window", [(0, 61, None), (45, 61, None), (31, 9, None), (40, 61, 33), (333, 40, 64)])
 def test_new_rows_are_stored_as_the_row_kernel_stores_them(kernels, ctx, rows, window):
