@@ -801,10 +801,11 @@ TilesPlan choose_tiles(const itak_pool *pool, uint64_t layer, const PlanInput *i
         uint32_t most_blocks = 0;
         for (uint32_t i = 0; i < n; ++i) most_blocks = std::max(most_blocks, item_block_count(b.item[i]));
         const bool appends = brings_rows && attn_prefill_f16_appends(pool->g, group, max_rows, most_blocks);
-        partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, appends);
+        attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, appends);
         if (cost >= b.plan_cost + kBlockLaunch + (brings_rows && !appends ? kBlockAppends : 0.0f)) return plan;
+        if (no_alloc) partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, false);
     }
-    // (The allocation-free call refuses what it refused: a step whose partials outgrow its workspace.)
+    // (The allocation-free call refuses a step by the same plans as without the tiles, see run_attention.)
     if (limit && partials * (pool->g.head_dim + 2) * sizeof(float) > limit) return plan;
     return form;
 }
@@ -851,9 +852,11 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         const uint32_t total_rows = start_batch(b, in + first, count, q_row0);
         q_row0 += total_rows;
         b.two_halves = prefill && pool->q_two_halves && pool->g.head_dim == 128 ? 1 : 0;
-        // (At head_dim 128 a step whose best plan outgrows the static workspace is refused; at the others it
-        // takes the best that fits.)
-        b.partial_limit = (need_only || pool->no_alloc_call) && pool->g.head_dim != 128 ? kScratchBytes - kScratchExchangeBytes : 0;
+        // (At head_dim 128 a step is refused when the best plan of a launch without its rows outgrows the static
+        // workspace; a launch that brings them along is cut otherwise, up to twice the partials, and takes the
+        // best plan that fits, as every launch at the other head dims does.)
+        b.partial_limit = (need_only || pool->no_alloc_call) && (pool->g.head_dim != 128 || k_new)
+                              ? kScratchBytes - kScratchExchangeBytes : 0;
         uint32_t partials = 0;
         if (tiles) {
             partials = attn_tiles_f16_plan(geom, b, uint32_t(q_heads), form);

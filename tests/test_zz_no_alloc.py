@@ -148,6 +148,48 @@ def test_a_step_beyond_the_static_workspace_is_refused_before_anything_changes()
     pool2.close()
 
 
+# Blocks whose launch brings the rows along and would be cut into more partials (9 to 16 MB) than the launch that
+# the call measures them by: they stay accepted, and within the static array's 8 MiB. The second is the block
+# kernel's, the others are tiles.
+@pytest.mark.parametrize("slots,rows,ctx", [(3, 61, 1500), (8, 9, 3000), (2, 64, 733)])
+def test_a_launch_that_brings_rows_keeps_its_partials_within_the_static_workspace(slots, rows, ctx, capfd):
+    rng = np.random.default_rng(slots)
+    pool = P().KvPool(1, KV_HEADS, D, elem="f16", max_slots=slots, capacity_rows=ctx + rows)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    caches = [pool.acquire() for _ in range(slots)]
+    k, v = normal(rng, ctx + slots * rows, ROW), normal(rng, ctx + slots * rows, ROW)
+    kd, vd = dev(k), dev(v)
+    for cache in caches:
+        pool.append_device(0, [(cache, ctx)], kd.data_ptr(), vd.data_ptr())
+    q = normal(rng, slots * rows, Q_HEADS * D)
+    qd = dev(q)
+    out = torch.full_like(qd, float("nan"))
+    lib = P()._native.load()
+    capfd.readouterr()
+    lib.itak_set_debug_enabled(1)
+    try:
+        st = call(pool, "itak_attention_step_device_noalloc", 0, [(c, rows) for c in caches], qd, kd[ctx:], vd[ctx:], out)
+    finally:
+        lib.itak_set_debug_enabled(0)
+    assert st == 0, lib.itak_last_error(pool._h)
+    pool.synchronize()
+    splits = [int(w[7:]) for w in capfd.readouterr().err.split() if w.startswith("splits=")]
+    assert len(splits) == 1
+    assert splits[0] == 1 or slots * rows * Q_HEADS * splits[0] * (D + 2) * 4 <= 8 << 20, splits
+    got = out.cpu().numpy()
+    for s in (0, slots - 1):
+        at = slice(s * rows, (s + 1) * rows)
+        new = slice(ctx + s * rows, ctx + (s + 1) * rows)
+        ref = oracle.KvCache.new([oracle.LayerKind.Global], KV_HEADS, D, store_f16=True)
+        ref.restore_bulk(0, 0, k[:ctx], v[:ctx])
+        want = oracle.attention_step(ref, 0, q[at], k[new], v[new], Q_HEADS, ctx, threads=8)
+        assert max_abs(got[at].reshape(-1), want) <= 2e-3, s
+        _, gk, gv = caches[s].read_rows(0, ctx, rows)
+        assert np.array_equal(gk.reshape(rows, ROW), oracle.f32_to_f16_array(k[new]))
+        assert np.array_equal(gv.reshape(rows, ROW), oracle.f32_to_f16_array(v[new]))
+    pool.close()
+
+
 def captured_on_first_use(pools, contexts, rows):
     """The callers the entry point is for: its very first call on a pool is made under stream
     capture (nothing before it has sized a workspace), the graph is replayed with new inputs
