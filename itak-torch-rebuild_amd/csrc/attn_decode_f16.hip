@@ -213,13 +213,19 @@ __device__ __forceinline__ void attn_decode_f16_body(const AttnParams &p, const 
             prep_trig(trig, double(pos), freq, trig_pairs);
         }
     }
-    // ---- Q^T as f16 through LDS while the block is in flight.
+    // ---- Q^T as f16 through LDS while the block is in flight. Queries that this launch prepares carry the scale
+    // with them, as in the split-K kernel's preparing forms: without a norm weight their channels may be beyond f16's
+    // largest. Others are scaled as scores.
+    const float softcap = p.softcap;
+    const float qscale = softcap > 0.0f ? p.scale : p.scale * kLog2e;
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
         const uint32_t f = tid + u * kWaves * 64, j = f >> 5, c4 = (f & 31) * 4;
         if constexpr (PREP) {
-            if (u == 0 || group > 8)  // (up to eight heads a group, the second half is padding)
-                qraw[u] = prep_chunk(qraw[u], fold.prep_q_weight != nullptr, wq, fold.prep_eps, c4, lane, prot, pinter, trig);
+            if (u == 0 || group > 8) {  // (up to eight heads a group, the second half is padding)
+                const float4 a = prep_chunk(qraw[u], fold.prep_q_weight != nullptr, wq, fold.prep_eps, c4, lane, prot, pinter, trig);
+                qraw[u] = make_float4(a.x * qscale, a.y * qscale, a.z * qscale, a.w * qscale);
+            }
         }
         half4 h{static_cast<_Float16>(qraw[u].x), static_cast<_Float16>(qraw[u].y),
                 static_cast<_Float16>(qraw[u].z), static_cast<_Float16>(qraw[u].w)};
@@ -263,8 +269,6 @@ __device__ __forceinline__ void attn_decode_f16_body(const AttnParams &p, const 
     }
 
     // ---- S^T = K . Q^T
-    const float softcap = p.softcap;
-    const float qscale = softcap > 0.0f ? p.scale : p.scale * kLog2e;
     floatx4 s[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -287,7 +291,7 @@ __device__ __forceinline__ void attn_decode_f16_body(const AttnParams &p, const 
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) sc[t * 4 + r] = s[t][r] * qscale;
+        for (int r = 0; r < 4; ++r) sc[t * 4 + r] = PREP ? s[t][r] : s[t][r] * qscale;
     if (softcap > 0.0f) {
         const float inv_cap = 1.0f / softcap;
 #pragma unroll

@@ -287,3 +287,31 @@ def test_bad_preparation_parameters_are_refused_by_name():
 def test_one_row_steps_prepared_in_the_launch(q_heads, kv_heads, ctx, norm, rope_base, rotary, gate, window, interleaved):
     run_case("f16", q_heads, kv_heads, 128, ctx=ctx, rows=1, norm=norm, rope_base=rope_base, interleaved=interleaved,
              rotary=rotary, gate=gate, seed=ctx, window=window)
+
+
+# Queries without a norm whose channels are beyond f16's largest value: prepared steps round them with the scale on.
+# Every head has one such channel, on keys of a few 2^-14 there (whole halves), so that its scores are of order one;
+# the one-row kernel whole and split, the split-K kernel's forms of several rows.
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+@pytest.mark.parametrize("ctx,rows", [(40, 1), (100, 1), (700, 1), (60, 3), (700, 3)])
+def test_queries_beyond_half_range_without_a_norm(ctx, rows, softcap):
+    q_heads, kv_heads, d = 32, 4, 128
+    rng = np.random.default_rng(ctx + rows)
+    k, v = normal(rng, ctx + rows, kv_heads, d), normal(rng, ctx + rows, kv_heads * d)
+    k[:, :, 5] = rng.integers(-3, 4, (ctx + rows, kv_heads)) * 2.0 ** -14
+    q = normal(rng, rows, q_heads, d)
+    q[:, :, 5] = 2.0e5
+    q, k = q.reshape(rows, -1), k.reshape(ctx + rows, -1)
+    pool = P().KvPool(1, kv_heads, d, elem="f16", capacity_rows=ctx + rows)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    cache, ref = pool.acquire(), oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, d, store_f16=True)
+    qd, kd, vd = dev(q), dev(k), dev(v)
+    pool.append_device(0, [(cache, ctx)], kd.data_ptr(), vd.data_ptr())
+    ref.restore_bulk(0, 0, k[:ctx], v[:ctx])
+    out = torch.full_like(qd, float("nan"))
+    pool.attention_prep_step_device(0, [(cache, rows)], qd.data_ptr(), kd[ctx:].data_ptr(), vd[ctx:].data_ptr(),
+                                    out.data_ptr(), q_heads, softcap=softcap)
+    torch.cuda.synchronize()
+    want = oracle.attention_step(ref, 0, q, k[ctx:], v[ctx:], q_heads, ctx, oracle.AttentionParams(softcap=softcap), threads=8)
+    assert max_abs(out.cpu().numpy().reshape(-1), np.asarray(want).reshape(-1)) <= 2e-3
+    pool.close()
