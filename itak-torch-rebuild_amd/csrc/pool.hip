@@ -767,9 +767,11 @@ uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t
 // LDS, the loads stream): steps of more vectors while the keys are at most one and a half blocks per compute
 // unit and the launch is its longest chain (7 rows at 300 9.7 -> 8.3, at 1,000 9.6 -> 8.6, 8 slots at 300 10.4 -> 9.7;
 // 160 shapes there 9 % faster on average, 7 % slower at worst). Beyond, each tile's pass over the keys shows
-// (keys that are not in the last-level cache: 4 slots of four rows at 8,192 20.4 against 21.7).
+// (keys that are not in the last-level cache: 4 slots of four rows at 8,192 20.4 against 21.7). Softcaps
+// outside [2, 1024] stay there too: the tiles round the queries with 2 log2(e) / softcap on, the split-K kernel caps the
+// scores, and beyond those the factor takes queries out of f16's range, or into its subnormals, that are inside it there.
 TilesPlan choose_tiles(const itak_pool *pool, uint64_t layer, const PlanInput *in, uint32_t n, uint64_t q_heads,
-                       bool prepares, bool brings_rows, bool no_alloc) {
+                       float softcap, bool prepares, bool brings_rows, bool no_alloc) {
     TilesPlan plan;
     const uint32_t group = uint32_t(q_heads / pool->g.kv_heads);
     uint32_t max_rows = 0;
@@ -783,6 +785,7 @@ TilesPlan choose_tiles(const itak_pool *pool, uint64_t layer, const PlanInput *i
         return plan;
     const bool splitk = takes_splitk_f16(pool, in, n, q_heads, nullptr);
     if (splitk && (prepares || pool->merge_in_launch || pool->die_merge || max_rows * group <= 16 ||
+                   (softcap > 0.0f && (softcap < 2.0f || softcap > 1024.0f)) ||
                    2 * blocks > 3 * uint64_t(compute_units())))
         return plan;
     const PoolGeom &geom = geom_of(pool, layer);
@@ -824,7 +827,7 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     // (A step has asked already, since who appends hangs on it.)
     const TilesPlan form = chosen ? *chosen
                            : q_pos_dev ? TilesPlan{}
-                                       : choose_tiles(pool, layer, in, n, q_heads, folded && folded->prep_on, false,
+                                       : choose_tiles(pool, layer, in, n, q_heads, softcap, folded && folded->prep_on, false,
                                                       need_only || pool->no_alloc_call);
     const bool tiles = form.sets != 0;
     const bool mfma = !tiles && takes_splitk_f16(pool, in, n, q_heads, q_pos_dev);
@@ -2733,7 +2736,7 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
     const bool splitk = takes_splitk_f16(pool, active.data(), uint32_t(active.size()), num_q_heads, nullptr);
     const bool any = !active.empty() &&
                      takes_splitk_any(pool, active.data(), uint32_t(active.size()), num_q_heads, q_dev, out_dev, nullptr);
-    const TilesPlan tiles = choose_tiles(pool, layer, active.data(), uint32_t(active.size()), num_q_heads,
+    const TilesPlan tiles = choose_tiles(pool, layer, active.data(), uint32_t(active.size()), num_q_heads, softcap,
                                          folded && folded->prep_on, true, no_alloc);
     // (With the queries as two halves the block kernel runs its two-tile form, which brings no
     // rows along: the append is a launch of its own.)

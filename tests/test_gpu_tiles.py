@@ -89,6 +89,24 @@ def test_against_the_oracle(kernels, ctxs, rows, q_heads, kv_heads, window, soft
     pool.close()
 
 
+# A softcap far from one: steps that the split-K kernel takes as well stay with it, whose queries do not carry
+# 2 log2(e) / softcap into their rounding (a factor of 261 on queries of some hundreds at the smallest one here).
+@pytest.mark.parametrize("softcap,kernel", [(2.0 ** -10, "splitk_f16"), (1.9, "splitk_f16"), (2.0, "tiles_f16"),
+                                            (1024.0, "tiles_f16"), (1100.0, "splitk_f16")])
+def test_steps_of_few_rows_with_a_softcap_far_from_one(kernels, softcap, kernel):
+    ctx, rows, q_heads, kv_heads = 290, 8, 32, 4
+    rng, pool, (cache,), (ref,) = setup([ctx], rows, kv_heads, None, 11)
+    q, k, v = (normal(rng, rows, w * D) for w in (q_heads, kv_heads, kv_heads))
+    if softcap < 1.0:
+        q *= 100.0
+    kernels()
+    got = step(pool, [cache], rows, q, k, v, q_heads, softcap)
+    assert kernels() == [kernel]
+    want = oracle.attention_step(ref, 0, q, k, v, q_heads, ctx, oracle.AttentionParams(softcap=softcap), threads=8)
+    assert max_abs(got.reshape(-1), np.asarray(want).reshape(-1)) <= 2e-3
+    pool.close()
+
+
 # Rings of one and two blocks, where two position blocks of a step are the same storage block: its old rows
 # are read beside the new ones' stores, and each row is in one place only.
 @pytest.mark.parametrize("ctx,rows,window,headroom", [(20, 20, 1, 31), (7, 30, 2, 30), (300, 31, 1, 31), (20, 40, 20, 40),
