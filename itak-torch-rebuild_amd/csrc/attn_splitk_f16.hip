@@ -182,16 +182,26 @@ static uint32_t variant_capacity(const Variant &v) {
 // costs half a microsecond. Eight wavefronts from the fifth block on. One-row steps: up to 12 blocks,
 // where the next wavefront's round begins to cost what the merge does (launches that prepare their rows as well:
 // 1 slot at 250 / 320 / 400 split 7.4 / 7.3 / 7.3, whole 6.5 / 7.4 / 8.4), 24 from 64 workgroups on (the merge of many
-// slots costs more). Steps of several rows, whose merge
+// slots costs more). Preparing steps keep 18 where splitting gains less: on pools whose preparing launches stay the
+// split-K kernel's (`may_tile` = false: queries as two halves, the merge in the launch), whose workgroups of one block
+// each spend 2 us on it, and from nine slots on, whose argument block is the large one for every split. Split -> whole
+// at 13 to 18 blocks, 32 Q / 4 KV heads, keys out of the caches: merged in the launch 1 / 4 / 15 slots 10.8 to
+// 10.4 -> 8.8 to 9.6, 11.7 to 11.2 -> 9.6 to 10.3, 13.3 to 13.7 -> 10.9 to 11.9; as two halves 1 / 4 / 15 slots 9.0 to 9.1 ->
+// 9.0 to 9.7, 10.6 -> 9.8 to 10.5, 12.8 -> 11.1 to 12.0; other pools 1 / 7 / 11 / 15 slots 7.9 -> 8.8 to 9.6, 10.2 to 10.4 ->
+// 10.0 to 10.9, 11.4 to 11.8 -> 10.4 to 11.3, 12.0 to 13.1 -> 10.8 to 12.0, one KV head, 50 slots 16.0 -> 12.8.
+// (Keys that are still in L2 favour whole contexts: 2 slots split 8.4, whole 7.8, where out of the caches 9.4 and 9.4 to 10.2.)
+// Steps of several rows, whose merge
 // is larger, up to 16, 24 from 128 workgroups on (up to 8 blocks in the forms that take a unit's vectors
 // together). One layer of 32 Q / 4 KV heads, us, split -> whole: 1 slot at 200 / 300 rows
 // 7.3 / 7.4 -> 5.1 / 5.4 (7.2 -> 7.2 at 400), 16 slots at 300 / 600 11.0 / 12.7 -> 8.7 / 11.1; seven rows at 150 / 350 / 500 8.6 / 8.9 / 8.9 ->
 // 6.8 / 7.2 / 7.8, 8 slots of them at 700 13.8 -> 13.1. Checked at 4, 8 and 1 KV heads and groups of 1 to 8 with
 // every shape forced either way: within 5 % of the better but for a few just past a line (16 slots of one
 // row at 900, 8 KV heads, split 19.1, whole 16.5).
-static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows, uint32_t tiles, bool may_tile) {
-    if (rows > 1) return !may_tile ? 8 : g.kv_heads * b.n * tiles >= 128 ? 24 : 16;
-    return g.kv_heads * b.n >= 64 ? 24 : 12;
+static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows, uint32_t tiles, bool prepares,
+                            bool may_tile, bool may) {
+    if (rows > 1) return !may ? 8 : g.kv_heads * b.n * tiles >= 128 ? 24 : 16;
+    if (g.kv_heads * b.n >= 64) return 24;
+    return prepares && (!may_tile || b.n > 8) ? 18 : 12;
 }
 
 // The tiled form gives every 16 query vectors of a unit (item, KV head) workgroups of their own, with one
@@ -233,7 +243,7 @@ uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads,
     const uint64_t cus = compute_units();
     const uint32_t tiles = (most_rows * group + 15) / 16;
     const bool may = may_tile && takes_tiles(g, b, tiles, blocks, cus, prepares && most_rows == 1);
-    const bool whole = most <= whole_limit(g, b, most_rows, tiles, may);
+    const bool whole = most <= whole_limit(g, b, most_rows, tiles, prepares, may_tile, may);
     b.whole_on_eight = whole && most > 4 && (may || most_rows == 1) ? 1 : 0;
     // (A whole one-row step has no second tile and hardly a second block: the form with two sets of
     // operands, whose next block is under way before the first is multiplied, is 0.4 us faster.)

@@ -315,3 +315,45 @@ def test_queries_beyond_half_range_without_a_norm(ctx, rows, softcap):
     want = oracle.attention_step(ref, 0, q, k[ctx:], v[ctx:], q_heads, ctx, oracle.AttentionParams(softcap=softcap), threads=8)
     assert max_abs(out.cpu().numpy().reshape(-1), np.asarray(want).reshape(-1)) <= 2e-3
     pool.close()
+
+
+# Blocks of keys up to which a preparing one-row step is left whole: 12 where it can run on the one-row kernel, 18 on
+# pools where the split-K kernel prepares, and for more than eight slots; the last length left whole and the next.
+@pytest.mark.parametrize("options,slots,whole", [
+    ({}, 1, 12), ({}, 8, 12), ({}, 9, 18), ({}, 15, 18), ({"merge_in_launch": True}, 1, 18), ({"merge_in_launch": True}, 3, 18),
+    ({"q_two_halves": True}, 1, 18), ({"q_two_halves": True}, 9, 18), ({"die_merge": True}, 1, 12)])
+def test_preparing_steps_left_whole(options, slots, whole, capfd):
+    q_heads, kv_heads, d = 32, 4, 128
+    rng = np.random.default_rng(slots)
+    w = (1.0 + 0.1 * normal(rng, d)).astype(np.float32)
+    wd, lib = dev(w), P()._native.load()
+    for blocks in (whole, whole + 1):
+        ctx = blocks * 32 - 1
+        pool = P().KvPool(1, kv_heads, d, elem="f16", max_slots=slots, capacity_rows=ctx + 1, **options)
+        pool.set_stream(torch.cuda.current_stream().cuda_stream)
+        caches = [pool.acquire() for _ in range(slots)]
+        k, v = normal(rng, ctx + slots, kv_heads * d), normal(rng, ctx + slots, kv_heads * d)
+        q = normal(rng, slots, q_heads * d)
+        qd, kd, vd = dev(q), dev(k), dev(v)
+        for cache in caches:
+            pool.append_device(0, [(cache, ctx)], kd.data_ptr(), vd.data_ptr())
+        out = torch.full_like(qd, float("nan"))
+        capfd.readouterr()
+        lib.itak_set_debug_enabled(1)
+        try:
+            pool.attention_prep_step_device(0, [(c, 1) for c in caches], qd.data_ptr(), kd[ctx:].data_ptr(),
+                                            vd[ctx:].data_ptr(), out.data_ptr(), q_heads, q_norm_ptr=wd.data_ptr(),
+                                            k_norm_ptr=wd.data_ptr(), rope_base=1e6)
+        finally:
+            lib.itak_set_debug_enabled(0)
+        torch.cuda.synchronize()
+        splits = [int(x[7:]) for x in capfd.readouterr().err.split() if x.startswith("splits=")]
+        assert len(splits) == 1 and (splits[0] == 1) == (blocks == whole), (blocks, splits)
+        for s in (0, slots - 1):
+            ref = oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, d, store_f16=True)
+            ref.restore_bulk(0, 0, k[:ctx], v[:ctx])
+            qp = oracle.attention_prep(q[s:s + 1], q_heads, d, ctx, w, 1e-6, 1e6, True, None)
+            kp = oracle.attention_prep(k[ctx + s:ctx + s + 1], kv_heads, d, ctx, w, 1e-6, 1e6, True, None)
+            want = oracle.attention_step(ref, 0, qp, kp, v[ctx + s:ctx + s + 1], q_heads, ctx, threads=8)
+            assert max_abs(out[s].cpu().numpy(), np.asarray(want).reshape(-1)) <= 2e-3
+        pool.close()
