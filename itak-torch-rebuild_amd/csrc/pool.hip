@@ -761,7 +761,12 @@ uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t
 // kernel by more than 2 %. 32 Q / 4 KV heads, us a layer, block kernel -> tiles: 61 rows on 0 / 300 / 1,000 12.4 / 17.9 /
 // 19.1 -> 7.5 / 8.9 / 12.3, on a window of 2,048 18.8 -> 15.9; 24 rows on 4,099 18.4 -> 14.1; 128 rows on 1,000
 // 24.5 -> 13.8; 512 rows on 0 20.1 -> 17.1. The block kernel keeps many rows on long contexts (192 rows on 12,000:
-// 62.5 against 73.3).
+// 62.5 against 73.3). The fit has no launches of several slots of which one brings 128 rows and more: there the
+// tiles take 3 to 8 us beyond their estimate, and `kLongBesideOthers` is added. Over 320 random steps of 1 to 42 slots, most
+// of them decode rows and short blocks beside a chunk, on which the estimates without it chose the tiles, these took 0.74 of
+// the block kernel's time and 14 steps more than 2 % longer (17 slots of seven rows beside 244 22.6 -> 27.4); with it 0.75,
+// and two, 8 % at most (320 others: one, 4 %). 3 / 31 / 7 decode rows at 500 / 1,500 / 2,000 beside 128 / 128 / 64 rows on 1,000 / 0 /
+// 2,000: 22.0 / 40.1 / 21.8 -> 14.2 / 31.7 / 16.7.
 //
 // Against the split-K kernel, whose 16-vector steps are the better ones throughout (the rows come in through
 // LDS, the loads stream): steps of more vectors while the keys are at most one and a half blocks per compute
@@ -800,12 +805,13 @@ TilesPlan choose_tiles(const itak_pool *pool, uint64_t layer, const PlanInput *i
     if (splitk) {
         if (no_alloc) partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads), false, true);
     } else {
-        constexpr float kBlockLaunch = 6.8f, kBlockAppends = 6.4f;
+        constexpr float kBlockLaunch = 6.8f, kBlockAppends = 6.4f, kLongBesideOthers = 5.0f;
         uint32_t most_blocks = 0;
         for (uint32_t i = 0; i < n; ++i) most_blocks = std::max(most_blocks, item_block_count(b.item[i]));
         const bool appends = brings_rows && attn_prefill_f16_appends(pool->g, group, max_rows, most_blocks);
         attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, appends);
-        if (cost >= b.plan_cost + kBlockLaunch + (brings_rows && !appends ? kBlockAppends : 0.0f)) return plan;
+        const float block = b.plan_cost + kBlockLaunch + (brings_rows && !appends ? kBlockAppends : 0.0f);
+        if (cost + (n > 1 && max_rows >= 128 ? kLongBesideOthers : 0.0f) >= block) return plan;
         if (no_alloc) partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, false);
     }
     // (The allocation-free call refuses a step by the same plans as without the tiles, see run_attention.)

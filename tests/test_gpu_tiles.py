@@ -107,6 +107,43 @@ def test_steps_of_few_rows_with_a_softcap_far_from_one(kernels, softcap, kernel)
     pool.close()
 
 
+# Steps of slots with different numbers of rows: a chunk of 128 rows and more beside others goes to the block kernel
+# unless the tiles are estimated to be well ahead; a short one, or a chunk alone, as before.
+@pytest.mark.parametrize("rows,ctxs,kernel", [
+    ([7] * 10 + [22, 244], [46] * 10 + [317, 67], "prefill_f16"), ([1] * 3 + [128], [500] * 3 + [1000], "tiles_f16"),
+    ([1] * 5 + [61], [300, 0, 77, 1500, 20, 333], "tiles_f16"), ([244], [67], "tiles_f16")])
+def test_slots_of_different_row_counts(kernels, rows, ctxs, kernel):
+    q_heads, kv_heads = 32, 8
+    P = pkg()
+    rng = np.random.default_rng(len(rows))
+    pool = P.KvPool(1, kv_heads, D, elem="f16", max_slots=len(rows), capacity_rows=max(ctxs) + max(rows))
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    caches = [pool.acquire() for _ in rows]
+    refs = [oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, D, store_f16=True) for _ in rows]
+    for cache, ref, n in zip(caches, refs, ctxs):
+        if n:
+            k, v = normal(rng, n, kv_heads * D), normal(rng, n, kv_heads * D)
+            cache.restore_bulk(0, 0, k, v)
+            ref.restore_bulk(0, 0, k, v)
+    q, k, v = (normal(rng, sum(rows), w * D) for w in (q_heads, kv_heads, kv_heads))
+    qd, kd, vd = dev(q), dev(k), dev(v)
+    out = torch.full_like(qd, float("nan"))
+    kernels()
+    pool.attention_step_device(0, list(zip(caches, rows)), qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), q_heads)
+    torch.cuda.synchronize()
+    assert kernels() == [kernel]
+    got, first = out.cpu().numpy(), 0
+    for cache, ref, n, ctx in zip(caches, refs, rows, ctxs):
+        at = slice(first, first + n)
+        first += n
+        want = oracle.attention_step(ref, 0, q[at], k[at], v[at], q_heads, ctx, threads=8)
+        assert max_abs(got[at].reshape(-1), np.asarray(want).reshape(-1)) <= 2e-3
+        _, gk, gv = cache.read_rows(0, ctx, n)
+        assert np.array_equal(gk.reshape(n, -1), oracle.f32_to_f16_array(k[at]))
+        assert np.array_equal(gv.reshape(n, -1), oracle.f32_to_f16_array(v[at]))
+    pool.close()
+
+
 # Rings of one and two blocks, where two position blocks of a step are the same storage block: its old rows
 # are read beside the new ones' stores, and each row is in one place only.
 @pytest.mark.parametrize("ctx,rows,window,headroom", [(20, 20, 1, 31), (7, 30, 2, 30), (300, 31, 1, 31), (20, 40, 20, 40),
