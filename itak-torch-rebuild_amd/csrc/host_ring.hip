@@ -7,11 +7,8 @@
 #include <atomic>
 #include <thread>
 
+#include "host_halves.h"
 #include "itkv.h"
-
-#if !defined(__HIP_DEVICE_COMPILE__)
-#include <immintrin.h>
-#endif
 
 namespace itak {
 
@@ -38,56 +35,6 @@ void HostRing::close() {
 }
 
 namespace {
-
-// n bytes of f32 values from n / 2 bytes of halves, and back: false where some value is no f16's (a NaN
-// counts as none: its payload would have to survive two conversions on either side).
-#if !defined(__HIP_DEVICE_COMPILE__)
-// (Streaming stores are no faster here: the pages are fresh, and the kernel has just cleared them.)
-__attribute__((target("avx,f16c"))) void widen_halves(unsigned char *out, const unsigned char *in, uint64_t n) {
-    uint64_t at = 0;
-    for (; at + 32 <= n; at += 32)
-        _mm256_storeu_ps(reinterpret_cast<float *>(out + at),
-                         _mm256_cvtph_ps(_mm_loadu_si128(reinterpret_cast<const __m128i *>(in + at / 2))));
-    for (; at < n; at += 4) {
-        uint16_t h;
-        memcpy(&h, in + at / 2, 2);
-        const float f = _mm_cvtss_f32(_mm_cvtph_ps(_mm_cvtsi32_si128(h)));
-        memcpy(out + at, &f, 4);
-    }
-}
-__attribute__((target("avx,f16c"))) bool narrow_floats(unsigned char *out, const unsigned char *in, uint64_t n) {
-    __m256 differ = _mm256_setzero_ps(), unordered = _mm256_setzero_ps();
-    uint64_t at = 0;
-    for (; at + 32 <= n; at += 32) {
-        const __m256 f = _mm256_loadu_ps(reinterpret_cast<const float *>(in + at));
-        const __m128i h = _mm256_cvtps_ph(f, _MM_FROUND_TO_NEAREST_INT);
-        _mm_storeu_si128(reinterpret_cast<__m128i *>(out + at / 2), h);
-        // (Bits, not values: a thread that takes subnormal f32 values as zero, as torch.set_flush_denormal asks for, would
-        // find them equal to the zeros they become.)
-        differ = _mm256_or_ps(differ, _mm256_xor_ps(f, _mm256_cvtph_ps(h)));
-        unordered = _mm256_or_ps(unordered, _mm256_cmp_ps(f, f, _CMP_UNORD_Q));
-    }
-    const __m256i bits = _mm256_castps_si256(differ);
-    bool exact = _mm256_testz_si256(bits, bits) && _mm256_movemask_ps(unordered) == 0;
-    for (; at < n; at += 4) {
-        float f;
-        memcpy(&f, in + at, 4);
-        const uint16_t h = uint16_t(_mm_cvtsi128_si32(_mm_cvtps_ph(_mm_set_ss(f), _MM_FROUND_TO_NEAREST_INT)));
-        memcpy(out + at / 2, &h, 2);
-        const float back = _mm_cvtss_f32(_mm_cvtph_ps(_mm_cvtsi32_si128(h)));
-        exact = exact && f == f && memcmp(&f, &back, 4) == 0;
-    }
-    return exact;
-}
-bool has_f16c() {
-    __builtin_cpu_init();
-    return __builtin_cpu_supports("avx") && __builtin_cpu_supports("f16c");
-}
-#else
-void widen_halves(unsigned char *, const unsigned char *, uint64_t) {}
-bool narrow_floats(unsigned char *, const unsigned char *, uint64_t) { return false; }
-bool has_f16c() { return false; }
-#endif
 
 // Part of a transfer that goes through one slot: bytes [at, at + bytes) of it.
 struct Chunk {
@@ -233,21 +180,15 @@ hipError_t ring_upload_narrow(HostRing &ring, const void *src, uint64_t bytes, v
     cut(bytes, true, [&](uint64_t at, uint64_t n) {
         chunks.push_back(Chunk{static_cast<const unsigned char *>(src) + at, static_cast<unsigned char *>(floats) + at, n, at});
     });
-    // One chunk with a value that is no f16's says what the rest holds: they are not tried any more.
+    // One value that is no f16's says what the rest holds: no thread tries any further.
     std::atomic<bool> worth_it{true};
     std::vector<unsigned char> narrowed(chunks.size(), 0);
     uint64_t from = 0, to = 0;  // arrived as halves and not reported
     return run_upload(
         ring, chunks.size(), stream,
         [&](uint64_t c, unsigned char *slot) {
-            if (worth_it.load(std::memory_order_relaxed)) {
-                if (narrow_floats(slot, chunks[c].src, chunks[c].bytes)) {
-                    narrowed[c] = 1;
-                    return;
-                }
-                worth_it.store(false, std::memory_order_relaxed);
-            }
-            memcpy(slot, chunks[c].src, chunks[c].bytes);
+            narrowed[c] = narrow_chunk(slot, chunks[c].src, chunks[c].bytes, worth_it);
+            if (!narrowed[c]) memcpy(slot, chunks[c].src, chunks[c].bytes);
         },
         [&](uint64_t c, unsigned char *slot, hipEvent_t moved, std::atomic<uint64_t> &enqueued) {
             const Chunk &k = chunks[c];
