@@ -441,7 +441,7 @@ itak_status itak_kv_capture_itkv_f16(itak_pool *pool, uint32_t slot, const char 
    slot (either format version; f16 rows go into an f16 pool as they are and are refused by
    an f32 pool): the snapshot's geometry must be the pool's, and, when expected_fingerprint is not
    NULL, its fingerprint the expected one. A payload of 128 KB and more goes to a device buffer of
-   its own size (half as much again where f32 rows cross the link to an f16 pool as halves, which
+   its own size (and up to 16 MB beside it where f32 rows cross the link to an f16 pool as halves, which
    they do chunk by chunk where that loses nothing) for the length of the call, is summed there (version 1; version 2 by host threads
    meanwhile) and gathered from there once the sum is known good; where that buffer cannot be had,
    and below that size, the host sums, and the rows are gathered from `bytes` in place when the device

@@ -43,9 +43,11 @@ struct RingSpan {
 hipError_t ring_upload(HostRing &ring, const std::vector<RingSpan> &spans, hipStream_t stream,
                        const std::function<hipError_t(uint64_t)> &after = nullptr);
 
-// f32 values at `src` to device memory, as halves at halves + at / 2 (16-byte aligned) while every value is an
-// f16's, else as they are at floats + at: `after(n, from, to)` is called like ring_upload's, with the bytes [from, to)
-// (of the f32 values) that have arrived as halves since the last call, all others among them as floats.
+// f32 values at `src` to device memory, as halves (16-byte aligned) while every value is an f16's, else as they are at
+// floats + at. The halves of each kRingChunk * kRingSlots bytes of values take the place of the last ones', at halves +
+// at % (kRingChunk * kRingSlots) / 2: `after(n, from, to)` is called like ring_upload's and at the end of each such
+// piece, with the bytes [from, to) (of the f32 values) that have arrived as halves since the last call, all others among
+// them as floats, and what it enqueues reads them before the next ones come.
 hipError_t ring_upload_narrow(HostRing &ring, const void *src, uint64_t bytes, void *floats, void *halves, hipStream_t stream,
                               const std::function<hipError_t(uint64_t, uint64_t, uint64_t)> &after);
 // Whether this host converts halves in its vector units (both calls that do need it).

@@ -192,7 +192,7 @@ hipError_t ring_upload_narrow(HostRing &ring, const void *src, uint64_t bytes, v
         },
         [&](uint64_t c, unsigned char *slot, hipEvent_t moved, std::atomic<uint64_t> &enqueued) {
             const Chunk &k = chunks[c];
-            void *dst = narrowed[c] ? static_cast<unsigned char *>(halves) + k.at / 2 : k.dst;
+            void *dst = narrowed[c] ? static_cast<unsigned char *>(halves) + k.at % (kRingChunk * kRingSlots) / 2 : k.dst;
             hipError_t e = hipMemcpyAsync(dst, slot, narrowed[c] ? k.bytes / 2 : k.bytes, hipMemcpyHostToDevice, stream);
             if (e == hipSuccess) e = hipEventRecord(moved, stream);
             if (e != hipSuccess) return e;

@@ -6,6 +6,7 @@
 #include "internal.h"
 #include "host_ring.h"
 #include "host_turns.h"
+#include "load_room.h"
 #include "itkv.h"
 
 #include <sys/mman.h>
@@ -2248,7 +2249,6 @@ itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *byt
     const ItkvSum sum_of = [&](const ItkvHeader &header, uint64_t payload) -> uint64_t {
         const uint64_t n = len - 8 - payload, piece = std::min(align_up(n, 256), kPayloadPiece);
         const bool device_sum = header.version == kItkvVersion;
-        const uint64_t scratch_at = align_up(n, 256) + 256;
         // Rows that an f16 pool wrote are halves again on their way over the link (ring_upload_narrow), and
         // f32 in device memory as the sum and the gather want them (16 layers of 2,000 rows: 3.9 -> 2.7 ms).
         const void *usable;
@@ -2256,17 +2256,20 @@ itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *byt
         // (Below, the narrowing and the device's launch take longer than the bytes saved: 1.9 MB 231 us as f32, 249
         // as halves, 4 MB 333 and 311.)
         constexpr uint64_t kNarrowBytes = 3ull << 20;
-        const bool narrow = device_sum && pool->elem_f16 && !pinned && n >= kNarrowBytes && host_has_f16();
-        const uint64_t halves_at = scratch_at + (device_sum ? align_up(fnv_scratch_bytes(piece), 256) : 0);
-        if (n < kDeviceSumBytes || rows.make(halves_at + (narrow ? align_up(n, 256) / 2 : 0)) != hipSuccess)
+        LoadRoom room;
+        if (n < kDeviceSumBytes ||
+            !take_load_room(n, piece, device_sum ? fnv_scratch_bytes(piece) : 0,
+                            device_sum && pool->elem_f16 && !pinned && n >= kNarrowBytes && host_has_f16(),
+                            [&](uint64_t want) { return rows.make(want) == hipSuccess; }, room))
             return itkv_trailer(header.version, b8, len - 8);
-        unsigned long long *state = reinterpret_cast<unsigned long long *>(rows.p + align_up(n, 256));
+        const bool narrow = room.halves_bytes != 0;
+        unsigned long long *state = reinterpret_cast<unsigned long long *>(rows.p + room.state_at);
         if (device_sum)
             moved = launch_fill_words(state, 1, fnv1a64(b8, payload, kFnvOffset), pool->stream);
         uint64_t summed = 0;
         const auto sum_up_to = [&](uint64_t sent) -> hipError_t {
             if (!device_sum || (sent < n && sent - summed < kPayloadPiece)) return hipSuccess;
-            hipError_t e = launch_fnv(rows.p + summed, (sent - summed) / kFnvRun * kFnvRun, rows.p + scratch_at, state, pool->stream);
+            hipError_t e = launch_fnv(rows.p + summed, (sent - summed) / kFnvRun * kFnvRun, rows.p + room.scratch_at, state, pool->stream);
             summed = sent;
             return e;
         };
@@ -2277,9 +2280,9 @@ itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *byt
                 if (moved == hipSuccess) moved = sum_up_to(at + here);
             }
         } else if (moved == hipSuccess && narrow) {
-            moved = ring_upload_narrow(pool->ring, b8 + payload, n, rows.p, rows.p + halves_at, pool->stream,
+            moved = ring_upload_narrow(pool->ring, b8 + payload, n, rows.p, rows.p + room.halves_at, pool->stream,
                                        [&](uint64_t sent, uint64_t from, uint64_t to) -> hipError_t {
-                                           hipError_t e = launch_widen_f16(reinterpret_cast<uint16_t *>(rows.p + halves_at + from / 2),
+                                           hipError_t e = launch_widen_f16(reinterpret_cast<uint16_t *>(rows.p + room.halves_at + from % kPayloadPiece / 2),
                                                                            reinterpret_cast<float *>(rows.p + from), (to - from) / 4,
                                                                            pool->stream);
                                            return e == hipSuccess && (sent == n || sent % kPayloadPiece == 0) ? sum_up_to(sent) : e;
