@@ -2236,7 +2236,8 @@ itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *byt
     // The decoder walks the bytes on the host (header fields, then the checksum over all of
     // them); a device-resident buffer would have to be copied first.
     const void *unused;
-    if (classify(bytes, &unused) == PtrKind::Device)
+    const PtrKind kind = classify(bytes, &unused);
+    if (kind == PtrKind::Device)
         return invalid_argument(pool->err, "an encoded snapshot is decoded on the host: pass host memory");
     ItkvHeader h;
     std::vector<ItkvLayer> ls;
@@ -2251,8 +2252,7 @@ itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *byt
         const bool device_sum = header.version == kItkvVersion;
         // Rows that an f16 pool wrote are halves again on their way over the link (ring_upload_narrow), and
         // f32 in device memory as the sum and the gather want them (16 layers of 2,000 rows: 3.9 -> 2.7 ms).
-        const void *usable;
-        const bool pinned = classify(b8, &usable) == PtrKind::PinnedHost;
+        const bool pinned = kind == PtrKind::PinnedHost;
         // (Below, the narrowing and the device's launch take longer than the bytes saved: 1.9 MB 231 us as f32, 249
         // as halves, 4 MB 333 and 311.)
         constexpr uint64_t kNarrowBytes = 3ull << 20;
