@@ -539,38 +539,64 @@ static uint32_t most_new_blocks(const AttnBatch &b) {
     return most;
 }
 
-static float cost_of(const PoolGeom &g, const AttnBatch &b, uint32_t q_heads, uint32_t window, const TileForm &f,
-                     uint32_t run, uint64_t cus, uint64_t *partial_bytes) {
-    const uint32_t group = q_heads / g.kv_heads, vectors = f.sets * 16;
-    uint64_t groups = 0, read = 0, partials = 0;
-    float longest = 0.0f, total = 0.0f;
+// What a form walks, whatever the split: an item's blocks, its tiles over all KV heads, and what one of them sees.
+struct TileItem {
+    uint32_t blocks, units;
+    float seen;
+};
+struct TileWork {
+    TileItem item[kMaxBatchItems];
+    uint64_t groups = 0, read = 0;  // workgroups of the whole contexts; bytes of keys and values, once
+    float total = 0.0f;             // blocks that all workgroups see
+};
+static void work_of(const PoolGeom &g, const AttnBatch &b, uint32_t group, uint32_t window, const TileForm &f, TileWork &w) {
+    const uint32_t vectors = f.sets * 16;
     for (uint32_t i = 0; i < b.n; ++i) {
         const AttnItem &it = b.item[i];
         const uint32_t blocks = item_block_count(it), tiles = (it.rows * group + vectors - 1) / vectors;
-        const uint32_t splits = std::max((blocks + run - 1) / run, 1u);
         const uint32_t units = g.kv_heads * tiles;
         // What a tile sees of them: its rows' window, or on average half the new rows less.
         const float seen = window ? float(std::min(blocks, (window + vectors / group + 62) / kBlockKeys))
                                   : std::max(float(blocks) - (tiles > 1 ? float(it.rows) / 64.0f : 0.0f), 1.0f);
-        groups += uint64_t(units) * splits;
-        longest = std::max(longest, std::min(float((blocks + splits - 1) / splits), seen));
-        total += float(units) * seen;
-        read += uint64_t(g.kv_heads) * blocks * 2 * kBlockKeys * kD * 2;
-        if (splits > 1) partials += uint64_t(it.rows) * q_heads * splits;
+        w.item[i] = {blocks, units, seen};
+        w.groups += units;
+        w.total += float(units) * seen;
+        w.read += uint64_t(g.kv_heads) * blocks * 2 * kBlockKeys * kD * 2;
+    }
+}
+// No split of the form takes less: its launch, what it reads, and the walks that share compute units.
+static float least_of(const TileForm &f, const TileWork &w, uint64_t cus) {
+    const float beside = w.groups > cus ? w.total * f.shared * (1.0f / float(cus) - 1.0f / float(w.groups)) : 0.0f;
+    return (f.fixed + float(w.read) / kReadRate + beside) * 0.9999f;  // (sums in another order than cost_of's)
+}
+static float cost_of(const AttnBatch &b, uint32_t q_heads, const TileForm &f, const TileWork &w, uint32_t run, uint64_t cus,
+                     uint64_t *partial_bytes) {
+    uint64_t groups = 0, partials = 0;
+    float longest = 0.0f;
+    for (uint32_t i = 0; i < b.n; ++i) {
+        const TileItem &it = w.item[i];
+        const uint32_t splits = std::max((it.blocks + run - 1) / run, 1u);
+        groups += uint64_t(it.units) * splits;
+        longest = std::max(longest, std::min(float((it.blocks + splits - 1) / splits), it.seen));
+        if (splits > 1) partials += uint64_t(b.item[i].rows) * q_heads * splits;
     }
     float walk = longest * f.alone;
     const uint64_t each_cu = (groups + cus - 1) / cus;
-    if (each_cu > 1) walk = kBeside * walk + float(each_cu - 1) * total / float(groups) * f.shared;
-    walk += float(read) / kReadRate;
+    if (each_cu > 1) walk = kBeside * walk + float(each_cu - 1) * w.total / float(groups) * f.shared;
+    walk += float(w.read) / kReadRate;
     const uint64_t held = cus * f.resident;
     *partial_bytes = partials * (kD + 2) * 4;
     return f.fixed + walk + float((groups + held - 1) / held - 1) * kRound +
            (partials ? kMergeLaunch + float(*partial_bytes) / kMergeRate : 0.0f);
 }
 
+// (Forms that cannot come under the least so far, or under `below`, are not searched: 32 slots of nine rows at 1,000, which
+// stay with the block kernel: 11.9 us of planning on one host core with the search unbounded and that kernel planned
+// twice, 6.5 so.)
 float attn_tiles_f16_choose(const PoolGeom &g, const AttnBatch &b, uint32_t q_heads, uint32_t window, bool brings_rows,
-                            bool few_rows, uint64_t partial_limit, TilesPlan &plan) {
+                            bool few_rows, uint64_t partial_limit, float below, TilesPlan &plan) {
     const uint64_t cus = compute_units();
+    const uint32_t group = q_heads / g.kv_heads;
     uint32_t most = 1, rows = 0;
     for (uint32_t i = 0; i < b.n; ++i) {
         most = std::max(most, item_block_count(b.item[i]));
@@ -578,12 +604,15 @@ float attn_tiles_f16_choose(const PoolGeom &g, const AttnBatch &b, uint32_t q_he
     }
     const uint32_t new_blocks = brings_rows ? most_new_blocks(b) : 0;
     constexpr uint8_t kCounts[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 20, 24, 32};
-    float least = INFINITY;
+    float least = below;
     for (const TileForm &f : kForms) {
-        if (f.sets == 2 && b.n == 1 && b.item[0].rows * (q_heads / g.kv_heads) <= 16) continue;
+        if (f.sets == 2 && b.n == 1 && b.item[0].rows * group <= 16) continue;
         // (A wavefront takes at most one block of new rows.)
         const bool appends = new_blocks <= f.waves;
         const float append = appends ? 0.0f : kAppendLaunch + kAppendRow * float(rows);
+        TileWork w;
+        work_of(g, b, group, window, f, w);
+        if (append + least_of(f, w, cus) >= least) continue;
         uint32_t before = 0;
         for (uint32_t c = 0; c < sizeof(kCounts); c += b.n > 8 ? 2 : 1) {
             const uint32_t run = (most + kCounts[c] - 1) / kCounts[c];
@@ -593,7 +622,7 @@ float attn_tiles_f16_choose(const PoolGeom &g, const AttnBatch &b, uint32_t q_he
             // (The split-K kernel's whole steps have eight wavefronts: no more blocks under one maximum here.)
             if (few_rows && f.waves == 4 && run > 4) continue;
             uint64_t partial_bytes = 0;
-            const float cost = append + cost_of(g, b, q_heads, window, f, run, cus, &partial_bytes);
+            const float cost = append + cost_of(b, q_heads, f, w, run, cus, &partial_bytes);
             if (partial_limit && partial_bytes > partial_limit) break;
             if (cost < least) {
                 least = cost;

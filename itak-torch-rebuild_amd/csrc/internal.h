@@ -561,11 +561,12 @@ struct TilesPlan {
     bool exact = false;   // the softmax keeps the exact running maximum
 };
 bool attn_tiles_f16_supports(const PoolGeom &g, uint32_t group, uint32_t most_rows);
-// The cheapest form for a batch (slot, rows, pos0, kv_len, kv_lo set) and its cost in us. `brings_rows`: the
+// The cheapest form for a batch (slot, rows, pos0, kv_len, kv_lo set) that costs less than `below` us, and its cost
+// (`below` and the plan as it was when there is none). `brings_rows`: the
 // step's rows are not in the cache yet (appended by the launch where the form can, else before it); `few_rows`: a
 // step the split-K kernel takes as well.
 float attn_tiles_f16_choose(const PoolGeom &g, const AttnBatch &b, uint32_t q_heads, uint32_t window, bool brings_rows,
-                            bool few_rows, uint64_t partial_limit, TilesPlan &plan);
+                            bool few_rows, uint64_t partial_limit, float below, TilesPlan &plan);
 uint32_t attn_tiles_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, const TilesPlan &plan);
 hipError_t launch_attn_tiles_f16(const AttnParams &p, const AttnBatch &b, uint32_t total_partials, const float *gate,
                                  hipStream_t stream);

@@ -194,6 +194,7 @@ struct itak_pool {
     HostRing ring;
     // Plan of the step in progress, and the slots it has named (by the number of the step).
     std::vector<PlanInput> plan, active;
+    AttnBatch block_plan;  // the block kernel's plan of the step at hand, where its price was asked (KernelChoice)
     std::vector<uint64_t> named;
     uint64_t step_number = 0;
     uint32_t call_number = 0;  // what the last host-pointer call asked to be told when done
@@ -776,9 +777,15 @@ uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t
 // (keys that are not in the last-level cache: 4 slots of four rows at 8,192 20.4 against 21.7). Softcaps
 // outside [2, 1024] stay there too: the tiles round the queries with 2 log2(e) / softcap on, the split-K kernel caps the
 // scores, and beyond those the factor takes queries out of f16's range, or into its subnormals, that are inside it there.
-TilesPlan choose_tiles(const itak_pool *pool, uint64_t layer, const PlanInput *in, uint32_t n, uint64_t q_heads,
-                       float softcap, bool prepares, bool brings_rows, bool no_alloc) {
-    TilesPlan plan;
+struct KernelChoice {
+    TilesPlan tiles;               // sets = 0: another kernel
+    bool block = false;            // pool->block_plan is the block kernel's plan of the step,
+    bool block_appends = false;    // in a launch that brings the rows along or not,
+    uint32_t block_partials = 0;   // and its partials
+};
+KernelChoice choose_tiles(itak_pool *pool, uint64_t layer, const PlanInput *in, uint32_t n, uint64_t q_heads, float softcap,
+                          bool prepares, bool brings_rows, bool no_alloc) {
+    KernelChoice choice;
     const uint32_t group = uint32_t(q_heads / pool->g.kv_heads);
     uint32_t max_rows = 0;
     uint64_t blocks = 0;
@@ -788,36 +795,39 @@ TilesPlan choose_tiles(const itak_pool *pool, uint64_t layer, const PlanInput *i
     }
     if (!pool->elem_f16 || pool->q_two_halves || n == 0 || n > uint32_t(kMaxBatchItems) ||
         !attn_tiles_f16_supports(pool->g, group, max_rows))
-        return plan;
+        return choice;
     const bool splitk = takes_splitk_f16(pool, in, n, q_heads, nullptr);
     if (splitk && (prepares || pool->merge_in_launch || pool->die_merge || max_rows * group <= 16 ||
                    (softcap > 0.0f && (softcap < 2.0f || softcap > 1024.0f)) ||
                    2 * blocks > 3 * uint64_t(compute_units())))
-        return plan;
+        return choice;
     const PoolGeom &geom = geom_of(pool, layer);
     const uint32_t window = uint32_t(std::min<uint64_t>(pool->layers[layer].window, 0xffffffffu));
     const uint64_t limit = no_alloc ? kScratchBytes - kScratchExchangeBytes : 0;
-    AttnBatch b;
+    AttnBatch &b = pool->block_plan;
     start_batch(b, in, n, 0);
-    TilesPlan form;
-    const float cost = attn_tiles_f16_choose(geom, b, uint32_t(q_heads), window, brings_rows, splitk, limit, form);
-    if (form.sets == 0) return plan;
-    uint64_t partials = 0;
-    if (splitk) {
-        if (no_alloc) partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads), false, true);
-    } else {
+    float below = INFINITY;
+    if (!splitk) {
         constexpr float kBlockLaunch = 6.8f, kBlockAppends = 6.4f, kLongBesideOthers = 5.0f;
         uint32_t most_blocks = 0;
         for (uint32_t i = 0; i < n; ++i) most_blocks = std::max(most_blocks, item_block_count(b.item[i]));
         const bool appends = brings_rows && attn_prefill_f16_appends(pool->g, group, max_rows, most_blocks);
-        attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, appends);
-        const float block = b.plan_cost + kBlockLaunch + (brings_rows && !appends ? kBlockAppends : 0.0f);
-        if (cost + (n > 1 && max_rows >= 128 ? kLongBesideOthers : 0.0f) >= block) return plan;
-        if (no_alloc) partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, false);
+        choice.block_partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, appends);
+        choice.block = true;
+        choice.block_appends = appends;
+        below = b.plan_cost + kBlockLaunch + (brings_rows && !appends ? kBlockAppends : 0.0f) -
+                (n > 1 && max_rows >= 128 ? kLongBesideOthers : 0.0f);
     }
-    // (The allocation-free call refuses a step by the same plans as without the tiles, see run_attention.)
-    if (limit && partials * (pool->g.head_dim + 2) * sizeof(float) > limit) return plan;
-    return form;
+    attn_tiles_f16_choose(geom, b, uint32_t(q_heads), window, brings_rows, splitk, limit, below, choice.tiles);
+    if (no_alloc && choice.tiles.sets) {
+        // (The allocation-free call refuses a step by the same plans as without the tiles, see run_attention.)
+        AttnBatch m;
+        start_batch(m, in, n, 0);
+        const uint64_t partials = splitk ? attn_splitk_f16_plan(geom, m, uint32_t(q_heads), false, true)
+                                         : attn_prefill_f16_plan(geom, m, group, uint32_t(q_heads), window, false);
+        if (partials * (pool->g.head_dim + 2) * sizeof(float) > limit) choice.tiles = TilesPlan{};
+    }
+    return choice;
 }
 
 // k_new / v_new non-null = the rows are not in the cache yet and the kernel appends them
@@ -827,15 +837,16 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
                           uint64_t q_heads, float scale, float softcap,
                           const float *k_new = nullptr, const float *v_new = nullptr,
                           const FoldedParams *folded = nullptr, WorkspaceNeed *need_only = nullptr,
-                          const TilesPlan *chosen = nullptr) {
+                          const KernelChoice *chosen = nullptr) {
     const uint32_t group = uint32_t(q_heads / pool->g.kv_heads);
     uint32_t max_rows = 0;
     for (uint32_t i = 0; i < n; ++i) max_rows = std::max(max_rows, in[i].rows);
     // (A step has asked already, since who appends hangs on it.)
-    const TilesPlan form = chosen ? *chosen
-                           : q_pos_dev ? TilesPlan{}
-                                       : choose_tiles(pool, layer, in, n, q_heads, softcap, folded && folded->prep_on, false,
-                                                      need_only || pool->no_alloc_call);
+    const KernelChoice choice = chosen ? *chosen
+                                : q_pos_dev ? KernelChoice{}
+                                            : choose_tiles(pool, layer, in, n, q_heads, softcap, folded && folded->prep_on,
+                                                           false, need_only || pool->no_alloc_call);
+    const TilesPlan &form = choice.tiles;
     const bool tiles = form.sets != 0;
     const bool mfma = !tiles && takes_splitk_f16(pool, in, n, q_heads, q_pos_dev);
     // Blocks of many rows (prefill chunks) on the same pools take the MFMA prefill kernel.
@@ -858,8 +869,16 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     uint32_t q_row0 = 0;
     for (uint32_t first = 0; first < n; first += kMaxBatchItems) {
         const uint32_t count = std::min<uint32_t>(kMaxBatchItems, n - first);
-        AttnBatch b;
-        const uint32_t total_rows = start_batch(b, in + first, count, q_row0);
+        // (Planned already where the choice has asked for the block kernel's price; such steps are one batch.)
+        const bool planned = prefill && choice.block && !need_only && !pool->no_alloc_call &&
+                             choice.block_appends == (k_new != nullptr);
+        AttnBatch own;
+        AttnBatch &b = planned ? pool->block_plan : own;
+        uint32_t total_rows = 0;
+        if (planned)
+            for (uint32_t i = 0; i < count; ++i) total_rows += in[i].rows;
+        else
+            total_rows = start_batch(b, in + first, count, q_row0);
         q_row0 += total_rows;
         b.two_halves = prefill && pool->q_two_halves && pool->g.head_dim == 128 ? 1 : 0;
         // (At head_dim 128 a step is refused when the best plan of a launch without its rows outgrows the static
@@ -868,7 +887,9 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         b.partial_limit = (need_only || pool->no_alloc_call) && (pool->g.head_dim != 128 || k_new)
                               ? kScratchBytes - kScratchExchangeBytes : 0;
         uint32_t partials = 0;
-        if (tiles) {
+        if (planned) {
+            partials = choice.block_partials;
+        } else if (tiles) {
             partials = attn_tiles_f16_plan(geom, b, uint32_t(q_heads), form);
         } else if (mfma) {
             partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads), folded && folded->prep_on,
@@ -2745,7 +2766,7 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
     const bool splitk = takes_splitk_f16(pool, active.data(), uint32_t(active.size()), num_q_heads, nullptr);
     const bool any = !active.empty() &&
                      takes_splitk_any(pool, active.data(), uint32_t(active.size()), num_q_heads, q_dev, out_dev, nullptr);
-    const TilesPlan tiles = choose_tiles(pool, layer, active.data(), uint32_t(active.size()), num_q_heads, softcap,
+    const KernelChoice choice = choose_tiles(pool, layer, active.data(), uint32_t(active.size()), num_q_heads, softcap,
                                          folded && folded->prep_on, true, no_alloc);
     // (With the queries as two halves the block kernel runs its two-tile form, which brings no
     // rows along: the append is a launch of its own.)
@@ -2753,7 +2774,7 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
         !splitk && !any && pool->elem_f16 && !active.empty() && !(pool->q_two_halves && pool->g.head_dim == 128) &&
         attn_prefill_f16_appends(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows, most_blocks);
     const bool fuse =
-        tiles.sets ? tiles.appends : splitk || block_fuses ||
+        choice.tiles.sets ? choice.tiles.appends : splitk || block_fuses ||
         (!pool->elem_f16 && !active.empty() &&
          attn_splitk_f32_supports(pool->g, uint32_t(num_q_heads / pool->g.kv_heads), most_rows)) ||
         (any && aligned16(k_dev) && aligned16(v_dev) &&
@@ -2769,7 +2790,7 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
         WorkspaceNeed need;
         itak_status st = run_attention(pool, layer, active.data(), uint32_t(active.size()), q_dev, out_dev,
                                        nullptr, num_q_heads, scale, softcap, nullptr, nullptr, folded,
-                                       &need, &tiles);
+                                       &need, &choice);
         if (st != ITAK_OK) return st;
         const uint64_t partial_bytes = need.partial_floats * sizeof(float);
         const uint64_t exchange_bytes = need.exchange_words * 8;
@@ -2794,12 +2815,12 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
         for (uint32_t i = 0; i < item_count; ++i)
             advance(pool->slots[items[i].slot], layer, items[i].rows);
         return run_attention(pool, layer, active.data(), uint32_t(active.size()), q_dev, out_dev,
-                             nullptr, num_q_heads, scale, softcap, k_dev, v_dev, folded, nullptr, &tiles);
+                             nullptr, num_q_heads, scale, softcap, k_dev, v_dev, folded, nullptr, &choice);
     }
     itak_status st = run_append(pool, layer, items, item_count, k_dev, v_dev);
     if (st != ITAK_OK) return st;
     return run_attention(pool, layer, active.data(), uint32_t(active.size()), q_dev, out_dev,
-                         nullptr, num_q_heads, scale, softcap, nullptr, nullptr, folded, nullptr, &tiles);
+                         nullptr, num_q_heads, scale, softcap, nullptr, nullptr, folded, nullptr, &choice);
 }
 
 // Validates one batched step and returns the per-item plan (positions before the append).
