@@ -972,8 +972,11 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             if (st != ITAK_OK) return st;
             ws = exchange_words ? reinterpret_cast<float *>(pool->xws) : pool->ws;
         }
-        // The reference's line (attention.rs:147-155) plus which kernel takes the launch.
+        // The reference's line (attention.rs:147-155) plus which kernel takes the launch, and in the forms that the
+        // planners of some choose between, its wavefronts a workgroup.
         if (diag_enabled()) {
+            const char *waves = tiles ? (b.tile_waves == 8 ? "8" : "4")
+                                : !f32fast && !any ? "-" : b.half_blocks ? "4,half_blocks" : b.on_eight ? "8" : "4";
             uint32_t splits = 0;
             uint64_t view_len = 0;
             for (uint32_t i = 0; i < count; ++i) {
@@ -982,11 +985,11 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             }
             diag_emit("gqa_attention layer=%llu items=%u queries=%u q_heads=%llu kv_heads=%llu "
                       "view_len=%llu window=%u scale=%g softcap=%g kernel=%s workgroups=%u splits=%u "
-                      "fused_append=%d merge=%s",
+                      "wavefronts=%s fused_append=%d merge=%s",
                       ULL(layer), count, total_rows, ULL(q_heads), ULL(pool->g.kv_heads), ULL(view_len),
                       window, double(scale), double(softcap),
                       tiles ? "tiles_f16" : mfma ? "splitk_f16" : prefill ? "prefill_f16" : f32fast ? "splitk_f32" : any ? "splitk_any" : "generic",
-                      bl.total_blocks, splits, int(k_new != nullptr && (tiles || mfma || f32fast || any || prefill)),
+                      bl.total_blocks, splits, waves, int(k_new != nullptr && (tiles || mfma || f32fast || any || prefill)),
                       partials == 0 ? "none" : on_die ? "on_die" : exchange_words ? "in_launch" : "launch");
         }
         AttnParams p{};

@@ -190,16 +190,30 @@ def test_rounds_of_wavefronts(elem, d, q_heads, kv_heads, ctx):
     pool.close()
 
 
-# Blocks of several tiles, cut by the estimates: contexts left whole that the even fill had split, fewer and
-# more splits than it, halves of blocks, eight wavefronts; contexts of one length, nearly so, and apart
-# (which keep the even fill). `most` = the splits that the launch may have.
-@pytest.mark.parametrize("elem,d,q_heads,kv_heads,rows,ctxs,most", [
-    ("f16", 192, 32, 4, 38, (198, 198, 198), 1), ("f16", 240, 8, 1, 33, (1206, 1190), 64), ("f16", 144, 8, 8, 25, (610,), 64),
-    ("f16", 80, 32, 4, 13, (911,) * 7, 1), ("f16", 48, 6, 2, 9, (333, 320), 64), ("f16", 112, 32, 4, 9, (700, 90), 64),
-    ("f32", 64, 32, 4, 12, (845, 840, 833, 845, 845, 845, 845, 831), 1), ("f32", 64, 24, 8, 3, (1500, 30), 64),
-    ("f32", 128, 32, 4, 19, (635,) * 6, 1), ("f32", 128, 8, 1, 15, (1900, 1891), 64), ("f32", 128, 32, 4, 3, (614,) * 7, 64),
+# Blocks of several tiles, cut by the estimates: contexts left whole that the even fill had split (on four and eight
+# wavefronts and on halves of blocks), fewer and more splits than it, another form at as many; contexts of one length,
+# nearly so, and far apart (which keep the even fill). `splits` and `wavefronts` are the launch's on 256 compute units,
+# the even fill's in the comment.
+@pytest.mark.parametrize("elem,d,q_heads,kv_heads,rows,ctxs,splits,wavefronts", [
+    ("f16", 192, 32, 4, 38, (198, 198, 198), 1, "4"),                  # 2, 4
+    ("f16", 240, 8, 1, 33, (1206, 1190), 6, "4"),                      # 10, 4
+    ("f16", 144, 8, 8, 25, (610,), 5, "4"),                            # the same
+    ("f16", 80, 32, 4, 13, (911,) * 7, 1, "8"),                        # 2, 4
+    ("f16", 48, 6, 2, 12, (507,), 1, "8"),                             # 5, 4
+    ("f16", 112, 32, 4, 19, (346,), 1, "4"),                           # 1, 8
+    ("f16", 112, 32, 4, 20, (1239,), 6, "4"),                          # 10, 4
+    ("f16", 48, 6, 2, 9, (333, 320), 1, "8"), ("f16", 112, 32, 4, 9, (700, 90), 1, "8"),  # the same, far apart
+    ("f32", 64, 32, 4, 12, (845, 840, 833, 845, 845, 845, 845, 831), 1, "8"),  # 2, 4
+    ("f32", 64, 32, 4, 28, (1191,), 4, "8"),                           # 8, 4
+    ("f32", 64, 24, 8, 3, (1500, 30), 24, "4,half_blocks"),            # the same, far apart
+    ("f32", 128, 32, 4, 19, (635,) * 6, 1, "4,half_blocks"),           # 2, 4
+    ("f32", 128, 8, 1, 25, (363, 345, 345, 345, 345), 7, "4,half_blocks"),  # 4, 4
+    ("f32", 128, 32, 4, 25, (675, 642, 642, 642, 642), 3, "4"),        # 2, 4
+    ("f32", 128, 32, 4, 21, (778, 778), 5, "4,half_blocks"),           # 5, 4
+    ("f32", 128, 8, 1, 15, (1900, 1891), 15, "4"),                     # the same
+    ("f32", 128, 32, 4, 3, (614,) * 7, 4, "4,half_blocks"),            # 5, 4
 ])
-def test_blocks_of_several_tiles(elem, d, q_heads, kv_heads, rows, ctxs, most, capfd):
+def test_blocks_of_several_tiles(elem, d, q_heads, kv_heads, rows, ctxs, splits, wavefronts, capfd):
     P = pkg()
     rng = np.random.default_rng(d + rows)
     pool = P.KvPool([P.LayerKind.Global], kv_heads, d, elem=elem, max_slots=len(ctxs), capacity_rows=max(ctxs) + rows + 8)
@@ -217,11 +231,13 @@ def test_blocks_of_several_tiles(elem, d, q_heads, kv_heads, rows, ctxs, most, c
     lib = P._native.load()
     capfd.readouterr()
     lib.itak_set_debug_enabled(1)
-    pool.attention_step_device(0, [(c, rows) for c in caches], qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), q_heads)
-    lib.itak_set_debug_enabled(0)
+    try:
+        pool.attention_step_device(0, [(c, rows) for c in caches], qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), q_heads)
+    finally:
+        lib.itak_set_debug_enabled(0)
     torch.cuda.synchronize()
-    splits = [int(w[7:]) for w in capfd.readouterr().err.split() if w.startswith("splits=")]
-    assert len(splits) == 1 and 1 <= splits[0] <= most
+    said = dict(w.split("=", 1) for w in capfd.readouterr().err.split() if "=" in w)
+    assert (int(said["splits"]), said["wavefronts"]) == (splits, wavefronts)
     got = out.cpu().numpy()
     for s, ref in enumerate(refs):
         at = slice(s * rows, (s + 1) * rows)

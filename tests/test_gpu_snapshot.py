@@ -249,9 +249,8 @@ def test_f16_snapshots_stay_with_f16_pools_and_go_through_the_store(tmp_path):
     f32_pool.close(); f16_pool.close()
 
 
-# Version 1 of an f16 pool crosses the link as halves. Every half there is goes out as the f32 value it is
-# (as the small captures, whose rows the device widens, have it), the sum holds, and comes back. Sizes
-# around the chunks of the ring and the pieces that are summed at a time.
+# Version 1 of an f16 pool crosses the link as halves, which host threads widen. Every half there is goes out as the
+# f32 value it is, the sum holds (over rows that the device widened for itself), and comes back.
 def test_every_half_through_a_version_1_snapshot():
     kv_heads, d, tokens = 4, 128, 256
     pool = P().KvPool(2, kv_heads, d, elem="f16", max_slots=3, capacity_rows=tokens)
@@ -278,6 +277,7 @@ def test_every_half_through_a_version_1_snapshot():
     pool.close()
 
 
+# Sizes around the chunks of the ring and the pieces that are summed at a time.
 @pytest.mark.parametrize("layers,tokens", [(1, 33), (2, 511), (2, 512), (2, 513), (4, 2048), (4, 2051), (5, 3333)])
 @pytest.mark.parametrize("exact", ["all", "first layer", "none"])
 def test_version_1_of_f16_pools_at_the_rings_edges(layers, tokens, exact):
