@@ -19,10 +19,9 @@
 #include <functional>
 #include <vector>
 
-namespace itak {
+#include "ring_cut.h"
 
-constexpr uint64_t kRingChunk = 4ull << 20;
-constexpr uint32_t kRingSlots = 8;
+namespace itak {
 
 struct HostRing {
     unsigned char *slot[kRingSlots] = {};  // pinned, kRingChunk bytes each

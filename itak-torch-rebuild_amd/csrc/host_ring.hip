@@ -44,21 +44,6 @@ struct Chunk {
     uint64_t at;
 };
 
-// A run of `bytes` bytes cut into chunks of kRingChunk, the first (`ramp_up`) or last one in four and its neighbour
-// in two. fn(at, n) for each in order. Runs of few chunks stay as they are: every chunk more is a helper more to
-// start, and a single chunk is moved by the calling thread (1.9 MB loaded 231 us in one, 264 in two).
-template <class F>
-void cut(uint64_t bytes, bool ramp_up, F fn) {
-    const uint64_t unit = kRingChunk, whole = (bytes + unit - 1) / unit;
-    const bool ramp = whole > kRingSlots / 2;
-    for (uint64_t c = 0; c < whole; ++c) {
-        const uint64_t from_end = ramp_up ? c : whole - 1 - c;
-        const uint64_t part = unit / (!ramp ? 1 : from_end == 0 ? 4 : from_end == 1 ? 2 : 1);
-        const uint64_t end = std::min(bytes, (c + 1) * unit);
-        for (uint64_t at = c * unit; at < end; at += part) fn(at, std::min(part, end - at));
-    }
-}
-
 // What the threads of one transfer share. Chunk c uses slot c % kRingSlots; thread w of `workers`
 // has the chunks w, w + workers, ..
 struct Transfer {
@@ -158,7 +143,7 @@ hipError_t ring_upload(HostRing &ring, const std::vector<RingSpan> &spans, hipSt
             chunks.push_back(Chunk{static_cast<const unsigned char *>(s.src) + at, static_cast<unsigned char *>(s.dst) + at, n, at});
         };
         if (i == 0)
-            cut(s.bytes, true, add);
+            ring_cut(s.bytes, RampAt::FirstOfMany, add);
         else
             for (uint64_t at = 0; at < s.bytes; at += kRingChunk) add(at, std::min(kRingChunk, s.bytes - at));
     }
@@ -177,7 +162,7 @@ hipError_t ring_upload(HostRing &ring, const std::vector<RingSpan> &spans, hipSt
 hipError_t ring_upload_narrow(HostRing &ring, const void *src, uint64_t bytes, void *floats, void *halves, hipStream_t stream,
                               const std::function<hipError_t(uint64_t, uint64_t, uint64_t)> &after) {
     std::vector<Chunk> chunks;
-    cut(bytes, true, [&](uint64_t at, uint64_t n) {
+    ring_cut(bytes, RampAt::First, [&](uint64_t at, uint64_t n) {
         chunks.push_back(Chunk{static_cast<const unsigned char *>(src) + at, static_cast<unsigned char *>(floats) + at, n, at});
     });
     // One value that is no f16's says what the rest holds: no thread tries any further.
@@ -216,7 +201,7 @@ hipError_t ring_download(HostRing &ring, void *out, uint64_t bytes, hipStream_t 
                          const std::function<hipError_t(uint64_t, uint64_t, const void **)> &source) {
     if (bytes == 0) return hipSuccess;
     std::vector<Chunk> list;
-    cut(bytes, false, [&](uint64_t at, uint64_t n) {
+    ring_cut(bytes, RampAt::Last, [&](uint64_t at, uint64_t n) {
         list.push_back(Chunk{nullptr, static_cast<unsigned char *>(out) + at, n, at});
     });
     const uint64_t chunks = list.size();
