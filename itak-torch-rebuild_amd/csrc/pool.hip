@@ -769,6 +769,10 @@ uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t
 // the block kernel's time and 14 steps more than 2 % longer (17 slots of seven rows beside 244 22.6 -> 27.4); with it 0.75,
 // and two, 8 % at most (320 others: one, 4 %). 3 / 31 / 7 decode rows at 500 / 1,500 / 2,000 beside 128 / 128 / 64 rows on 1,000 / 0 /
 // 2,000: 22.0 / 40.1 / 21.8 -> 14.2 / 31.7 / 16.7.
+// Estimates within 5 % of each other are the block kernel's (`kAhead`): near ties on contexts beyond the fit were not
+// ties (71 rows on 18,376 44.0 -> 51.5, 248 on 8,241 at 8 KV heads 55.6 -> 64.4). Over 814 random steps, 176 with the keys
+// out of the caches, the tiles' took 0.742 of the block kernel's time without the margin and eight more than 2 % longer; with
+// it 0.747, and one.
 //
 // Against the split-K kernel, whose 16-vector steps are the better ones throughout (the rows come in through
 // LDS, the loads stream): steps of more vectors while the keys are at most one and a half blocks per compute
@@ -808,14 +812,14 @@ KernelChoice choose_tiles(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     start_batch(b, in, n, 0);
     float below = INFINITY;
     if (!splitk) {
-        constexpr float kBlockLaunch = 6.8f, kBlockAppends = 6.4f, kLongBesideOthers = 5.0f;
+        constexpr float kBlockLaunch = 6.8f, kBlockAppends = 6.4f, kLongBesideOthers = 5.0f, kAhead = 0.95f;
         uint32_t most_blocks = 0;
         for (uint32_t i = 0; i < n; ++i) most_blocks = std::max(most_blocks, item_block_count(b.item[i]));
         const bool appends = brings_rows && attn_prefill_f16_appends(pool->g, group, max_rows, most_blocks);
         choice.block_partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, appends);
         choice.block = true;
         choice.block_appends = appends;
-        below = b.plan_cost + kBlockLaunch + (brings_rows && !appends ? kBlockAppends : 0.0f) -
+        below = kAhead * (b.plan_cost + kBlockLaunch + (brings_rows && !appends ? kBlockAppends : 0.0f)) -
                 (n > 1 && max_rows >= 128 ? kLongBesideOthers : 0.0f);
     }
     attn_tiles_f16_choose(geom, b, uint32_t(q_heads), window, brings_rows, splitk, limit, below, choice.tiles);

@@ -111,7 +111,8 @@ def test_steps_of_few_rows_with_a_softcap_far_from_one(kernels, softcap, kernel)
 # unless the tiles are estimated to be well ahead; a short one, or a chunk alone, as before.
 @pytest.mark.parametrize("rows,ctxs,kernel", [
     ([7] * 10 + [22, 244], [46] * 10 + [317, 67], "prefill_f16"), ([1] * 3 + [128], [500] * 3 + [1000], "tiles_f16"),
-    ([1] * 5 + [61], [300, 0, 77, 1500, 20, 333], "tiles_f16"), ([244], [67], "tiles_f16")])
+    ([1] * 5 + [61], [300, 0, 77, 1500, 20, 333], "tiles_f16"), ([244], [67], "tiles_f16"),
+    ([11], [8553], "prefill_f16")])  # (a near tie: the tiles' estimate is 3 % ahead)
 def test_slots_of_different_row_counts(kernels, rows, ctxs, kernel):
     q_heads, kv_heads = 32, 8
     P = pkg()
