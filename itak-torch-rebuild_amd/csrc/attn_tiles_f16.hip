@@ -620,7 +620,8 @@ float attn_tiles_f16_choose(const PoolGeom &g, const AttnBatch &b, uint32_t q_he
             if (c && run * 2 < f.waves) break;
             before = run;
             // (The split-K kernel's whole steps have eight wavefronts: no more blocks under one maximum here.)
-            if (few_rows && f.waves == 4 && run > 4) continue;
+            if (few_rows && run > (f.waves == 4 ? 4u : g.kv_heads >= 8 ? 8u : 16u)) continue;
+            if (few_rows && run < most && b.n > 1) break;
             uint64_t partial_bytes = 0;
             const float cost = append + cost_of(b, q_heads, f, w, run, cus, &partial_bytes);
             if (partial_limit && partial_bytes > partial_limit) break;

@@ -769,6 +769,7 @@ uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t
 // the block kernel's time and 14 steps more than 2 % longer (17 slots of seven rows beside 244 22.6 -> 27.4); with it 0.75,
 // and two, 8 % at most (320 others: one, 4 %). 3 / 31 / 7 decode rows at 500 / 1,500 / 2,000 beside 128 / 128 / 64 rows on 1,000 / 0 /
 // 2,000: 22.0 / 40.1 / 21.8 -> 14.2 / 31.7 / 16.7.
+//
 // Estimates within 5 % of each other are the block kernel's (`kAhead`): near ties on contexts beyond the fit were not
 // ties (71 rows on 18,376 44.0 -> 51.5, 248 on 8,241 at 8 KV heads 55.6 -> 64.4). Over 814 random steps, 176 with the keys
 // out of the caches, the tiles' took 0.742 of the block kernel's time without the margin and eight more than 2 % longer; with
@@ -776,9 +777,14 @@ uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t
 //
 // Against the split-K kernel, whose 16-vector steps are the better ones throughout (the rows come in through
 // LDS, the loads stream): steps of more vectors while the keys are at most one and a half blocks per compute
-// unit and the launch is its longest chain (7 rows at 300 9.7 -> 8.3, at 1,000 9.6 -> 8.6, 8 slots at 300 10.4 -> 9.7;
-// 160 shapes there 9 % faster on average, 7 % slower at worst). Beyond, each tile's pass over the keys shows
-// (keys that are not in the last-level cache: 4 slots of four rows at 8,192 20.4 against 21.7). Softcaps
+// unit and the launch is its longest chain (7 rows at 300 9.7 -> 8.3, at 1,000 9.6 -> 8.6, 8 slots at 300 10.4 -> 9.7).
+// Beyond, each tile's pass over the keys shows (keys that are not in the last-level cache: 4 slots of four rows at 8,192
+// 20.4 against 21.7). Several slots: contexts that kernel leaves whole, and as whole tiles, so up to 16 blocks, 8 from
+// eight KV heads on, where it has twice the workgroups; one slot also split, from 17 blocks on. With the keys out of the
+// caches, split-K -> tiles, 400 positions (13 blocks): 4 KV heads 1 / 3 slots of eight rows 8.8 / 9.7 -> 8.4 / 9.3, 8 KV
+// heads 2 of six 9.2 -> 10.0; a window of 512 (17 blocks): 1 slot of eight rows 9.5 -> 9.0 split (10.6 whole), 2 / 5 of
+// three 9.9 / 10.6 -> 10.8 / 11.5 split (11.4 / 11.8 whole). 160 random steps there 6 % faster on average, 7 % slower at worst,
+// 120 with the keys in the caches 7 and 6 %. Softcaps
 // outside [2, 1024] stay there too: the tiles round the queries with 2 log2(e) / softcap on, the split-K kernel caps the
 // scores, and beyond those the factor takes queries out of f16's range, or into its subnormals, that are inside it there.
 struct KernelChoice {
@@ -793,9 +799,12 @@ KernelChoice choose_tiles(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     const uint32_t group = uint32_t(q_heads / pool->g.kv_heads);
     uint32_t max_rows = 0;
     uint64_t blocks = 0;
+    uint32_t most = 0;
     for (uint32_t i = 0; i < n; ++i) {
         max_rows = std::max(max_rows, in[i].rows);
-        blocks += uint64_t(pool->g.kv_heads) * ((in[i].kv_len + 31) / 32 - in[i].kv_lo / 32);
+        const uint32_t held = (in[i].kv_len + 31) / 32 - in[i].kv_lo / 32;
+        most = std::max(most, held);
+        blocks += uint64_t(pool->g.kv_heads) * held;
     }
     if (!pool->elem_f16 || pool->q_two_halves || n == 0 || n > uint32_t(kMaxBatchItems) ||
         !attn_tiles_f16_supports(pool->g, group, max_rows))
@@ -803,6 +812,7 @@ KernelChoice choose_tiles(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     const bool splitk = takes_splitk_f16(pool, in, n, q_heads, nullptr);
     if (splitk && (prepares || pool->merge_in_launch || pool->die_merge || max_rows * group <= 16 ||
                    (softcap > 0.0f && (softcap < 2.0f || softcap > 1024.0f)) ||
+                   (most > (pool->g.kv_heads >= 8 ? 8u : 16u) && (n > 1 || most <= 16)) ||
                    2 * blocks > 3 * uint64_t(compute_units())))
         return choice;
     const PoolGeom &geom = geom_of(pool, layer);

@@ -107,6 +107,25 @@ def test_steps_of_few_rows_with_a_softcap_far_from_one(kernels, softcap, kernel)
     pool.close()
 
 
+# Steps the split-K kernel takes as well: tiles for contexts of up to 16 blocks (8 from eight KV heads on), beyond them
+# for one slot.
+@pytest.mark.parametrize("slots,rows,ctx,q_heads,kv_heads,kernel", [
+    (2, 3, 509, 32, 4, "tiles_f16"), (2, 3, 510, 32, 4, "splitk_f16"), (1, 3, 510, 32, 4, "tiles_f16"),
+    (1, 5, 251, 32, 8, "tiles_f16"), (1, 5, 252, 32, 8, "splitk_f16"), (2, 5, 252, 32, 8, "splitk_f16"),
+    (1, 5, 507, 32, 8, "splitk_f16"), (1, 5, 508, 32, 8, "tiles_f16"), (2, 5, 508, 32, 8, "splitk_f16")])
+def test_steps_of_few_rows_by_blocks_and_slots(kernels, slots, rows, ctx, q_heads, kv_heads, kernel):
+    rng, pool, caches, refs = setup([ctx] * slots, rows, kv_heads, None, ctx)
+    q, k, v = (normal(rng, slots * rows, w * D) for w in (q_heads, kv_heads, kv_heads))
+    kernels()
+    got = step(pool, caches, rows, q, k, v, q_heads).reshape(slots, -1)
+    assert kernels() == [kernel]
+    for i, ref in enumerate(refs):
+        at = slice(i * rows, (i + 1) * rows)
+        want = oracle.attention_step(ref, 0, q[at], k[at], v[at], q_heads, ctx, threads=8)
+        assert max_abs(got[i], np.asarray(want).reshape(-1)) <= 2e-3
+    pool.close()
+
+
 # Steps of slots with different numbers of rows: a chunk of 128 rows and more beside others goes to the block kernel
 # unless the tiles are estimated to be well ahead; a short one, or a chunk alone, as before.
 @pytest.mark.parametrize("rows,ctxs,kernel", [
