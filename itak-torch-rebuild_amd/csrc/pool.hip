@@ -759,7 +759,7 @@ uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t
 //
 // Against the block kernel the two planners' costs decide; `kBlockLaunch` and `kBlockAppends` put that
 // kernel's walk and merge on the tiles' scale (medians over the shapes the tiles' figures were fitted on). The pick is
-// 1.4 % behind the better of the two kernels there and in two of 549 shapes slower than the block
+// 1.4 % behind the better of the two kernels there, before the margins below, and in two of 549 shapes slower than the block
 // kernel by more than 2 %. 32 Q / 4 KV heads, us a layer, block kernel -> tiles: 61 rows on 0 / 300 / 1,000 12.4 / 17.9 /
 // 19.1 -> 7.5 / 8.9 / 12.3, on a window of 2,048 18.8 -> 15.9; 24 rows on 4,099 18.4 -> 14.1; 128 rows on 1,000
 // 24.5 -> 13.8; 512 rows on 0 20.1 -> 17.1. The block kernel keeps many rows on long contexts (192 rows on 12,000:
@@ -770,10 +770,10 @@ uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t
 // and two, 8 % at most (320 others: one, 4 %). 3 / 31 / 7 decode rows at 500 / 1,500 / 2,000 beside 128 / 128 / 64 rows on 1,000 / 0 /
 // 2,000: 22.0 / 40.1 / 21.8 -> 14.2 / 31.7 / 16.7.
 //
-// Estimates within 5 % of each other are the block kernel's (`kAhead`): near ties on contexts beyond the fit were not
-// ties (71 rows on 18,376 44.0 -> 51.5, 248 on 8,241 at 8 KV heads 55.6 -> 64.4). Over 814 random steps, 176 with the keys
-// out of the caches, the tiles' took 0.742 of the block kernel's time without the margin and eight more than 2 % longer; with
-// it 0.747, and one.
+// Estimates within 8 % of each other are the block kernel's (`kAhead`): near ties on contexts beyond the fit were not
+// ties (71 rows on 18,376 44.0 -> 51.5, 248 on 8,241 at 8 KV heads 55.6 -> 64.4). Over 1,255 random steps, 617 with the keys
+// out of the caches, the tiles took 0.749 of the block kernel's time without the margin, 15 more than 2 % longer and 17 % at
+// worst; with it 0.754, six and 6 %.
 //
 // Against the split-K kernel, whose 16-vector steps are the better ones throughout (the rows come in through
 // LDS, the loads stream): steps of more vectors while the keys are at most one and a half blocks per compute
@@ -822,7 +822,7 @@ KernelChoice choose_tiles(itak_pool *pool, uint64_t layer, const PlanInput *in, 
     start_batch(b, in, n, 0);
     float below = INFINITY;
     if (!splitk) {
-        constexpr float kBlockLaunch = 6.8f, kBlockAppends = 6.4f, kLongBesideOthers = 5.0f, kAhead = 0.95f;
+        constexpr float kBlockLaunch = 6.8f, kBlockAppends = 6.4f, kLongBesideOthers = 5.0f, kAhead = 0.92f;
         uint32_t most_blocks = 0;
         for (uint32_t i = 0; i < n; ++i) most_blocks = std::max(most_blocks, item_block_count(b.item[i]));
         const bool appends = brings_rows && attn_prefill_f16_appends(pool->g, group, max_rows, most_blocks);
