@@ -13,9 +13,10 @@
 // all its vectors (8 MB, and a merge launch that reads them). Here the same block is 124 units of
 // 16 vectors whose eight wavefronts already are an eightfold split, merged in LDS: short contexts stay whole
 // (no partials, no second launch), longer ones are cut in two or four. The price is that a tile reads the keys for
-// 16 (32) vectors where the block kernel's ring feeds 64 (128): what bounds this kernel is the
-// 64 bytes a clock that come into a compute unit through its vector cache, 16 KB in 0.2 us, so
-// long contexts under many rows stay with the block kernel; the planner below weighs the two.
+// 16 (32) vectors where the block kernel's ring feeds 64 (128): long walks are bound by the
+// 64 bytes a clock that come into a compute unit through its vector cache, 16 KB in 0.11 us (`shared` below), so
+// long contexts under many rows stay with the block kernel; the planner below weighs the two. Short ones are mostly what
+// a launch takes whatever it walks (`fixed`, 5.4 to 7.3 us) and, split, the merge launch.
 //
 // New rows (AttnParams::k_new / v_new): the step's own keys and values are read where the caller left
 // them, as f32 straight into the operand registers of the wavefronts whose first block holds them
