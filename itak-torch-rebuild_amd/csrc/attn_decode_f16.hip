@@ -110,7 +110,7 @@ __device__ __forceinline__ void attn_decode_f16_body(const AttnParams &p, const 
     if (N == 1 && PREP)
         asm volatile("" ::"s"(fold.prep_q_weight), "s"(fold.prep_k_weight), "s"(fold.prep_eps), "s"(fold.prep_rot),
                      "s"(fold.prep_interleaved), "s"(fold.prep_freq_step), "s"(fold.prep_freq), "s"(fold.gate));
-    const AttnItem item = b.item[b.find_by_block(blockIdx.x)];
+    const AttnItem item = b.of_block(blockIdx.x);
     const uint32_t local = blockIdx.x - item.block0;
     // Workgroups reach the device in the order of their index and the launch ends with its
     // slowest: the last split of every KV head, which holds the new position and has the most to

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kThreads) void attn_generic_kernel(AttnParams p, At
     const uint32_t tid = threadIdx.x;
 
     // ---- which work item is this workgroup? -------------------------------------
-    const AttnItem item = b.item[b.find_by_block(blockIdx.x)];
+    const AttnItem item = b.of_block(blockIdx.x);
     const uint32_t local = blockIdx.x - item.block0;
     const uint32_t split = local % item.splits;
     const uint32_t rest = local / item.splits;

@@ -130,7 +130,7 @@ __global__ __launch_bounds__(kWaves * 64, D <= 128 ? 2 : 1) void attn_prefill_f1
     ITAK_MARK_BEGIN
     ITAK_MARK(0)
 
-    const AttnItem item = b.item[b.find_by_block(blockIdx.x)];
+    const AttnItem item = b.of_block(blockIdx.x);
     // A query row's heads of one KV group fill `gp` consecutive columns: the group size padded
     // to the next divisor of 16 (a group of 5 takes 8 columns, three of them zero queries whose
     // results are dropped), so that a row never straddles two MFMA tiles.

@@ -75,7 +75,7 @@ __global__ __launch_bounds__(W * 64, DP <= 128 ? 8 / W : 1) void attn_splitk_hal
     const uint32_t g = lane >> 4, jl = lane & 15;
     const uint32_t D = p.g.head_dim, chunks = D / 8;
 
-    const AttnItem item = b.item[b.find_by_block(blockIdx.x)];
+    const AttnItem item = b.of_block(blockIdx.x);
     const uint32_t local = blockIdx.x - item.block0;
     const uint32_t unit = local / item.splits, split = local % item.splits;
     const uint32_t group = p.group, nvec = item.rows * group;

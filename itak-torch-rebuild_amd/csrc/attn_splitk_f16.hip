@@ -429,7 +429,7 @@ __global__ __launch_bounds__(kCombineThreads) void attn_combine_kernel(AttnParam
     const uint32_t D = p.g.head_dim;
     const uint32_t pair = blockIdx.x;
     const uint32_t grow = pair / p.q_heads, head = pair % p.q_heads;
-    const AttnItem item = b.item[b.find_by_row(grow)];
+    const AttnItem item = b.of_row(grow);
     if (item.splits == 1) return;
     const uint32_t row = grow - (item.q_row0 - b.base_row);
     const uint64_t ps0 = item.ws0 + (uint64_t(row) * p.q_heads + head) * item.splits;
@@ -578,7 +578,7 @@ __device__ __forceinline__ void attn_combine128_body(const AttnParams &p, const 
                      "s"(b.base_row), "s"(b.item[0].q_row0), "s"(b.item[0].splits),
                      "s"(b.item[0].ws0));
     if (N == 1 && GATE) asm volatile("" ::"s"(gate));
-    const AttnItem item = b.item[b.find_by_row(grow)];
+    const AttnItem item = b.of_row(grow);
     const uint32_t S = item.splits;
     if (S == 1) return;
     const uint32_t row = grow - (item.q_row0 - b.base_row);
@@ -713,7 +713,7 @@ __global__ __launch_bounds__(256) void attn_combine128_wave_kernel(AttnParams p,
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t head = blockIdx.x * 4 + wave, grow = blockIdx.y;
     if (head >= p.q_heads) return;
-    const AttnItem item = b.item[b.find_by_row(grow)];
+    const AttnItem item = b.of_row(grow);
     const uint32_t S = item.splits;
     if (S == 1) return;
     const uint32_t row = grow - (item.q_row0 - b.base_row);

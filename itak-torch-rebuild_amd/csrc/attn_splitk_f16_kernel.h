@@ -526,13 +526,11 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
         if (idx >= count) return;
         kv_head = die & ((1u << dm.shift) - 1u);
 #pragma unroll 1
-        while (item_at + 1 < item_end && idx >= b.block0[item_at + 1]) ++item_at;
+        while (item_at + 1 < item_end && idx >= b.item[item_at + 1].block0) ++item_at;
         if (tid == 0 && (compute_die() & (kDieCount - 1)) != die)
             __hip_atomic_fetch_add(dm.faults, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-        item_at = b.find_by_block(blockIdx.x);
     }
-    const AttnItem item = b.item[item_at];
+    const AttnItem item = DIE ? b.item[item_at] : b.of_block(blockIdx.x);
     const uint32_t nvec = item.rows * group;
     if constexpr (DIE) {
         split = blockIdx.x / kDieCount - item.block0;

@@ -199,7 +199,7 @@ __global__ __launch_bounds__(WAVES * 64, NQ == 1 && WAVES == 4 ? 3 : 2) void att
         tile_store_new<WAVES * 64>(p, item, kv_head, kb, kplane, kplane + p.g.side_stride);
         return;
     }
-    const AttnItem item = b.item[b.find_by_block(blockIdx.x)];
+    const AttnItem item = b.of_block(blockIdx.x);
     const uint32_t nvec = item.rows * group;
     // Eight units (KV head, split) after eight others, and within the eight a tile after the other:
     // workgroup i runs on compute die i mod 8, so the tiles of a unit, which read the same keys and

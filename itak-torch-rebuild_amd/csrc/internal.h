@@ -314,43 +314,55 @@ struct AttnBatch {
 };
 // The kernel argument form of AttnBatch, sized to the batch: kernel arguments are
 // expensive to read on this GPU (a 2.6 KB argument block costs about a microsecond per
-// launch, a scan through 40-byte items several), so small batches get a small block and
-// the workgroup-to-item search runs over a compact array of first-workgroup indices.
+// launch, a scan through 40-byte items several), so small batches get a small block.
+//
+// A workgroup finds its item in one trip to memory: every lane reads an item, the lanes compare side by side, and
+// the fields come out of the lane that has it. Argument lines are cold at every launch and a trip to one costs 0.3 to 0.5 us;
+// a walk over the items' first indices with the item's fields behind it was one trip an item and two more. One row of
+// each slot, 32 Q / 4 KV heads, us a layer of attention and merge, walk -> this: 2 slots at 2,000 positions 8.2 -> 7.7, 8 at
+// 500 9.0 -> 8.0, 16 of up to 1,000 12.0 -> 10.6, 32 at 300 10.7 -> 8.8, 16 of up to 16,384 58.5 -> 57.1; four slots of seven
+// rows at 8,192 24.4 -> 23.7; f32, 8 KV heads, 6 slots at 900 16.5 -> 15.4.
 template <int N>
 struct AttnBatchT {
     uint32_t n;
     uint32_t total_blocks;
     uint32_t rows_per_block;
     uint32_t base_row;  // q_row0 of item 0
-    uint32_t block0[N];
-    uint32_t row0[N];   // q_row0 - base_row
-    AttnItem item[N];
+    AttnItem item[N];   // (those beyond n hold nothing)
 
     explicit AttnBatchT(const AttnBatch &b)
         : n(b.n), total_blocks(b.total_blocks), rows_per_block(b.rows_per_block),
           base_row(b.n ? b.item[0].q_row0 : 0) {
-        for (int i = 0; i < N; ++i) {
-            const bool live = uint32_t(i) < b.n;
-            item[i] = live ? b.item[i] : AttnItem{};
-            block0[i] = live ? b.item[i].block0 : 0xffffffffu;
-            row0[i] = live ? b.item[i].q_row0 - base_row : 0xffffffffu;
-        }
+        for (uint32_t i = 0; i < b.n; ++i) item[i] = b.item[i];
     }
-    __device__ __forceinline__ uint32_t find_by_block(uint32_t block) const {
-        uint32_t it = 0;
-        if (N > 1) {
-#pragma unroll 1
-            while (it + 1 < n && block >= block0[it + 1]) ++it;
-        }
-        return it;
+    // The item of a workgroup, or of a row of the batch: the last that does not begin beyond it. All lanes of the
+    // wavefront ask together.
+    __device__ __forceinline__ AttnItem of_block(uint32_t block) const {
+        return fetch([=](const AttnItem &x) { return block >= x.block0; });
     }
-    __device__ __forceinline__ uint32_t find_by_row(uint32_t row) const {
-        uint32_t it = 0;
-        if (N > 1) {
-#pragma unroll 1
-            while (it + 1 < n && row >= row0[it + 1]) ++it;
+    __device__ __forceinline__ AttnItem of_row(uint32_t row) const {
+        const uint32_t at = base_row + row;
+        return fetch([=](const AttnItem &x) { return at >= x.q_row0; });
+    }
+
+private:
+    template <typename F>
+    __device__ __forceinline__ AttnItem fetch(F begun) const {
+        if constexpr (N == 1) {
+            return item[0];
+        } else {
+            static_assert(N <= 64 && (N & (N - 1)) == 0, "an item a lane");
+            const uint32_t lane = __lane_id() % N;
+            const AttnItem mine = item[lane];
+            const uint64_t mask = __builtin_amdgcn_ballot_w64(lane < n && begun(mine)) & (N == 64 ? ~0ull : (1ull << N) - 1);
+            const uint32_t at = uint32_t(__builtin_popcountll(mask)) - 1u;
+            AttnItem it;
+#define ITAK_FIELD(f) it.f = __builtin_amdgcn_readlane(mine.f, at)
+            ITAK_FIELD(slot), ITAK_FIELD(rows), ITAK_FIELD(pos0), ITAK_FIELD(q_row0), ITAK_FIELD(kv_len), ITAK_FIELD(splits);
+            ITAK_FIELD(keys_per_split), ITAK_FIELD(block0), ITAK_FIELD(ws0), ITAK_FIELD(splits_magic), ITAK_FIELD(kv_lo);
+#undef ITAK_FIELD
+            return it;
         }
-        return it;
     }
 };
 
