@@ -107,52 +107,69 @@ __device__ __forceinline__ void tile_take_new(BlockOperands &b, const float *kn,
     }
 }
 
-// One 32-key block's new rows of one KV head, converted and stored to the planes by a workgroup.
-template <int THREADS>
+// One 32-key block's new rows of one KV head, converted and stored to the planes by four wavefronts: two take the
+// values, eight keys of four channels a lane, two the keys, eight channels of four rows a lane, every load issued
+// before the first is waited for. A workgroup stores up to kStoreTurns blocks for every four wavefronts it has, one
+// after the other beside the walks of the others: with a workgroup a block, 61 rows on 2,040 positions were 248 tiles
+// and 12 of these on 256 compute units that hold one each, and some ran a second round:
+// 15.4 -> 14.5 us a layer (with a window of 2,048 around them 16.2 -> 15.8); 20 rows on 500 of four slots 9.4 -> 8.9,
+// 61 rows on none 6.3 -> 6.1, 500 on none 15.1 -> 14.7.
+constexpr uint32_t kStoreTurns = 2;
 __device__ __forceinline__ void tile_store_new(const AttnParams &p, const AttnItem &item, uint32_t kv_head, uint32_t kb,
                                                uint16_t *kplane, uint16_t *vplane) {
+    const uint32_t tid = threadIdx.x & 255;
     const uint32_t row_width = p.g.kv_heads * kD;
-    const float *kn = p.k_new + uint64_t(item.q_row0) * row_width + kv_head * kD;
-    const float *vn = p.v_new + uint64_t(item.q_row0) * row_width + kv_head * kD;
     const uint32_t sb = p.ring_blocks ? kb % p.ring_blocks : kb;
-    uint16_t *kdst = kplane + uint64_t(sb) * (kBlockKeys * kD), *vdst = vplane + uint64_t(sb) * (kBlockKeys * kD);
-    const uint32_t pos0 = item.pos0, end = item.pos0 + item.rows;
-#pragma unroll 1
-    for (uint32_t piece = threadIdx.x; piece < 2 * kBlockKeys * kD / 8; piece += THREADS) {
-        uint16_t h[8];
-        if (piece < kBlockKeys * kD / 8) {  // keys: row `kin`, channels 8 * chunk ..
-            const uint32_t kin = piece >> 4, chunk = piece & 15, key = kb * kBlockKeys + kin;
-            if (key < pos0 || key >= end) continue;
-            const float *src = kn + uint64_t(key - pos0) * row_width + chunk * 8;
-            const floatx4 a = *reinterpret_cast<const floatx4 *>(src), c = *reinterpret_cast<const floatx4 *>(src + 4);
+    const uint32_t first = kb * kBlockKeys - item.pos0, rows = item.rows;  // row of the block's first key (may wrap)
+    const uint32_t lane = tid & 127;
+    const uint64_t at = uint64_t(item.q_row0) * row_width + kv_head * kD;
+    floatx4 x[8];
+    if (tid < 128) {  // values: keys 8 * eight .., channels 4 * c ..
+        const uint32_t eight = lane >> 5, c = (lane & 31) * 4;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) h[e] = f32_to_f16_bits(a[e]), h[e + 4] = f32_to_f16_bits(c[e]);
-            const uint32_t kt = (kin >> 2) & 1, ki = (kin >> 3) * 4 + (kin & 3);
-            uint4 w;
-            w.x = h[0] | uint32_t(h[1]) << 16, w.y = h[2] | uint32_t(h[3]) << 16;
-            w.z = h[4] | uint32_t(h[5]) << 16, w.w = h[6] | uint32_t(h[7]) << 16;
-            *reinterpret_cast<uint4 *>(kdst + ((kt * 16 + chunk) * 16 + ki) * 8) = w;
-        } else {  // values: channel c, keys 8 * eight ..
-            const uint32_t x = piece - kBlockKeys * kD / 8, c = x & (kD - 1), eight = x >> 7;
-            const uint32_t key0 = kb * kBlockKeys + eight * 8;
-            uint16_t *dst = vdst + c * kBlockKeys + eight * 8;
-            uint32_t there = 0;
+        for (uint32_t e = 0; e < 8; ++e) {
+            const uint32_t r = first + eight * 8 + e;
+            x[e] = *reinterpret_cast<const floatx4 *>(p.v_new + at + uint64_t(r < rows ? r : 0) * row_width + c);
+        }
+        uint32_t there = 0;
 #pragma unroll
-            for (uint32_t e = 0; e < 8; ++e) {
-                const bool is_new = key0 + e >= pos0 && key0 + e < end;
-                there |= is_new ? 1u << e : 0u;
-                h[e] = f32_to_f16_bits(vn[uint64_t(is_new ? key0 + e - pos0 : 0) * row_width + c]);
-            }
+        for (uint32_t e = 0; e < 8; ++e) there |= first + eight * 8 + e < rows ? 1u << e : 0u;
+        uint16_t *dst = vplane + uint64_t(sb) * (kBlockKeys * kD) + c * kBlockKeys + eight * 8;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint16_t h[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) h[e] = f32_to_f16_bits(x[e][j]);
             if (there == 0xffu) {
                 uint4 w;
                 w.x = h[0] | uint32_t(h[1]) << 16, w.y = h[2] | uint32_t(h[3]) << 16;
                 w.z = h[4] | uint32_t(h[5]) << 16, w.w = h[6] | uint32_t(h[7]) << 16;
-                *reinterpret_cast<uint4 *>(dst) = w;
+                *reinterpret_cast<uint4 *>(dst + j * kBlockKeys) = w;
             } else {
 #pragma unroll
-                for (uint32_t e = 0; e < 8; ++e)
-                    if (there >> e & 1u) dst[e] = h[e];
+                for (int e = 0; e < 8; ++e)
+                    if (there >> e & 1u) dst[j * kBlockKeys + e] = h[e];
             }
+        }
+    } else {  // keys: channels 8 * chunk .. of rows kin, kin + 8, ..
+        const uint32_t chunk = lane & 15;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t r = first + (lane >> 4) + 8 * u;
+            const float *src = p.k_new + at + uint64_t(r < rows ? r : 0) * row_width + chunk * 8;
+            x[2 * u] = *reinterpret_cast<const floatx4 *>(src), x[2 * u + 1] = *reinterpret_cast<const floatx4 *>(src + 4);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t kin = (lane >> 4) + 8 * u, kt = (kin >> 2) & 1, ki = (kin >> 3) * 4 + (kin & 3);
+            uint16_t h[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) h[e] = f32_to_f16_bits(x[2 * u + (e >> 2)][e & 3]);
+            uint4 w;
+            w.x = h[0] | uint32_t(h[1]) << 16, w.y = h[2] | uint32_t(h[3]) << 16;
+            w.z = h[4] | uint32_t(h[5]) << 16, w.w = h[6] | uint32_t(h[7]) << 16;
+            if (first + kin < rows)
+                *reinterpret_cast<uint4 *>(kplane + uint64_t(sb) * (kBlockKeys * kD) + ((kt * 16 + chunk) * 16 + ki) * 8) = w;
         }
     }
 }
@@ -163,7 +180,7 @@ constexpr size_t tiles_lds(int nq, int waves) {
 
 struct TilesExtra {
     const float *gate;    // the output is multiplied by sigmoid(gate) where this launch writes it, or null
-    uint32_t new_blocks;  // blocks that hold new rows, per item at most (0: nothing to append)
+    uint32_t stores;      // workgroups that store an item's new rows, a KV head (0: nothing to append)
     float slack;
 };
 
@@ -187,16 +204,18 @@ __global__ __launch_bounds__(WAVES * 64, NQ == 1 && WAVES == 4 ? 3 : 2) void att
                      "s"(b.total_blocks), "s"(b.item[0].slot), "s"(b.item[0].rows), "s"(b.item[0].pos0),
                      "s"(b.item[0].q_row0), "s"(b.item[0].kv_len), "s"(b.item[0].splits), "s"(b.item[0].keys_per_split),
                      "s"(b.item[0].block0), "s"(b.item[0].ws0), "s"(b.item[0].splits_magic), "s"(b.item[0].kv_lo),
-                     "s"(p.window), "s"(p.ring_blocks), "s"(extra.gate), "s"(extra.new_blocks), "s"(extra.slack));
+                     "s"(p.window), "s"(p.ring_blocks), "s"(extra.gate), "s"(extra.stores), "s"(extra.slack));
     const uint32_t group = p.group, magic = p.group_magic, kv_heads = p.g.kv_heads;
-    if (blockIdx.x >= b.total_blocks) {  // (item, KV head, block) of the new rows, to the planes
-        const uint32_t at = blockIdx.x - b.total_blocks, unit = at / extra.new_blocks;
+    if (blockIdx.x >= b.total_blocks) {  // (item, KV head, some blocks) of the new rows, to the planes
+        const uint32_t at = blockIdx.x - b.total_blocks, unit = at / extra.stores;
         const AttnItem item = b.item[N == 1 ? 0 : unit / kv_heads];
-        const uint32_t kv_head = unit % kv_heads, kb = item.pos0 / kBlockKeys + (at - unit * extra.new_blocks);
-        if (kb * kBlockKeys >= item.pos0 + item.rows) return;
+        const uint32_t kv_head = unit % kv_heads;
         uint16_t *kplane = static_cast<uint16_t *>(const_cast<void *>(p.layer_base)) + item.slot * p.g.slot_stride +
                            kv_head * p.g.head_stride;
-        tile_store_new<WAVES * 64>(p, item, kv_head, kb, kplane, kplane + p.g.side_stride);
+        uint32_t kb = item.pos0 / kBlockKeys + (at - unit * extra.stores) * (WAVES / 4) * kStoreTurns + tid / 256;
+#pragma unroll 1
+        for (uint32_t turn = 0; turn < kStoreTurns && kb * kBlockKeys < item.pos0 + item.rows; ++turn, kb += WAVES / 4)
+            tile_store_new(p, item, kv_head, kb, kplane, kplane + p.g.side_stride);
         return;
     }
     const AttnItem item = b.of_block(blockIdx.x);
@@ -480,7 +499,7 @@ hipError_t launch_tiles(const AttnParams &p, const AttnBatch &b, uint32_t total_
         hipFuncSetAttribute(reinterpret_cast<const void *>(&attn_tiles_f16_kernel<NQ, WAVES, N, RING>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (granted != hipSuccess) return granted;
-    launch_kernel(attn_tiles_f16_kernel<NQ, WAVES, N, RING>, b.total_blocks + b.n * p.g.kv_heads * extra.new_blocks,
+    launch_kernel(attn_tiles_f16_kernel<NQ, WAVES, N, RING>, b.total_blocks + b.n * p.g.kv_heads * extra.stores,
                   WAVES * 64, lds, stream, p, AttnBatchT<N>(b), total_partials, extra);
     return hipGetLastError();
 }
@@ -645,8 +664,9 @@ uint32_t attn_tiles_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, 
 hipError_t launch_attn_tiles_f16(const AttnParams &p, const AttnBatch &b, uint32_t total_partials, const float *gate,
                                  hipStream_t stream) {
     if (b.total_blocks == 0) return hipSuccess;
-    const TilesExtra extra{gate, p.k_new ? most_new_blocks(b) : 0, b.tile_exact ? 0.0f : kTileSlack};
-    if (extra.new_blocks > b.tile_waves) return hipErrorInvalidValue;  // (the planner brings no more)
+    const uint32_t new_blocks = p.k_new ? most_new_blocks(b) : 0, stored = b.tile_waves / 4 * kStoreTurns;
+    if (new_blocks > b.tile_waves) return hipErrorInvalidValue;  // (the planner brings no more)
+    const TilesExtra extra{gate, (new_blocks + stored - 1) / stored, b.tile_exact ? 0.0f : kTileSlack};
     hipError_t e = hipSuccess;
 #define ITAK_TILES(NQ, W)                                                                          \
     do {                                                                                           \

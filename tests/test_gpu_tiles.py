@@ -89,6 +89,14 @@ def test_against_the_oracle(kernels, ctxs, rows, q_heads, kv_heads, window, soft
     pool.close()
 
 
+# New rows of more blocks than a workgroup of eight (four) wavefronts stores, first and last block begun or full.
+@pytest.mark.parametrize("ctxs,rows,q_heads,kv_heads", [
+    ([500], 200, 32, 4), ([1005], 140, 16, 4), ([480], 256, 8, 4), ([511], 129, 32, 4), ([600, 37], 130, 16, 4),
+    ([1], 65, 16, 2)])
+def test_new_rows_of_many_blocks(kernels, ctxs, rows, q_heads, kv_heads):
+    test_against_the_oracle(kernels, ctxs, rows, q_heads, kv_heads, None, 0.0)
+
+
 # A softcap far from one: steps that the split-K kernel takes as well stay with it, whose queries do not carry
 # 2 log2(e) / softcap into their rounding (a factor of 261 on queries of some hundreds at the smallest one here).
 @pytest.mark.parametrize("softcap,kernel", [(2.0 ** -10, "splitk_f16"), (1.9, "splitk_f16"), (2.0, "tiles_f16"),
