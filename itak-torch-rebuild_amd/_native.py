@@ -10,6 +10,7 @@ import os
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libitak_hip_kv.so")
+FRONT_PATH = os.path.join(HERE, "lib", "_itak_front.so")
 
 OK = 0
 STATUS_NAMES = {
@@ -197,6 +198,22 @@ PROTOTYPES = {
 }
 
 _lib = None
+
+
+def load_front(lib, cache_type):
+    """The module of the calls made per layer and per round (csrc/front.cpp), bound to `lib`."""
+    import importlib.machinery
+    import importlib.util
+
+    if not os.path.exists(FRONT_PATH):
+        raise ImportError(f"{FRONT_PATH} is missing: build it with `python {os.path.join(HERE, 'build.py')}`.")
+    loader = importlib.machinery.ExtensionFileLoader("_itak_front", FRONT_PATH)
+    front = importlib.util.module_from_spec(importlib.util.spec_from_loader("_itak_front", loader))
+    loader.exec_module(front)
+    front.bind(cache_type, *(C.cast(getattr(lib, name), C.c_void_p).value for name in (
+        "itak_attention_step_device", "itak_attention_prep_step_device", "itak_kv_truncate",
+        "itak_compute_attention", "itak_gqa_attention")))
+    return front
 
 
 def load():

@@ -17,6 +17,8 @@ LIB_PATH = os.path.join(LIB_DIR, "libitak_hip_kv.so")
 TIMELINE_LIB_PATH = os.path.join(LIB_DIR, "libitak_hip_kv_timeline.so")
 OBJ_DIR = os.path.join(HERE, "build")
 
+FRONT_PATH = os.path.join(LIB_DIR, "_itak_front.so")
+
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # Packed FP32 VALU forms are kept off: ordinary float code must compile to scalar FP32 ops.
@@ -68,6 +70,23 @@ def _compile(src: str, timeline: bool = False) -> str:
     return obj
 
 
+def build_front() -> str:
+    """Compiles csrc/front.cpp, the Python module of the per-layer calls, for this interpreter."""
+    import sysconfig
+
+    import numpy
+
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           f"-I{sysconfig.get_paths()['include']}", f"-I{numpy.get_include()}",
+           os.path.join(CSRC, "front.cpp"), "-o", FRONT_PATH]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on front.cpp:\n{res.stderr}")
+    if res.stderr.strip():
+        sys.stderr.write(res.stderr + "\n")
+    return FRONT_PATH
+
+
 def build(verbose: bool = False, timeline: bool = False) -> str:
     """Builds lib/libitak_hip_kv.so; with `timeline`, lib/libitak_hip_kv_timeline.so instead: the
     same library with stage timestamps compiled into the attention kernels (csrc/timeline.h),
@@ -76,6 +95,8 @@ def build(verbose: bool = False, timeline: bool = False) -> str:
     os.makedirs(OBJ_DIR + ("_timeline" if timeline else ""), exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     srcs = sources()
+    if not timeline:
+        build_front()
     with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as pool:
         objs = list(pool.map(lambda src: _compile(src, timeline), srcs))
     lib_path = TIMELINE_LIB_PATH if timeline else LIB_PATH

@@ -205,6 +205,15 @@ def _ptr(a: Optional[np.ndarray]):
 
 _ITEM_PACK = {}
 _NAN = math.nan
+_front = None  # csrc/front.cpp's module, once a pool has loaded the library
+
+
+def _load():
+    global _front
+    lib = N.load()
+    if _front is None:
+        _front = N.load_front(lib, KvCache)
+    return lib
 
 
 class KvPool:
@@ -253,11 +262,13 @@ class KvPool:
         cfg.ring_headroom = ring_headroom
         handle = C.c_void_p()
         self._h = None
-        self._lib = N.load()
+        self._hv = 0  # the handle as the front module takes it
+        self._lib = _load()
         status = self._lib.itak_pool_create(C.byref(cfg), C.byref(handle))
         if status != N.OK:
             _raise_last(None)
         self._h = handle
+        self._hv = handle.value
         self.num_kv_heads = num_kv_heads
         self.head_dim = head_dim
         self.row = num_kv_heads * head_dim
@@ -266,6 +277,7 @@ class KvPool:
         if self._h:
             self._lib.itak_pool_destroy(self._h)
             self._h = None
+            self._hv = 0
 
     def __del__(self):
         try:
@@ -314,10 +326,12 @@ class KvPool:
                               out_ptr: int, num_q_heads: int, scale: Optional[float] = None,
                               softcap: float = 0.0) -> None:
         """Append each item's rows, then attend causally; device pointers, pool's stream."""
-        raw, n = self._items(items)
-        status = self._lib.itak_attention_step_device(
-            self._h, layer, raw, n, q_ptr, k_ptr, v_ptr, out_ptr, num_q_heads,
-            _NAN if scale is None else scale, softcap)
+        status = _front.step(self._hv, layer, items, q_ptr, k_ptr, v_ptr, out_ptr, num_q_heads, scale, softcap)
+        if status < 0:  # arguments that the front module leaves to ctypes
+            raw, n = self._items(items)
+            status = self._lib.itak_attention_step_device(
+                self._h, layer, raw, n, q_ptr, k_ptr, v_ptr, out_ptr, num_q_heads,
+                _NAN if scale is None else scale, softcap)
         if status:
             _raise_last(self._h)
 
@@ -338,12 +352,15 @@ class KvPool:
                                    scale: float = float("nan"), softcap: float = 0.0) -> None:
         """Per-head RMSNorm + RoPE of the raw Q/K projections, append, attention, gate: the
         steps of muse-glimmer/src/model.rs:445-464 around Compute::attention, device tensors."""
-        arr, n = self._items(items)
-        prep = N.PrepParams(q_norm_ptr or None, k_norm_ptr or None, eps, rope_base,
-                            1 if interleaved else 0, rotary_dim)
-        status = self._lib.itak_attention_prep_step_device(
-            self._h, layer, arr, n, q_ptr, k_ptr, v_ptr, gate_ptr or None, out_ptr, num_q_heads,
-            scale, softcap, C.byref(prep))
+        status = _front.prep_step(self._hv, layer, items, q_ptr, k_ptr, v_ptr, gate_ptr, out_ptr, num_q_heads, scale,
+                                  softcap, q_norm_ptr, k_norm_ptr, eps, rope_base, interleaved, rotary_dim)
+        if status < 0:
+            arr, n = self._items(items)
+            prep = N.PrepParams(q_norm_ptr or None, k_norm_ptr or None, eps, rope_base,
+                                1 if interleaved else 0, rotary_dim)
+            status = self._lib.itak_attention_prep_step_device(
+                self._h, layer, arr, n, q_ptr, k_ptr, v_ptr, gate_ptr or None, out_ptr, num_q_heads,
+                scale, softcap, C.byref(prep))
         if status:
             _raise_last(self._h, "attention")
 
@@ -360,6 +377,11 @@ class KvPool:
         _check(self._h, self._lib.itak_kv_append_device(self._h, layer, raw, n, k_ptr, v_ptr))
 
     def truncate(self, slots, new_lengths) -> None:
+        status = _front.truncate(self._hv, slots, new_lengths)
+        if status >= 0:
+            if status:
+                _raise_last(self._h)
+            return
         n = len(slots)
         s = array("I", [x.slot if isinstance(x, KvCache) else int(x) for x in slots])
         try:
@@ -426,6 +448,7 @@ class KvCache:
         self._owns_pool = owns_pool
         self._lib = pool._lib
         self._h = pool._h
+        self._hv = pool._hv
 
     @staticmethod
     def new(pattern: Sequence[LayerKind], num_kv_heads: int, head_dim: int, *, elem: str = "f32",
@@ -619,6 +642,12 @@ class CacheView:
 def gqa_attention(q, num_queries: int, num_q_heads: int, query_positions: Sequence[int],
                   view: CacheView, params: AttentionParams = AttentionParams()) -> np.ndarray:
     """attention::gqa_attention (attention.rs:104-215) on the device; flat f32 output."""
+    c = view._c
+    got = _front.gqa(c._hv, c.slot, view._layer, q, num_queries, num_q_heads, query_positions, params.scale, params.softcap)
+    if got.__class__ is not int:
+        return got if num_queries else got[:0]
+    if got >= 0:
+        _raise_last(c._h)
     q = _as_f32(q)
     try:
         pos = array("Q", query_positions)
@@ -627,7 +656,6 @@ def gqa_attention(q, num_queries: int, num_q_heads: int, query_positions: Sequen
         pos = np.asarray(query_positions, dtype=np.uint64).reshape(-1)
         pos_ptr, pos_size = _ptr(pos), pos.size
     out = np.empty(q.size, dtype=_F32)  # every element is written, or the call raises
-    c = view._c
     status = c._lib.itak_gqa_attention(
         c._h, c.slot, view._layer, _ptr(q), q.size, num_queries, num_q_heads, pos_ptr if pos_size else None,
         pos_size, _NAN if params.scale is None else float(params.scale), float(params.softcap), _ptr(out))
@@ -754,7 +782,9 @@ class HipCompute:
         if kind is not req.kind and kind != req.kind:
             raise StepFailed(step, f"request kind {req.kind} does not match the config's kind for "
                                    f"layer {req.layer}")
-        q, k, v = _as_f32(req.q), _as_f32(req.k), _as_f32(req.v)
+        q, k, v = req.q, req.k, req.v
+        if not (q.__class__ is k.__class__ is v.__class__ is np.ndarray and q.dtype is k.dtype is v.dtype is _F32):
+            q, k, v = _as_f32(q), _as_f32(k), _as_f32(v)
         if self._shape is None:
             self._build(cfg, step)
         elif ((self._layers != cfg.layers or self._widths != (cfg.kv_heads, cfg.key_length, cfg.value_length,
@@ -763,8 +793,15 @@ class HipCompute:
             raise StepFailed(step, "this HipCompute already serves a model of a different shape; "
                                    "construct a fresh HipCompute per model (or reset this one) "
                                    "instead of retargeting it mid-sequence")
-        out = np.empty(q.size, dtype=_F32)  # every element is written, or the call raises
         c = self._cache
+        got = _front.compute(c._hv, c.slot, req.layer, q, k, v, cfg.q_heads, cache.position(), self._softcap,
+                             cfg.rope_freq_base_swa)
+        if got.__class__ is not int:
+            return got
+        if got >= 0:
+            _raise_last(c._h, step)
+        q, k, v = _as_f32(q), _as_f32(k), _as_f32(v)
+        out = np.empty(q.size, dtype=_F32)  # every element is written, or the call raises
         status = c._lib.itak_compute_attention(
             c._h, c.slot, req.layer, _ptr(q), q.size, _ptr(k), k.size, _ptr(v), v.size,
             cfg.q_heads, cache.position(), self._softcap, cfg.rope_freq_base_swa, _ptr(out))
