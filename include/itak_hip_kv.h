@@ -442,8 +442,8 @@ itak_status itak_kv_capture_itkv_f16(itak_pool *pool, uint32_t slot, const char 
    an f32 pool): the snapshot's geometry must be the pool's, and, when expected_fingerprint is not
    NULL, its fingerprint the expected one. A payload of 128 KB and more goes to a device buffer of
    its own size (and up to 16 MB beside it where f32 rows cross the link to an f16 pool as halves, which
-   they do chunk by chunk where that loses nothing) for the length of the call, is summed there (version 1; version 2 by host threads
-   meanwhile) and gathered from there once the sum is known good; where that buffer cannot be had,
+   they do chunk by chunk where that loses nothing) for the length of the call, is summed there
+   and gathered from there once the sum is known good; where that buffer cannot be had,
    and below that size, the host sums, and the rows are gathered from `bytes` in place when the device
    can read them there (pinned memory, 4-byte aligned payload), otherwise staged. An f32 snapshot into
    an f16 pool converts exactly as append does. */

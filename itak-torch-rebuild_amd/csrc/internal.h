@@ -188,6 +188,11 @@ hipError_t launch_read_runs(const void *base, const void *base_w, int elem_f16, 
 constexpr uint32_t kFnvRun = 64;
 uint64_t fnv_scratch_bytes(uint64_t bytes);
 hipError_t launch_fnv(const void *data, uint64_t bytes, void *scratch, unsigned long long *state, hipStream_t stream);
+// The sums of a file's 1 MiB blocks, states[k] = FNV-1a of block k, piece by piece and in order: `bytes` bytes of the
+// file from file_at on (a multiple of kFnvRun but for the last piece). A block that begins in the piece starts there; one
+// that does not goes on from states[k], which for the file's first block the caller sets.
+hipError_t launch_fnv_blocks(const void *data, uint64_t bytes, uint64_t file_at, void *scratch, unsigned long long *states,
+                             hipStream_t stream);
 
 // ---- ring rows aside and back (checkpoints deeper than a ring's headroom) -----------------
 // Copies rows of windowed layers between their rings and a side buffer that holds, per entry,

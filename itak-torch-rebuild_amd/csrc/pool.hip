@@ -2112,9 +2112,10 @@ itak_status itak_kv_capture_itkv_f16(itak_pool *pool, uint32_t slot, const char 
 }
 
 // A snapshot's payload passes through device memory this many bytes at a time (a multiple of the
-// ring's chunk and of the hash's runs). From kDeviceSumBytes on version 1's checksum is the
+// ring's chunk and of the hash's runs). From kDeviceSumBytes on the checksum is the
 // device's: the ten launches take 40 us there, what a host core needs for 48 KiB, and the rule
-// leaves a margin for their coming one behind the other on a busy stream.
+// leaves a margin for their coming one behind the other on a busy stream. (Version 2's was
+// the host threads' until its blocks' sums came to the device: fnv_kernels.hip.)
 constexpr uint64_t kPayloadPiece = 32ull << 20;
 constexpr uint64_t kDeviceSumBytes = 128ull << 10;
 static_assert(kPayloadPiece == kRingChunk * kRingSlots && kRingChunk % kFnvRun == 0, "pieces are whole chunks and runs");
@@ -2126,6 +2127,10 @@ static void advise_huge_pages(void *p, uint64_t bytes) {
     const uint64_t from = align_up(reinterpret_cast<uint64_t>(p), huge), to = (reinterpret_cast<uint64_t>(p) + bytes) / huge * huge;
     if (to > from && to - from >= 4 * huge) (void)madvise(reinterpret_cast<void *>(from), to - from, MADV_HUGEPAGE);
 }
+
+// Version 2's block sums can be made on the device where the header ends in the first block.
+static uint64_t sum_blocks(uint64_t file_bytes) { return (file_bytes + kItkvSumBlock - 1) / kItkvSumBlock; }
+static bool device_sums(uint32_t version, uint64_t payload_at) { return version == kItkvVersion || payload_at < kItkvSumBlock; }
 
 static itak_status finish_capture(uint8_t *bytes, uint64_t total, uint32_t version, bool with_checksum,
                                   const uint64_t *known) {
@@ -2186,15 +2191,18 @@ static itak_status capture_itkv(itak_pool *pool, uint32_t slot, const char *fing
     // summed there when the trailer is version 1's, and goes out through the pinned ring.
     const uint64_t payload = ls[0].keys_offset, payload_bytes = total - 8 - payload;
     const uint64_t piece = std::min(align_up(payload_bytes, 256), kPayloadPiece);
-    const bool device_sum = with_checksum && h.version == kItkvVersion && payload_bytes >= kDeviceSumBytes;
+    const bool device_sum = with_checksum && payload_bytes >= kDeviceSumBytes && device_sums(h.version, payload);
+    const uint64_t blocks = device_sum && h.version != kItkvVersion ? sum_blocks(total - 8) : 0;
     // f32 rows of an f16 pool cross the link as the halves they are and are widened by the host threads that
     // empty the ring (16 layers of 2,000 rows: 4.0 -> 3.05 ms); the sum is over f32 rows made beside them.
     const bool widen = !f16_rows && pool->elem_f16 && host_has_f16();
     const uint64_t halves_bytes = widen ? align_up(piece / 2, 256) : 0;
-    itak_status st = ensure_stage(pool, piece + 256 + halves_bytes + (device_sum ? fnv_scratch_bytes(piece) : 0));
+    const uint64_t scratch_bytes = device_sum ? fnv_scratch_bytes(piece) : 0;
+    itak_status st = ensure_stage(pool, piece + 256 + halves_bytes + scratch_bytes + blocks * 8);
     if (st != ITAK_OK) return st;
-    unsigned long long *state = reinterpret_cast<unsigned long long *>(pool->stage);
     unsigned char *rows_dev = pool->stage + 256, *halves_dev = rows_dev + piece, *scratch = halves_dev + halves_bytes;
+    // (Version 1's one chain, or version 2's of each block.)
+    unsigned long long *state = reinterpret_cast<unsigned long long *>(blocks ? scratch + scratch_bytes : pool->stage);
     advise_huge_pages(bytes, total);
     if (device_sum)
         HIP_TRY(pool, launch_fill_words(state, 1, fnv1a64(bytes, payload, kFnvOffset), pool->stream), "start checksum");
@@ -2229,7 +2237,9 @@ static itak_status capture_itkv(itak_pool *pool, uint32_t slot, const char *fing
                 b.n = 0;
             }
         }
-        return device_sum ? launch_fnv(rows_dev, bytes_here / kFnvRun * kFnvRun, scratch, state, pool->stream) : hipSuccess;
+        if (!device_sum) return hipSuccess;
+        return blocks ? launch_fnv_blocks(rows_dev, bytes_here, payload + at, scratch, state, pool->stream)
+                      : launch_fnv(rows_dev, bytes_here / kFnvRun * kFnvRun, scratch, state, pool->stream);
     };
     HIP_TRY(pool,
             ring_download(pool->ring, bytes + payload, payload_bytes, pool->stream, widen,
@@ -2240,9 +2250,14 @@ static itak_status capture_itkv(itak_pool *pool, uint32_t slot, const char *fing
                           }),
             "download snapshot rows");
     if (!device_sum) return finish_capture(bytes, total, h.version, with_checksum, nullptr);
-    uint64_t sum = 0;
-    HIP_TRY(pool, hipMemcpyAsync(&sum, state, 8, hipMemcpyDeviceToHost, pool->stream), "download checksum");
+    std::vector<uint64_t> sums(std::max<uint64_t>(blocks, 1));
+    HIP_TRY(pool, hipMemcpyAsync(sums.data(), state, sums.size() * 8, hipMemcpyDeviceToHost, pool->stream), "download checksum");
     HIP_TRY(pool, hipStreamSynchronize(pool->stream), "synchronize after readback");
+    uint64_t sum = sums[0];
+    if (blocks) {
+        sum = fnv1a64_of_sums(sums.data(), blocks);
+        return finish_capture(bytes, total, h.version, true, &sum);
+    }
     const uint64_t tail = payload_bytes % kFnvRun;  // only the last piece can have one
     sum = fnv1a64(bytes + total - 8 - tail, tail, sum);
     return finish_capture(bytes, total, h.version, true, &sum);
@@ -2281,13 +2296,15 @@ itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *byt
     std::vector<ItkvLayer> ls;
     ItkvError err;
     const uint8_t *b8 = static_cast<const uint8_t *>(bytes);
-    // From kDeviceSumBytes on the payload goes to the device first, is summed there (version 1) or
-    // by host threads meanwhile (version 2), and is gathered from there once the sum is known good.
+    // From kDeviceSumBytes on the payload goes to the device first, is summed there, and is gathered from there
+    // once the sum is known good.
     DeviceBuffer rows;
     hipError_t moved = hipSuccess;
     const ItkvSum sum_of = [&](const ItkvHeader &header, uint64_t payload) -> uint64_t {
         const uint64_t n = len - 8 - payload, piece = std::min(align_up(n, 256), kPayloadPiece);
-        const bool device_sum = header.version == kItkvVersion;
+        const bool device_sum = device_sums(header.version, payload);
+        const uint64_t blocks = header.version != kItkvVersion && device_sum ? sum_blocks(len - 8) : 0;
+        const uint64_t scratch_bytes = device_sum ? fnv_scratch_bytes(piece) : 0;
         // Rows that an f16 pool wrote are halves again on their way over the link (ring_upload_narrow), and
         // f32 in device memory as the sum and the gather want them (16 layers of 2,000 rows: 3.9 -> 2.7 ms).
         const bool pinned = kind == PtrKind::PinnedHost;
@@ -2296,18 +2313,21 @@ itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *byt
         constexpr uint64_t kNarrowBytes = 3ull << 20;
         LoadRoom room;
         if (n < kDeviceSumBytes ||
-            !take_load_room(n, piece, device_sum ? fnv_scratch_bytes(piece) : 0,
-                            device_sum && pool->elem_f16 && !pinned && n >= kNarrowBytes && host_has_f16(),
+            !take_load_room(n, piece, scratch_bytes + blocks * 8,
+                            header.version == kItkvVersion && pool->elem_f16 && !pinned && n >= kNarrowBytes && host_has_f16(),
                             [&](uint64_t want) { return rows.make(want) == hipSuccess; }, room))
             return itkv_trailer(header.version, b8, len - 8);
         const bool narrow = room.halves_bytes != 0;
-        unsigned long long *state = reinterpret_cast<unsigned long long *>(rows.p + room.state_at);
+        unsigned long long *state = reinterpret_cast<unsigned long long *>(
+            rows.p + (blocks ? room.scratch_at + scratch_bytes : room.state_at));
         if (device_sum)
             moved = launch_fill_words(state, 1, fnv1a64(b8, payload, kFnvOffset), pool->stream);
         uint64_t summed = 0;
         const auto sum_up_to = [&](uint64_t sent) -> hipError_t {
             if (!device_sum || (sent < n && sent - summed < kPayloadPiece)) return hipSuccess;
-            hipError_t e = launch_fnv(rows.p + summed, (sent - summed) / kFnvRun * kFnvRun, rows.p + room.scratch_at, state, pool->stream);
+            unsigned char *scratch = rows.p + room.scratch_at;
+            hipError_t e = blocks ? launch_fnv_blocks(rows.p + summed, sent - summed, payload + summed, scratch, state, pool->stream)
+                                  : launch_fnv(rows.p + summed, (sent - summed) / kFnvRun * kFnvRun, scratch, state, pool->stream);
             summed = sent;
             return e;
         };
@@ -2328,14 +2348,14 @@ itak_status itak_kv_restore_itkv(itak_pool *pool, uint32_t slot, const void *byt
         } else if (moved == hipSuccess) {
             moved = ring_upload(pool->ring, {RingSpan{b8 + payload, rows.p, n}}, pool->stream, sum_up_to);
         }
-        uint64_t sum = 0;
-        if (!device_sum) sum = itkv_trailer(header.version, b8, len - 8);
+        std::vector<uint64_t> sums(std::max<uint64_t>(blocks, 1));
+        if (!device_sum) sums[0] = itkv_trailer(header.version, b8, len - 8);
         if (moved == hipSuccess && device_sum)
-            moved = hipMemcpyAsync(&sum, state, 8, hipMemcpyDeviceToHost, pool->stream);
+            moved = hipMemcpyAsync(sums.data(), state, sums.size() * 8, hipMemcpyDeviceToHost, pool->stream);
         const hipError_t done = hipStreamSynchronize(pool->stream);
         if (moved == hipSuccess) moved = done;
-        if (device_sum) sum = fnv1a64(b8 + len - 8 - n % kFnvRun, n % kFnvRun, sum);
-        return sum;
+        if (blocks) return fnv1a64_of_sums(sums.data(), blocks);
+        return device_sum ? fnv1a64(b8 + len - 8 - n % kFnvRun, n % kFnvRun, sums[0]) : sums[0];
     };
     const bool decoded = itkv_decode(b8, len, h, ls, err, nullptr, sum_of);
     if (moved != hipSuccess) return hip_error(pool->err, moved, "move snapshot rows to the device");
