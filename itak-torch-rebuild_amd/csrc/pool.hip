@@ -2113,7 +2113,7 @@ itak_status itak_kv_capture_itkv_f16(itak_pool *pool, uint32_t slot, const char 
 
 // A snapshot's payload passes through device memory this many bytes at a time (a multiple of the
 // ring's chunk and of the hash's runs). From kDeviceSumBytes on the checksum is the
-// device's: the ten launches take 40 us there, what a host core needs for 48 KiB, and the rule
+// device's: its six launches take 30 us there, what a host core needs for 36 KiB, and the rule
 // leaves a margin for their coming one behind the other on a busy stream. (Version 2's was
 // the host threads' until its blocks' sums came to the device: fnv_kernels.hip.)
 constexpr uint64_t kPayloadPiece = 32ull << 20;

@@ -13,9 +13,8 @@ constexpr uint32_t kRingSlots = 8;
 // `bytes` bytes cut into chunks of kRingChunk, one at the end that the link waits for in four and its neighbour in two:
 // the first of an upload, the last of a download. fn(at, n) for each in order. Runs of few chunks stay as they are: every
 // chunk more is a helper more to start, and a single chunk is moved by the calling thread (1.9 MB loaded 231 us in one,
-// 264 in two). Uploads of bytes as they lie only from nine chunks on: up to eight are a thread each, and version 2 loads,
-// whose sum the host's threads begin when the upload's are done, took 5 to 10 % longer with theirs cut (16 layers of
-// 520 / 640 / 900 rows 1.39 / 1.51 / 1.71 -> 1.33 / 1.38 / 1.49 ms); halves, which are narrowed on the way, from five.
+// 264 in two). Uploads of bytes as they lie only from nine chunks on: up to eight are a thread each, and version 2
+// loads took 4 % longer with theirs cut (16 layers of 520 / 700 rows, least of 50, 0.87 / 1.00 -> 0.83 / 0.96 ms); halves, which are narrowed on the way, from five.
 enum class RampAt { First, FirstOfMany, Last };
 template <class F>
 void ring_cut(uint64_t bytes, RampAt ramp_at, F fn) {
