@@ -178,8 +178,8 @@ __device__ __forceinline__ void accumulate_by_row(floatx4 (&o)[8], const BlockOp
 // hi), and every score is K.hi + K.lo: the queries' rounding to f16, which is relative to each
 // channel and so grows with the scores, leaves the scores (the keys are exact, they are stored
 // as f16). The low halves are read from LDS (sm_q_lo) block by block.
-template <int NQ, bool FIRST, bool RING, bool BYROW, bool QLO>
-__device__ __forceinline__ void process_block(WaveState<NQ> &st, BlockOperands &b,
+template <int NQ, bool FIRST, bool RING, bool BYROW, bool QLO, typename NextKeys>
+__device__ __forceinline__ void process_block(WaveState<NQ> &st, BlockOperands &b, [[maybe_unused]] NextKeys next_keys,
                                               const half8 *qreg, const _Float16 *sm_q,
                                               [[maybe_unused]] const _Float16 *sm_q_lo,
                                               uint32_t kb, uint32_t g, uint32_t jl,
@@ -315,6 +315,7 @@ __device__ __forceinline__ void process_block(WaveState<NQ> &st, BlockOperands &
         }
     }
     if constexpr (NQ > 2) {
+        next_keys();
         if (tail) zero_tail();
         // (The values are looked at after the tail is cleared: what lies past the stored rows
         // is nobody's to see.)
@@ -763,6 +764,9 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
     WaveState<NQ> st;
     const RowSpan span{item.pos0, row_first, row_last + 1, vec0, window, kv_lo, magic, fused, new_not_finite};
     if constexpr (!TILED) {
+    [[maybe_unused]] auto next_keys = [&] {
+        if (kb + WAVES < kb_end) load_block_keys(buf_a, kplane, storage_block(kb + WAVES, ring_blocks), g, jl);
+    };
 #define ITAK_BLOCK(FIRST, BUF, KB)                                                               \
     do {                                                                                         \
         if (fused && ((KB) + 1) * kBlockKeys > item.pos0)                                        \
@@ -772,17 +776,17 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
            same keys, so that every other block runs code that knows nothing of it. */        \
         if constexpr (NQ > 2) { /* (no room for two copies beside 128 accumulators; the one copy  \
            costs the 7-row verify block 3 %: 23.7 -> 24.5 us per layer, same box) */             \
-            process_block<NQ, FIRST, RING, true, QLO>(st, BUF, qreg, sm_q, sm_q_lo, KB, g, jl, colpos, \
+            process_block<NQ, FIRST, RING, true, QLO>(st, BUF, next_keys, qreg, sm_q, sm_q_lo, KB, g, jl, colpos, \
                                  collo, first_pos, seen_end, lo_min,    \
                                  lo_max, softcap, inv_cap, span);                                \
         } else if (WAVES != 8 && row_last > row_first &&                                         \
             (((KB) + 1) * kBlockKeys > first_pos + 1 ||                                          \
              (RING && (KB) * kBlockKeys < lo_max)))                                              \
-            process_block<NQ, FIRST, RING, WAVES != 8, QLO>(st, BUF, qreg, sm_q, sm_q_lo, KB, g, jl, colpos, \
+            process_block<NQ, FIRST, RING, WAVES != 8, QLO>(st, BUF, next_keys, qreg, sm_q, sm_q_lo, KB, g, jl, colpos, \
                                  collo, first_pos, seen_end, lo_min,    \
                                  lo_max, softcap, inv_cap, span);                                \
         else                                                                                     \
-            process_block<NQ, FIRST, RING, false, QLO>(st, BUF, qreg, sm_q, sm_q_lo, KB, g, jl, colpos, collo, \
+            process_block<NQ, FIRST, RING, false, QLO>(st, BUF, next_keys, qreg, sm_q, sm_q_lo, KB, g, jl, colpos, collo, \
                                  first_pos, seen_end, lo_min, lo_max,   \
                                  softcap, inv_cap, span);                                        \
     } while (0)
@@ -804,9 +808,12 @@ __device__ __forceinline__ void attn_splitk_f16_body(const AttnParams &p, const 
                 ITAK_BLOCK(false, buf_a, kb3);
             }
         } else {
+            // The next block's keys are asked for when the scores of all tiles have used this one's, its values when
+            // the products have. (Both behind the products, a wavefront had nothing on its way while it multiplied: 4
+            // slots of seven rows at 8,192 23.7 -> 22.7 us a layer, 8 of six 33.3 -> 32.5, 2 of eight at 30,000 32.1 -> 31.2.)
             ITAK_BLOCK(true, buf_a, kb);
             for (kb += WAVES; kb < kb_end; kb += WAVES) {
-                load_block(buf_a, kplane, vplane, storage_block(kb, ring_blocks), g, jl);
+                load_block_values(buf_a, vplane, storage_block(kb, ring_blocks), g, jl);
                 ITAK_BLOCK(false, buf_a, kb);
             }
         }
