@@ -558,6 +558,76 @@ __device__ __forceinline__ float split_lanes_sum(float v) {
     const auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(c[0]) + __uint_as_float(c[1]);
 }
+// Partials of one (row, head) from split s0 on, U per lane: split s0 + sl + u * SL. Only the last of them can lie beyond
+// the S splits; it then reads the last split's partial again, weighs nothing and is cleared, or a value in it that is not finite
+// (which the rows that see the key are due) would make the product NaN. Every load is issued before the first is
+// waited for, and all addresses are 32-bit offsets from the pair's own.
+struct Merge {
+    float m = -INFINITY, l = 0.0f;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+};
+template <int U, int SL, bool FIRST, bool BASE2, bool ONCE>
+__device__ __forceinline__ void merge_trip(Merge &r, const float *acc_at, const float *ml_at, uint32_t dim, uint32_t c4,
+                                           uint32_t sl, uint32_t s0, uint32_t S) {
+    typedef float f4v __attribute__((ext_vector_type(4)));
+    f4v x[U];
+    float2 ml[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t at = s0 + sl + u * SL, s = u + 1 < U ? at : min(at, S - 1);
+        const f4v *from = reinterpret_cast<const f4v *>(reinterpret_cast<const char *>(acc_at) + (s * dim + c4) * 4u);
+        x[u] = ONCE ? __builtin_nontemporal_load(from) : *from;
+        ml[u] = *reinterpret_cast<const float2 *>(reinterpret_cast<const char *>(ml_at) + s * 8u);
+    }
+    // (Nothing below may move above this line and no load below it: left to itself the scheduler issues half of the
+    // accumulator loads after the first weights are computed.)
+    if (!ONCE) __builtin_amdgcn_sched_barrier(0);
+    const bool there = s0 + sl + (U - 1) * SL < S;
+    ml[U - 1].x = there ? ml[U - 1].x : -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[U - 1][e] = there ? x[U - 1][e] : 0.0f;
+    float mx = FIRST ? ml[0].x : fmaxf(r.m, ml[0].x);
+#pragma unroll
+    for (int u = 1; u < U; ++u) mx = fmaxf(mx, ml[u].x);
+    // Nothing visible in these splits (nor before): every weight below is exp(-inf) = 0 against a finite stand-in.
+    const float ref = mx == -INFINITY ? 0.0f : mx;
+    if (!FIRST) {
+        const float alpha = BASE2 ? fast_exp2(r.m - ref) : __expf(r.m - ref);
+        r.acc.x *= alpha, r.acc.y *= alpha, r.acc.z *= alpha, r.acc.w *= alpha;
+        r.l *= alpha;
+    }
+    r.m = mx;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const float w = BASE2 ? fast_exp2(ml[u].x - ref) : __expf(ml[u].x - ref);  // exp(-inf) = 0
+        r.l = fmaf(ml[u].y, w, r.l);
+        r.acc.x = fmaf(x[u][0], w, r.acc.x);
+        r.acc.y = fmaf(x[u][1], w, r.acc.y);
+        r.acc.z = fmaf(x[u][2], w, r.acc.z);
+        r.acc.w = fmaf(x[u][3], w, r.acc.w);
+    }
+}
+// The last trip, of as many partials a lane as there are: with eight for every count, a merge of two splits asked for
+// eight times what it needs, and one of 33 for 64. With the addresses as offsets and no branch around the clearing, us a layer, before -> now:
+// one row at 500 / 2,040 / 4,096 (4, 16 and 33 splits) 6.8 / 6.9 / 7.15 -> 6.3 / 6.5 / 7.0, 8 slots at 500 8.0 -> 7.6, 61 rows on
+// 2,040 14.5 -> 13.7, head_dim 64 / 80 / 256 7.7 / 12.0 / 12.9 -> 7.3 / 11.5 / 12.6. (Two or eight wavefronts an output
+// instead of four: 33 splits 7.2 and 7.1, four splits 6.2 and 6.4.)
+template <int SL, bool FIRST, bool BASE2, bool ONCE>
+__device__ __forceinline__ void merge_rest(Merge &r, const float *acc_at, const float *ml_at, uint32_t dim, uint32_t c4,
+                                           uint32_t sl, uint32_t s0, uint32_t S) {
+    switch ((S - s0 + SL - 1) / SL) {
+#define ITAK_TRIP(U) merge_trip<U, SL, FIRST, BASE2, ONCE>(r, acc_at, ml_at, dim, c4, sl, s0, S); break
+        case 1: ITAK_TRIP(1);
+        case 2: ITAK_TRIP(2);
+        case 3: ITAK_TRIP(3);
+        case 4: ITAK_TRIP(4);
+        case 5: ITAK_TRIP(5);
+        case 6: ITAK_TRIP(6);
+        case 7: ITAK_TRIP(7);
+        default: ITAK_TRIP(8);
+#undef ITAK_TRIP
+    }
+}
 // D = head_dim (64, 96, 128 or 256): a wavefront owns D/4 channels, i.e. D/16 chunks, in the next
 // power of two of lanes (at 96 two of eight sit idle), and the other lane bits are split lanes.
 // D = 0: any multiple of four, from the pool's geometry, in CL chunk lanes.
@@ -588,60 +658,24 @@ __device__ __forceinline__ void attn_combine128_body(const AttnParams &p, const 
     // Chunk of 4 channels; lanes beyond the wavefront's chunks or head_dim read one that is there.
     const bool holds = cl < kChunks && (D || wave * kChunks + cl < dim / 4);
     const uint32_t c = D ? wave * kChunks + min(cl, kChunks - 1) : min(wave * kChunks + min(cl, kChunks - 1), dim / 4 - 1);
-    const float *ws_acc = p.ws + ps0 * dim + c * 4;
-    const float2 *ws_ml = reinterpret_cast<const float2 *>(p.ws + uint64_t(total_partials) * dim) + ps0;
+    const float *ws_acc = p.ws + ps0 * dim, *ws_ml = p.ws + uint64_t(total_partials) * dim + ps0 * 2;
     const uint64_t at = (uint64_t(item.q_row0 + row) * p.q_heads + head) * dim + c * 4;
     // The gate of the lanes that write the output, fetched with the partials.
     [[maybe_unused]] float4 gt = make_float4(0.f, 0.f, 0.f, 0.f);
     if (GATE && sl == 0 && holds) gt = *reinterpret_cast<const float4 *>(gate + at);
     ITAK_MARK(1)
 
-    float m_run = -INFINITY, l_run = 0.0f;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (uint32_t s0 = 0; s0 < S; s0 += 8 * SL) {
-        float4 x[8];
-        float2 ml[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {  // clamped, so the loads need no branch
-            const uint32_t s = min(s0 + sl + u * SL, S - 1);
-            x[u] = *reinterpret_cast<const float4 *>(ws_acc + uint64_t(s) * dim);
-            ml[u] = ws_ml[s];
-        }
-        // Nothing below may move above this line and no load below it: left to itself the
-        // scheduler issues half of the accumulator loads after the first weights are computed.
-        __builtin_amdgcn_sched_barrier(0);
-        if (s0 == 0) { ITAK_MARK(2) }
-        float mx = m_run;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            // A lane past the last split holds a second copy of that split's partial: its
-            // weight is zero, and so must the copy be, or a value in it that is not finite
-            // (which the rows that see the key are due) would make the product NaN.
-            if (s0 + sl + u * SL >= S) {
-                ml[u].x = -INFINITY;
-                x[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-            mx = fmaxf(mx, ml[u].x);
-        }
-        // Nothing visible in these splits (nor before): every weight below is exp(-inf) = 0
-        // against a finite stand-in. No branch around the arithmetic: behind one the compiler
-        // fetches the maxima first and the accumulators after it has looked at them, two memory
-        // round trips instead of one.
-        const float ref = mx == -INFINITY ? 0.0f : mx;
-        const float alpha = BASE2 ? fast_exp2(m_run - ref) : __expf(m_run - ref);  // 0 at first
-        acc.x *= alpha, acc.y *= alpha, acc.z *= alpha, acc.w *= alpha;
-        l_run *= alpha;
-        m_run = mx;
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const float w = BASE2 ? fast_exp2(ml[u].x - ref) : __expf(ml[u].x - ref);  // exp(-inf) = 0
-            l_run = fmaf(ml[u].y, w, l_run);
-            acc.x = fmaf(x[u].x, w, acc.x);
-            acc.y = fmaf(x[u].y, w, acc.y);
-            acc.z = fmaf(x[u].z, w, acc.z);
-            acc.w = fmaf(x[u].w, w, acc.w);
-        }
+    Merge r;
+    if (S <= 8 * SL) {
+        merge_rest<SL, true, BASE2, false>(r, ws_acc, ws_ml, dim, c * 4, sl, 0, S);
+    } else {
+        merge_trip<8, SL, true, BASE2, false>(r, ws_acc, ws_ml, dim, c * 4, sl, 0, S);
+        uint32_t s0 = 8 * SL;
+        for (; S - s0 > 8 * SL; s0 += 8 * SL) merge_trip<8, SL, false, BASE2, false>(r, ws_acc, ws_ml, dim, c * 4, sl, s0, S);
+        merge_rest<SL, false, BASE2, false>(r, ws_acc, ws_ml, dim, c * 4, sl, s0, S);
     }
+    const float m_run = r.m, l_run = r.l;
+    const float4 acc = r.acc;
     ITAK_MARK(7)
     // The eight split lanes of a chunk: a common maximum, then the weighted sums.
     const float M = split_lanes_max<SL>(m_run);
@@ -697,20 +731,14 @@ __device__ __forceinline__ float half_sum(float v) {
     const auto c = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(c[0]) + __uint_as_float(c[1]);
 }
-// A load with the streaming hint: split partials are read once, by the merge, and what they
-// would otherwise displace from L2 on their way through is the next layer's use (measured with
-// the hint on the wave kernel's loads: the verify block 23.85 -> 23.23 us per layer, the 64-row
-// chunk 20.16 -> 19.56; the decode merge, a twentieth of the bytes, does not change).
-__device__ __forceinline__ float4 load_once4(const float *p) {
-    typedef float f4v __attribute__((ext_vector_type(4)));
-    const f4v v = __builtin_nontemporal_load(reinterpret_cast<const f4v *>(p));
-    return make_float4(v[0], v[1], v[2], v[3]);
-}
+// (The partials are loaded with the streaming hint: they are read once, and what they would otherwise displace from
+// L2 on their way through is the next layer's use: the verify block 23.85 -> 23.23 us per layer, the 64-row
+// chunk 20.16 -> 19.56; the decode merge, a twentieth of the bytes, does not change.)
 template <int N, bool BASE2, bool GATE>
 __global__ __launch_bounds__(256) void attn_combine128_wave_kernel(AttnParams p, AttnBatchT<N> b,
                                                                    uint32_t total_partials,
                                                                    const float *gate) {
-    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const uint32_t head = blockIdx.x * 4 + wave, grow = blockIdx.y;
     if (head >= p.q_heads) return;
     const AttnItem item = b.of_row(grow);
@@ -719,43 +747,16 @@ __global__ __launch_bounds__(256) void attn_combine128_wave_kernel(AttnParams p,
     const uint32_t row = grow - (item.q_row0 - b.base_row);
     const uint64_t ps0 = item.ws0 + (uint64_t(row) * p.q_heads + head) * S;
     const uint32_t c = lane & 31, sl = lane >> 5;
-    const float *ws_acc = p.ws + ps0 * 128 + c * 4;
-    const float2 *ws_ml = reinterpret_cast<const float2 *>(p.ws + uint64_t(total_partials) * 128) + ps0;
     const uint64_t at = (uint64_t(item.q_row0 + row) * p.q_heads + head) * 128 + c * 4;
     [[maybe_unused]] float4 gt = make_float4(0.f, 0.f, 0.f, 0.f);
     if (GATE && sl == 0) gt = *reinterpret_cast<const float4 *>(gate + at);
-    float4 x[8];
-    float2 ml[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {  // clamped, so the loads need no branch
-        const uint32_t s = min(sl + u * 2, S - 1);
-        x[u] = load_once4(ws_acc + uint64_t(s) * 128);
-        ml[u] = ws_ml[s];
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        if (sl + u * 2 >= S) {  // a second copy of the last split: weight zero, and cleared
-            ml[u].x = -INFINITY;
-            x[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        mx = fmaxf(mx, ml[u].x);
-    }
-    const float M = half_max(mx);
-    float l = 0.0f;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const float w = ml[u].x == -INFINITY ? 0.0f : (BASE2 ? fast_exp2(ml[u].x - M) : __expf(ml[u].x - M));
-        l = fmaf(ml[u].y, w, l);
-        acc.x = fmaf(x[u].x, w, acc.x);
-        acc.y = fmaf(x[u].y, w, acc.y);
-        acc.z = fmaf(x[u].z, w, acc.z);
-        acc.w = fmaf(x[u].w, w, acc.w);
-    }
-    const float inv = 1.0f / half_sum(l);
-    float4 o = make_float4(half_sum(acc.x) * inv, half_sum(acc.y) * inv, half_sum(acc.z) * inv,
-                           half_sum(acc.w) * inv);
+    Merge r;
+    merge_rest<2, true, BASE2, true>(r, p.ws + ps0 * 128, p.ws + uint64_t(total_partials) * 128 + ps0 * 2, 128, c * 4, sl, 0, S);
+    const float M = half_max(r.m);
+    const float w = r.m == -INFINITY ? 0.0f : (BASE2 ? fast_exp2(r.m - M) : __expf(r.m - M));
+    const float inv = 1.0f / half_sum(r.l * w);
+    float4 o = make_float4(half_sum(r.acc.x * w) * inv, half_sum(r.acc.y * w) * inv, half_sum(r.acc.z * w) * inv,
+                           half_sum(r.acc.w * w) * inv);
     if (sl == 0) {
         if (GATE)
             o = make_float4(o.x * sigmoid_fast(gt.x), o.y * sigmoid_fast(gt.y),
