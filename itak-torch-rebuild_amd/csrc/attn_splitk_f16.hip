@@ -179,7 +179,7 @@ static uint32_t variant_capacity(const Variant &v) {
 // Blocks up to which a batch's items stay whole: one workgroup per KV head (and 16 query vectors) walks
 // the context, and there is neither a partial nor a merge launch. A compute unit reads 16 KB of keys and
 // values (a block) in 0.25 us, a merge launch costs 3 us in a single-slot step; a wavefront's second block
-// costs half a microsecond. Eight wavefronts from the fifth block on. One-row steps: up to 12 blocks,
+// costs half a microsecond. Eight wavefronts from the fifth block on. One-row steps (those that `whole_parts` leaves): up to 12 blocks,
 // where the next wavefront's round begins to cost what the merge does (launches that prepare their rows as well:
 // 1 slot at 250 / 320 / 400 split 7.4 / 7.3 / 7.3, whole 6.5 / 7.4 / 8.4), 24 from 64 workgroups on (the merge of many
 // slots costs more). Preparing steps keep 18 where splitting gains less: on pools whose preparing launches stay the
@@ -202,6 +202,23 @@ static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows
     if (rows > 1) return !may ? 8 : g.kv_heads * b.n * tiles >= 128 ? 24 : 16;
     if (g.kv_heads * b.n >= 64) return 24;
     return prepares && (!may_tile || b.n > 8) ? 18 : 12;
+}
+
+// Parts of the channels (attn_whole_f16.hip) in which one-row steps are left whole; 0 = the forms of this file. As many parts
+// as leave every workgroup a compute unit (of 2 / 4 / 8, one slot of 4 KV heads at 500 positions 6.3 / 5.4 / 5.2, 16 slots
+// with 2 / 4 at 500 7.9 / 7.6; two parts at 128 units, 256 workgroups, lose to whole units on the split-K kernel, 8.8 and
+// 11.0 at 300 and 500 -> 8.9 and 11.6, and at 96 win, 8.5 and 10.5 -> 7.4 and 9.8; more workgroups than compute units lose
+// throughout, 24 slots of four parts at 300 8.5 -> 9.0). Up to three blocks a wavefront; where a merge has few outputs, below
+// 16 units, splitting wins before that: one slot at 620 / 700 split 6.3 / 6.3, whole 6.2 / 6.5, 4 slots 7.2 / 7.2 against
+// 6.5 / 6.9 (a fourth block each: 16 slots at 1,000 12.0 -> 13.8). Preparing steps are left whole as far as
+// they were, up to `whole_limit`.
+static uint32_t whole_parts(const PoolGeom &g, const AttnBatch &b, uint32_t group, uint32_t most, bool prepares, uint64_t cus) {
+    const uint64_t units = uint64_t(g.kv_heads) * b.n;
+    const uint32_t limit = prepares ? whole_limit(g, b, 1, 1, true, true, true) : units < 16 ? 20 : kWholeMostBlocks;
+    if (group > 16 || most > limit) return 0;
+    for (uint32_t i = 0; i < b.n; ++i)
+        if (b.item[i].pos0 + 1 != b.item[i].kv_len) return 0;
+    return units * 8 <= cus ? 8 : units * 4 <= cus ? 4 : units * 8 <= cus * 3 ? 2 : 0;
 }
 
 // The tiled form gives every 16 query vectors of a unit (item, KV head) workgroups of their own, with one
@@ -229,8 +246,8 @@ static bool takes_tiles(const PoolGeom &g, const AttnBatch &b, uint32_t tiles, u
 // Every unit is cut into equal runs of at most T blocks, T the smallest run for which the whole
 // batch fits the device in one wave of dispatch; a run is never shorter than one block per wavefront.
 // may_tile = false keeps the forms that the exchange inside the launch and the queries as two
-// halves are written for.
-uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares, bool may_tile) {
+// halves are written for; may_part = false those that a merge on the compute dies can take.
+uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares, bool may_tile, bool may_part) {
     const uint32_t group = q_heads / g.kv_heads;
     uint32_t most = 0, most_rows = 0;
     uint64_t blocks = 0;
@@ -243,13 +260,14 @@ uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads,
     const uint64_t cus = compute_units();
     const uint32_t tiles = (most_rows * group + 15) / 16;
     const bool may = may_tile && takes_tiles(g, b, tiles, blocks, cus, prepares && most_rows == 1);
-    const bool whole = most <= whole_limit(g, b, most_rows, tiles, prepares, may_tile, may);
+    b.parts = may_part && most_rows == 1 ? whole_parts(g, b, group, most, prepares, cus) : 0;
+    const bool whole = b.parts || most <= whole_limit(g, b, most_rows, tiles, prepares, may_tile, may);
     b.whole_on_eight = whole && most > 4 && (may || most_rows == 1) ? 1 : 0;
     // (A whole one-row step has no second tile and hardly a second block: the form with two sets of
     // operands, whose next block is under way before the first is multiplied, is 0.4 us faster.)
     b.tiled = !may || (whole && most_rows == 1) ? 0
               : (whole ? b.whole_on_eight != 0 : tiles == 1 && blocks >= 16 * cus) ? 8 : 4;
-    auto units_of = [&](const AttnItem &it) { return g.kv_heads * (b.tiled ? (it.rows * group + 15) / 16 : 1u); };
+    auto units_of = [&](const AttnItem &it) { return g.kv_heads * (b.parts ? b.parts : b.tiled ? (it.rows * group + 15) / 16 : 1u); };
     auto groups_at = [&](uint32_t run) {
         uint64_t groups = 0;
         for (uint32_t i = 0; i < b.n; ++i)
@@ -337,6 +355,7 @@ hipError_t launch_attn_splitk_f16(const AttnParams &p, const AttnBatch &b, uint3
     if (b.total_blocks == 0) return hipSuccess;
     const Variant v = pick_variant(p.g, b, p.group);
     const bool prep = folded && folded->prep_on;
+    if (b.parts) return launch_attn_whole_f16(p, b, stream, prep ? folded : nullptr);
     if (v.index == 0 && (!prep || (!q_two_halves && !p.exchange)) && attn_decode_f16_takes(p, b))
         return launch_attn_decode_f16(p, b, total_partials, stream, q_two_halves, prep ? folded : nullptr);
     if (q_two_halves) return launch_attn_splitk_f16_qlo(p, b, total_partials, stream, folded);

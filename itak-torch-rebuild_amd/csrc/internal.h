@@ -310,6 +310,7 @@ struct AttnBatch {
     uint32_t half_blocks; // host side only: the rows kernel's wavefronts take half a block each
     uint32_t tiled; // host side only: the split-K plan gives every 16 query vectors their own workgroups
     uint32_t whole_on_eight; // host side only: the split-K plan leaves every item whole on eight wavefronts
+    uint32_t parts; // host side only: and gives every (item, KV head) that many workgroups, a part of the channels each
     uint32_t tile_sets;  // host side only: the tiles kernel's plan, sets of 16 query vectors a tile
     uint32_t tile_waves; // and wavefronts a workgroup
     uint32_t tile_exact; // and whether the softmax keeps the exact running maximum
@@ -467,7 +468,8 @@ uint32_t attn_generic_tile(uint32_t head_dim);
 // Partials are in log2 domain (combine with base2 = 1).
 bool attn_splitk_f16_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
 // (`prepares`: the launch prepares Q and the new K rows itself.)
-uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares = false, bool may_tile = false);
+uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares = false, bool may_tile = false,
+                              bool may_part = false);
 // After attn_splitk_f16_plan: whether the batch can merge its splits inside the split-K launch
 // (AttnParams::exchange). Returns the 64-bit words the exchange buffer must hold and re-bases
 // the items' ws0 on it, or 0 (items untouched) when the batch keeps the merge launch.
@@ -528,6 +530,9 @@ uint32_t attn_decode_f16_resident_groups();
 // `prepares`: Q and the new K rows are prepared by the launch (not with q_two_halves or an exchange).
 hipError_t launch_attn_decode_f16(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream, bool q_two_halves = false, const FoldedParams *prepares = nullptr);
+// Whole one-row steps by channels (attn_whole_f16.hip): AttnBatch::parts is 2 or 4.
+constexpr uint32_t kWholeMostBlocks = 24;
+hipError_t launch_attn_whole_f16(const AttnParams &p, const AttnBatch &b, hipStream_t stream, const FoldedParams *prepares);
 // f32 MFMA split-K path: f32 pools (row-major planes), head_dim 128, rows*group <= 16, implied
 // query positions. Partials are in log2 domain (combine with base2 = 1).
 bool attn_splitk_f32_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);

@@ -735,7 +735,7 @@ bool takes_splitk_any(const itak_pool *pool, const PlanInput *in, uint32_t n, ui
 // Clears a batch's plan and names its items' places; q rows counted from q_row0. Returns their rows.
 uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t q_row0) {
     b.n = count;  // (cleared item by item: all 64 are three kilobytes)
-    b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.tiled = b.on_eight = b.half_blocks = 0;
+    b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.parts = b.tiled = b.on_eight = b.half_blocks = 0;
     b.two_halves = b.tile_sets = b.tile_waves = b.tile_exact = 0;
     b.plan_cost = 0.0f;
     b.partial_limit = 0;
@@ -907,7 +907,8 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             partials = attn_tiles_f16_plan(geom, b, uint32_t(q_heads), form);
         } else if (mfma) {
             partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads), folded && folded->prep_on,
-                                            !pool->q_two_halves && !pool->merge_in_launch);
+                                            !pool->q_two_halves && !pool->merge_in_launch,
+                                            !pool->q_two_halves && !pool->merge_in_launch && !pool->die_merge);
         } else if (prefill) {
             partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, k_new != nullptr);
         } else if (f32fast || any) {
