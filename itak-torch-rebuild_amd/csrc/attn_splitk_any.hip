@@ -48,20 +48,6 @@ namespace itak {
 
 namespace {
 
-
-// x = h[0] + h[1] + h[2] up to 2^-33 of the largest x the halves hold. A half that is not finite
-// has nothing left to say.
-__device__ __forceinline__ void split3(float x, _Float16 &a, _Float16 &b, _Float16 &c) {
-    a = static_cast<_Float16>(x);
-    const float r = x - float(a);
-    b = static_cast<_Float16>(r);
-    c = static_cast<_Float16>(r - float(b));
-}
-
-// Weights carry this many powers of two (so that their third halves are no subnormals); sums and
-// outputs carry them too, and lose them in the division.
-constexpr float kWeightShift = 15.0f;
-
 template <int DP, int W, int N>
 __global__ __launch_bounds__(W * 64, DP <= 128 ? 8 / W : 1) void attn_splitk_halves_kernel(AttnParams p, AttnBatchT<N> b,
                                                                                           uint32_t total_partials) {
@@ -420,6 +406,7 @@ bool attn_splitk_any_appends(const PoolGeom &g, int elem_f16, uint32_t group, ui
 hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream) {
     if (b.total_blocks == 0) return hipSuccess;
+    if (b.parts) return launch_attn_whole_halves(p, b, stream);
     const uint32_t d = p.g.head_dim;
     // (Batches of one item take the eight-item argument block: 0.1 us on a launch of 5.)
 #define ITAK_ANY(W, ...)                                                                          \

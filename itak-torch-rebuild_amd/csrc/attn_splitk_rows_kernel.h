@@ -61,6 +61,19 @@ __device__ __forceinline__ float lanes4_sum(float v) {
     return __uint_as_float(c[0]) + __uint_as_float(c[1]);
 }
 
+// x = h[0] + h[1] + h[2] up to 2^-33 of the largest x the halves hold. A half that is not finite
+// has nothing left to say.
+__device__ __forceinline__ void split3(float x, _Float16 &a, _Float16 &b, _Float16 &c) {
+    a = static_cast<_Float16>(x);
+    const float r = x - float(a);
+    b = static_cast<_Float16>(r);
+    c = static_cast<_Float16>(r - float(b));
+}
+
+// Weights carry this many powers of two (so that their third halves are no subnormals); sums and
+// outputs carry them too, and lose them in the division.
+constexpr float kWeightShift = 15.0f;
+
 // Four channels of a row. K/V rows that one workgroup alone reads (a step of one tile of vectors
 // per KV head: decode rows, short blocks) are read with the streaming hint, so that they do not
 // displace the kernel's code, arguments and split partials in L2 (decode at context 4096 13.6 ->

@@ -72,3 +72,58 @@ def test_short_preparing_steps_by_channels(q_heads, kv_heads, slots, window):
     for i, n in enumerate((0, 1, 31, 32, 255, 256, 383, 440, 500, 580)):
         run_case("f16", q_heads, kv_heads, D, n, 1, norm=True, rope_base=(1e4, 0.0, 5e5)[i % 3],
                  interleaved=bool(i & 1), rotary=(0, 64)[i % 2], gate=i % 4 != 2, seed=n, slots=slots, window=window)
+
+
+# Other head dims on blocked f16 planes: queries and weights as three halves, so the bar is what f32 sums of a thousand
+# terms leave, 2^-23 * 1024 of |v| <= 4 at most and a tenth of that as they are of either sign: 5e-5. Every count of
+# channel tiles, parts of one tile and of several (the last of which may be part empty), one to four rounds; `bad`
+# plants an infinity in a stored key and value and in the new row, whose rows then are the oracle's, infinities and NaN as they are.
+@pytest.mark.parametrize("bad", [False, True])
+@pytest.mark.parametrize("d,q_heads,kv_heads,slots", [(16, 8, 2, 1), (32, 8, 8, 2), (64, 32, 4, 1), (64, 16, 1, 9), (80, 32, 8, 1),
+                                                      (80, 9, 3, 10), (96, 32, 4, 3), (112, 14, 2, 1), (112, 32, 4, 8), (144, 8, 4, 1),
+                                                      (192, 32, 4, 1), (208, 8, 8, 3), (256, 32, 4, 1), (256, 16, 2, 12)])
+@pytest.mark.parametrize("window", [None, 100])
+def test_short_steps_at_other_head_dims(d, q_heads, kv_heads, slots, window, bad):
+    P = pkg()
+    row = kv_heads * d
+    kind = P.LayerKind.Global if window is None else P.LayerKind.windowed(window)
+    okind = oracle.LayerKind.Global if window is None else oracle.LayerKind.windowed(window)
+    for n in (0, 31, 32, 255, 256, 511, 767, 800, 1023):
+        rng = np.random.default_rng(n + 1000 * slots + d)
+        pool = P.KvPool([kind], kv_heads, d, elem="f16", max_slots=slots, capacity_rows=1030)
+        pool.set_stream(torch.cuda.current_stream().cuda_stream)
+        caches, refs, lengths = [], [], []
+        for s in range(slots):
+            length = max(n - 37 * s, 0)
+            first = 0 if window is None else max(0, length - window)
+            cache, ref = pool.acquire(), oracle.KvCache.new([okind], kv_heads, d, store_f16=True)
+            if length:
+                k, v = normal(rng, length - first, row), normal(rng, length - first, row)
+                if bad:
+                    v[rng.integers(length - first), rng.integers(row)] = np.inf
+                    k[rng.integers(length - first), rng.integers(row)] = -np.inf
+                cache.restore_bulk(0, first, k, v)
+                ref.restore_bulk(0, first, k, v)
+            caches.append(cache), refs.append(ref), lengths.append(length)
+        for step in range(2):
+            q, k, v = normal(rng, slots, q_heads * d), normal(rng, slots, row), normal(rng, slots, row)
+            if bad:
+                v[0, rng.integers(row)] = -np.inf
+            qd, kd, vd = dev(q), dev(k), dev(v)
+            out = torch.full_like(qd, 7.0)
+            softcap = 30.0 * step
+            pool.attention_step_device(0, [(c, 1) for c in caches], qd.data_ptr(), kd.data_ptr(), vd.data_ptr(),
+                                       out.data_ptr(), q_heads, softcap=softcap)
+            torch.cuda.synchronize()
+            got = out.cpu().numpy()
+            for s, ref in enumerate(refs):
+                at = lengths[s] + step
+                want = np.asarray(oracle.attention_step(ref, 0, q[s:s + 1], k[s:s + 1], v[s:s + 1], q_heads, at,
+                                                        oracle.AttentionParams(softcap=softcap))).reshape(-1)
+                finite = np.isfinite(want)
+                assert np.array_equal(got[s][~finite], want[~finite], equal_nan=True), (n, s, at)
+                assert not finite.any() or max_abs(got[s][finite], want[finite]) <= 5e-5, (n, s, at)
+                _, gk, gv = caches[s].read_rows(0, caches[s].stored_len(0) - 1, 1)
+                assert np.array_equal(gk.reshape(-1), oracle.f32_to_f16_array(k[s]))
+                assert np.array_equal(gv.reshape(-1), oracle.f32_to_f16_array(v[s]))
+        pool.close()
