@@ -1,22 +1,26 @@
-// GQA flash-decode for gfx950 over short contexts on f16 pools at the head dims attn_splitk_halves_kernel serves (blocked
-// planes, head_dim a multiple of 16): one row per sequence, no split of the context and no merge launch.
+// GQA flash-decode for gfx950 on f16 pools at the head dims attn_splitk_halves_kernel serves (blocked planes, head_dim a
+// multiple of 16): one row per sequence, while the work is at most one workgroup per compute unit.
 //
 // The work is cut as in attn_whole_f16.hip: each workgroup of a (slot, KV head) works out all scores and the output of KT of
-// its channel tiles, eight wavefronts of up to four blocks each, every load asked for before anything is waited for. The
+// its channel tiles, eight wavefronts of up to four blocks each, every load asked for before anything is waited for.
+// Contexts beyond are cut into runs of eight blocks, one a wavefront, and merged by a second launch. The
 // arithmetic is attn_splitk_halves_kernel's (attn_splitk_any.hip): queries and weights as three halves each, a
-// wavefront whose sums come out not finite walks its keys again on the f32 pipe. What cost that kernel's short steps
+// wavefront whose sums come out not finite walks its keys again on the f32 pipe. What cost that kernel's steps
 // most, beside the merge launch, was done once per wavefront there and is done once per workgroup here: the queries' split
 // into halves (64 channels a lane at head_dim 256; 4 or 8 here, shared through LDS), and the new row, which was stored,
 // waited for and read back and is patched into the operands now.
-// 32 Q / 4 KV heads, us a layer, attn_splitk_halves_kernel whole or split -> this: one slot at 60 / 200 / 400 / 700 positions,
-// head_dim 64 4.9 / 5.6 / 6.6 / 7.0 -> 4.1 / 4.3 / 5.0 / 5.8, head_dim 80 5.2 / 6.4 / 7.7 / 7.5 -> 4.3 / 4.5 / 5.4 / 6.5,
-// head_dim 112 5.8 / 7.4 / 8.9 / 8.2 -> 4.4 / 4.7 / 5.8 / 7.2; at 60 / 200 / 400 head_dim 192 8.0 / 9.4 / 10.4 ->
-// 5.0 / 5.4 / 7.4, head_dim 256 9.6 / 11.5 / 12.0 -> 5.5 / 5.8 / 8.5; 8 slots at 200 / 700, head_dim 80 6.9 / 9.5 -> 4.9 / 7.1.
+// 32 Q / 4 KV heads, us a layer, attn_splitk_halves_kernel whole or split -> this. Whole, one slot at 60 / 200 / 400 / 700
+// positions, head_dim 64 4.9 / 5.6 / 6.6 / 7.0 -> 4.2 / 4.4 / 5.2 / 6.0, head_dim 80 5.2 / 6.4 / 7.7 / 7.5 -> 4.4 / 4.6 / 5.5 / 6.5,
+// head_dim 112 5.8 / 7.4 / 8.9 / 8.2 -> 4.6 / 4.8 / 6.0 / 7.3; at 60 / 200 / 400 head_dim 192 8.0 / 9.4 / 10.4 ->
+// 5.3 / 5.5 / 7.5, head_dim 256 9.6 / 11.5 / 12.0 -> 5.7 / 5.9 / 8.6; 8 slots at 200 / 700, head_dim 80 6.9 / 9.5 -> 5.0 / 7.2.
+// Split, one slot at 1,500 / 3,000, head_dim 64 7.0 / 7.5 -> 6.5 / 7.0, head_dim 80 8.1 / 8.5 -> 7.2 / 7.6, head_dim 112 8.9 / 9.1 ->
+// 7.7 / 7.9, head_dim 256 12.5 / 12.8 -> 8.6 / 9.1; 4 slots at 1,500 head_dim 80 9.2 -> 8.1, head_dim 192 12.9 -> 11.3; 8 slots
+// at 1,500 head_dim 96 11.1 -> 9.7.
 // What bounds it now: launch and first trips to memory, 2.5 us, the products of eight wavefronts on one compute unit's
-// matrix pipes (0.3 us a round at head_dim 80, three for one with f32's precision), and the keys each part reads.
+// matrix pipes (0.3 us a round at head_dim 80, three for one with f32's precision), the keys each part reads, and the merge.
 //
 // Semantics: gqa_attention in crates/attention/src/attention.rs:104-215, softcap as
-// crates/torch-math/src/logits.rs:26-37.
+// crates/torch-math/src/logits.rs:26-37. Partials are in the log2 domain.
 #include "attn_splitk_rows_kernel.h"
 
 #include <math.h>
@@ -39,9 +43,11 @@ __device__ __forceinline__ float row_max32(float v) {
     return fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
 }
 
-// DP: head_dim rounded up to a multiple of 32; KT: channel tiles of a workgroup; R: blocks of a wavefront.
-template <int DP, int KT, int R, int N>
-__global__ __launch_bounds__(kWaves * 64) void attn_whole_halves_kernel(AttnParams p, AttnBatchT<N> b) {
+// DP: head_dim rounded up to a multiple of 32; KT: channel tiles of a workgroup; R: blocks of a wavefront; SPLIT: contexts may be
+// cut (without it the whole forms were 2 % slower).
+template <int DP, int KT, int R, bool SPLIT, int N>
+__global__ __launch_bounds__(kWaves * 64) void attn_parts_halves_kernel(AttnParams p, AttnBatchT<N> b,
+                                                                        uint32_t total_partials) {
     constexpr int kS = DP / 32;       // steps of a key row
     constexpr int kStride = DP + 8;   // LDS row stride of the staged queries (halves)
     constexpr int kQ = DP > 128 ? 2 : 1;  // pieces of four channels of a query a thread stages
@@ -57,7 +63,14 @@ __global__ __launch_bounds__(kWaves * 64) void attn_whole_halves_kernel(AttnPara
 
     const AttnItem item = b.of_block(blockIdx.x);
     const uint32_t local = blockIdx.x - item.block0, heads = p.g.kv_heads, group = p.group;
-    const uint32_t part = heads > 1 ? __umulhi(local, item.splits_magic) : local, kv_head = local - part * heads;
+    // Part after part, and within one split after split, so that with a multiple of eight (KV head, split) pairs the parts of one
+    // run on one compute die.
+    const uint32_t pairs = SPLIT ? heads * item.splits : heads, part = pairs > 1 ? __umulhi(local, item.splits_magic) : local;
+    uint32_t kv_head = local - part * pairs, split = 0;
+    if (SPLIT && item.splits > 1) {  // (a thousand pairs at most: a float holds the quotient)
+        split = __builtin_amdgcn_readfirstlane(int((float(kv_head) + 0.5f) * __builtin_amdgcn_rcpf(float(heads))));
+        kv_head -= split * heads;
+    }
 
     uint16_t *kplane = static_cast<uint16_t *>(const_cast<void *>(p.layer_base)) + item.slot * p.g.slot_stride +
                        kv_head * p.g.head_stride;
@@ -65,7 +78,8 @@ __global__ __launch_bounds__(kWaves * 64) void attn_whole_halves_kernel(AttnPara
     const uint32_t ring_blocks = p.ring_blocks;
     const uint32_t pos = min(item.pos0, item.kv_len - 1);  // the newest position the query sees, and the oldest
     const uint32_t lo = lowest_visible(item.pos0, p.window, item.kv_lo);
-    const uint32_t kb_begin = lo / kBlockKeys, kb_end = pos / kBlockKeys + 1;
+    const uint32_t run = SPLIT ? item.keys_per_split / kBlockKeys : 0, kb_begin = lo / kBlockKeys + split * run;
+    const uint32_t kb_end = SPLIT ? min(pos / kBlockKeys + 1, kb_begin + run) : pos / kBlockKeys + 1;
     auto block_at = [&](uint32_t kb) { return uint64_t(ring_blocks ? kb % ring_blocks : kb) * (kVBlock * D); };
 
     // ---- every load: the new row (its keys' pieces, then its values'), the queries (32 threads a vector; vectors beyond
@@ -305,17 +319,19 @@ __global__ __launch_bounds__(kWaves * 64) void attn_whole_halves_kernel(AttnPara
         sm_l[wave * 16 + jl] = l_col;
     }
     lds_barrier();
-    // Value tid + 512 u of the part's outputs, [tile][lane][row of the lane] (of one tile half the threads do).
-    constexpr int kF = KT == 4 ? 2 : 1;
-    const uint32_t fid = KT == 1 ? tid & 255 : tid, fcol = (fid >> 2) & 15;
-    const uint32_t fch = part * KT * 16 + (fid >> 8) * 16 + ((fid >> 6) & 3) * 4 + (fid & 3);
+    // Value tid + 64 kWaves u of the part's outputs, [tile][lane][row of the lane].
+    static_assert(KT == 1 || KT % 2 == 0, "every thread has as many values");
+    constexpr int kValues = KT * 256, kF = (KT + 1) / 2;
+    const bool final_out = !SPLIT || item.splits == 1;
+    if (wave * 64 >= kValues) return;
+    const uint32_t fcol = (tid >> 2) & 15, fch = part * KT * 16 + (tid >> 8) * 16 + ((tid >> 6) & 3) * 4 + (tid & 3);
     float mw[kWaves], lw[kWaves], ow[kF][kWaves];
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
         mw[w] = sm_m[w * 16 + fcol];
         lw[w] = sm_l[w * 16 + fcol];
 #pragma unroll
-        for (int u = 0; u < kF; ++u) ow[u][w] = sm_o[w * KT * 256 + u * 512 + fid];
+        for (int u = 0; u < kF; ++u) ow[u][w] = sm_o[w * kValues + u * kWaves * 64 + tid];
     }
     float M = mw[0];
 #pragma unroll
@@ -330,15 +346,19 @@ __global__ __launch_bounds__(kWaves * 64) void attn_whole_halves_kernel(AttnPara
 #pragma unroll
         for (int u = 0; u < kF; ++u) fin[u] = fmaf(ow[u][w], wgt, fin[u]);
     }
-    if (fcol < group && (KT != 1 || tid < 256)) {
-        const float post = 1.0f / L;
-        float *dst = p.out + (uint64_t(item.q_row0) * p.q_heads + kv_head * group + fcol) * D;
+    if (fcol < group) {
+        const uint32_t head = kv_head * group + fcol;
+        const uint64_t ps = item.ws0 + uint64_t(head) * item.splits + split;
+        const float post = final_out ? 1.0f / L : 1.0f;
+        float *dst = final_out ? p.out + (uint64_t(item.q_row0) * p.q_heads + head) * D : p.ws + ps * D;
 #pragma unroll
         for (int u = 0; u < kF; ++u)
-            if (fch + 32 * u < D) dst[fch + 32 * u] = fin[u] * post;
+            if (fch + 4 * kWaves * u < D) dst[fch + 4 * kWaves * u] = fin[u] * post;
+        if (!final_out && part == 0 && tid < 64 && (tid & 3) == 0)
+            *reinterpret_cast<float2 *>(p.ws + uint64_t(total_partials) * D + ps * 2) = make_float2(M, L);
     }
     // The new row goes to the planes as append lays it out; nothing in this launch reads it from there.
-    if (fused && part == 0 && tid < 2 * quads) {
+    if (fused && part == 0 && (!SPLIT || new_kb - kb_begin < kb_end - kb_begin) && tid < 2 * quads) {
         const uint64_t blk = block_at(new_kb);
         if (nside == 0) {
             *reinterpret_cast<uint2 *>(kplane + blk + ((t_new * chunks + nc4 / 8) * 16 + i_new) * 8 + nc4 % 8) = packed;
@@ -352,17 +372,22 @@ __global__ __launch_bounds__(kWaves * 64) void attn_whole_halves_kernel(AttnPara
     }
 }
 
-// Blocks of a wavefront, by the registers they take (a third one at head_dim 192 and above spills). Where a merge has few outputs, below
-// 16 units, splitting wins from the fourth block on: one slot at 800 / 1,000, head_dim 80, split 7.5 / 7.5, whole 7.5 / 7.8,
-// head_dim 112 8.4 / 8.6 against 8.3 / 8.7, 8 slots at 1,000 9.3 and 10.3 -> 8.3 and 9.4.
-uint32_t most_rounds(uint32_t d, uint64_t units) { return d > 128 ? 2 : units < 16 ? 3 : 4; }
+// Channel tiles a workgroup may have: one, two, four or all up to head_dim 128; two, four or eight beyond, where the keys
+// are the larger part of what a workgroup reads.
+uint32_t next_tiles(uint32_t d, uint32_t kt) {
+    if (kt == 0) return d <= 128 ? 1 : 2;
+    if (kt < (d <= 128 ? 4u : 8u)) return 2 * kt;
+    const uint32_t all = (d + 31) / 32 * 2;
+    return d <= 128 && kt < all ? all : 0;
+}
 
 }  // namespace
 
-// Leaves a batch of one-row steps whole in parts of channels, when the blocks fit the wavefronts and every workgroup has a compute
-// unit: parts of one channel tile, of two otherwise (two and four above head_dim 128, where the keys are the larger
-// part of what a workgroup reads). More workgroups than compute units stay with attn_splitk_halves_kernel.
-bool attn_whole_halves_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads) {
+// Takes a batch of one-row steps when every workgroup has a compute unit to itself: whole contexts, or runs of eight blocks, one
+// for each wavefront, with as few channel tiles a workgroup as that allows. (More workgroups than compute units lose to
+// attn_splitk_halves_kernel: 8 slots at 3,000, head_dim 80, 384 workgroups of all tiles 13.1 against 12.6; runs of 10 or 12 blocks on
+// as many wavefronts are no faster than that kernel either, 10.2 against 10.3 where runs of eight take 9.1.)
+bool attn_parts_halves_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uint32_t *partials) {
     const uint32_t d = g.head_dim, tiles = d / 16;
     if (!g.v_block || d % 16 != 0 || d > 256 || q_heads / g.kv_heads > 16) return false;
     uint32_t most = 0;
@@ -370,68 +395,110 @@ bool attn_whole_halves_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads) {
         if (b.item[i].rows != 1) return false;
         most = std::max(most, item_block_count(b.item[i]));
     }
-    const uint64_t units = uint64_t(g.kv_heads) * b.n;
-    if (most > most_rounds(d, units) * kWaves) return false;
-    const uint32_t fewest = d <= 128 ? 1 : 2;
-    for (uint32_t kt = fewest; kt <= 2 * fewest && !b.parts; kt *= 2)
-        if (units * ((tiles + kt - 1) / kt) <= compute_units()) b.parts = kt;
-    if (!b.parts) return false;
-    uint32_t block0 = 0;
+    const uint64_t units = uint64_t(g.kv_heads) * b.n, cus = compute_units();
+    auto groups_at = [&](uint32_t run, uint32_t kt) {
+        uint64_t pairs = 0;
+        for (uint32_t i = 0; i < b.n; ++i)
+            pairs += uint64_t(g.kv_heads) * std::max((item_block_count(b.item[i]) + run - 1) / run, 1u);
+        return pairs * ((tiles + kt - 1) / kt);
+    };
+    uint32_t T = 0;
+    auto fits = [&](uint32_t run, uint32_t most_kt) {
+        for (uint32_t kt = next_tiles(d, 0); kt && kt <= most_kt; kt = next_tiles(d, kt))
+            if (groups_at(run, kt) <= cus) {
+                b.parts = kt;
+                T = run;
+                return true;
+            }
+        return false;
+    };
+    // Whole first: two rounds above head_dim 128 (a third spills), three below; a fourth where a merge has many outputs, from 16 units on, at
+    // head_dim 64 before and at others after the cut. Below 16 units the cut wins from the fourth on: one slot at 800,
+    // head_dim 64 / 112, split 6.6 / 7.2, whole 6.6 / 8.3. Cut second, where a context has a fourth round: the general forms leave up
+    // to 24 blocks whole from 16 units on, and better so (24 slots at 400, head_dim 80, 8.4 whole, 9.4 split).
+    const uint32_t whole_kt = d <= 128 ? 2 : 4, rounds = (most + kWaves - 1) / kWaves;
+    const bool many = d <= 128 && units >= 16;
+    const uint32_t whole_rounds = d > 128 ? 2 : many && d <= 64 ? 4 : 3;
+    if (!(rounds <= whole_rounds && fits(most, whole_kt)) && !(rounds > (many ? 3u : 1u) && fits(kWaves, 16)) &&
+        !(many && rounds <= 4 && fits(most, whole_kt)))
+        return false;
+    uint32_t block0 = 0, ws0 = 0;
     for (uint32_t i = 0; i < b.n; ++i) {
         AttnItem &it = b.item[i];
-        it.splits = 1;
-        it.keys_per_split = std::max(item_block_count(it), 1u) * kBlockKeys;
-        it.splits_magic = g.kv_heads > 1 ? uint32_t(((uint64_t(1) << 32) + g.kv_heads - 1) / g.kv_heads) : 0;
+        const uint32_t nblocks = std::max(item_block_count(it), 1u);
+        it.splits = (nblocks + T - 1) / T;
+        const uint32_t run = (nblocks + it.splits - 1) / it.splits;
+        it.splits = (nblocks + run - 1) / run;
+        it.keys_per_split = run * kBlockKeys;
+        const uint64_t pairs = uint64_t(g.kv_heads) * it.splits;
+        it.splits_magic = pairs > 1 ? uint32_t(((uint64_t(1) << 32) + pairs - 1) / pairs) : 0;
         it.block0 = block0;
-        it.ws0 = 0;
-        block0 += g.kv_heads * ((tiles + b.parts - 1) / b.parts);
+        it.ws0 = ws0;
+        block0 += g.kv_heads * ((tiles + b.parts - 1) / b.parts) * it.splits;
+        if (it.splits > 1) ws0 += q_heads * it.splits;
     }
     b.total_blocks = block0;
     b.rows_per_block = 0;
+    *partials = ws0;
     return true;
 }
 
-hipError_t launch_attn_whole_halves(const AttnParams &p, const AttnBatch &b, hipStream_t stream) {
+hipError_t launch_attn_parts_halves(const AttnParams &p, const AttnBatch &b, uint32_t total_partials, hipStream_t stream) {
     uint32_t most = 1;
-    for (uint32_t i = 0; i < b.n; ++i) most = std::max(most, item_block_count(b.item[i]));
+    bool split = false;
+    for (uint32_t i = 0; i < b.n; ++i) {
+        most = std::max(most, b.item[i].keys_per_split / kBlockKeys);
+        split = split || b.item[i].splits > 1;
+    }
     const uint32_t rounds = (most + kWaves - 1) / kWaves, d = p.g.head_dim;
-    if (rounds > (d > 128 ? 2u : 4u)) return hipErrorInvalidValue;  // (the planner asks for no more)
-#define ITAK_WHOLE(DP, KT, R)                                                                                          \
+#define ITAK_PARTS(DP, KT, R, SPLIT)                                                                                   \
     do {                                                                                                               \
         if (b.n <= 8)                                                                                                  \
-            launch_kernel(attn_whole_halves_kernel<DP, KT, R, 8>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<8>(b)); \
+            launch_kernel(attn_parts_halves_kernel<DP, KT, R, SPLIT, 8>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<8>(b), total_partials); \
         else                                                                                                           \
-            launch_kernel(attn_whole_halves_kernel<DP, KT, R, 64>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<64>(b)); \
+            launch_kernel(attn_parts_halves_kernel<DP, KT, R, SPLIT, 64>, b.total_blocks, kWaves * 64, 0, stream, p, AttnBatchT<64>(b), total_partials); \
+        return hipGetLastError();                                                                                      \
     } while (0)
-#define ITAK_WHOLE_R(DP, KT)                                                 \
-    do {                                                                     \
-        if (rounds == 1) ITAK_WHOLE(DP, KT, 1);                              \
-        else if (rounds == 2) ITAK_WHOLE(DP, KT, 2);                         \
-        else if constexpr (DP <= 128) {                                      \
-            if (rounds == 3) ITAK_WHOLE(DP, KT, 3);                          \
-            else ITAK_WHOLE(DP, KT, 4);                                      \
-        }                                                                    \
-    } while (0)
-#define ITAK_WHOLE_T(DP)                                                     \
-    do {                                                                     \
-        constexpr int kFew = DP <= 128 ? 1 : 2;                              \
-        if (b.parts == kFew) ITAK_WHOLE_R(DP, kFew);                         \
-        else ITAK_WHOLE_R(DP, 2 * kFew);                                     \
+// (Split runs are one round; WHOLE = the rounds of whole contexts, of which the forms of most tiles have none.)
+#define ITAK_PARTS_R(DP, KT, WHOLE)                                              \
+    if (b.parts == KT) {                                                         \
+        if (split && rounds == 1) ITAK_PARTS(DP, KT, 1, true);                   \
+        if constexpr (WHOLE >= 2) {                                              \
+            if (!split && rounds == 1) ITAK_PARTS(DP, KT, 1, false);             \
+            if (!split && rounds == 2) ITAK_PARTS(DP, KT, 2, false);             \
+        }                                                                        \
+        if constexpr (WHOLE >= 4) {                                              \
+            if (!split && rounds == 3) ITAK_PARTS(DP, KT, 3, false);             \
+            if (!split && rounds == 4) ITAK_PARTS(DP, KT, 4, false);             \
+        }                                                                        \
+    }
+#define ITAK_PARTS_T(DP)                                                 \
+    do {                                                                 \
+        if constexpr (DP <= 128) {                                       \
+            ITAK_PARTS_R(DP, 1, 4)                                       \
+            ITAK_PARTS_R(DP, 2, 4)                                       \
+            ITAK_PARTS_R(DP, 4, 0)                                       \
+            if constexpr (DP > 64) ITAK_PARTS_R(DP, (DP / 16), 0)        \
+        } else {                                                         \
+            ITAK_PARTS_R(DP, 2, 2)                                       \
+            ITAK_PARTS_R(DP, 4, 2)                                       \
+            ITAK_PARTS_R(DP, 8, 0)                                       \
+        }                                                                \
     } while (0)
     switch ((d + 31) / 32) {
-        case 1: ITAK_WHOLE_T(32); break;
-        case 2: ITAK_WHOLE_T(64); break;
-        case 3: ITAK_WHOLE_T(96); break;
-        case 4: ITAK_WHOLE_T(128); break;
-        case 5: ITAK_WHOLE_T(160); break;
-        case 6: ITAK_WHOLE_T(192); break;
-        case 7: ITAK_WHOLE_T(224); break;
-        default: ITAK_WHOLE_T(256); break;
+        case 1: ITAK_PARTS_T(32); break;
+        case 2: ITAK_PARTS_T(64); break;
+        case 3: ITAK_PARTS_T(96); break;
+        case 4: ITAK_PARTS_T(128); break;
+        case 5: ITAK_PARTS_T(160); break;
+        case 6: ITAK_PARTS_T(192); break;
+        case 7: ITAK_PARTS_T(224); break;
+        default: ITAK_PARTS_T(256); break;
     }
-#undef ITAK_WHOLE_T
-#undef ITAK_WHOLE_R
-#undef ITAK_WHOLE
-    return hipGetLastError();
+#undef ITAK_PARTS_T
+#undef ITAK_PARTS_R
+#undef ITAK_PARTS
+    return hipErrorInvalidValue;  // (the planner asks for no others)
 }
 
 }  // namespace itak

@@ -406,7 +406,7 @@ bool attn_splitk_any_appends(const PoolGeom &g, int elem_f16, uint32_t group, ui
 hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream) {
     if (b.total_blocks == 0) return hipSuccess;
-    if (b.parts) return launch_attn_whole_halves(p, b, stream);
+    if (b.parts) return launch_attn_parts_halves(p, b, total_partials, stream);
     const uint32_t d = p.g.head_dim;
     // (Batches of one item take the eight-item argument block: 0.1 us on a launch of 5.)
 #define ITAK_ANY(W, ...)                                                                          \

@@ -75,7 +75,8 @@ static const CutCosts *cut_costs(const PoolGeom &g, int elem_f16) {
 // such a cut may take (0 = any).
 uint32_t attn_splitk_f32_plan(const PoolGeom &g, int elem_f16, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu,
                               uint64_t partial_bytes) {
-    if (elem_f16 && attn_whole_halves_plan(g, b, q_heads)) return 0;
+    uint32_t in_parts = 0;
+    if (elem_f16 && attn_parts_halves_plan(g, b, q_heads, &in_parts)) return in_parts;
     const uint64_t cus = compute_units();
     uint64_t capacity = groups_per_cu * cus;
     const uint32_t group = q_heads / g.kv_heads;

@@ -311,7 +311,7 @@ struct AttnBatch {
     uint32_t tiled; // host side only: the split-K plan gives every 16 query vectors their own workgroups
     uint32_t whole_on_eight; // host side only: the split-K plan leaves every item whole on eight wavefronts
     uint32_t parts; // host side only: items are left whole in parts of channels: how many (attn_whole_f16.hip), or the channel
-                    // tiles of one (attn_whole_halves.hip)
+                    // tiles of one (attn_parts_halves.hip)
     uint32_t tile_sets;  // host side only: the tiles kernel's plan, sets of 16 query vectors a tile
     uint32_t tile_waves; // and wavefronts a workgroup
     uint32_t tile_exact; // and whether the softmax keeps the exact running maximum
@@ -552,9 +552,10 @@ uint32_t attn_splitk_any_groups_per_cu(const PoolGeom &g);
 // True when such a launch also appends the step's rows (k_new / v_new in its parameters); launches of
 // the f32 kernel always do.
 bool attn_splitk_any_appends(const PoolGeom &g, int elem_f16, uint32_t group, uint32_t max_rows);
-// Whole one-row steps by channels on blocked f16 planes at other head dims (attn_whole_halves.hip); `plan` = whether it took the batch.
-bool attn_whole_halves_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads);
-hipError_t launch_attn_whole_halves(const AttnParams &p, const AttnBatch &b, hipStream_t stream);
+// One-row steps by channels on blocked f16 planes at other head dims (attn_parts_halves.hip); `plan` = whether it took the
+// batch, and its partials.
+bool attn_parts_halves_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uint32_t *partials);
+hipError_t launch_attn_parts_halves(const AttnParams &p, const AttnBatch &b, uint32_t total_partials, hipStream_t stream);
 hipError_t launch_attn_splitk_any(int elem_f16, const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream);
 // MFMA block path (speculative blocks and prefill chunks): same pools, any number of rows,

@@ -76,21 +76,22 @@ def test_short_preparing_steps_by_channels(q_heads, kv_heads, slots, window):
 
 # Other head dims on blocked f16 planes: queries and weights as three halves, so the bar is what f32 sums of a thousand
 # terms leave, 2^-23 * 1024 of |v| <= 4 at most and a tenth of that as they are of either sign: 5e-5. Every count of
-# channel tiles, parts of one tile and of several (the last of which may be part empty), one to four rounds; `bad`
-# plants an infinity in a stored key and value and in the new row, whose rows then are the oracle's, infinities and NaN as they are.
+# channel tiles, parts of one tile and of several (the last of which may be part empty), one to four rounds, and runs of
+# eight blocks merged by a second launch, of slots whole beside split ones; `bad` plants an infinity in a stored key and value and in the
+# new row, whose rows then are the oracle's, infinities and NaN as they are.
 @pytest.mark.parametrize("bad", [False, True])
 @pytest.mark.parametrize("d,q_heads,kv_heads,slots", [(16, 8, 2, 1), (32, 8, 8, 2), (64, 32, 4, 1), (64, 16, 1, 9), (80, 32, 8, 1),
                                                       (80, 9, 3, 10), (96, 32, 4, 3), (112, 14, 2, 1), (112, 32, 4, 8), (144, 8, 4, 1),
-                                                      (192, 32, 4, 1), (208, 8, 8, 3), (256, 32, 4, 1), (256, 16, 2, 12)])
+                                                      (192, 32, 4, 1), (208, 8, 8, 3), (256, 32, 4, 1), (256, 16, 2, 12), (80, 32, 8, 5), (112, 8, 8, 6)])
 @pytest.mark.parametrize("window", [None, 100])
 def test_short_steps_at_other_head_dims(d, q_heads, kv_heads, slots, window, bad):
     P = pkg()
     row = kv_heads * d
     kind = P.LayerKind.Global if window is None else P.LayerKind.windowed(window)
     okind = oracle.LayerKind.Global if window is None else oracle.LayerKind.windowed(window)
-    for n in (0, 31, 32, 255, 256, 511, 767, 800, 1023):
+    for n in (0, 31, 32, 255, 256, 511, 767, 800, 1023, 1056):
         rng = np.random.default_rng(n + 1000 * slots + d)
-        pool = P.KvPool([kind], kv_heads, d, elem="f16", max_slots=slots, capacity_rows=1030)
+        pool = P.KvPool([kind], kv_heads, d, elem="f16", max_slots=slots, capacity_rows=1060)
         pool.set_stream(torch.cuda.current_stream().cuda_stream)
         caches, refs, lengths = [], [], []
         for s in range(slots):
