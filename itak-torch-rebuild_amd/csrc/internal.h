@@ -531,7 +531,7 @@ uint32_t attn_decode_f16_resident_groups();
 // `prepares`: Q and the new K rows are prepared by the launch (not with q_two_halves or an exchange).
 hipError_t launch_attn_decode_f16(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream, bool q_two_halves = false, const FoldedParams *prepares = nullptr);
-// Whole one-row steps by channels (attn_whole_f16.hip): AttnBatch::parts is 2 or 4.
+// Whole one-row steps by channels (attn_whole_f16.hip): AttnBatch::parts is 2, 4 or 8.
 constexpr uint32_t kWholeMostBlocks = 24;
 hipError_t launch_attn_whole_f16(const AttnParams &p, const AttnBatch &b, hipStream_t stream, const FoldedParams *prepares);
 // f32 MFMA split-K path: f32 pools (row-major planes), head_dim 128, rows*group <= 16, implied
