@@ -204,10 +204,14 @@ __global__ __launch_bounds__(kWaves * 64) void attn_parts_halves_kernel(AttnPara
             sc[r][e] = acc[e / 4][e % 4] * colscale;
             if (softcap > 0.0f) sc[r][e] = softcap_log2(sc[r][e], softcap, inv_cap);
         }
-        if ((kb + 1) * kBlockKeys > pos + 1 || kb * kBlockKeys < lo) {  // (so are blocks beyond the last)
+        // Keys the query does not see score nothing, and neither does what a wavefront loaded in place of a block beyond its
+        // run: whole contexts' and the last run's end at `pos`, the others' before it. (As the end that keys are compared with it
+        // costs nothing, one slot at 1,500, head_dim 64 / 80 / 256, 6.9 / 7.4 / 8.6 us a layer; as a condition beside them 0.2 us.)
+        const uint32_t end = SPLIT && kb >= kb_end ? 0 : pos + 1;
+        if ((kb + 1) * kBlockKeys > end || kb * kBlockKeys < lo) {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                if (key0 + e > pos || key0 + e < lo) sc[r][e] = -INFINITY;
+                if (key0 + e >= end || key0 + e < lo) sc[r][e] = -INFINITY;
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) mx = fmaxf(mx, sc[r][e]);

@@ -128,3 +128,50 @@ def test_short_steps_at_other_head_dims(d, q_heads, kv_heads, slots, window, bad
                 assert np.array_equal(gk.reshape(-1), oracle.f32_to_f16_array(k[s]))
                 assert np.array_equal(gv.reshape(-1), oracle.f32_to_f16_array(v[s]))
         pool.close()
+
+
+# Contexts cut into runs of fewer than eight blocks, so that some wavefronts of a workgroup have none: 33 and 34 blocks are five
+# runs of seven and a rest, 41 six, 9 beside them two of five. Keys that are large in one channel of every row, as a
+# bias on their projection leaves them, or in the first eight, with queries of one sign: a score made up from a part of a row is far
+# from every true one.
+#
+# The bar: a score is a sum of d terms, and f32 leaves it off by 2^-24 * d^.5 of the sum of their sizes; an output, a mean of
+# |v| <= 4, by as much of 4 on either side of the comparison, beside the 5e-5 above.
+@pytest.mark.parametrize("contexts", [(1040,), (1060,), (1300,), (1300, 270), (270, 1060, 1040)])
+@pytest.mark.parametrize("d,q_heads,kv_heads", [(64, 32, 4), (80, 32, 4), (112, 14, 2), (256, 32, 4), (256, 8, 2)])
+@pytest.mark.parametrize("keys", ["a bias on one channel", "eight large channels"])
+def test_runs_of_fewer_blocks_than_wavefronts(d, q_heads, kv_heads, contexts, keys):
+    P = pkg()
+    row, slots, group = kv_heads * d, len(contexts), q_heads // kv_heads
+    rng = np.random.default_rng(d + sum(contexts))
+    bias = np.zeros((kv_heads, d), np.float32)
+    if keys == "eight large channels":
+        bias[:, :8] = 4.5
+    else:
+        for h in range(kv_heads):
+            bias[h, rng.integers(8)] = rng.choice([-1, 1]) * rng.integers(150, 400)
+    def some_keys(n):
+        return 0.25 * normal(rng, n, row) + bias.reshape(1, row)
+    pool = P.KvPool([P.LayerKind.Global], kv_heads, d, elem="f16", max_slots=slots, capacity_rows=1320)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    caches, refs, stored = [], [], []
+    for length in contexts:
+        cache, ref = pool.acquire(), oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, d, store_f16=True)
+        k, v = some_keys(length), normal(rng, length, row)
+        cache.restore_bulk(0, 0, k, v)
+        ref.restore_bulk(0, 0, k, v)
+        caches.append(cache), refs.append(ref), stored.append(np.abs(k).reshape(length, kv_heads, d).max(0))
+    q = 2 * normal(rng, slots, q_heads * d) if keys == "a bias on one channel" else 4 + 0.5 * normal(rng, slots, q_heads * d)
+    k, v = some_keys(slots), normal(rng, slots, row)
+    qd, kd, vd = dev(q), dev(k), dev(v)
+    out = torch.full_like(qd, float("nan"))
+    pool.attention_step_device(0, [(c, 1) for c in caches], qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), q_heads)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    for s, ref in enumerate(refs):
+        want = oracle.attention_step(ref, 0, q[s:s + 1], k[s:s + 1], v[s:s + 1], q_heads, contexts[s])
+        most = np.maximum(stored[s], np.abs(k[s]).reshape(kv_heads, d)).repeat(group, 0)
+        size = float((np.abs(q[s]).reshape(q_heads, d) * most).sum(1).max()) / d ** 0.5
+        bar = 5e-5 + 2 * 4 * size * 2.0 ** -24 * d ** 0.5
+        assert max_abs(got[s], want) <= bar, (s, contexts[s], max_abs(got[s], want), bar)
+    pool.close()
