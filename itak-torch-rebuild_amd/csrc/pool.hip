@@ -990,8 +990,13 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         // The reference's line (attention.rs:147-155) plus which kernel takes the launch, and in the forms that the
         // planners of some choose between, its wavefronts a workgroup.
         if (diag_enabled()) {
-            const char *waves = tiles ? (b.tile_waves == 8 ? "8" : "4")
+            // (Steps by channels run on eight, in that many parts of the channels, or of that many channel tiles each.)
+            char by_channels[24];
+            snprintf(by_channels, sizeof by_channels, mfma ? "8,parts=%u" : "8,tiles=%u", b.parts);
+            const char *waves = b.parts ? by_channels : tiles ? (b.tile_waves == 8 ? "8" : "4")
                                 : !f32fast && !any ? "-" : b.half_blocks ? "4,half_blocks" : b.on_eight ? "8" : "4";
+            const char *kernel = tiles ? "tiles_f16" : mfma ? (b.parts ? "whole_f16" : "splitk_f16") : prefill ? "prefill_f16"
+                                 : f32fast ? "splitk_f32" : any ? (b.parts ? "parts_halves" : "splitk_any") : "generic";
             uint32_t splits = 0;
             uint64_t view_len = 0;
             for (uint32_t i = 0; i < count; ++i) {
@@ -1003,8 +1008,7 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
                       "wavefronts=%s fused_append=%d merge=%s",
                       ULL(layer), count, total_rows, ULL(q_heads), ULL(pool->g.kv_heads), ULL(view_len),
                       window, double(scale), double(softcap),
-                      tiles ? "tiles_f16" : mfma ? "splitk_f16" : prefill ? "prefill_f16" : f32fast ? "splitk_f32" : any ? "splitk_any" : "generic",
-                      bl.total_blocks, splits, waves, int(k_new != nullptr && (tiles || mfma || f32fast || any || prefill)),
+                      kernel, bl.total_blocks, splits, waves, int(k_new != nullptr && (tiles || mfma || f32fast || any || prefill)),
                       partials == 0 ? "none" : on_die ? "on_die" : exchange_words ? "in_launch" : "launch");
         }
         AttnParams p{};

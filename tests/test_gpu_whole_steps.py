@@ -175,3 +175,54 @@ def test_runs_of_fewer_blocks_than_wavefronts(d, q_heads, kv_heads, contexts, ke
         bar = 5e-5 + 2 * 4 * size * 2.0 ** -24 * d ** 0.5
         assert max_abs(got[s], want) <= bar, (s, contexts[s], max_abs(got[s], want), bar)
     pool.close()
+
+
+@pytest.fixture
+def launches(capfd):
+    """(kernel, wavefronts) of the attention launches since the last look, from the diagnostic channel."""
+    lib = pkg()._native.load()
+    lib.itak_set_debug_enabled(1)
+    capfd.readouterr()
+
+    def since():
+        words = [w.split("=", 1) for w in capfd.readouterr().err.split()]
+        return list(zip([w[1] for w in words if w[0] == "kernel"], [w[1] for w in words if w[0] == "wavefronts"]))
+    yield since
+    lib.itak_set_debug_enabled(0)
+
+
+# The lines of the two planners on a device of 256 compute units: which kernel a step goes to and how it is cut there.
+@pytest.mark.parametrize("d,q_heads,kv_heads,slots,n,form,kernel,wavefronts", [
+    (128, 32, 4, 1, 0, {}, "whole_f16", "8,parts=8"), (128, 32, 4, 1, 639, {}, "whole_f16", "8,parts=8"),
+    (128, 32, 4, 1, 640, {}, "splitk_f16", "-"), (128, 32, 4, 8, 767, {}, "whole_f16", "8,parts=8"),
+    (128, 32, 4, 8, 768, {}, "splitk_f16", "-"), (128, 32, 4, 9, 500, {}, "whole_f16", "8,parts=4"),
+    (128, 32, 4, 16, 767, {}, "whole_f16", "8,parts=4"), (128, 32, 4, 17, 500, {}, "whole_f16", "8,parts=2"),
+    (128, 32, 4, 24, 500, {}, "whole_f16", "8,parts=2"), (128, 32, 4, 25, 500, {}, "splitk_f16", "-"),
+    (128, 32, 1, 1, 300, {}, "splitk_f16", "-"), (128, 32, 4, 1, 300, {"merge_in_launch": True}, "splitk_f16", "-"),
+    (128, 32, 4, 1, 300, {"q_two_halves": True}, "splitk_f16", "-"), (128, 32, 4, 1, 300, {"die_merge": True}, "splitk_f16", "-"),
+    (128, 32, 4, 1, 383, {"prep": True}, "whole_f16", "8,parts=8"), (128, 32, 4, 1, 384, {"prep": True}, "splitk_f16", "-"),
+    (64, 32, 4, 1, 767, {}, "parts_halves", "8,tiles=1"), (80, 32, 8, 1, 800, {}, "parts_halves", "8,tiles=1"),
+    (80, 32, 8, 6, 700, {}, "parts_halves", "8,tiles=1"), (80, 32, 8, 8, 700, {}, "parts_halves", "8,tiles=2"),
+    (80, 32, 8, 8, 1500, {}, "splitk_any", "4"), (256, 32, 4, 1, 511, {}, "parts_halves", "8,tiles=2"),
+    (256, 32, 4, 1, 1500, {}, "parts_halves", "8,tiles=2"), (256, 32, 4, 4, 1500, {}, "parts_halves", "8,tiles=8")])
+def test_which_steps_go_by_channels(launches, d, q_heads, kv_heads, slots, n, form, kernel, wavefronts):
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are counted in compute units")
+    form = dict(form)
+    prep = form.pop("prep", False)
+    pool = pkg().KvPool(1, kv_heads, d, elem="f16", max_slots=slots, capacity_rows=n + 1,
+                        **{"q_two_halves": False, "die_merge": False, **form})
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    items = [(pool.acquire(), 1) for _ in range(slots)]
+    rows = torch.ones(max(slots * n, 1), kv_heads * d, device="cuda")
+    if n:
+        pool.append_device(0, [(c, n) for c, _ in items], rows.data_ptr(), rows.data_ptr())
+    q, k = torch.ones(slots, q_heads * d, device="cuda"), torch.ones(slots, kv_heads * d, device="cuda")
+    out = torch.zeros_like(q)
+    launches()
+    step = pool.attention_prep_step_device if prep else pool.attention_step_device
+    step(0, items, q.data_ptr(), k.data_ptr(), k.data_ptr(), out.data_ptr(), q_heads)
+    torch.cuda.synchronize()
+    assert launches() == [(kernel, wavefronts)]
+    assert torch.allclose(out, torch.ones_like(out), atol=1e-3)  # every value row is ones
+    pool.close()
