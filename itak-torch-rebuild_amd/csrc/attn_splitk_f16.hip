@@ -246,7 +246,7 @@ static bool takes_tiles(const PoolGeom &g, const AttnBatch &b, uint32_t tiles, u
 // Every unit is cut into equal runs of at most T blocks, T the smallest run for which the whole
 // batch fits the device in one wave of dispatch; a run is never shorter than one block per wavefront.
 // may_tile = false keeps the forms that the exchange inside the launch and the queries as two
-// halves are written for; may_part = false those that a merge on the compute dies can take.
+// halves are written for; may_part = false those that a merge on the compute dies and an output over the inputs can take.
 uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, bool prepares, bool may_tile, bool may_part) {
     const uint32_t group = q_heads / g.kv_heads;
     uint32_t most = 0, most_rows = 0;

@@ -72,11 +72,11 @@ static const CutCosts *cut_costs(const PoolGeom &g, int elem_f16) {
 // most T blocks, T the smallest run for which the batch is at most groups_per_cu workgroups per
 // compute unit, and never shorter than one block per wavefront; blocks of
 // several tiles by what the cuts are estimated to take (cut_costs). `partial_bytes` = the most the partials of
-// such a cut may take (0 = any).
+// such a cut may take (0 = any). `may_part` = false keeps one-row steps from attn_parts_halves.hip.
 uint32_t attn_splitk_f32_plan(const PoolGeom &g, int elem_f16, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu,
-                              uint64_t partial_bytes) {
+                              uint64_t partial_bytes, bool may_part) {
     uint32_t in_parts = 0;
-    if (elem_f16 && attn_parts_halves_plan(g, b, q_heads, &in_parts)) return in_parts;
+    if (elem_f16 && may_part && attn_parts_halves_plan(g, b, q_heads, &in_parts)) return in_parts;
     const uint64_t cus = compute_units();
     uint64_t capacity = groups_per_cu * cus;
     const uint32_t group = q_heads / g.kv_heads;

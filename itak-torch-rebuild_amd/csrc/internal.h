@@ -538,9 +538,9 @@ hipError_t launch_attn_whole_f16(const AttnParams &p, const AttnBatch &b, hipStr
 // query positions. Partials are in log2 domain (combine with base2 = 1).
 bool attn_splitk_f32_supports(const PoolGeom &g, uint32_t group, uint32_t max_rows);
 // (`groups_per_cu` workgroups of four wavefronts share a compute unit; `partial_bytes`: the workspace of a call
-// that may not grow it, 0 = any.)
+// that may not grow it, 0 = any; `may_part` = false: no steps by channels, attn_parts_halves.hip.)
 uint32_t attn_splitk_f32_plan(const PoolGeom &g, int elem_f16, AttnBatch &b, uint32_t q_heads, uint32_t groups_per_cu,
-                              uint64_t partial_bytes);
+                              uint64_t partial_bytes, bool may_part);
 hipError_t launch_attn_splitk_f32(const AttnParams &p, const AttnBatch &b, uint32_t total_partials,
                                   hipStream_t stream);
 // f32-arithmetic MFMA split-K path for the other shapes (attn_splitk_any.hip): f16 and f32 pools,

@@ -732,6 +732,22 @@ bool takes_splitk_any(const itak_pool *pool, const PlanInput *in, uint32_t n, ui
            attn_splitk_any_supports(pool->g, group, max_rows);
 }
 
+// Whether a call's output lies over its queries, or over new rows that its launch brings along. Steps by channels
+// (attn_whole_f16.hip, attn_parts_halves.hip) have several workgroups read what one of them writes over, whichever comes
+// first; the other forms read all of a (slot, KV head)'s inputs in the workgroup that writes its output, or a launch before the
+// merge that does. (The gate is read by the thread that writes over it.)
+bool shares_memory(const itak_pool *pool, const PlanInput *in, uint32_t n, uint64_t q_heads, const float *out_dev,
+                   const float *q_dev, const float *k_new, const float *v_new) {
+    uint64_t rows = 0;
+    for (uint32_t i = 0; i < n; ++i) rows += in[i].rows;
+    const uint64_t q_bytes = rows * q_heads * pool->g.head_dim * sizeof(float), kv_bytes = rows * pool->row * sizeof(float);
+    auto over = [&](const float *p, uint64_t bytes) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(p), o = reinterpret_cast<uintptr_t>(out_dev);
+        return p && a < o + q_bytes && o < a + bytes;
+    };
+    return over(q_dev, q_bytes) || over(k_new, kv_bytes) || over(v_new, kv_bytes);
+}
+
 // Clears a batch's plan and names its items' places; q rows counted from q_row0. Returns their rows.
 uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t q_row0) {
     b.n = count;  // (cleared item by item: all 64 are three kilobytes)
@@ -788,6 +804,7 @@ uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t
 // outside [2, 1024] stay there too: the tiles round the queries with 2 log2(e) / softcap on, the split-K kernel caps the
 // scores, and beyond those the factor takes queries out of f16's range, or into its subnormals, that are inside it there.
 struct KernelChoice {
+    bool in_place = false;         // out shares memory with what the launch reads (`shares_memory`)
     TilesPlan tiles;               // sets = 0: another kernel
     bool block = false;            // pool->block_plan is the block kernel's plan of the step,
     bool block_appends = false;    // in a launch that brings the rows along or not,
@@ -860,6 +877,7 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
                                 : q_pos_dev ? KernelChoice{}
                                             : choose_tiles(pool, layer, in, n, q_heads, softcap, folded && folded->prep_on,
                                                            false, need_only || pool->no_alloc_call);
+    const bool in_place = chosen ? choice.in_place : shares_memory(pool, in, n, q_heads, out_dev, q_dev, k_new, v_new);
     const TilesPlan &form = choice.tiles;
     const bool tiles = form.sets != 0;
     const bool mfma = !tiles && takes_splitk_f16(pool, in, n, q_heads, q_pos_dev);
@@ -908,13 +926,14 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
         } else if (mfma) {
             partials = attn_splitk_f16_plan(geom, b, uint32_t(q_heads), folded && folded->prep_on,
                                             !pool->q_two_halves && !pool->merge_in_launch,
-                                            !pool->q_two_halves && !pool->merge_in_launch && !pool->die_merge);
+                                            !pool->q_two_halves && !pool->merge_in_launch && !pool->die_merge && !in_place);
         } else if (prefill) {
             partials = attn_prefill_f16_plan(geom, b, group, uint32_t(q_heads), window, k_new != nullptr);
         } else if (f32fast || any) {
             partials = attn_splitk_f32_plan(geom, pool->elem_f16, b, uint32_t(q_heads),
                                             any && max_rows * group <= 16 ? attn_splitk_any_groups_per_cu(geom) : 2,
-                                            need_only || pool->no_alloc_call ? kScratchBytes - kScratchExchangeBytes : 0);
+                                            need_only || pool->no_alloc_call ? kScratchBytes - kScratchExchangeBytes : 0,
+                                            !in_place);
         } else {
             b.rows_per_block = rpb;
             uint64_t key_work = 0;
@@ -2808,8 +2827,9 @@ static itak_status step_on_device(itak_pool *pool, uint64_t layer, const itak_ba
     const bool splitk = takes_splitk_f16(pool, active.data(), uint32_t(active.size()), num_q_heads, nullptr);
     const bool any = !active.empty() &&
                      takes_splitk_any(pool, active.data(), uint32_t(active.size()), num_q_heads, q_dev, out_dev, nullptr);
-    const KernelChoice choice = choose_tiles(pool, layer, active.data(), uint32_t(active.size()), num_q_heads, softcap,
-                                         folded && folded->prep_on, true, no_alloc);
+    KernelChoice choice = choose_tiles(pool, layer, active.data(), uint32_t(active.size()), num_q_heads, softcap,
+                                       folded && folded->prep_on, true, no_alloc);
+    choice.in_place = shares_memory(pool, active.data(), uint32_t(active.size()), num_q_heads, out_dev, q_dev, k_dev, v_dev);
     // (With the queries as two halves the block kernel runs its two-tile form, which brings no
     // rows along: the append is a launch of its own.)
     const bool block_fuses =

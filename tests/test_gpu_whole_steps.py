@@ -226,3 +226,52 @@ def test_which_steps_go_by_channels(launches, d, q_heads, kv_heads, slots, n, fo
     assert launches() == [(kernel, wavefronts)]
     assert torch.allclose(out, torch.ones_like(out), atol=1e-3)  # every value row is ones
     pool.close()
+
+
+# Outputs over the queries, or over the new rows where there are as many heads of either: steps by channels, whose workgroups would
+# read what others have written over, leave them to the forms that took them before. Memory that only adjoins is no such case.
+# Bars as above.
+IN_PLACE = [(128, 32, 4, (300,)), (128, 8, 8, (90, 700, 31)), (128, 16, 4, (500,) * 17), (64, 16, 16, (400,)), (80, 32, 8, (400, 90)),
+            (256, 8, 8, (300,)), (112, 14, 2, (1300, 200))]
+
+
+@pytest.mark.parametrize("d,heads,kv_heads,contexts,over", [
+    (*shape, over) for shape in IN_PLACE for over in ("q", "k", "v", "nothing") if over not in "kv" or shape[1] == shape[2]])
+@pytest.mark.parametrize("form", ["step", "preparing", "allocation-free"])
+def test_outputs_over_the_inputs(launches, d, heads, kv_heads, contexts, over, form):
+    P = pkg()
+    rng = np.random.default_rng(d + sum(contexts))
+    row, slots = kv_heads * d, len(contexts)
+    pool = P.KvPool(1, kv_heads, d, elem="f16", max_slots=slots, capacity_rows=1400, q_two_halves=False, die_merge=False)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    caches, refs = [], []
+    for length in contexts:
+        cache, ref = pool.acquire(), oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, d, store_f16=True)
+        k, v = normal(rng, length, row), normal(rng, length, row)
+        cache.restore_bulk(0, 0, k, v)
+        ref.restore_bulk(0, 0, k, v)
+        caches.append(cache), refs.append(ref)
+    q, k, v = normal(rng, slots, heads * d), normal(rng, slots, row), normal(rng, slots, row)
+    memory = torch.from_numpy(np.concatenate([q.ravel(), k.ravel(), v.ravel(), np.zeros(q.size, np.float32)])).cuda()
+    at, size = {}, {"q": q.size, "k": k.size, "v": v.size, "nothing": q.size}
+    first = 0
+    for name, n in size.items():
+        at[name] = memory[first:first + n]
+        first += n
+    step = {"step": pool.attention_step_device, "preparing": pool.attention_prep_step_device,
+            "allocation-free": pool.attention_step_device_noalloc}[form]
+    launches()
+    step(0, [(c, 1) for c in caches], at["q"].data_ptr(), at["k"].data_ptr(), at["v"].data_ptr(), at[over].data_ptr(), heads)
+    torch.cuda.synchronize()
+    by_channels, other = ("whole_f16", "splitk_f16") if d == 128 else ("parts_halves", "splitk_any")
+    # (Prepared queries and keys of the other head dims are the pool's own memory, and preparing steps stay whole up to 12 blocks.)
+    apart = over == "nothing" or (form == "preparing" and d != 128 and over != "v")
+    if form != "preparing" or d != 128 or max(contexts) < 384:
+        assert [kernel for kernel, _ in launches()] == [by_channels if apart else other]
+    got = at[over].cpu().numpy().reshape(slots, -1)
+    for s, ref in enumerate(refs):
+        want = oracle.attention_step(ref, 0, q[s:s + 1], k[s:s + 1], v[s:s + 1], heads, contexts[s])
+        assert max_abs(got[s], want) <= (2e-3 if d == 128 else 5e-5), (s, max_abs(got[s], want))
+        for rows, new in zip(caches[s].read_rows(0, contexts[s], 1)[1:], (k, v)):
+            assert np.array_equal(rows.reshape(-1), oracle.f32_to_f16_array(new[s]))
+    pool.close()
