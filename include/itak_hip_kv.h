@@ -93,7 +93,9 @@ enum {
    the reference's own rounding.
    An f16 pool rounds the rows it stores to f16 (round to nearest even, as the reference's f16
    session does) and its attention kernels feed Q and the softmax weights to the matrix pipe as
-   f16 too (scores, softmax state and accumulators stay f32): outputs are within 2e-3 (max abs)
+   f16 too (scores, softmax state and accumulators stay f32; Q as it is in the one-row steps of up to four
+   32-position blocks and in those whose contexts the library would split, Q * scale in others: a channel
+   beyond f16's range either way is no query that every step takes): outputs are within 2e-3 (max abs)
    of f32 arithmetic over the same rounded rows as long as the scaled scores q.k*scale have a
    standard deviation of at most about 3 (3e-5 at unit scale, 1.5e-3 at 3, above the bar from
    about 4.5 on). Q and K normed per head, as the reference's model norms them, stay at unit

@@ -261,7 +261,11 @@ uint32_t attn_splitk_f16_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads,
     const uint32_t tiles = (most_rows * group + 15) / 16;
     const bool may = may_tile && takes_tiles(g, b, tiles, blocks, cus, prepares && most_rows == 1);
     b.parts = may_part && most_rows == 1 ? whole_parts(g, b, group, most, prepares, cus) : 0;
-    const bool whole = b.parts || most <= whole_limit(g, b, most_rows, tiles, prepares, may_tile, may);
+    const bool whole_units = most <= whole_limit(g, b, most_rows, tiles, prepares, may_tile, may);
+    const bool whole = b.parts || whole_units;
+    // What a step by channels rounds to f16 is what it would otherwise: the one-row kernel, which takes what is short or split,
+    // scales scores, the split-K kernel's whole steps on eight wavefronts scaled queries.
+    b.scale_scores = b.parts && !prepares && (most <= 4 || !whole_units) ? 1 : 0;
     b.whole_on_eight = whole && most > 4 && (may || most_rows == 1) ? 1 : 0;
     // (A whole one-row step has no second tile and hardly a second block: the form with two sets of
     // operands, whose next block is under way before the first is multiplied, is 0.4 us faster.)

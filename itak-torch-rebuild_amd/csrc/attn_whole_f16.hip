@@ -8,8 +8,9 @@
 // 8 + 8 / P KB to a compute unit, and nothing is left to merge but the workgroup's own wavefronts.
 //   - eight wavefronts, R = 1 to 3 blocks each, every load asked for before the first is waited for: no loop, one maximum
 //     over a wavefront's blocks, nothing rescaled;
-//   - S^T = K . Q^T and O^T = V^T . P^T as in attn_decode_f16.hip; queries of more than four blocks are scaled on their way
-//     to f16, as in the split-K kernel;
+//   - S^T = K . Q^T and O^T = V^T . P^T as in attn_decode_f16.hip; the scale goes to the scores, as there, or to the queries
+//     on their way to f16, as in the split-K kernel: to what it goes in the form that the step has where it may not go by
+//     channels, so that channels which fit f16 only with the scale on, or only without it, fit in either;
 //   - wavefront 0 of every workgroup converts the new position's row, the wavefront that has its block patches it into its
 //     operands, and the first part's workgroup stores it.
 // The parts of up to eight KV heads follow one another that many workgroups apart: workgroup i runs on compute die
@@ -68,8 +69,8 @@ __device__ __forceinline__ void attn_whole_f16_body(const AttnParams &p, const A
     if (N == 1)
         asm volatile("" ::"s"(p.layer_base), "s"(p.q), "s"(p.out), "s"(p.k_new), "s"(p.v_new), "s"(p.g.slot_stride),
                      "s"(p.g.head_stride), "s"(p.g.side_stride), "s"(p.g.kv_heads), "s"(p.q_heads), "s"(p.group), "s"(p.scale),
-                     "s"(p.softcap), "s"(b.item[0].slot), "s"(b.item[0].q_row0), "s"(b.item[0].kv_len), "s"(b.item[0].kv_lo),
-                     "s"(p.window), "s"(p.ring_blocks));
+                     "s"(p.softcap), "s"(p.scale_scores), "s"(b.item[0].slot), "s"(b.item[0].q_row0), "s"(b.item[0].kv_len),
+                     "s"(b.item[0].kv_lo), "s"(p.window), "s"(p.ring_blocks));
     if (N == 1 && PREP)
         asm volatile("" ::"s"(fold.prep_q_weight), "s"(fold.prep_k_weight), "s"(fold.prep_eps), "s"(fold.prep_rot),
                      "s"(fold.prep_interleaved), "s"(fold.prep_freq_step), "s"(fold.prep_freq), "s"(fold.gate));
@@ -129,6 +130,7 @@ __device__ __forceinline__ void attn_whole_f16_body(const AttnParams &p, const A
 #pragma unroll
             for (int s = 0; s < 4; ++s)
                 bk[r][t][s] = *reinterpret_cast<const half8 *>(base + ((t * 16 + s * 4) * 16) * 8);
+        __builtin_amdgcn_sched_barrier(0);  // (in their order: the first block's products wait for the first loads alone)
     }
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -153,10 +155,9 @@ __device__ __forceinline__ void attn_whole_f16_body(const AttnParams &p, const A
 
     const float softcap = p.softcap;
     const float scale = softcap > 0.0f ? p.scale : p.scale * kLog2e;
-    // Up to four blocks the scale goes to the scores and the queries are rounded as they are, as in attn_decode_f16.hip, whose
-    // steps these are on pools that merge in the launch: one result whichever way a pool merges.
-    const bool scale_scores = !PREP && R == 1 && kb_end - kb_begin <= 4;
-    const float qscale = scale_scores ? 1.0f : scale;
+    // The queries are rounded to f16 with the scale on, or as they are and the scale goes to the scores, as the planner says.
+    const bool scale_scores = !PREP && p.scale_scores != 0;
+    const float qscale = scale_scores ? 1.0f : scale, score_scale = scale_scores ? scale : 1.0f;
     [[maybe_unused]] PrepTrig trig;
     if constexpr (PREP) {
         if (prot) {
@@ -213,7 +214,7 @@ __device__ __forceinline__ void attn_whole_f16_body(const AttnParams &p, const A
 #pragma unroll
             for (int k = 0; k < 4; ++k) s = __builtin_amdgcn_mfma_f32_16x16x32_f16(bk[r][t][k], qb[k], s, 0, 0, 0);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sc[r][t * 4 + e] = scale_scores ? s[e] * scale : s[e];
+            for (int e = 0; e < 4; ++e) sc[r][t * 4 + e] = PREP ? s[e] : s[e] * score_scale;
         }
         if (softcap > 0.0f) {
             const float inv_cap = 1.0f / softcap;

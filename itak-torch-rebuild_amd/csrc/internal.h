@@ -312,6 +312,7 @@ struct AttnBatch {
     uint32_t whole_on_eight; // host side only: the split-K plan leaves every item whole on eight wavefronts
     uint32_t parts; // host side only: items are left whole in parts of channels: how many (attn_whole_f16.hip), or the channel
                     // tiles of one (attn_parts_halves.hip)
+    uint32_t scale_scores; // host side only: AttnParams::scale_scores of a step in parts at head_dim 128
     uint32_t tile_sets;  // host side only: the tiles kernel's plan, sets of 16 query vectors a tile
     uint32_t tile_waves; // and wavefronts a workgroup
     uint32_t tile_exact; // and whether the softmax keeps the exact running maximum
@@ -420,6 +421,9 @@ struct AttnParams {
     // holds (so the next step will not find them there): kernels that read each row once may ask
     // for them with the streaming hint.
     uint32_t kv_streams;
+    // Whole steps by channels (attn_whole_f16.hip) only: the queries are rounded to f16 as they are, and the scale goes
+    // to the scores. Else the queries are rounded with the scale on.
+    uint32_t scale_scores;
 };
 // What the reference's model does around the step (muse-glimmer/src/model.rs:445-464),
 // folded into the step's own launches instead of running as launches of their own. `gate`

@@ -751,7 +751,7 @@ bool shares_memory(const itak_pool *pool, const PlanInput *in, uint32_t n, uint6
 // Clears a batch's plan and names its items' places; q rows counted from q_row0. Returns their rows.
 uint32_t start_batch(AttnBatch &b, const PlanInput *in, uint32_t count, uint32_t q_row0) {
     b.n = count;  // (cleared item by item: all 64 are three kilobytes)
-    b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.parts = b.tiled = b.on_eight = b.half_blocks = 0;
+    b.total_blocks = b.rows_per_block = b.tiles = b.fold_units = b.whole_on_eight = b.parts = b.scale_scores = b.tiled = b.on_eight = b.half_blocks = 0;
     b.two_halves = b.tile_sets = b.tile_waves = b.tile_exact = 0;
     b.plan_cost = 0.0f;
     b.partial_limit = 0;
@@ -1049,6 +1049,7 @@ itak_status run_attention(itak_pool *pool, uint64_t layer, const PlanInput *in, 
             p.kv_streams = layer_bytes * pool->layers.size() > (uint64_t(512) << 20) ? 1 : 0;  // twice the cache: well clear of it
         }
         p.spin_limit = pool->spin_limit;
+        p.scale_scores = b.scale_scores;
         p.k_new = (tiles || mfma || f32fast || any || prefill) ? k_new : nullptr;  // the caller passes them only to
         p.v_new = (tiles || mfma || f32fast || any || prefill) ? v_new : nullptr;  // launches that append themselves
         p.q_heads = uint32_t(q_heads);

@@ -275,3 +275,51 @@ def test_outputs_over_the_inputs(launches, d, heads, kv_heads, contexts, over, f
         for rows, new in zip(caches[s].read_rows(0, contexts[s], 1)[1:], (k, v)):
             assert np.array_equal(rows.reshape(-1), oracle.f32_to_f16_array(new[s]))
     pool.close()
+
+
+# Queries near the ends of f16's range: what is rounded to f16 is the query or the query with the scale on, by the step's blocks
+# (a batch's longest counts), and channels that fit in one of the two alone must find it. `most`: the largest channel.
+#
+# The bar: rounding moves a score by 2^-11 of its largest term at most, here of `term`, and a weight by 2^-11 of itself, so an
+# output, a mean of |v| <= 5, by 2 * 5 * 2^-11 * (term + 1).
+@pytest.mark.parametrize("contexts,q_heads,kv_heads,scale,most", [
+    ((60,), 32, 4, 1.0, 6e4), ((127,), 32, 4, 1.0, 6e4), ((384,), 32, 4, 1.0, 6e4), ((639,), 16, 4, 1.0, 6e4),  # as they are
+    ((767, 30) * 6, 8, 4, 1.0, 6e4), ((520,) * 15, 32, 4, 1.0, 6e4),
+    ((128,), 32, 4, None, 4e5), ((383,), 32, 4, None, 4e5), ((90, 200), 16, 4, None, 4e5),                      # with the scale on
+    ((60, 700) * 8, 8, 4, None, 4e5), ((300,) * 17, 8, 4, None, 4e5)])
+def test_queries_at_the_ends_of_f16(launches, contexts, q_heads, kv_heads, scale, most):
+    P = pkg()
+    rng = np.random.default_rng(sum(contexts))
+    row, slots, term = kv_heads * D, len(contexts), 0.5
+    pool = P.KvPool(1, kv_heads, D, elem="f16", max_slots=slots, capacity_rows=800, q_two_halves=False, die_merge=False)
+    pool.set_stream(torch.cuda.current_stream().cuda_stream)
+    at = scale or D ** -0.5
+    large = rng.integers(D)
+
+    def some_keys(n):
+        k = 0.01 * normal(rng, n, row).reshape(n, kv_heads, D)
+        k[:, :, large] = rng.uniform(-term, term, (n, kv_heads)) / (most * at)
+        return k.reshape(n, row)
+    q = normal(rng, slots, q_heads * D)
+    q.reshape(slots, q_heads, D)[:, :, large] = rng.choice([-1, 1], (slots, q_heads)) * rng.uniform(0.9, 1, (slots, q_heads)) * most
+    caches, refs = [], []
+    for length in contexts:
+        cache, ref = pool.acquire(), oracle.KvCache.new([oracle.LayerKind.Global], kv_heads, D, store_f16=True)
+        k, v = some_keys(length), normal(rng, length, row)
+        cache.restore_bulk(0, 0, k, v)
+        ref.restore_bulk(0, 0, k, v)
+        caches.append(cache), refs.append(ref)
+    k, v = some_keys(slots), normal(rng, slots, row)
+    qd, kd, vd = dev(q), dev(k), dev(v)
+    out = torch.full_like(qd, float("nan"))
+    launches()
+    pool.attention_step_device(0, [(c, 1) for c in caches], qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), out.data_ptr(), q_heads,
+                               scale=scale)
+    torch.cuda.synchronize()
+    assert [kernel for kernel, _ in launches()] == ["whole_f16"]
+    got = out.cpu().numpy()
+    for s, ref in enumerate(refs):
+        want = oracle.attention_step(ref, 0, q[s:s + 1], k[s:s + 1], v[s:s + 1], q_heads, contexts[s],
+                                     oracle.AttentionParams(scale=scale))
+        assert max_abs(got[s], want) <= 2 * 5 * 2.0 ** -11 * (term + 1), (s, max_abs(got[s], want))
+    pool.close()
