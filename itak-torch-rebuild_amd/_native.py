@@ -1,16 +1,22 @@
 """ctypes binding of libitak_hip_kv.so (the C ABI declared in include/itak_hip_kv.h).
 
 There is no fallback: if the library is missing or does not export a declared symbol,
-import fails with an error that says how to build it.
+import fails with an error that says how to build it. (The front module beside it, which saves host time in some
+calls, may be missing.)
 """
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
+import sysconfig
+import warnings
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "lib", "libitak_hip_kv.so")
-FRONT_PATH = os.path.join(HERE, "lib", "_itak_front.so")
+# (For one interpreter, and named for it: another looks for its own.)
+FRONT_PATH = os.path.join(HERE, "lib", "_itak_front" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 OK = 0
 STATUS_NAMES = {
@@ -200,16 +206,23 @@ PROTOTYPES = {
 _lib = None
 
 
-def load_front(lib, cache_type):
-    """The module of the calls made per layer and per round (csrc/front.cpp), bound to `lib`."""
-    import importlib.machinery
-    import importlib.util
+class NoFront:
+    """In place of the front module: every call is left to ctypes."""
 
-    if not os.path.exists(FRONT_PATH):
-        raise ImportError(f"{FRONT_PATH} is missing: build it with `python {os.path.join(HERE, 'build.py')}`.")
-    loader = importlib.machinery.ExtensionFileLoader("_itak_front", FRONT_PATH)
-    front = importlib.util.module_from_spec(importlib.util.spec_from_loader("_itak_front", loader))
-    loader.exec_module(front)
+    step = prep_step = truncate = compute = gqa = staticmethod(lambda *_: -1)
+
+
+def load_front(lib, cache_type):
+    """The module of the calls made per layer and per round (csrc/front.cpp), bound to `lib`. It saves host time and nothing
+    else: where it is missing or does not load, the same calls are made through ctypes."""
+    try:
+        loader = importlib.machinery.ExtensionFileLoader("_itak_front", FRONT_PATH)
+        front = importlib.util.module_from_spec(importlib.util.spec_from_loader("_itak_front", loader))
+        loader.exec_module(front)
+    except (ImportError, RuntimeError) as e:  # (numpy refuses a module built for another of its ABIs with either)
+        warnings.warn(f"calls go through ctypes, 1 to 2 us more host time each: {FRONT_PATH} does not load ({e}); "
+                      f"build it with `python {os.path.join(HERE, 'build.py')}`", RuntimeWarning, stacklevel=3)
+        return NoFront
     front.bind(cache_type, *(C.cast(getattr(lib, name), C.c_void_p).value for name in (
         "itak_attention_step_device", "itak_attention_prep_step_device", "itak_kv_truncate",
         "itak_compute_attention", "itak_gqa_attention")))

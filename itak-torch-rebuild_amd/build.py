@@ -6,8 +6,10 @@ built in-tree so that it travels with the source tree; nothing is installed.
 from __future__ import annotations
 
 import os
+import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -16,8 +18,7 @@ LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libitak_hip_kv.so")
 TIMELINE_LIB_PATH = os.path.join(LIB_DIR, "libitak_hip_kv_timeline.so")
 OBJ_DIR = os.path.join(HERE, "build")
-
-FRONT_PATH = os.path.join(LIB_DIR, "_itak_front.so")
+FRONT_PATH = os.path.join(LIB_DIR, "_itak_front" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -70,15 +71,24 @@ def _compile(src: str, timeline: bool = False) -> str:
     return obj
 
 
-def build_front() -> str:
-    """Compiles csrc/front.cpp, the Python module of the per-layer calls, for this interpreter."""
-    import sysconfig
+def build_front() -> str | None:
+    """Compiles csrc/front.cpp, the Python module of the per-layer calls, for this interpreter. Where there is no g++ or the
+    headers of Python or numpy are missing, the library does without it and its calls go through ctypes."""
+    include = sysconfig.get_paths()["include"]
+    try:
+        import numpy
 
-    import numpy
-
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
-           f"-I{sysconfig.get_paths()['include']}", f"-I{numpy.get_include()}",
-           os.path.join(CSRC, "front.cpp"), "-o", FRONT_PATH]
+        missing = [what for what, there in (("g++", shutil.which("g++")), (
+            "Python.h", os.path.exists(os.path.join(include, "Python.h")))) if not there]
+    except ImportError:
+        missing = ["numpy"]
+    if missing:
+        sys.stderr.write(f"csrc/front.cpp is not built, calls go through ctypes: {', '.join(missing)} not found\n")
+        if os.path.exists(FRONT_PATH):  # (one of an older source)
+            os.remove(FRONT_PATH)
+        return None
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden", f"-I{include}",
+           f"-I{numpy.get_include()}", os.path.join(CSRC, "front.cpp"), "-o", FRONT_PATH]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"g++ failed on front.cpp:\n{res.stderr}")
@@ -95,8 +105,7 @@ def build(verbose: bool = False, timeline: bool = False) -> str:
     os.makedirs(OBJ_DIR + ("_timeline" if timeline else ""), exist_ok=True)
     os.makedirs(LIB_DIR, exist_ok=True)
     srcs = sources()
-    if not timeline:
-        build_front()
+    build_front()
     with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as pool:
         objs = list(pool.map(lambda src: _compile(src, timeline), srcs))
     lib_path = TIMELINE_LIB_PATH if timeline else LIB_PATH

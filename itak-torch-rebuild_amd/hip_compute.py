@@ -205,7 +205,7 @@ def _ptr(a: Optional[np.ndarray]):
 
 _ITEM_PACK = {}
 _NAN = math.nan
-_front = None  # csrc/front.cpp's module, once a pool has loaded the library
+_front = None  # csrc/front.cpp's module or what stands in for it, once a pool has loaded the library
 
 
 def _load():

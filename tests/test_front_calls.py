@@ -1,5 +1,7 @@
 """The per-layer calls of the Python front end, made by its compiled module for plain arguments and through ctypes
 for every other kind: both make the same call."""
+import warnings
+
 import numpy as np
 import pytest
 import torch
@@ -52,6 +54,76 @@ def test_only_plain_arguments_are_taken():
     assert f.gqa(0, 0, 0, x, 2, 1, np.array([0, 1]), None, 0.0) == -1
     with pytest.raises(TypeError):
         f.step(0, 0, items)
+
+
+
+# A library without its front module, or with one that is not this interpreter's, makes every call through ctypes and says so once.
+@pytest.mark.parametrize("there", [None, b"", b"\x7fELF not a module"])
+def test_a_library_without_its_front_module(monkeypatch, tmp_path, there):
+    P = pkg()
+    path = tmp_path / "front.so"
+    if there is not None:
+        path.write_bytes(there)
+    monkeypatch.setattr(P._native, "FRONT_PATH", str(path))
+    monkeypatch.setattr(P.hip_compute, "_front", None)
+    with pytest.warns(RuntimeWarning, match="go through ctypes"):
+        assert P.hip_compute._load() is P._native.load()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        f = front()  # (said once)
+    x = np.zeros((2, 8), np.float32)
+    assert f.step(0, 0, [(0, 1)], 1, 2, 3, 4, 8, None, 0.0) == f.truncate(0, [0], [5]) == -1
+    assert f.compute(0, 0, 0, x, x, x, 1, 0, 0.0, 1e4) == f.gqa(0, 0, 0, x, 2, 1, [0, 1], None, 0.0) == -1
+    assert f.prep_step(0, 0, [(0, 1)], 1, 2, 3, 0, 4, 8, 1.0, 0.0, 0, 0, 1e-6, 0.0, True, 0) == -1
+
+
+@pytest.mark.parametrize("missing", ["g++", "Python.h"])
+def test_a_build_without_what_the_front_module_needs(monkeypatch, tmp_path, capfd, missing):
+    from __graft_entry__ import _load_builder
+
+    build = _load_builder()
+    built = tmp_path / "front.so"
+    built.write_bytes(b"of an older source")
+    monkeypatch.setattr(build, "FRONT_PATH", str(built))
+    if missing == "g++":
+        monkeypatch.setattr(build.shutil, "which", lambda name: None)
+    else:
+        monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    assert build.build_front() is None
+    assert f"{missing} not found" in capfd.readouterr().err and not built.exists()
+
+
+def test_both_builds_of_the_library_bring_the_front_module(monkeypatch, tmp_path):
+    from __graft_entry__ import _load_builder
+
+    build, made = _load_builder(), []
+    monkeypatch.setattr(build, "OBJ_DIR", str(tmp_path / "build"))
+    monkeypatch.setattr(build, "sources", lambda: ["one.hip"])
+    monkeypatch.setattr(build.subprocess, "run", lambda *a, **kw: type("Done", (), {"returncode": 0, "stderr": ""}))
+    monkeypatch.setattr(build, "build_front", lambda: made.append(1))
+    build.build(), build.build(timeline=True)
+    assert made == [1, 1]
+
+
+@gpu
+def test_steps_without_the_front_module_give_the_same(monkeypatch):
+    P, rng = pkg(), np.random.default_rng(3)
+    front()
+    q, k, v = normal(rng, 1, 8 * 128), normal(rng, 1, 256), normal(rng, 1, 256)
+    d = [torch.from_numpy(x).cuda() for x in (q, k, v)]
+    outs = []
+    for f in (P.hip_compute._front, P._native.NoFront):
+        monkeypatch.setattr(P.hip_compute, "_front", f)
+        pool = P.KvPool(1, 2, 128, capacity_rows=64)
+        pool.set_stream(torch.cuda.current_stream().cuda_stream)
+        cache, out = pool.acquire(), torch.full_like(d[0], float("nan"))
+        for _ in range(3):
+            pool.attention_step_device(0, [(cache, 1)], *(x.data_ptr() for x in d), out.data_ptr(), 8)
+            pool.attention_prep_step_device(0, [(cache, 1)], *(x.data_ptr() for x in d), out.data_ptr(), 8, rope_base=1e4)
+        pool.truncate([cache], [5])
+        outs += [out.cpu().numpy(), P.gqa_attention(q, 1, 8, [4], cache.view(0))]
+        pool.close()
+    assert np.array_equal(outs[0], outs[2]) and np.array_equal(outs[1], outs[3])
 
 
 @gpu
