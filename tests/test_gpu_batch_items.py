@@ -51,7 +51,9 @@ def test_every_workgroup_finds_its_item(elem, d, slots):
             err = max_abs(got[at:at + n].reshape(-1), want)
             if elem == "f32":
                 err /= float(np.abs(want).max())
-            assert err <= (2e-3 if elem == "f16" else 1e-5), (slots, s, n, contexts[s], err)
+            # (Of f16 pools only head_dim 128 rounds queries and weights to f16: the others' arithmetic is f32's.)
+            bar = 1e-5 if elem == "f32" else 2e-3 if d == 128 else 5e-5
+            assert err <= bar, (slots, s, n, contexts[s], err)
             at += n
             contexts[s] += n
     pool.close()
