@@ -58,7 +58,8 @@ static uint32_t unit_block_count(const AttnItem &it, uint32_t rows_per_group, ui
 // blocks: 5 to 14 % behind the best plan, up to 65; with their own 1.2 to 2 %, up to 23. Us a layer: head_dim
 // 256, four rows at 400 20.3 -> 12.5; head_dim 96, four rows on a window of 512 14.0 -> 10.1; head_dim 64, 5
 // slots of seven rows at 1,100 17.1 -> 14.0. (The other way: head_dim 64, 16 slots of seven at 1,100 17.8 ->
-// 20.9.)
+// 20.9.) `merge` is of a merge launch that asked for eight partials a lane whatever there were; it takes 0.3 to 0.8 us
+// less now.
 struct PlanCost {
     float alone[2], shared[2], merge;
     float rate;              // bytes a microsecond

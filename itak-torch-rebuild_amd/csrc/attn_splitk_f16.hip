@@ -196,7 +196,8 @@ static uint32_t variant_capacity(const Variant &v) {
 // 7.3 / 7.4 -> 5.1 / 5.4 (7.2 -> 7.2 at 400), 16 slots at 300 / 600 11.0 / 12.7 -> 8.7 / 11.1; seven rows at 150 / 350 / 500 8.6 / 8.9 / 8.9 ->
 // 6.8 / 7.2 / 7.8, 8 slots of them at 700 13.8 -> 13.1. Checked at 4, 8 and 1 KV heads and groups of 1 to 8 with
 // every shape forced either way: within 5 % of the better but for a few just past a line (16 slots of one
-// row at 900, 8 KV heads, split 19.1, whole 16.5).
+// row at 900, 8 KV heads, split 19.1, whole 16.5). The split figures are of a merge launch that asked for eight partials a lane
+// whatever there were; it has been 0.3 to 0.5 us shorter since (`merge_rest`), and the lines have not been moved for it.
 static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows, uint32_t tiles, bool prepares,
                             bool may_tile, bool may) {
     if (rows > 1) return !may ? 8 : g.kv_heads * b.n * tiles >= 128 ? 24 : 16;
@@ -209,8 +210,9 @@ static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows
 // with 2 / 4 at 500 7.9 / 7.6; two parts at 128 units, 256 workgroups, lose to whole units on the split-K kernel, 8.8 and
 // 11.0 at 300 and 500 -> 8.9 and 11.6, and at 96 win, 8.5 and 10.5 -> 7.4 and 9.8; more workgroups than compute units lose
 // throughout, 24 slots of four parts at 300 8.5 -> 9.0). Up to three blocks a wavefront; where a merge has few outputs, below
-// 16 units, splitting wins before that: one slot at 620 / 700 split 6.3 / 6.3, whole 6.2 / 6.5, 4 slots 7.2 / 7.2 against
-// 6.5 / 6.9 (a fourth block each: 16 slots at 1,000 12.0 -> 13.8). Preparing steps are left whole as far as
+// 16 units, up to 20: one slot at 660 / 700 / 760 (21 to 24 blocks) split 6.1 / 6.2 / 6.3, whole 6.2 / 6.1 / 6.3; 2 and 3
+// slots would be better whole there as well, 6.8 to 7.2 against 6.3 to 6.6. 4 slots at 620 / 700 split 7.2 / 7.2, whole
+// 6.4 / 6.9 (a fourth block each: 16 slots at 1,000 12.0 -> 13.8). Preparing steps are left whole as far as
 // they were, up to `whole_limit`.
 static uint32_t whole_parts(const PoolGeom &g, const AttnBatch &b, uint32_t group, uint32_t most, bool prepares, uint64_t cus) {
     const uint64_t units = uint64_t(g.kv_heads) * b.n;

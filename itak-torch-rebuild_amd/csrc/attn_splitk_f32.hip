@@ -51,7 +51,8 @@ struct CutCosts {
 // The even fill is far off for contexts just past the line, which it splits whatever the merge costs:
 // 3 slots of 38 rows at 198, head_dim 192, 32 Q / 4 KV heads 31.6 -> 13.9 us, 4 of 21 at 839 38.2 -> 21.6;
 // head_dim 80, 7 slots of 13 rows at 911 24.4 -> 14.6; f32, head_dim 64, 8 of 12 at 845 27.7 -> 17.2.
-// Row-major f16 planes keep the line: their estimates missed by up to a half.
+// Row-major f16 planes keep the line: their estimates missed by up to a half. (`merge`, and the split figures of whole_limit, are
+// of a merge launch that asked for eight partials a lane whatever there were; it takes 0.3 to 0.5 us less now.)
 static const CutCosts *cut_costs(const PoolGeom &g, int elem_f16) {
     static const CutCosts kBlocked{{5.04f, 2.56f, 0.55f, 0.49f, 0.137f, 3.17f, 2.85f},
                                    {4.98f, 4.00f, 1.04f, 0.34f, 0.169f, 3.07f, 5.64f},

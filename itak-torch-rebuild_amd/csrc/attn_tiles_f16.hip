@@ -537,7 +537,10 @@ static uint32_t fill_plan(const PoolGeom &g, AttnBatch &b, uint32_t q_heads, uin
 // unit to itself, `shared` what a block of every further workgroup there adds. The figures are a fit to
 // 780 shapes (9 to 1,024 rows on 0 to 12,000 positions, 2 to 8 rows of 1 to 8 slots on 100 to 8,192, windows of 512
 // and 2,048, five head layouts, as many layers as the last-level cache does not hold; every form and up
-// to thirteen counts of splits timed for each): 6 % off on average, the pick 0.8 % behind the best.
+// to thirteen counts of splits timed for each): 6 % off on average, the pick 0.8 % behind the best. Both figures are of the
+// launches as they were timed. Since then the merge launch asks for the partials there are (0.3 to 0.8 us less) and a
+// chunk's rows are stored by fewer workgroups (0.2 to 0.9 us less), the same in each form: splits and these forms are priced a
+// little too high, which costs steps near a line and no others.
 struct TileForm {
     uint32_t sets, waves, resident;  // resident: workgroups a compute unit holds
     float fixed, alone, shared;

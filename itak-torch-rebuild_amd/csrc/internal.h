@@ -291,7 +291,8 @@ struct AttnItem {
     uint32_t keys_per_split;
     uint32_t block0;        // first workgroup index of the item
     uint32_t ws0;           // first partial index of the item
-    uint32_t splits_magic;  // ceil(2^32 / splits) for splits > 1: x / splits == mulhi(x, magic), x < 2^16
+    uint32_t splits_magic;  // ceil(2^32 / splits) for splits > 1: x / splits == mulhi(x, magic), x < 2^16. Of a batch that
+                            // attn_parts_halves_plan took, of kv_heads * splits in place of splits
     uint32_t kv_lo;         // oldest position any query of the item may see (0 on global layers)
 };
 // Key blocks (32 positions) an item's queries can touch: [first, end).

@@ -2213,7 +2213,7 @@ static itak_status capture_itkv(itak_pool *pool, uint32_t slot, const char *fing
     itkv_write_header(bytes, h, fingerprint, ls.data());
     if (token_count == 0) return finish_capture(bytes, total, h.version, with_checksum, nullptr);
     // The payload (every layer's keys, then its values) is made in device memory 32 MiB at a time,
-    // summed there when the trailer is version 1's, and goes out through the pinned ring.
+    // summed there from kDeviceSumBytes on (version 1's chain, or version 2's blocks), and goes out through the pinned ring.
     const uint64_t payload = ls[0].keys_offset, payload_bytes = total - 8 - payload;
     const uint64_t piece = std::min(align_up(payload_bytes, 256), kPayloadPiece);
     const bool device_sum = with_checksum && payload_bytes >= kDeviceSumBytes && device_sums(h.version, payload);
