@@ -213,13 +213,18 @@ static uint32_t whole_limit(const PoolGeom &g, const AttnBatch &b, uint32_t rows
 // 16 units, up to 20: one slot at 660 / 700 / 760 (21 to 24 blocks) split 6.1 / 6.2 / 6.3, whole 6.2 / 6.1 / 6.3; 2 and 3
 // slots would be better whole there as well, 6.8 to 7.2 against 6.3 to 6.6. 4 slots at 620 / 700 split 7.2 / 7.2, whole
 // 6.4 / 6.9 (a fourth block each: 16 slots at 1,000 12.0 -> 13.8). Preparing steps are left whole as far as
-// they were, up to `whole_limit`.
+// they were, up to `whole_limit`. Four blocks are one for each wavefront of the one-row kernel, which has them on a fourth or
+// an eighth of the workgroups: with at most two queries a KV head, and beyond 32 units, it is the faster one (keys out of the caches, 126
+// positions, by channels / one-row: 1 slot of 1 query and KV head, 8 / 16 heads 4.8 / 4.4 and 5.0 / 4.5, 4 slots of 8
+// 5.2 / 4.8, 4 of 16 heads of 4 queries 5.4 / 5.1; 1 slot of 4 heads of 4 4.2 / 4.3), preparing steps of few queries only from 16 units on
+// (8 / 16 units 5.1 / 5.1 and 5.4 / 5.2).
 static uint32_t whole_parts(const PoolGeom &g, const AttnBatch &b, uint32_t group, uint32_t most, bool prepares, uint64_t cus) {
     const uint64_t units = uint64_t(g.kv_heads) * b.n;
     const uint32_t limit = prepares ? whole_limit(g, b, 1, 1, true, true, true) : units < 16 ? 20 : kWholeMostBlocks;
     if (group > 16 || most > limit) return 0;
     for (uint32_t i = 0; i < b.n; ++i)
         if (b.item[i].pos0 + 1 != b.item[i].kv_len) return 0;
+    if (most == 4 && (units * 8 > cus || (group <= 2 && (!prepares || units >= 16)))) return 0;
     return units * 8 <= cus ? 8 : units * 4 <= cus ? 4 : units * 8 <= cus * 3 ? 2 : 0;
 }
 

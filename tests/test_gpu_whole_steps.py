@@ -198,6 +198,11 @@ def launches(capfd):
     (128, 32, 4, 8, 768, {}, "splitk_f16", "-"), (128, 32, 4, 9, 500, {}, "whole_f16", "8,parts=4"),
     (128, 32, 4, 16, 767, {}, "whole_f16", "8,parts=4"), (128, 32, 4, 17, 500, {}, "whole_f16", "8,parts=2"),
     (128, 32, 4, 24, 500, {}, "whole_f16", "8,parts=2"), (128, 32, 4, 25, 500, {}, "splitk_f16", "-"),
+    (128, 8, 8, 1, 95, {}, "whole_f16", "8,parts=8"), (128, 8, 8, 1, 96, {}, "splitk_f16", "-"), (128, 2, 1, 1, 127, {}, "splitk_f16", "-"),
+    (128, 8, 8, 1, 128, {}, "whole_f16", "8,parts=8"), (128, 3, 1, 1, 127, {}, "whole_f16", "8,parts=8"),
+    (128, 32, 4, 8, 127, {}, "whole_f16", "8,parts=8"), (128, 32, 4, 9, 127, {}, "splitk_f16", "-"),
+    (128, 32, 4, 9, 128, {}, "whole_f16", "8,parts=4"), (128, 8, 8, 1, 127, {"prep": True}, "whole_f16", "8,parts=8"),
+    (128, 8, 8, 2, 127, {"prep": True}, "splitk_f16", "-"),
     (128, 32, 1, 1, 300, {}, "splitk_f16", "-"), (128, 32, 4, 1, 300, {"merge_in_launch": True}, "splitk_f16", "-"),
     (128, 32, 4, 1, 300, {"q_two_halves": True}, "splitk_f16", "-"), (128, 32, 4, 1, 300, {"die_merge": True}, "splitk_f16", "-"),
     (128, 32, 4, 1, 383, {"prep": True}, "whole_f16", "8,parts=8"), (128, 32, 4, 1, 384, {"prep": True}, "splitk_f16", "-"),
