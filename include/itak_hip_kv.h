@@ -143,9 +143,9 @@ enum {
        itak_pool_synchronize reports ITAK_STEP_FAILED if a workgroup ran elsewhere (seen
        rarely, on small launches between other work; the pool then keeps the merge launch). Results
        agree with the merge launch's to the rounding of another split plan. On an MI355X it is
-       2 to 4 % faster than the merge launch on batches of a hundred MB of KV per layer and more,
-       level or slower below (the launch's own tail and a slower start cost what the second
-       launch costs), so it is not the default. */
+       level with the merge launch on batches of 200 MB of KV per layer and more and slower below (32
+       slots of 4,096 positions 49.2 us against 48.0, 4 slots 14.0 against 11.7), and one-row steps over
+       short contexts are not cut by channels, so it is not the default. */
     ITAK_POOL_DIE_MERGE = 4u,
     /* f16 pools at head_dim 128, every step (decode rows, blocks, prefill chunks):
        the queries enter the score products as two f16 halves, q = hi + lo, and every score is
@@ -153,8 +153,10 @@ enum {
        that grows with the scores: outputs meet the 2e-3 bar up to scaled scores of standard
        deviation 3 (see ITAK_ELEM_F16). With it the queries are good to 2^-22 and what is left is
        the rounding of the softmax weights to f16. The decode and split-K kernels wait for
-       memory more than for the matrix pipe: the second product costs 1 % on a decode step or a
-       ragged batch and 7 % on a speculative block of 64 query vectors per KV head. Longer
+       memory more than for the matrix pipe: the second product costs 1 to 3 % on a ragged batch, nothing
+       on one slot of 4,096 positions (8 % on four), and 7 % on a speculative block of 64 query vectors per
+       KV head; one-row steps over short contexts are not cut by channels (one slot of 200 positions 5.2
+       us a layer in place of 3.8). Longer
        blocks and prefill chunks (the block kernel, which the matrix pipe bounds) take 22 to
        26 % longer, and blocks of 9 to 64 rows are appended by a launch of their own instead of
        inside the attention launch. Other head dims ignore the flag. One thing it changes for keys
